@@ -457,7 +457,8 @@ __device__ __forceinline__ double sensor_rows(int Nelem, int e0, const SensorCon
         }
     }
     __syncthreads();
-    if (act && r < 4) sSum[el][r] = sensor_sum<NGL, RB::RS, true>(T, r);
+    if (act)
+        for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum<NGL, RB::RS, true>(T, w);   // (NGL = 3: lane 0 two)
     __syncthreads();
     double v = 0.0;
     if (act && r == 0) {

@@ -382,12 +382,14 @@ __global__ void __launch_bounds__(256) k_pos_pres(int Nelem, double tol, double 
         sMin[el][r] = mn;
     }
     __syncthreads();
-    if (act && r < 3) {
-        const double* P = sP[r] + el * NN;
-        double a = 0.0;
-        for (int l = 0; l < NGL; ++l)
-            for (int k = 0; k < NGL; ++k) a += P[k * NGL + l];
-        sSum[el][r] = a;
+    if (act) {
+        for (int v = r; v < 3; v += NGL) {     // (NGL = 2: lane 0 two)
+            const double* P = sP[v] + el * NN;
+            double a = 0.0;
+            for (int l = 0; l < NGL; ++l)
+                for (int k = 0; k < NGL; ++k) a += P[k * NGL + l];
+            sSum[el][v] = a;
+        }
     }
     __syncthreads();
     if (act) {

@@ -421,13 +421,15 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
             // h w (hu w, hv w) of plane v and plane 3 in the okl's serial order (xi outer, eta
             // inner) into the padding slot of row 0 of plane v; then every lane limits its column
             __syncthreads();
-            if (act && r < 3) {
-                const double* P = S + r * C::PLANE;
-                const double* W = S + 3 * C::PLANE;
-                double a = 0.0;
-                for (int l = 0; l < NGL; ++l)
-                    for (int k = 0; k < NGL; ++k) a += P[k * C::RS + l] * W[k * C::RS + l];
-                S[r * C::PLANE + NGL] = a;
+            if (act) {
+                for (int v = r; v < 3; v += NGL) {     // (NGL = 2: lane 0 two)
+                    const double* P = S + v * C::PLANE;
+                    const double* W = S + 3 * C::PLANE;
+                    double a = 0.0;
+                    for (int l = 0; l < NGL; ++l)
+                        for (int k = 0; k < NGL; ++k) a += P[k * C::RS + l] * W[k * C::RS + l];
+                    S[v * C::PLANE + NGL] = a;
+                }
             }
             __syncthreads();
             if (act) {
@@ -534,7 +536,8 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
                     }
                 }
                 __syncthreads();
-                if (act && r < 4) sSum[el][r] = sensor_sum<NGL, C::RS, true>(Tm, r);
+                if (act)
+                    for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum<NGL, C::RS, true>(Tm, w);
                 __syncthreads();
                 if (act && r == 0) {
                     const double v = sensor_ramp(sSum[el][0], sSum[el][1], sSum[el][2], sSum[el][3], si.sc);

@@ -418,3 +418,18 @@ def test_captured_fused_step_equals_eager(dev, learned):
     assert np.array_equal(va, vb)
     if not learned:
         assert (va > 0).any()
+
+
+@pytest.mark.parametrize("fused", SCHEDULES, ids=SCHEDULE_IDS)
+@pytest.mark.parametrize("N,av,pos", [(1, 0, 1), (2, 1, 0), (2, 1, 1)])
+def test_lowest_degrees(dev, N, av, pos, fused):
+    """Elements with fewer rows than the sensor's four energy sums and the limiter's three means."""
+    if fused == 2 and N < 2:
+        pytest.skip("the single-kernel stage starts at N = 2")
+    case = Case.flood(N=N, nel=12, seed=4) if pos else Case.dam_break(N=N, nel=12, noise=1e-3, seed=4)
+    rp = RunParams(num_flux=3, artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05,
+                   positivity=pos, pos_pres_tol=1e-3, CFL=0.1 if pos else 0.5)
+    qo, no, to, _ = O.timeloop(case, rp, 6)
+    qg, ng, tg = run_gpu(dev, case, rp, 6, fused=fused)
+    assert ng == no == 6 and abs(tg - to) <= 1e-12 * to
+    assert max(fields_rel_l2(case, qg, qo)) <= 1e-12
