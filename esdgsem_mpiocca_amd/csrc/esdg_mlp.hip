@@ -250,10 +250,10 @@ struct MaskedSensor {
     double T = 0.0;
     int clock_mode = 0;
     // a scenario of a batched ensemble: an element given viscosity marks itself and its face
-    // neighbours with `mark`; with stage0 its viscosity also enters the scenario's maximum
+    // neighbours with `mark`; in stage 0 its viscosity also enters the scenario's maximum
     const StageScn* scn = nullptr;
     int mark = 0;
-    int stage0 = 0;
+    int stage = 0;
 };
 
 // The indicator over elements e0 .. e0 + FEPB - 1 of one state (all 256 threads of the block).
@@ -326,12 +326,12 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
             glob(MS.visc)[e] = v;
             if (MS.visc_plot) glob(MS.visc_plot)[e] = v;
             if (MS.scn) {
-                if (v != 0.0) mark_reach(*MS.scn, e, MS.mark);
+                if (v != 0.0) mark_reach(*MS.scn, e, MS.mark, MS.stage);
                 // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
-                if (MS.stage0 && v > 0.0) atomicMax(&sMax, (unsigned long long)__double_as_longlong(v));
+                if (MS.stage == 0 && v > 0.0) atomicMax(&sMax, (unsigned long long)__double_as_longlong(v));
             }
         }
-        const bool to_max = MS.scn && MS.stage0;
+        const bool to_max = MS.scn && MS.stage == 0;
         if (MS.counters || to_max) {
             __syncthreads();
             if (threadIdx.x == 0) {
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
     MS.counters = counters;
     MS.scn = &S;
     MS.mark = *mark + stage;
-    MS.stage0 = stage == 0;
+    MS.stage = stage;
     mlp_indicator_block(S.Nelem, tk.e0, glob((const double*)S.q[src]), glob(S.B), glob(S.VdmInv), W, lo, hi, nullptr,
                         nullptr, MS);
 }

@@ -44,6 +44,11 @@ struct StageScn {
     double* Qv;         // viscous volume term [Nelem][2][ngl^2] (hu, hv)
     double* SPV;        // viscous face fluxes [Nfaces][2][ngl]
     int* active;        // == mark: viscosity on the element or a face neighbour this stage
+    // the stage's marked elements, each once, with those of every scenario of the same degree and
+    // indicator (learned or not): mlist[0 .. mcount[s]) = {scenario, element} at stage s of a step
+    int2* mlist;
+    int* mcount;
+    int id;             // this scenario's index in the batch
     unsigned long long* emax;   // bit pattern of the step's max viscosity
     // per element side, what its face flux needs from the connectivity (built by StageBatch::init
     // from E2E, EOR, EMS and EdgeData; one record per side, shared by the scenarios of a mesh):
@@ -59,17 +64,30 @@ struct StageTask {
 
 // An element with viscosity marks itself and its face neighbours for this stage (the elements whose
 // viscous terms can be non-zero), as the fused face pass does for both elements of every face with
-// viscosity on either side.  Plain stores of one value: concurrent marks agree.
-__device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m) {
-    const gptr<int> active = glob(S.active);
-    active[e] = m;
+// viscosity on either side.  The first to mark an element this stage also lists it.
+__device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m, int stage) {
+    auto mark = [&](int k) {
+        if (atomicExch(S.active + k, m) != m) S.mlist[atomicAdd(S.mcount + stage, 1)] = make_int2(S.id, k);
+    };
+    mark(e);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const gptr<const int> E = glob(S.EdgeData) + 8 * (int64_t)(glob(S.E2E)[e * 4 + s] - 1);
-        if (E[5] == 0) active[E[0]] = m;
-        if (E[6] == 0) active[E[1]] = m;
+        if (E[5] == 0) mark(E[0]);
+        if (E[6] == 0) mark(E[1]);
     }
 }
+
+// The marked-element lists of a batch: one for the modal-sensor scenarios of each degree (ngl - 3)
+// and one for the learned ones (MARK_LISTS - 1).  A pass over them takes, of each list, the blocks
+// [first, first + blocks) of its grid.
+constexpr int MARK_LISTS = 7;
+constexpr int MARK_STAGES = 8;          // counter slots of a list, one per stage of a step
+struct MarkLists {
+    const int2* list[MARK_LISTS];
+    const int* count[MARK_LISTS];
+    int ngl[MARK_LISTS], first[MARK_LISTS], blocks[MARK_LISTS];
+};
 
 // How the tasks of a stage are ordered and launched (the autotuner's search space).
 struct StageSchedule {
@@ -108,19 +126,21 @@ class StageBatch {
     int ntask = 0;
     int ncu = 0;
     hipGraphExec_t exec[2] = {nullptr, nullptr};   // graph of two steps, one per starting parity
-    // artificial viscosity: element tiles of the AV scenarios for the sensor (row tiles), the
-    // learned indicator (32-element tiles of learned scenarios), the gradient pass (256-element tiles) and
-    // the viscous face pass; the step's mark counter lives on the device (graph replays advance it)
+    // artificial viscosity: element tiles of the AV scenarios for the sensor (row tiles) and the
+    // learned indicator (32-element tiles of learned scenarios); the gradient and the viscous face
+    // pass run over the lists of marked elements; the step's mark counter lives on the device
+    // (graph replays advance it)
     bool has_av = false;
-    StageTask *d_sens = nullptr, *d_ind = nullptr, *d_grad = nullptr, *d_vface = nullptr;
-    int nsens = 0, nind = 0, ngrad = 0, nvface = 0;
+    StageTask *d_sens = nullptr, *d_ind = nullptr;
+    int nsens = 0, nind = 0;
+    int2* d_mlist = nullptr;                       // the marked-element lists, one after another
+    int* d_mcount = nullptr;                       // MARK_LISTS x MARK_STAGES lengths
+    int64_t mfirst[MARK_LISTS + 1] = {0};          // where each list starts in d_mlist
     // With both modal-sensor and learned scenarios the stage runs as two streams of work: the
     // other scenarios (sensor pass, their AV terms, their stage launches) on the second stream and
     // the learned ones (indicator pass, AV terms, stage launches) on the main stream, so the
-    // indicator overlaps the other scenarios' stage.  The gradient and viscous-face task lists hold
-    // the other scenarios' tasks first (ngrad_o, nvface_o of them).
+    // indicator overlaps the other scenarios' stage.  Their marked elements are in lists of their own.
     bool split = false;
-    int ngrad_o = 0, nvface_o = 0;
     int* d_mark = nullptr;
     unsigned long long* d_icount = nullptr;        // learned indicator counts (5, as the solver's)
     const esdg_mlp* mlp = nullptr;
@@ -137,9 +157,9 @@ class StageBatch {
     int build_av_tasks(esdg_ctx* ctx);
     int reset_marks(esdg_ctx* ctx);
     int av_pass(esdg_ctx* ctx, int src, int stage);     // viscosity of the stage's state + marks
-    int av_terms(esdg_ctx* ctx, int src, int stage);    // gradients, viscous volume and face terms
-    // the same over the learned (1) or the other (0) scenarios only, on stream st
-    int av_terms_group(esdg_ctx* ctx, int src, int stage, int learned, hipStream_t st);
+    // gradients, viscous volume and face terms of the marked elements, of the lists [l0, l1), on
+    // stream st
+    int av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipStream_t st);
 };
 
 }  // namespace esdg

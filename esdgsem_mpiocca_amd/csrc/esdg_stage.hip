@@ -539,12 +539,13 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
 // traces read from the state instead of a side-trace buffer: the same bits.
 // ---------------------------------------------------------------------------------------------
 
-// Elements per task of the gradient pass (one flag per thread decides whether a tile has work)
-constexpr int GRAD_TILE = 256;
-
 // The marks of a step: stage s of the step marks with *mark + s.  Advanced by 8 at each step on
-// the device, so that replays of a captured step take fresh marks.
-__global__ void k_stage_mark(int* mark) { *mark += 8; }
+// the device, so that replays of a captured step take fresh marks; the lists of every stage start
+// empty.
+__global__ void k_stage_mark(int* mark, int* mcount) {
+    if (threadIdx.x == 0) *mark += 8;
+    if (threadIdx.x < MARK_LISTS * MARK_STAGES) mcount[threadIdx.x] = 0;
+}
 
 template <int LO, int HI>
 struct MaxRowLds {
@@ -556,7 +557,7 @@ struct MaxRowLds<HI, HI> {
 };
 
 template <int NGL>
-__device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int src, int m, bool stage0, double* sV,
+__device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int src, int m, int stage, double* sV,
                                                 double* sT, double (*sSum)[4], unsigned long long* sMax) {
     if (threadIdx.x < NGL * NGL) sV[threadIdx.x] = glob(S.VdmInv)[threadIdx.x];
     const double v = sensor_rows<NGL>(S.Nelem, e0, S.sc, glob((const double*)S.q[src]), glob(S.B), sV, sT, sSum);
@@ -564,9 +565,9 @@ __device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int s
     const int e = e0 + el;
     if (el < RowBlock<NGL>::EPB && e < S.Nelem && r == 0) {
         glob(S.visc)[e] = v;
-        if (v != 0.0) mark_reach(S, e, m);
+        if (v != 0.0) mark_reach(S, e, m, stage);
         // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
-        if (stage0 && v > 0.0) atomicMax(sMax, (unsigned long long)__double_as_longlong(v));
+        if (stage == 0 && v > 0.0) atomicMax(sMax, (unsigned long long)__double_as_longlong(v));
     }
 }
 
@@ -590,7 +591,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
-        if constexpr (n >= LO && n <= HI) ens_sensor_body<n>(S, tk.e0, src, m, stage == 0, sV, sT, sSum, &sMax); \
+        if constexpr (n >= LO && n <= HI) ens_sensor_body<n>(S, tk.e0, src, m, stage, sV, sT, sSum, &sMax); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -602,48 +603,49 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
     }
 }
 
+// One list's marked elements, ElemBlock<NGL>::EPB at a time, one thread per node; the elements of a
+// block may be of different scenarios, so every element brings its own operators and pointers.
 template <int NGL>
-__device__ __forceinline__ void ens_grad_body(const StageScn& S, int e0, int src, int m, double* sDh, double* sDs,
-                                              double* sA, double* sB, double* sC, double* sE, double* sEps) {
+__device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns, const int2* __restrict__ list, int cnt,
+                                              int blk, int nblk, int src, double* sDh, double* sDs, double* sA,
+                                              double* sB, double* sC, double* sE, double* sEps) {
     using EB = ElemBlock<NGL>;
     constexpr int NN = NGL * NGL;
-    const int e1 = min(e0 + GRAD_TILE, S.Nelem);
-    // most tiles hold no marked element: one flag per thread, one barrier, and the block is done
-    const int et = e0 + (int)threadIdx.x;
-    if (!__syncthreads_or(et < e1 && S.active[et] == m)) return;
-    if (threadIdx.x < NN) {
-        sDh[threadIdx.x] = S.Dhat[threadIdx.x];
-        sDs[threadIdx.x] = S.Dstrong[threadIdx.x];
-    }
-    const AvMesh M{S.q[src], S.Jac, S.Yxi, S.Yeta, S.Xxi, S.Xeta, S.E2E, S.EMS, S.EOR, S.EdgeData,
-                   S.nx, S.ny, S.scal, S.bL, S.bR, GatherConsts{S.bc, S.h_zero}, S.geomFace, S.tol, S.gtr, S.Qv};
-    const int el = threadIdx.x / NN;
-    for (int g = e0; g < e1; g += EB::EPB) {
-        const int e = g + el;
-        const bool act = el < EB::EPB && e < e1 && S.active[e] == m;
-        // the first barrier also publishes sDh, sDs; a group without a marked element is skipped
-        if (!__syncthreads_or(act)) continue;
-        av_element_block<NGL>(M, TraceFromState{S.q[src]}, e, act, act ? S.visc[e] : 0.0, sDh, sDs, sA, sB, sC, sE,
-                              sEps);
+    const int el = threadIdx.x / NN, n = threadIdx.x % NN;
+    for (int g = blk * EB::EPB; g < cnt; g += nblk * EB::EPB) {
+        const bool act = el < EB::EPB && g + el < cnt;
+        const int2 me = list[act ? g + el : g];
+        const StageScn& S = scns[me.x];
+        if (el < EB::EPB) {
+            sDh[threadIdx.x] = S.Dhat[n];
+            sDs[threadIdx.x] = S.Dstrong[n];
+        }
+        const AvMesh M{S.q[src], S.Jac, S.Yxi, S.Yeta, S.Xxi, S.Xeta, S.E2E, S.EMS, S.EOR, S.EdgeData,
+                       S.nx, S.ny, S.scal, S.bL, S.bR, GatherConsts{S.bc, S.h_zero}, S.geomFace, S.tol, S.gtr, S.Qv};
+        const int o = (el < EB::EPB ? el : 0) * NN;
+        av_element_block<NGL>(M, TraceFromState{S.q[src]}, me.y, act, act ? S.visc[me.y] : 0.0, sDh + o, sDs + o, sA,
+                              sB, sC, sE, sEps);
     }
 }
 
-// The gradient pass over tiles of GRAD_TILE elements (tasks: {scenario, first element, ngl}): the
-// marked elements of each tile, in groups of ElemBlock<ngl>::EPB elements, one thread per node.
+// The gradient pass over the lists of marked elements.  A list's blocks stride over it, so a front
+// that crosses one part of a mesh spreads over the chip (one block per 256-element tile worked
+// through the tile's marked elements in sequence, 248 us for each launch of ten scenarios).
 template <int LO, int HI>
-__global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns,
-                                                  const StageTask* __restrict__ tasks, int src,
-                                                  const int* __restrict__ markp, int stage) {
-    __shared__ double sDh[HI * HI], sDs[HI * HI];
+__global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src,
+                                                  int stage) {
+    __shared__ double sDh[256], sDs[256];
     __shared__ double sA[256], sB[256], sC[256], sE[256];
     __shared__ double sEps[ElemBlock<LO>::EPB];
-    const StageTask tk = tasks[blockIdx.x];
-    const StageScn& S = scns[tk.scn];
-    const int m = *markp + stage;
-    switch (tk.ngl) {
+    int l = l0;
+    while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
+    const int blk = (int)blockIdx.x - L.first[l], cnt = L.count[l][stage];
+    if (blk >= L.blocks[l]) return;
+    switch (L.ngl[l]) {
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
-        if constexpr (n >= LO && n <= HI) ens_grad_body<n>(S, tk.e0, src, m, sDh, sDs, sA, sB, sC, sE, sEps); \
+        if constexpr (n >= LO && n <= HI)                                                     \
+            ens_grad_body<n>(scns, L.list[l], cnt, blk, L.blocks[l], src, sDh, sDs, sA, sB, sC, sE, sEps); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -651,25 +653,30 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
     }
 }
 
-// The viscous face fluxes over tiles of 256 faces (tasks: {scenario, first face, ngl}), one thread
-// per face: a face is evaluated (all its nodes) when either of its elements is marked; the faces a
-// marked element reads are exactly those.
-__global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ scns,
-                                                   const StageTask* __restrict__ tasks,
+// The viscous face fluxes over the side nodes of the listed elements; each face node once, by the
+// face's left element if that is marked, else by its right one (the faces a marked element reads
+// are exactly those).
+__global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1,
                                                    const int* __restrict__ markp, int stage) {
-    const StageTask tk = tasks[blockIdx.x];
-    const StageScn& S = scns[tk.scn];
-    const int m = *markp + stage;
-    const int ngl = tk.ngl;
-    const int f = tk.e0 + (int)threadIdx.x;
-    if (f >= S.Nfaces) return;
-    const int* E = S.EdgeData + 8 * (int64_t)f;
-    const int iel = E[0], ier = E[1], cpuL = E[5], cpuR = E[6];
-    if (!((cpuL == 0 && S.active[iel] == m) || (cpuR == 0 && S.active[ier] == m))) return;
-    const int isl = E[2], isr = E[3], rv = E[4];
-    for (int i = 0; i < ngl; ++i)
+    int l = l0;
+    while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
+    const int blk = (int)blockIdx.x - L.first[l];
+    if (blk >= L.blocks[l]) return;
+    const int m = *markp + stage, ngl = L.ngl[l];
+    const int64_t items = (int64_t)L.count[l][stage] * 4 * ngl;
+    for (int64_t it = (int64_t)blk * 256 + threadIdx.x; it < items; it += (int64_t)L.blocks[l] * 256) {
+        const int li = (int)(it / (4 * ngl)), rem = (int)(it % (4 * ngl));
+        const int side = rem / ngl, i = rem % ngl;
+        const int2 me = L.list[l][li];
+        const StageScn& S = scns[me.x];
+        const int f = S.E2E[me.y * 4 + side] - 1;
+        const int* E = S.EdgeData + 8 * (int64_t)f;
+        const int iel = E[0], ier = E[1], isl = E[2], isr = E[3], rv = E[4], cpuL = E[5], cpuR = E[6];
+        const int owner = (cpuL == 0 && S.active[iel] == m) ? iel : ier;
+        if (me.y != owner) continue;
         viscous_face_node(f, i, ngl, S.geomFace, iel, ier, isl, isr, rv, cpuL, cpuR, S.gtr, S.visc, S.nx, S.ny, S.scal,
                           S.SPV);
+    }
 }
 
 // Loads each degree's D into c_stage_D once per device; a later batch must bring the same D.
@@ -758,29 +765,40 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
     return rc;
 }
 
-// Element and face tiles of the AV scenarios for the sensor (RowBlock tiles), the learned
-// indicator (32-element tiles), the gradient pass (GRAD_TILE elements) and the viscous face pass
-// (256 faces).
+// Element tiles of the AV scenarios for the sensor (RowBlock tiles) and the learned indicator
+// (32-element tiles), and the layout of the marked-element lists.
 int StageBatch::build_av_tasks(esdg_ctx* ctx) {
-    std::vector<StageTask> sens, ind, grad, vface;
-    // gradient and viscous-face tasks: the non-learned scenarios' first, then the learned ones'
-    for (int pass = 0; pass < 2; ++pass) {
-        for (int s = 0; s < (int)host.size(); ++s) {
-            const StageScn& S = host[s];
-            if (!S.av || S.learned != pass) continue;
-            const int ngl = S.ngl;
-            if (S.learned)
-                for (int e0 = 0; e0 < S.Nelem; e0 += 32) ind.push_back(StageTask{s, e0, ngl, 0});
-            else
-                for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
-            for (int e0 = 0; e0 < S.Nelem; e0 += GRAD_TILE) grad.push_back(StageTask{s, e0, ngl, 0});
-            for (int f0 = 0; f0 < S.Nfaces; f0 += 256) vface.push_back(StageTask{s, f0, ngl, 0});
-        }
-        if (pass == 0) {
-            ngrad_o = (int)grad.size();
-            nvface_o = (int)vface.size();
-        }
+    std::vector<StageTask> sens, ind;
+    int64_t total[MARK_LISTS] = {0}, all = 0;
+    auto list_of = [](const StageScn& S) { return S.learned ? MARK_LISTS - 1 : S.ngl - 3; };
+    for (int s = 0; s < (int)host.size(); ++s) {
+        const StageScn& S = host[s];
+        if (!S.av) continue;
+        const int ngl = S.ngl;
+        if (S.learned)
+            for (int e0 = 0; e0 < S.Nelem; e0 += 32) ind.push_back(StageTask{s, e0, ngl, 0});
+        else
+            for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
+        total[list_of(S)] += S.Nelem;
+        all += S.Nelem;
     }
+    // the lists hold every element of their scenarios at most once a stage; their total size does
+    // not depend on which scenarios are learned
+    if (!d_mlist) {
+        int rc = esdg_malloc(ctx, (void**)&d_mlist, (size_t)all * sizeof(int2));
+        if (!rc) rc = esdg_malloc(ctx, (void**)&d_mcount, MARK_LISTS * MARK_STAGES * sizeof(int));
+        if (rc) return rc;
+    }
+    for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + total[l];
+    for (int s = 0; s < (int)host.size(); ++s) {
+        StageScn& S = host[s];
+        S.id = s;
+        if (!S.av) continue;
+        S.mlist = d_mlist + mfirst[list_of(S)];
+        S.mcount = d_mcount + MARK_STAGES * list_of(S);
+    }
+    int rcs = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
+    if (rcs) return rcs;
     auto put = [&](const std::vector<StageTask>& v, StageTask*& d, int& n) -> int {
         if (d) esdg_free(ctx, d);
         d = nullptr;
@@ -792,8 +810,6 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     };
     int rc = put(sens, d_sens, nsens);
     if (!rc) rc = put(ind, d_ind, nind);
-    if (!rc) rc = put(grad, d_grad, ngrad);
-    if (!rc) rc = put(vface, d_vface, nvface);
     return rc;
 }
 
@@ -810,8 +826,9 @@ int StageBatch::set_indicator(esdg_ctx* ctx, const esdg_mlp* m, float lo, float 
     ind_lo = lo;
     ind_hi = hi;
     drop_graphs();
-    int rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
-    if (!rc && has_av) rc = build_av_tasks(ctx);
+    int rc = ESDG_OK;
+    if (has_av) rc = build_av_tasks(ctx);
+    else rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (!rc) rc = set_schedule(ctx, sched);   // the stage launches split by group (or not)
     return rc;
 }
@@ -852,30 +869,36 @@ int StageBatch::av_pass(esdg_ctx* ctx, int src, int stage) {
     return ESDG_OK;
 }
 
-int StageBatch::av_terms_group(esdg_ctx* ctx, int src, int stage, int learned, hipStream_t st) {
-    const int gb = learned ? ngrad_o : 0, gn = learned ? ngrad - ngrad_o : ngrad_o;
-    const int vb = learned ? nvface_o : 0, vn = learned ? nvface - nvface_o : nvface_o;
-    if (gn) {
-        k_ens_grad<3, 8><<<gn, 256, 0, st>>>(d_scn, d_grad + gb, src, d_mark, stage);
-        int rc = launch_check(ctx, "ens_grad");
-        if (rc) return rc;
-    }
-    if (vn) {
-        k_ens_vface<<<vn, 256, 0, st>>>(d_scn, d_vface + vb, d_mark, stage);
-        return launch_check(ctx, "ens_viscous_face");
-    }
-    return ESDG_OK;
-}
-
-int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage) {
+int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipStream_t st) {
+    // blocks per list: enough for a front's elements in one pass (the lists' lengths are known on
+    // the device only), never more than the list could use
+    auto lay_out = [&](int cap, auto per_block) {
+        MarkLists L{};
+        int n = 0;
+        for (int l = l0; l < l1; ++l) {
+            L.ngl[l] = l == MARK_LISTS - 1 ? 8 : l + 3;
+            L.list[l] = d_mlist + mfirst[l];
+            L.count[l] = d_mcount + MARK_STAGES * l;
+            L.first[l] = n;
+            L.blocks[l] = (int)std::min<int64_t>(cap, per_block(mfirst[l + 1] - mfirst[l], L.ngl[l]));
+            n += L.blocks[l];
+        }
+        return std::make_pair(L, n);
+    };
     {
+        const auto [L, n] = lay_out(1024, [](int64_t e, int ngl) {
+            const int epb = std::max(1, 256 / (ngl * ngl));
+            return (e + epb - 1) / epb;
+        });
+        if (n == 0) return ESDG_OK;
         KernelScope ks(ctx, "ens_grad");
-        k_ens_grad<3, 8><<<ngrad, 256, 0, ctx->stream>>>(d_scn, d_grad, src, d_mark, stage);
+        k_ens_grad<3, 8><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, stage);
         int rc = launch_check(ctx, "ens_grad");
         if (rc) return rc;
     }
+    const auto [L, n] = lay_out(512, [](int64_t e, int ngl) { return (e * 4 * ngl + 255) / 256; });
     KernelScope ks(ctx, "ens_viscous_face");
-    k_ens_vface<<<nvface, 256, 0, ctx->stream>>>(d_scn, d_vface, d_mark, stage);
+    k_ens_vface<<<n, 256, 0, st>>>(d_scn, L, l0, l1, d_mark, stage);
     return launch_check(ctx, "ens_viscous_face");
 }
 
@@ -1015,7 +1038,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
     if (has_av) {
         // the step's marks, then the viscosity of the step's state (its maximum enters the dt)
         KernelScope ks(ctx, "stage_mark");
-        k_stage_mark<<<1, 1, 0, ctx->stream>>>(d_mark);
+        k_stage_mark<<<1, 64, 0, ctx->stream>>>(d_mark, d_mcount);
         int rc = launch_check(ctx, "stage_mark");
         if (!rc) rc = av_pass(ctx, src, 0);
         if (rc) return rc;
@@ -1037,7 +1060,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
                 k_ens_sensor<3, 8><<<nsens, 256, 0, ctx->side>>>(d_scn, d_sens, src, d_mark, s);
                 rc = launch_check(ctx, "ens_sensor");
             }
-            if (!rc) rc = av_terms_group(ctx, src, s, 0, ctx->side);
+            if (!rc) rc = av_terms(ctx, src, s, 0, MARK_LISTS - 1, ctx->side);
             for (const Range& r : ranges)
                 if (!rc && !r.learned) {
                     launch_ranges<true>(ctx->side, *this, r, src, A[s], C[s], last, s);
@@ -1047,7 +1070,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
             if (!rc && s > 0)
                 rc = mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit,
                                             d_icount);
-            if (!rc) rc = av_terms_group(ctx, src, s, 1, ctx->stream);
+            if (!rc) rc = av_terms(ctx, src, s, MARK_LISTS - 1, MARK_LISTS, ctx->stream);
             for (const Range& r : ranges)
                 if (!rc && r.learned) {
                     launch_ranges<true>(ctx->stream, *this, r, src, A[s], C[s], last, s);
@@ -1060,7 +1083,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
         }
         if (has_av) {
             int rc = (s > 0) ? av_pass(ctx, src, s) : ESDG_OK;
-            if (!rc) rc = av_terms(ctx, src, s);
+            if (!rc) rc = av_terms(ctx, src, s, 0, MARK_LISTS, ctx->stream);
             if (rc) return rc;
         }
         for (const Range& r : ranges) {
@@ -1120,13 +1143,17 @@ int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages,
 
 void StageBatch::release(esdg_ctx* ctx) {
     drop_graphs();
-    for (StageTask** p : {&d_task, &d_sens, &d_ind, &d_grad, &d_vface})
+    for (StageTask** p : {&d_task, &d_sens, &d_ind})
         if (*p) { esdg_free(ctx, *p); *p = nullptr; }
     if (d_scn) esdg_free(ctx, d_scn);
     for (int4* p : srec_bufs) esdg_free(ctx, p);
     srec_bufs.clear();
     if (d_mark) esdg_free(ctx, d_mark);
     if (d_icount) esdg_free(ctx, d_icount);
+    if (d_mlist) esdg_free(ctx, d_mlist);
+    if (d_mcount) esdg_free(ctx, d_mcount);
+    d_mlist = nullptr;
+    d_mcount = nullptr;
     d_scn = nullptr;
     d_mark = nullptr;
     d_icount = nullptr;

@@ -205,3 +205,21 @@ def test_single_kernel_schedule_with_av_equals_fused(dev, mem, learned):
             pa = alone(dev, case, rp, q, STEPS, fused=1, plot=True)[3]
             pb = alone(dev, case, rp, q, STEPS, fused=2, plot=True)[3]
             assert np.array_equal(pa, pb), i
+
+
+@pytest.mark.parametrize("learned", [False, True], ids=["sensor", "learned"])
+def test_every_element_marked(dev, learned):
+    """Sensor bounds that give every element viscosity: the lists of marked elements then hold whole
+    meshes, two scenarios in one list among them, and are longer than one pass of the gradient and
+    viscous face blocks over a list (4096 elements, 131072 side nodes at N = 7)."""
+    kw = dict(sigma_min=-40.0, sigma_max=-2.5, eps0=1e-4, DFL=0.05)
+    big = Case.dam_break(N=7, nel=66, noise=1e-3, seed=8, ratio=2.0, angle=0.4)
+    q2 = dam_break_state(big, 3.0, 1.0, 1e-3, np.random.default_rng(12))
+    d4 = Case.dam_break(N=4, nel=9, noise=1e-3, seed=9, ratio=2.0, angle=0.4)
+    mem = [(big, av(**kw), None), (d4, av(**kw), None), (big, av(**kw), q2)]
+    seed, lo, hi = (3, -1.0, 2.0) if learned else (None, 0.5, 0.5)     # every element unsure
+    res, _ = run_ensemble(dev, mem, 2, net_seed=seed, lo=lo, hi=hi)
+    for (case, rp, q), (got, t, n) in zip(mem, res):
+        want, nw, tw, _ = alone(dev, case, rp, q, 2)
+        assert n == nw == 2 and t == tw
+        assert np.array_equal(got, want)
