@@ -186,3 +186,35 @@ def test_indicator_bands_reduce_to_known_schedules(dev):
     assert np.array_equal(no_av, smooth)
     assert c0["viscous"] == 0 and c0["false_negatives"] == c0["sensor_positives"] > 0
     assert c0["not_smooth"] == 0
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 1000, 32 * 1024 + 45])
+def test_loss_gradient_batch_sizes(dev, state, n):
+    """Batches below, at and above the samples of one pass of a block (32) and above one pass of
+    the whole grid (32768): loss and gradient against the oracle, and twice the same bits."""
+    case, rp, q = state
+    w = random_params(17)
+    rng = np.random.default_rng(18)
+    X = np.concatenate([rng.uniform(-1, 1, (n, 64)), rng.uniform(-2, 0, (n, 8))], axis=1).astype(np.float32)
+    y = (rng.uniform(size=n) < 0.25).astype(np.float32)
+    idx = rng.permutation(n).astype(np.int32)
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        net = dev.MLP(ctx, params=w)
+        dX, dy, di = ctx.array(X), ctx.array(y), ctx.array(idx)
+        got = []
+        for _ in range(2):
+            dg, dl = ctx.empty(M.NPARAM, np.float32), ctx.empty(1, np.float32)
+            net.loss_grad(n, dX, dy, di, 4.0, dg, dl)
+            got.append((dg.download(), dl.download()[0]))
+        net.close()
+    finally:
+        ctx.close()
+    g, L = got[0]
+    assert np.array_equal(g, got[1][0]) and L == got[1][1]
+    Lo, go = M.loss_grad(w.astype(np.float64), X.astype(np.float64), y.astype(np.float64), 4.0)
+    assert abs(L - Lo) <= 1e-4 * abs(Lo), (L, Lo)
+    for a, b in ((M.OFF_W1, M.OFF_B1), (M.OFF_B1, M.OFF_W2), (M.OFF_W2, M.OFF_B2), (M.OFF_B2, M.OFF_W3),
+                 (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.NPARAM)):
+        scale = np.abs(go[a:b]).max()
+        assert np.abs(g[a:b] - go[a:b]).max() <= 2e-3 * scale + 1e-9, (a, np.abs(g[a:b] - go[a:b]).max(), scale)
