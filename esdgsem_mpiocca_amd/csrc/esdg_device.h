@@ -491,11 +491,11 @@ struct PairOut {
 };
 
 __device__ __forceinline__ PairOut ec_pair_scaled(double g, double hL, double huL, double hvL, double uL, double vL,
-                                                  double YL, double XL, double hR, double huR, double hvR, double uR,
-                                                  double vR, double YR, double XR) {
+                                                  double hR, double huR, double hvR, double uR, double vR, double SY,
+                                                  double SX) {
     const double Sh = hL + hR;
     const double P4 = (g * Sh) * Sh - g * (hL * hL + hR * hR);
-    const double Shu = huL + huR, Shv = hvL + hvR, Su = uL + uR, Sv = vL + vR, SY = YL + YR, SX = XL + XR;
+    const double Shu = huL + huR, Shv = hvL + hvR, Su = uL + uR, Sv = vL + vR;
     const double XV = SX * Shv;
     PairOut o;
     o.f1 = SY * Shu - XV;
@@ -516,20 +516,36 @@ struct VolCfg {
     static constexpr int ESZ = 4 * PLANE + ((8 - (4 * PLANE) % 16) + 16) % 16;
 };
 
+// The metric sums Y_c + Y_l, X_c + X_l of a pair of line nodes: of two node arrays, or of a line whose
+// metrics are the same at every node (then one sum serves all pairs, with the same bits).
+template <int NGL>
+struct LineMetrics {
+    const double (&Y)[NGL];
+    const double (&X)[NGL];
+    __device__ __forceinline__ double sy(int c, int l) const { return Y[c] + Y[l]; }
+    __device__ __forceinline__ double sx(int c, int l) const { return X[c] + X[l]; }
+};
+struct ConstMetrics {
+    double SY, SX;
+    __device__ __forceinline__ ConstMetrics(double Y, double X) : SY(Y + Y), SX(X + X) {}
+    __device__ __forceinline__ double sy(int, int) const { return SY; }
+    __device__ __forceinline__ double sx(int, int) const { return SX; }
+};
+
 // All pairs of one line of NGL nodes; acc[k] += sgn * D(k,l) F(k,l), l ascending for every k, with
 // the sums scaled as ec_pair_scaled's outputs are (4, 8, 8).
-template <int NGL, bool NEG>
+template <int NGL, bool NEG, class Metrics>
 __device__ __forceinline__ void line_sweep(const double* __restrict__ D, double g,
                                            const double (&h)[NGL], const double (&hu)[NGL], const double (&hv)[NGL],
                                            const double (&u)[NGL], const double (&v)[NGL],
-                                           const double (&Y)[NGL], const double (&X)[NGL], double (&a1)[NGL],
+                                           const Metrics& M, double (&a1)[NGL],
                                            double (&a2)[NGL], double (&a3)[NGL]) {
 #pragma unroll
     for (int c = 0; c < NGL; ++c) {
 #pragma unroll
         for (int l = c; l < NGL; ++l) {
-            const PairOut F = ec_pair_scaled(g, h[c], hu[c], hv[c], u[c], v[c], Y[c], X[c], h[l], hu[l], hv[l], u[l],
-                                             v[l], Y[l], X[l]);
+            const PairOut F = ec_pair_scaled(g, h[c], hu[c], hv[c], u[c], v[c], h[l], hu[l], hv[l], u[l], v[l],
+                                             M.sy(c, l), M.sx(c, l));
             const double dcl = NEG ? -D[c * NGL + l] : D[c * NGL + l];
             a1[c] += dcl * F.f1;
             a2[c] += dcl * F.f2;

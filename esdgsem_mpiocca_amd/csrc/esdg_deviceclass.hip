@@ -468,7 +468,7 @@ class deviceclass {
             stage_.drop_graphs();
         }
         // the state is in o_q at every entry; the clock restarts from the host's t
-        double ck[8] = {0.0, t, 0.0, last_dt, 0.0, 0.0, 0.0, 0.0};
+        double ck[8] = {0.0, t, 0.0, last_dt, 0.0, 0.0, 0.0, (double)max_steps};
         rc = esdg_memcpy(ctx_, o_clock, ck, sizeof ck, ESDG_H2D);
         if (!rc) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_lmax), 0.0, 1);
         int src = 0;

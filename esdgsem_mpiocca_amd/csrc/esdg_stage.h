@@ -30,7 +30,8 @@ struct StageScn {
     double* q[2];       // ping-pong state buffers
     double* gRK;
     double* clock;      // [0] dt of the current step (0 once t >= T), [1] t, [2] steps taken,
-                        // [3] dt of the last step taken, [4] 1 if a dt was not positive and finite
+                        // [3] dt of the last step taken, [4] 1 if a dt was not positive and finite,
+                        // [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
     unsigned long long* lmax;   // bit pattern of max lambda (non-negative doubles order as integers)
     // artificial viscosity (av = 1): the modal sensor, or with learned = 1 (N = 7) the learned
     // indicator with the sensor as fallback, evaluated on each stage's state; BR1 gradients and the
@@ -55,7 +56,10 @@ struct StageScn {
     // x face, y EdgeData[0] (left element), z EdgeData[1] (right element), w bits: [0,2) left
     // side, [2,4) right side, 4 EdgeData[4] (reversed), 5 EOR, 6 EMS > 0, [8,16) EdgeData[5] + 2,
     // [16,24) EdgeData[6] + 2
+    // (24: the face's geometry is one record of fgeo)
     const int4* srec;
+    // one record per element and per face of a mesh with element-wise constant metrics (else null)
+    const double *geo, *fgeo;
 };
 
 struct StageTask {
@@ -117,6 +121,7 @@ class StageBatch {
     struct Range {
         int beg, n, lo, hi, grid, persistent;
         int learned;   // 1: the tasks of learned-indicator scenarios (see `split`)
+        int affine;    // 1: every scenario of the range has element records (StageScn::geo)
     };
     std::vector<StageScn> host;
     StageSchedule sched;
@@ -153,7 +158,7 @@ class StageBatch {
     void drop_graphs();
 
   private:
-    std::vector<int4*> srec_bufs;   // side records, one buffer per distinct mesh
+    std::vector<void*> rec_bufs;    // side, element and face records, per distinct mesh
     int build_av_tasks(esdg_ctx* ctx);
     int reset_marks(esdg_ctx* ctx);
     int av_pass(esdg_ctx* ctx, int src, int stage);     // viscosity of the stage's state + marks

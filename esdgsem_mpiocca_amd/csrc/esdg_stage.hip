@@ -20,12 +20,6 @@
 
 namespace esdg {
 
-// Flux-differencing D of each degree (ngl 3..8) in constant memory: read through the scalar cache
-// into SGPRs, as a kernel argument would be, whatever scenario of the batch a block serves.  It
-// depends on the degree only; StageBatch::init fills it and refuses a batch whose D differs from
-// the one already loaded for that degree.
-__constant__ double c_stage_D[9][64];
-
 // Per element: the four planes of the volume sweep (VolCfg::ESZ), reused for the face fluxes
 // [side][v][k] once the sweeps have read them, and 16 doubles for the limiter's element means
 // (keeping consecutive elements 8 doubles apart modulo 16, as ESZ does).  At N = 7 a block of 8
@@ -54,15 +48,19 @@ struct MaxLds<HI, HI> {
 // face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
 // parameters are __restrict__ so that the geometry loads schedule as in a kernel taking them as
 // arguments, and global (gptr) so that they compile to global loads and stores.
-template <int NGL, bool AV, class Faces, class Early>
+// AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
+// record per element instead of five doubles per node; the bottom slopes too where they are constant.
+// The kernel moves its bytes at what streaming kernels reach here, so bytes are time.
+template <int NGL, bool AV, bool AFF, class Faces, class Early>
 __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, const Faces& faces, const Early& early,
                                            double g, double tol,
                                            double zero_tol, int positivity, double rkA, double rkC, double dt, bool last,
-                                           gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
+                                           bool keep, gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
                                            gptr<double> __restrict__ gRK, gptr<const double> __restrict__ Yeta,
                                            gptr<const double> __restrict__ Xeta, gptr<const double> __restrict__ Yxi,
                                            gptr<const double> __restrict__ Xxi, gptr<const double> __restrict__ Jac,
                                            gptr<const double> __restrict__ Bx, gptr<const double> __restrict__ By,
+                                           gptr<const double> __restrict__ geo,
                                            gptr<const double> __restrict__ EleSizes,
                                            gptr<const double> __restrict__ GLw,
                                            gptr<unsigned long long> __restrict__ lmax, const StageScn* SV, int mark,
@@ -71,8 +69,10 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
     double* FS = P;                  // face fluxes, after the sweeps (the planes are free then)
     double* MS = P + C::ESZ;         // the limiter's element means
     const int lane = threadIdx.x;
-    double h[NGL], hu[NGL], hv[NGL], u[NGL], v[NGL], Y[NGL], X[NGL];
+    double h[NGL], hu[NGL], hv[NGL], u[NGL], v[NGL];
+    double Y[AFF ? 1 : NGL], X[AFF ? 1 : NGL];
     double a1[NGL], a2[NGL], a3[NGL];
+    double G[8];                     // the element's geometry record (AFF)
 #pragma unroll
     for (int c = 0; c < NGL; ++c) { a1[c] = 0.0; a2[c] = 0.0; a3[c] = 0.0; }
 
@@ -80,13 +80,25 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
     if (act) {
         const int64_t qb = (int64_t)e * C::NN * 3 + r * NGL;
         const int64_t xb = (int64_t)e * C::NN + r * NGL;
+        if constexpr (AFF) {
+            using d2v = double __attribute__((ext_vector_type(2)));
+            const gptr<const d2v> gp = (gptr<const d2v>)(geo + (int64_t)e * 8);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const d2v t = gp[k];
+                G[2 * k] = t.x;
+                G[2 * k + 1] = t.y;
+            }
+        }
 #pragma unroll
         for (int c = 0; c < NGL; ++c) {
             h[c] = qi[qb + c];
             hu[c] = qi[qb + C::NN + c];
             hv[c] = qi[qb + 2 * C::NN + c];
-            Y[c] = Yeta[xb + c];
-            X[c] = Xeta[xb + c];
+            if constexpr (!AFF) {
+                Y[c] = Yeta[xb + c];
+                X[c] = Xeta[xb + c];
+            }
         }
         early();   // LDS stores of values loaded beside the row data
 #pragma unroll
@@ -99,7 +111,8 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             P[2 * C::PLANE + r * C::RS + c] = hv[c];
             P[3 * C::PLANE + r * C::RS + c] = inv;
         }
-        line_sweep<NGL, false>(D, g, h, hu, hv, u, v, Y, X, a1, a2, a3);
+        if constexpr (AFF) line_sweep<NGL, false>(D, g, h, hu, hv, u, v, ConstMetrics(G[0], G[1]), a1, a2, a3);
+        else line_sweep<NGL, false>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, a1, a2, a3);
     }
     __syncthreads();
 
@@ -114,8 +127,10 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             const double inv = P[3 * C::PLANE + k * C::RS + r];
             u[k] = hu[k] * inv;
             v[k] = hv[k] * inv;
-            Y[k] = Yxi[xb + k * NGL];
-            X[k] = Xxi[xb + k * NGL];
+            if constexpr (!AFF) {
+                Y[k] = Yxi[xb + k * NGL];
+                X[k] = Xxi[xb + k * NGL];
+            }
         }
     }
     __syncthreads();
@@ -136,14 +151,29 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             b2[k] = P[1 * C::PLANE + k * C::RS + r];
             b3[k] = P[2 * C::PLANE + k * C::RS + r];
         }
-        line_sweep<NGL, true>(D, g, h, hu, hv, u, v, Y, X, b1, b2, b3);
+        if constexpr (AFF) line_sweep<NGL, true>(D, g, h, hu, hv, u, v, ConstMetrics(G[2], G[3]), b1, b2, b3);
+        else line_sweep<NGL, true>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, b1, b2, b3);
+        // the bottom slopes: with AFF from the record where they are the same at every node (a choice of
+        // address: a branch here makes the compiler move the whole sweep behind it and spill)
+        gptr<const double> bxp = Bx + xb, byp = By + xb;
+        int bst = NGL;
+        if constexpr (AFF) {
+            if (G[7] != 0.0) { bxp = geo + (int64_t)e * 8 + 5; byp = bxp + 1; bst = 0; }
+        }
+        double bx[NGL], by[NGL];
+#pragma unroll
+        for (int k = 0; k < NGL; ++k) {
+            if constexpr (AFF) rJ[k] = G[4];
+            else rJ[k] = Jac[xb + k * NGL];
+            bx[k] = bxp[k * bst];
+            by[k] = byp[k * bst];
+        }
 #pragma unroll
         for (int k = 0; k < NGL; ++k) {
             unscale_sums(b1[k], b2[k], b3[k]);
-            rJ[k] = Jac[xb + k * NGL];
             b1[k] = -rJ[k] * b1[k];
-            b2[k] = -rJ[k] * b2[k] - g * h[k] * Bx[xb + k * NGL];
-            b3[k] = -rJ[k] * b3[k] - g * h[k] * By[xb + k * NGL];
+            b2[k] = -rJ[k] * b2[k] - g * h[k] * bx[k];
+            b3[k] = -rJ[k] * b3[k] - g * h[k] * by[k];
         }
     }
     // the face fluxes of the element's sides (from the stage-start state) into the planes, which
@@ -217,18 +247,32 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         // lane's column input (h, hu, hv): the same bits, without a second read of q
         const double cdt = rkC * dt;
         const int64_t ob = (int64_t)e * C::NN * 3 + r;
+        // A step's first stage has A = 0: the register starts from Qt and is not read.  What the last
+        // stage would leave in it is read by nobody but a checkpoint: it is stored where the caller
+        // asks for it.
+        if (rkA != 0.0) {
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) {
+                const int64_t id = ob + k * NGL;
+                b1[k] = rkA * gRK[id] + b1[k];
+                b2[k] = rkA * gRK[id + C::NN] + b2[k];
+                b3[k] = rkA * gRK[id + 2 * C::NN] + b3[k];
+            }
+        }
+        if (!last || keep) {
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) {
+                const int64_t id = ob + k * NGL;
+                gRK[id] = b1[k];
+                gRK[id + C::NN] = b2[k];
+                gRK[id + 2 * C::NN] = b3[k];
+            }
+        }
 #pragma unroll
         for (int k = 0; k < NGL; ++k) {
-            const int64_t id = ob + k * NGL;
-            const double g1 = rkA * gRK[id] + b1[k];
-            const double g2 = rkA * gRK[id + C::NN] + b2[k];
-            const double g3 = rkA * gRK[id + 2 * C::NN] + b3[k];
-            gRK[id] = g1;
-            gRK[id + C::NN] = g2;
-            gRK[id + 2 * C::NN] = g3;
-            b1[k] = h[k] + cdt * g1;
-            b2[k] = hu[k] + cdt * g2;
-            b3[k] = hv[k] + cdt * g3;
+            b1[k] = h[k] + cdt * b1[k];
+            b2[k] = hu[k] + cdt * b2[k];
+            b3[k] = hv[k] + cdt * b3[k];
         }
     }
     if (positivity) {
@@ -240,7 +284,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 P[0 * C::PLANE + k * C::RS + r] = b1[k];
                 P[1 * C::PLANE + k * C::RS + r] = b2[k];
                 P[2 * C::PLANE + k * C::RS + r] = b3[k];
-                P[3 * C::PLANE + k * C::RS + r] = Jac[xb + k * NGL];
+                P[3 * C::PLANE + k * C::RS + r] = rJ[k];
             }
         }
         __syncthreads();
@@ -314,14 +358,14 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 }
 
 
-template <int NGL, bool AV>
+template <int NGL, bool AV, bool AFF>
 __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, int src, double rkA,
                                            double rkC, bool last, int mark) {
     using C = VolCfg<NGL>;
     using SC = StageCfg<NGL>;
     const int lane = threadIdx.x;
     // D of this degree in LDS (wave-uniform reads, broadcast): keeps it out of the scalar registers
-    for (int t = lane; t < NGL * NGL; t += 64) sD[t] = c_stage_D[NGL][t];
+    for (int t = lane; t < NGL * NGL; t += 64) sD[t] = glob(S.D)[t];
     const int el = lane / NGL, r = lane % NGL;
     const int e = e0 + el;
     const bool act = (el < C::EPW) && (e < S.Nelem);
@@ -383,7 +427,18 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
             d.ir = (1 - rv) * (NGL - 1 - i) + rv * i;
             const int64_t t = (int64_t)f * NGL + i;
             face_side_traces(qi, NGL, d.E, i, d.Li, d.Ri);
-            d.nx = nxp[t]; d.ny = nyp[t]; d.sc = scp[t]; d.bl = bLp[t]; d.br = bRp[t];
+            if constexpr (AFF) {
+                // a face whose five values are the same at every node has them in one 64-byte record
+                const bool one = (d.w >> 24) & 1u;
+                const gptr<const double> fg = glob(S.fgeo) + (int64_t)f * 8;
+                d.nx = one ? fg[0] : nxp[t];
+                d.ny = one ? fg[1] : nyp[t];
+                d.sc = one ? fg[2] : scp[t];
+                d.bl = one ? fg[3] : bLp[t];
+                d.br = one ? fg[4] : bRp[t];
+            } else {
+                d.nx = nxp[t]; d.ny = nyp[t]; d.sc = scp[t]; d.bl = bLp[t]; d.br = bRp[t];
+            }
         };
         // The element's NGL lanes (one wave) hold the face's NGL nodes: each lane also evaluates
         // the right trace at its own node, and lane r takes node ir's from the lane holding it
@@ -413,19 +468,20 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     };
 
     __syncthreads();   // sD written
-    stage_core<NGL, AV>(e, r, act, P, faces, early, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, glob(S.clock)[0], last,
-                        qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi), glob(S.Xxi), glob(S.Jac),
-                        glob(S.Bx), glob(S.By), glob(S.EleSizes), glob(S.GLw), glob(S.lmax), &S, mark, sD);
+    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, glob(S.clock)[0],
+                             last, glob(S.clock)[6] != 0.0, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
+                             glob(S.Xxi), glob(S.Jac), glob(S.Bx), glob(S.By), glob(S.geo), glob(S.EleSizes), glob(S.GLw),
+                             glob(S.lmax), &S, mark, sD);
 }
 
-template <int LO, int HI, bool AV>
+template <int LO, int HI, bool AV, bool AFF>
 __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, const StageTask& tk, double* lds,
                                            double* sD, int src, double rkA, double rkC, bool last, int mark) {
     const StageScn& S = scns[tk.scn];
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                \
     case n:                                                                         \
-        if constexpr (n >= LO && n <= HI) stage_body<n, AV>(S, tk.e0, lds, sD, src, rkA, rkC, last, mark);    \
+        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, rkA, rkC, last, mark);    \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -441,7 +497,7 @@ __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, co
 // on XCD x (b mod 8 = x) take part x, so tasks that are adjacent in the list (one element tile of
 // several scenarios that share geometry) meet in the same L2.  Every block leaves after a bounded
 // number of tasks.
-template <int LO, int HI, bool PERSIST, bool AV>
+template <int LO, int HI, bool PERSIST, bool AV, bool AFF>
 __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ scns, const StageTask* __restrict__ tasks,
                                                  int n, int xcd, int tile, int src, double rkA, double rkC,
                                                  int last, const int* __restrict__ markp, int stage) {
@@ -458,14 +514,14 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
         stride = gridDim.x >> 3;
     }
     if constexpr (!PERSIST) {
-        if (i0 < cnt) stage_task<LO, HI, AV>(scns, tasks[beg + i0], lds, sD, src, rkA, rkC, last != 0, mark);
+        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i0], lds, sD, src, rkA, rkC, last != 0, mark);
     } else {
         const int nch = (cnt + tile - 1) / tile;
         for (int c = i0; c < nch; c += stride) {
             const int i1 = min(cnt, (c + 1) * tile);
             for (int i = c * tile; i < i1; ++i) {
                 if (i != i0 * tile) __syncthreads();   // LDS of the previous task is free
-                stage_task<LO, HI, AV>(scns, tasks[beg + i], lds, sD, src, rkA, rkC, last != 0, mark);
+                stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i], lds, sD, src, rkA, rkC, last != 0, mark);
             }
         }
     }
@@ -523,6 +579,8 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
             ck[1] = t + dt;
             ck[2] += 1.0;
             ck[3] = dt;
+            // the step that ends the run leaves its RK register for a checkpoint
+            ck[6] = (ck[2] == ck[7] || t + dt >= S.T) ? 1.0 : 0.0;
         }
     }
     ck[0] = dt;
@@ -679,8 +737,8 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
     }
 }
 
-// Loads each degree's D into c_stage_D once per device; a later batch must bring the same D.
-static int load_degree_operators(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
+// Each degree has one D per device: a later batch must bring the same.
+static int check_degree_operators(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
     static std::mutex mtx;
     static std::map<int, std::map<int, std::vector<double>>> loaded;   // device -> ngl -> D
     std::lock_guard<std::mutex> lock(mtx);
@@ -691,12 +749,6 @@ static int load_degree_operators(esdg_ctx* ctx, const std::vector<StageScn>& scn
         if (rc) return rc;
         auto& slot = loaded[ctx->device][S.ngl];
         if (slot.empty()) {
-            rc = hip_check(ctx, hipSetDevice(ctx->device), "set device");
-            if (!rc)
-                rc = hip_check(ctx, hipMemcpyToSymbol(HIP_SYMBOL(c_stage_D), D.data(), n2 * sizeof(double),
-                                                      (size_t)S.ngl * 64 * sizeof(double), hipMemcpyHostToDevice),
-                               "D to constant memory");
-            if (rc) return rc;
             slot = D;
         } else if (std::memcmp(slot.data(), D.data(), n2 * sizeof(double)) != 0) {
             return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage: D differs from the one loaded for this degree");
@@ -705,17 +757,65 @@ static int load_degree_operators(esdg_ctx* ctx, const std::vector<StageScn>& scn
     return ESDG_OK;
 }
 
+// One record per element (StageScn::geo) of a mesh whose metrics are the same, bit for bit, at all nodes
+// of each element: {Yeta, Xeta, Yxi, Xxi, 1/J, Bx, By, 1 if Bx and By are the same at all nodes}.  *bad is
+// set where an element's metrics vary: the mesh then has no records.  One wave per element.
+__global__ void __launch_bounds__(64) k_geo_records(int Nelem, int nn, const double* __restrict__ Yeta,
+                                                    const double* __restrict__ Xeta, const double* __restrict__ Yxi,
+                                                    const double* __restrict__ Xxi, const double* __restrict__ Jac,
+                                                    const double* __restrict__ Bx, const double* __restrict__ By,
+                                                    double* __restrict__ geo, int* __restrict__ bad) {
+    const int n = threadIdx.x;      // nn <= 64
+    const double* a[7] = {Yeta, Xeta, Yxi, Xxi, Jac, Bx, By};
+    for (int e = blockIdx.x; e < Nelem; e += gridDim.x) {
+        bool metrics = true, slopes = true;
+        double first[7];
+        for (int k = 0; k < 7; ++k) {
+            const double v = a[k][(int64_t)e * nn + (n < nn ? n : 0)];
+            first[k] = a[k][(int64_t)e * nn];
+            const bool same = __all(__double_as_longlong(v) == __double_as_longlong(first[k]));
+            if (k < 5) metrics = metrics && same;
+            else slopes = slopes && same;
+        }
+        if (n == 0) {
+            for (int k = 0; k < 7; ++k) geo[8 * (int64_t)e + k] = first[k];
+            geo[8 * (int64_t)e + 7] = slopes ? 1.0 : 0.0;
+            if (!metrics) *bad = 1;
+        }
+    }
+}
+
+// One record per face of such a mesh: {nx, ny, scal, bL, bR, -, -, 1 if all five are the same at all
+// nodes of the face}.
+__global__ void __launch_bounds__(256) k_face_records(int Nfaces, int ngl, const double* __restrict__ nx,
+                                                      const double* __restrict__ ny, const double* __restrict__ scal,
+                                                      const double* __restrict__ bL, const double* __restrict__ bR,
+                                                      double* __restrict__ fgeo) {
+    const int f = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (f >= Nfaces) return;
+    const double* a[5] = {nx, ny, scal, bL, bR};
+    bool same = true;
+    for (int k = 0; k < 5; ++k) {
+        const double* p = a[k] + (int64_t)f * ngl;
+        const long long first = __double_as_longlong(p[0]);
+        for (int i = 1; i < ngl; ++i) same = same && __double_as_longlong(p[i]) == first;
+        fgeo[8 * (int64_t)f + k] = p[0];
+    }
+    fgeo[8 * (int64_t)f + 7] = same ? 1.0 : 0.0;
+}
+
 // One record per element side (StageScn::srec) from the connectivity arrays.
 __global__ void __launch_bounds__(256) k_side_records(int Nelem, const int* __restrict__ E2E, const int* __restrict__ EOR,
                                                       const int* __restrict__ EMS, const int* __restrict__ ED,
-                                                      int4* __restrict__ rec) {
+                                                      const double* __restrict__ fgeo, int4* __restrict__ rec) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t)Nelem * 4) return;
     const int f = E2E[t] - 1;
     const int* E = ED + 8 * (int64_t)f;
     const unsigned w = (unsigned)(E[2] & 3) | ((unsigned)(E[3] & 3) << 2) | ((unsigned)(E[4] & 1) << 4) |
                        ((unsigned)(EOR[t] & 1) << 5) | ((EMS[t] > 0 ? 1u : 0u) << 6) |
-                       (((unsigned)(E[5] + 2) & 255u) << 8) | (((unsigned)(E[6] + 2) & 255u) << 16);
+                       (((unsigned)(E[5] + 2) & 255u) << 8) | (((unsigned)(E[6] + 2) & 255u) << 16) |
+                       ((fgeo && fgeo[8 * (int64_t)f + 7] != 0.0 ? 1u : 0u) << 24);
     rec[t] = make_int4(f, E[0], E[1], (int)w);
 }
 
@@ -726,24 +826,62 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
         if (S.ngl < 3 || S.ngl > 8) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage supports 2 <= N <= 7");
         if (S.Nelem <= 0) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one element");
     }
-    int rc = load_degree_operators(ctx, scns);
+    int rc = check_degree_operators(ctx, scns);
     if (rc) return rc;
-    // side records, once per distinct connectivity
+    // element and face records, once per distinct mesh and bottom (a mesh with varying metrics has
+    // none), and side records, once per distinct connectivity and face records
+    auto same_mesh = [](const StageScn& A, const StageScn& B) {
+        return A.ngl == B.ngl && A.Nelem == B.Nelem && A.Nfaces == B.Nfaces && A.E2E == B.E2E && A.EOR == B.EOR &&
+               A.EMS == B.EMS && A.EdgeData == B.EdgeData && A.Yeta == B.Yeta && A.Xeta == B.Xeta && A.Yxi == B.Yxi &&
+               A.Xxi == B.Xxi && A.Jac == B.Jac && A.Bx == B.Bx && A.By == B.By && A.nx == B.nx && A.ny == B.ny &&
+               A.scal == B.scal && A.bL == B.bL && A.bR == B.bR;
+    };
+    auto buffer = [&](size_t bytes) {
+        void* d = nullptr;
+        if (!rc) rc = esdg_malloc(ctx, &d, bytes);
+        if (!rc) rec_bufs.push_back(d);
+        return d;
+    };
     for (size_t a = 0; a < host.size() && !rc; ++a) {
         StageScn& S = host[a];
-        S.srec = nullptr;
-        for (size_t b = 0; b < a; ++b)
-            if (host[b].E2E == S.E2E && host[b].EdgeData == S.EdgeData && host[b].Nelem == S.Nelem) {
-                S.srec = host[b].srec;
-                break;
+        size_t b = 0;
+        while (b < a && !same_mesh(host[b], S)) ++b;
+        if (b < a) {
+            S.geo = host[b].geo;
+            S.fgeo = host[b].fgeo;
+            S.srec = host[b].srec;
+            continue;
+        }
+        S.geo = S.fgeo = nullptr;
+        int bad = 0;
+        double* geo = (double*)buffer((size_t)S.Nelem * 8 * sizeof(double));
+        int* dbad = (int*)buffer(sizeof(int));      // zero-filled
+        if (!rc) {
+            k_geo_records<<<(unsigned)std::min(S.Nelem, 16384), 64, 0, ctx->stream>>>(
+                S.Nelem, S.ngl * S.ngl, S.Yeta, S.Xeta, S.Yxi, S.Xxi, S.Jac, S.Bx, S.By, geo, dbad);
+            rc = launch_check(ctx, "geometry records");
+        }
+        if (!rc) rc = esdg_memcpy(ctx, &bad, dbad, sizeof bad, ESDG_D2H);
+        auto drop = [&](void* d) {
+            rec_bufs.erase(std::find(rec_bufs.begin(), rec_bufs.end(), d));
+            esdg_free(ctx, d);
+        };
+        if (!rc) drop(dbad);
+        if (!rc && bad) drop(geo);
+        if (!rc && !bad) {
+            S.geo = geo;
+            double* fgeo = (double*)buffer((size_t)S.Nfaces * 8 * sizeof(double));
+            if (!rc) {
+                k_face_records<<<blocks_for(S.Nfaces, 256), 256, 0, ctx->stream>>>(S.Nfaces, S.ngl, S.nx, S.ny, S.scal,
+                                                                                   S.bL, S.bR, fgeo);
+                rc = launch_check(ctx, "face records");
             }
-        if (S.srec) continue;
-        int4* d = nullptr;
-        rc = esdg_malloc(ctx, (void**)&d, (size_t)S.Nelem * 4 * sizeof(int4));
+            S.fgeo = fgeo;
+        }
+        int4* d = (int4*)buffer((size_t)S.Nelem * 4 * sizeof(int4));
         if (rc) break;
-        srec_bufs.push_back(d);
-        k_side_records<<<(unsigned)(((int64_t)S.Nelem * 4 + 255) / 256), 256, 0, ctx->stream>>>(S.Nelem, S.E2E, S.EOR,
-                                                                                              S.EMS, S.EdgeData, d);
+        k_side_records<<<blocks_for((int64_t)S.Nelem * 4, 256), 256, 0, ctx->stream>>>(S.Nelem, S.E2E, S.EOR, S.EMS,
+                                                                                     S.EdgeData, S.fgeo, d);
         rc = launch_check(ctx, "side records");
         S.srec = d;
     }
@@ -956,7 +1094,9 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     int cur_learned = 0;
     auto add_range = [&](int beg, int n, int lo, int hi) {
         if (n <= 0) return;
-        Range r{beg, n, lo, hi, n, 0, cur_learned};
+        Range r{beg, n, lo, hi, n, 0, cur_learned, 1};
+        for (int i = beg; i < beg + n; ++i)
+            if (!host[tasks[i].scn].geo) { r.affine = 0; break; }
         // chunks of sc.tile tasks; with xcd every XCD's part is chunked on its own
         const int nch = sc.xcd ? 8 * (((n + 7) / 8 + sc.tile - 1) / sc.tile) : (n + sc.tile - 1) / sc.tile;
         const int pgrid = sc.blocks_per_cu * ncu;
@@ -1012,11 +1152,15 @@ template <int LO, int HI, bool AV>
 static void launch_stage(hipStream_t st, const StageBatch& b, const StageBatch::Range& r, int src, double rkA,
                          double rkC, int last, int stage) {
     if (r.persistent)
-        k_stage<LO, HI, true, AV><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd,
-                                                                   b.sched.tile, src, rkA, rkC, last, b.d_mark, stage);
+        // (the records of a Cartesian mesh serve the launches of one block per task)
+        k_stage<LO, HI, true, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, b.sched.tile,
+                                                                src, rkA, rkC, last, b.d_mark, stage);
+    else if (r.affine)
+        k_stage<LO, HI, false, AV, true><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, 1, src, rkA,
+                                                                rkC, last, b.d_mark, stage);
     else
-        k_stage<LO, HI, false, AV><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, 1,
-                                                                    src, rkA, rkC, last, b.d_mark, stage);
+        k_stage<LO, HI, false, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, 1, src, rkA,
+                                                                 rkC, last, b.d_mark, stage);
 }
 
 template <bool AV>
@@ -1146,8 +1290,8 @@ void StageBatch::release(esdg_ctx* ctx) {
     for (StageTask** p : {&d_task, &d_sens, &d_ind})
         if (*p) { esdg_free(ctx, *p); *p = nullptr; }
     if (d_scn) esdg_free(ctx, d_scn);
-    for (int4* p : srec_bufs) esdg_free(ctx, p);
-    srec_bufs.clear();
+    for (void* p : rec_bufs) esdg_free(ctx, p);
+    rec_bufs.clear();
     if (d_mark) esdg_free(ctx, d_mark);
     if (d_icount) esdg_free(ctx, d_icount);
     if (d_mlist) esdg_free(ctx, d_mlist);

@@ -189,7 +189,7 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
         }
     }
     __syncthreads();   // sD written
-    if (act) line_sweep<NGL, false>(D, g, h, hu, hv, u, v, Y, X, a1, a2, a3);
+    if (act) line_sweep<NGL, false>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, a1, a2, a3);
     __syncthreads();
 
     // ---- column phase: xi-column r, nodes (k, r) -------------------------------------------
@@ -255,7 +255,7 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
         }
     }
     if (act) {
-        line_sweep<NGL, true>(D, g, h, hu, hv, u, v, Y, X, b1, b2, b3);
+        line_sweep<NGL, true>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, b1, b2, b3);
         const int64_t xb = (int64_t)e * C::NN + r;
         const int64_t ob = (int64_t)e * C::NN * ESDG_NEQ + r;
 #pragma unroll
