@@ -9,7 +9,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <tuple>
 #include <vector>
 
 #include "esdg_device_setup.h"
@@ -64,22 +63,21 @@ class deviceclass {
             if (rc == ESDG_OK) rc = esdg_fill(ctx_, o_ArrivalTimings, 1000.0, nodes);
         }
         if (rp.maximum_elevation) A(&o_MaximumElevation, nodes);
-        if (rc == ESDG_OK && rp.fused == 1) rc = fused_.init(ctx_, Nelem, Nfaces, rp.artificial_viscosity != 0);
-        if (rp.fused == 2) {
-            // single-kernel stage: second state buffer (ping-pong), device clock, lambda_max cell
-            A(&o_q2, nodes * 3); A(&o_clock, 8); A(reinterpret_cast<double**>(&o_lmax), 1);
+        if (rc == ESDG_OK && rp.fused == 1 && !element_stage())
+            rc = fused_.init(ctx_, Nelem, Nfaces, rp.artificial_viscosity != 0);
+        if (rp.fused) A(&o_clock, 8);   // the device clock
+        if (element_stage()) {
+            // the stage kernel: second state buffer (ping-pong), lambda_max cell
+            A(&o_q2, nodes * 3); A(reinterpret_cast<double**>(&o_lmax), 1);
             if (rp.artificial_viscosity) {
-                // the stage's gradient side traces, marks and viscosity maximum (the viscous volume
-                // term goes to qGradientX, the viscous face fluxes to SurfacePartsVisc)
+                // the stage's gradient side traces, marks (one array per state buffer) and viscosity
+                // maximum (the viscous volume term goes to qGradientX, the viscous face fluxes to
+                // SurfacePartsVisc); allocations are zero-filled
                 A(&o_gtr, (size_t)Nelem * 16 * ngl);
-                A(reinterpret_cast<double**>(&o_active), ((size_t)Nelem + 1) / 2);
+                for (int*& a : o_active) A(reinterpret_cast<double**>(&a), ((size_t)Nelem + 1) / 2);
                 A(reinterpret_cast<double**>(&o_emax), 1);
-                if (rc == ESDG_OK) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_active), 0.0, ((size_t)Nelem + 1) / 2);
-                if (rc == ESDG_OK) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_emax), 0.0, 1);
-                if (rc == ESDG_OK) rc = esdg_fill(ctx_, o_ViscPara, 0.0, Nelem);
             }
         }
-        if (rp.fused == 1) A(&o_clock, 8);   // the fused schedule's device clock
         return rc;
     }
 
@@ -109,6 +107,13 @@ class deviceclass {
         C(o_EdgeReversed, in.EdgeReversed, Nfaces * sizeof(int));
         return rc;
     }
+
+    // Both fused schedules run on the element-centric stage kernel (esdg_stage.hip) where it is compiled,
+    // 2 <= N <= 7; outside that the fused schedule runs its face and element passes (esdg_fused.hip).
+    // It reads the state once where the passes write and read face fluxes and side traces: per step at 512 x
+    // 512, N = 7, with viscosity 3.73 ms on the passes and 3.26 on the stage kernel, at 301 x 223, N = 4, with
+    // viscosity 685 and 505 us, at 93 x 71, N = 5, without 115 and 94.
+    bool element_stage() const { return rp_.fused == 2 || (rp_.fused == 1 && ngl >= 3 && ngl <= 8); }
 
     // buildDeviceKernels (src/deviceclass.cpp:349-544): kernels are compiled ahead of time; here the
     // run flags are checked against what is implemented.
@@ -161,16 +166,9 @@ class deviceclass {
         return ESDG_OK;
     }
 
-    // The element viscosity of the current state (ShockCapturing, src/deviceclass.cpp:918 and
-    // :1045): the modal sensor, or with the learned indicator the network's classes and the sensor
-    // where the network does not settle the element as smooth.
-    // clock_mode (the device clock of the fused schedule; 0 without it): the learned indicator skips
-    // a step issued after T (1: the step's first evaluation, 2: before a later stage)
-    // stream (learned indicator only; null: the context's stream)
-    int viscosity(int clock_mode = 0, hipStream_t stream = nullptr) {
-        if (!ind_) return esdg_shock_capturing(ctx_, Nelem, o_q, o_B, o_VdmInv, o_EleSizes, o_ViscPara, o_ViscForPlot);
-        return mlp_classify_sensor(ctx_, ind_, Nelem, o_q, o_B, o_VdmInv, ind_lo, ind_hi, o_estat, ind_audit, o_icount,
-                                   o_ViscPara, o_ViscForPlot, clock_mode ? o_clock : nullptr, rp_.T, clock_mode, stream);
+    // The element viscosity of the current state (ShockCapturing, src/deviceclass.cpp:918 and :1045).
+    int viscosity() {
+        return esdg_shock_capturing(ctx_, Nelem, o_q, o_B, o_VdmInv, o_EleSizes, o_ViscPara, o_ViscForPlot);
     }
 
     // One time step's dt (src/deviceclass.cpp:899-928), reductions on the device.
@@ -259,7 +257,7 @@ class deviceclass {
             if (rc) return rc;
             bottom_done = true;
         }
-        if (rp_.fused == 2) return stage_timeloop(max_steps, steps_taken);
+        if (element_stage()) return stage_timeloop(max_steps, steps_taken);
         if (rp_.fused == 1) {
             rc = fused_.begin(ctx_, o_q, o_ElemToEdge, o_EdgeData);
             if (rc) return rc;
@@ -272,7 +270,7 @@ class deviceclass {
         // The fused state update (or the limiter after it) evaluates the sensor (every stage) and
         // the wave speeds (last stage) of the state it writes, in place of the separate passes.
         const bool fuse_next = rp_.fused == 1;
-        const bool fuse_sensor = fuse_next && rp_.artificial_viscosity && !ind_;
+        const bool fuse_sensor = fuse_next && rp_.artificial_viscosity;
         int n = 0;
         while (t < rp_.T && n < max_steps) {
             double dt = 0.0;
@@ -320,9 +318,7 @@ class deviceclass {
     // issued after t reaches T change nothing and are not counted.  Same arithmetic as DGtimeloop.
     int clock_timeloop(int max_steps, int* steps_taken) {
         lambda_fresh = visc_fresh = false;
-        // with the learned indicator the network's classes come before the sensor, so the
-        // indicator pass runs before every stage instead of the sensor fused into the update
-        const bool fuse_sensor = rp_.artificial_viscosity && !ind_;
+        const bool fuse_sensor = rp_.artificial_viscosity;
         const double dti = rp_.min_ele_size / (ngl) * rp_.CFL;
         const double dvc = rp_.DFL / (std::pow(ngl, 2)) * std::pow(rp_.min_ele_size, 2);
         double ck[8] = {0.0, t, 0.0, last_dt, 0.0, 0.0, 0.0, 0.0};
@@ -332,19 +328,12 @@ class deviceclass {
             int r = lambda_fresh ? ESDG_OK : esdg_find_lambda_max(ctx_, Nelem, o_q, o_LambdaMax);
             if (!r) r = esdg_reduce_max(ctx_, Nelem, o_LambdaMax, o_red);
             if (!r && rp_.artificial_viscosity) {
-                if (!visc_fresh) r = viscosity(1);
+                if (!visc_fresh) r = viscosity();
                 if (!r) r = esdg_reduce_max(ctx_, Nelem, o_ViscPara, o_red + 1);
             }
             if (!r) r = fused_clock(ctx_, o_red, o_clock, dti, dvc, rp_.artificial_viscosity, rp_.T);
             for (int s = 0; s < stages && !r; ++s) {
                 FusedArgs fa = fused_args();
-                if (rp_.artificial_viscosity && s > 0 && !visc_fresh) {
-                    // the learned indicator of this stage's state: issued by the stage beside its
-                    // face fluxes (which do not read the viscosity)
-                    if (ind_) fa.visc_pass = [this](hipStream_t st) { return viscosity(2, st); };
-                    else r = viscosity(2);
-                }
-                if (r) break;
                 if (fuse_sensor) { fa.next_visc = o_ViscPara; fa.next_visc_plot = o_ViscForPlot; }
                 if (s == stages - 1) fa.next_lambda = o_LambdaMax;
                 fa.dt_dev = o_clock;
@@ -363,7 +352,6 @@ class deviceclass {
                 // and the stage marks live on the device): that step is captured once as a graph
                 // and replayed.  Profiling runs, and a capture the runtime refuses, stay eager.
                 if (lambda_fresh && !ctx_->profile && graph_ok) {
-                    if (graph_stale()) drop_step_graph();
                     if (!step_exec) {
                         rc = capture_step(issue_step);
                         if (rc) break;
@@ -413,20 +401,14 @@ class deviceclass {
         }
         if (g) (void)hipGraphDestroy(g);
         // the capture issued nothing: the step is launched from the graph by the caller
-        graph_key = current_graph_key();
         return ESDG_OK;
     }
-    // what a captured step depends on beyond its buffers: the learned indicator's settings
-    std::tuple<const void*, float, float, int> current_graph_key() const {
-        return std::make_tuple((const void*)ind_, ind_lo, ind_hi, ind_audit);
-    }
-    bool graph_stale() const { return step_exec && graph_key != current_graph_key(); }
     void drop_step_graph() {
         if (step_exec) (void)hipGraphExecDestroy(step_exec);
         step_exec = nullptr;
     }
 
-    // The same time loop with the single-kernel stage: dt and t live on the device, steps run in
+    // The time loop on the element-centric stage kernel: dt and t live on the device, steps run in
     // chunks (pairs replayed from a hipGraph) and the clock is read back after each chunk.  Steps
     // issued after t reaches T leave the state unchanged and are not counted.
     int stage_timeloop(int max_steps, int* steps_taken) {
@@ -444,24 +426,27 @@ class deviceclass {
             S.EdgeData = o_EdgeData; S.E2E = o_ElemToEdge; S.EMS = o_ElemEdgeMasterSlave; S.EOR = o_ElemEdgeOrientation;
             S.q[0] = o_q; S.q[1] = o_q2; S.gRK = o_gRK; S.clock = o_clock; S.lmax = o_lmax;
             S.emax = o_emax;
+            S.B = o_B;
+            S.arrival = o_ArrivalTimings; S.maxelev = o_MaximumElevation;
+            if (rp_.fused == 1) { S.lam = o_LambdaMax; S.freeze = 1; }
             if (rp_.artificial_viscosity) {
                 S.av = 1;
                 S.dvc = rp_.DFL / (std::pow(ngl, 2)) * std::pow(rp_.min_ele_size, 2);
                 S.sc = SensorConsts{ctx_->p.ZeroTOL, ctx_->p.eps0, ctx_->p.sigmaMin, ctx_->p.sigmaMax};
-                S.B = o_B; S.VdmInv = o_VdmInv; S.Dhat = o_Dhat; S.Dstrong = o_Dstrong;
-                S.visc = o_ViscPara; S.gtr = o_gtr; S.Qv = o_qGradientX; S.SPV = o_SurfacePartsVisc;
-                S.active = o_active;
+                S.VdmInv = o_VdmInv; S.Dhat = o_Dhat; S.Dstrong = o_Dstrong;
+                S.visc = o_ViscPara; S.visc_plot = o_ViscForPlot; S.gtr = o_gtr; S.Qv = o_qGradientX;
+                S.SPV = o_SurfacePartsVisc;
+                S.active[0] = o_active[0]; S.active[1] = o_active[1];
             }
-            rc = stage_.init(ctx_, std::vector<StageScn>{S});
+            rc = stage_.init(ctx_, std::vector<StageScn>{S}, rp_.fused == 1);
             if (rc) return rc;
             stage_ready = true;
-            stage_ind = nullptr;
         }
         // the learned indicator as last set on the solver
-        if (rp_.artificial_viscosity && (stage_ind != ind_ || stage_lo != ind_lo || stage_hi != ind_hi)) {
+        if (rp_.artificial_viscosity && ind_changed) {
             rc = stage_.set_indicator(ctx_, ind_, ind_lo, ind_hi);
             if (rc) return rc;
-            stage_ind = ind_; stage_lo = ind_lo; stage_hi = ind_hi;
+            ind_changed = false;
         }
         if (stage_.ind_audit != ind_audit) {
             stage_.ind_audit = ind_audit;
@@ -473,6 +458,7 @@ class deviceclass {
         if (!rc) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_lmax), 0.0, 1);
         int src = 0;
         if (!rc) rc = stage_.lambda(ctx_, src);
+        stage_.primed = false;   // q may have been set since the last call
         int issued = 0;
         while (!rc && issued < max_steps && ck[1] < rp_.T && ck[4] == 0.0) {
             const int chunk = std::min(max_steps - issued, 64);
@@ -483,15 +469,13 @@ class deviceclass {
         if (!rc && src == 1)
             rc = hip_check(ctx_, hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double), hipMemcpyDeviceToDevice,
                                                 ctx_->stream), "state copy");
-        // ViscPara / ViscForPlot of the final state, as the fused schedule leaves them
-        if (!rc && rp_.artificial_viscosity && !ind_)
-            rc = esdg_shock_capturing(ctx_, Nelem, o_q, o_B, o_VdmInv, o_EleSizes, o_ViscPara, o_ViscForPlot);
         if (!rc) rc = esdg_finish(ctx_);
         if (rc) return rc;
         t = ck[1];
         last_dt = ck[3];
         if (steps_taken) *steps_taken = (int)ck[2];
-        if (ck[4] != 0.0) return set_error(ctx_, ESDG_ERR_STATE, "time step is not positive and finite");
+        if (ck[4] != 0.0)
+            return set_error(ctx_, ESDG_ERR_STATE, "time step is not positive and finite (dt = " + std::to_string(ck[5]) + ")");
         return ESDG_OK;
     }
 
@@ -507,13 +491,12 @@ class deviceclass {
             if (p) esdg_free(ctx_, p);
         fused_.release(ctx_);
         stage_.release(ctx_);
-        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_estat, (void*)o_icount, (void*)o_gtr,
-                        (void*)o_active, (void*)o_emax})
+        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_gtr,
+                        (void*)o_active[0], (void*)o_active[1], (void*)o_emax})
             if (p) esdg_free(ctx_, p);
         o_q2 = o_clock = o_gtr = nullptr;
-        o_lmax = o_icount = o_emax = nullptr;
-        o_active = nullptr;
-        o_estat = nullptr;
+        o_lmax = o_emax = nullptr;
+        o_active[0] = o_active[1] = nullptr;
         o_q = o_Qt = o_gRK = o_Qtmp = nullptr;
         return ESDG_OK;
     }
@@ -549,6 +532,11 @@ class deviceclass {
         if (n == "MaximumElevation") return o_MaximumElevation;
         if (n == "qGradientX") return o_qGradientX;
         if (n == "qGradientY") return o_qGradientY;
+        if (element_stage()) {
+            if (n == "Grad") return o_gtr;
+            if (n == "FVisc") return o_SurfacePartsVisc;
+            if (n == "QVisc") return o_qGradientX;
+        }
         return fused_.buffer(n);
     }
 
@@ -565,22 +553,18 @@ class deviceclass {
     bool stage_ready = false;
     // learned troubled-cell indicator (esdg_mlp.h)
     esdg_mlp* ind_ = nullptr;
+    bool ind_changed = false;                // since the stage batch was given it
     float ind_lo = 0.0f, ind_hi = 1.0f;
     int ind_audit = 0;
-    signed char* o_estat = nullptr;
-    unsigned long long* o_icount = nullptr;
     double *o_q2 = nullptr, *o_clock = nullptr;
     unsigned long long* o_lmax = nullptr;
     // single-kernel stage with artificial viscosity
     double* o_gtr = nullptr;
-    int* o_active = nullptr;
+    int* o_active[2] = {nullptr, nullptr};
     unsigned long long* o_emax = nullptr;
-    const esdg_mlp* stage_ind = nullptr;     // the indicator the stage batch was last given
-    float stage_lo = 0.0f, stage_hi = 0.0f;
     // a captured step of the fused schedule (clock_timeloop) and the settings it was captured with
     hipGraphExec_t step_exec = nullptr;
     bool graph_ok = true;
-    std::tuple<const void*, float, float, int> graph_key{nullptr, 0.0f, 0.0f, 0};
     double *o_q = nullptr, *o_Qt = nullptr, *o_gRK = nullptr, *o_Qtmp = nullptr;
     double *o_D = nullptr, *o_Dstrong = nullptr, *o_Dhat = nullptr, *o_VdmInv = nullptr, *o_GLw = nullptr;
     double *o_Jac = nullptr, *o_Yxi = nullptr, *o_Yeta = nullptr, *o_Xxi = nullptr, *o_Xeta = nullptr;
@@ -734,6 +718,7 @@ int esdg_solver_set_indicator(esdg_solver* s, esdg_mlp* m, float lo, float hi) {
     if (!s) return set_error(nullptr, ESDG_ERR_ARG, "esdg_solver_set_indicator: null solver");
     deviceclass& d = s->dc;
     if (!m) {
+        d.ind_changed = d.ind_changed || d.ind_;
         d.ind_ = nullptr;
         return ESDG_OK;
     }
@@ -741,11 +726,8 @@ int esdg_solver_set_indicator(esdg_solver* s, esdg_mlp* m, float lo, float hi) {
         return set_error(d.ctx_, ESDG_ERR_ARG, "the learned indicator needs a fused schedule (1 or 2) with artificial viscosity");
     if (d.ngl != 8) return set_error(d.ctx_, ESDG_ERR_ARG, "the learned indicator is defined for N = 7");
     if (!(lo <= hi)) return set_error(d.ctx_, ESDG_ERR_ARG, "esdg_solver_set_indicator: lo > hi");
-    int rc = ESDG_OK;
-    if (!d.o_estat) rc = esdg_malloc(d.ctx_, (void**)&d.o_estat, (size_t)d.Nelem);
-    if (!rc && !d.o_icount) rc = esdg_malloc(d.ctx_, (void**)&d.o_icount, 5 * sizeof(unsigned long long));
-    if (rc) return rc;
     d.ind_ = m;
+    d.ind_changed = true;
     d.ind_lo = lo;
     d.ind_hi = hi;
     return ESDG_OK;
@@ -762,7 +744,7 @@ int esdg_solver_indicator_counts(esdg_solver* s, int64_t* viscous, int64_t* fals
     if (!s) return set_error(nullptr, ESDG_ERR_ARG, "esdg_solver_indicator_counts: null solver");
     deviceclass& d = s->dc;
     unsigned long long c[5] = {0, 0, 0, 0, 0};
-    unsigned long long* ic = d.rp_.fused == 2 ? d.stage_.d_icount : d.o_icount;
+    unsigned long long* ic = d.stage_.d_icount;
     if (ic) {
         int rc = esdg_memcpy(d.ctx_, c, ic, sizeof c, ESDG_D2H);
         if (!rc) rc = esdg_fill(d.ctx_, reinterpret_cast<double*>(ic), 0.0, 5);

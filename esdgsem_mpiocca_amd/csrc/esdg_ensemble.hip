@@ -191,9 +191,9 @@ int esdg_ensemble_create(esdg_ctx* ctx, int nscn, const esdg_params* params, con
             if (!rc) S.gtr = (double*)E->alloc((size_t)in.Nelem * 16 * ngl * dd, &rc);
             if (!rc) S.Qv = (double*)E->alloc(nodes * 2 * dd, &rc);
             if (!rc) S.SPV = (double*)E->alloc(fn * 2 * dd, &rc);
-            if (!rc) S.active = (int*)E->alloc(((size_t)in.Nelem + 1) / 2 * dd, &rc);
+            for (int*& a : S.active)     // (zero-filled)
+                if (!rc) a = (int*)E->alloc(((size_t)in.Nelem + 1) / 2 * dd, &rc);
             if (!rc) rc = esdg_fill(ctx, S.visc, 0.0, in.Nelem);
-            if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(S.active), 0.0, ((size_t)in.Nelem + 1) / 2);
             if (rc) break;
         }
         E->scn.push_back(S);
@@ -334,8 +334,9 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
             best_t = ms;
             best_s = s;
         }
-        // back to the snapshot (the state sits in buffer src0 again)
+        // back to the snapshot (the state sits in buffer src0 again; its viscosity is evaluated anew)
         E->src = src0;
+        E->batch.primed = false;
         if (!rc) rc = copy_all(false);
     };
     for (const StageSchedule& s : cand) {

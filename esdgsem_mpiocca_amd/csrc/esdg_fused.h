@@ -1,7 +1,6 @@
 // esdg_fused.h -- fused per-stage kernels (a faster schedule of the same per-stage arithmetic).
 #pragma once
 
-#include <functional>
 #include <string>
 
 #include "esdg_internal.h"
@@ -27,11 +26,6 @@ struct FusedArgs {
     // issued after T), the update using C_stage * dt; a step with dt = 0 changes nothing.
     const double* dt_dev = nullptr;
     double C_stage = 0.0;
-    // Optional (with AV): the pass that evaluates the stage's element viscosity (ViscPara), issued
-    // by the stage itself on the stream it is given.  The face fluxes do not read the viscosity, so
-    // with the context's second stream (and no per-launch profiling) it runs there beside the
-    // face-flux pass, and the face marks follow once both are done.
-    std::function<int(hipStream_t)> visc_pass;
 };
 
 // The device clock of the fused schedule: clock = {dt, t, steps, last dt, error, bad dt, -, -}.
@@ -39,6 +33,15 @@ struct FusedArgs {
 // (src/deviceclass.cpp:899-930, with the host's operation order), t += dt; once t >= T, or after
 // a dt that is not positive and finite (flagged), dt = 0.
 int fused_clock(esdg_ctx* ctx, const double* red, double* clock, double dti, double dvc, int av, double T);
+
+// The degrees that run on these passes: the others take the element-centric stage kernel.
+#define ESDG_FUSED_DISPATCH(ngl, FN, ...)            \
+    switch (ngl) {                                   \
+        case 2: FN<2>(__VA_ARGS__); break;           \
+        case 9: FN<9>(__VA_ARGS__); break;           \
+        case 10: FN<10>(__VA_ARGS__); break;         \
+        default: break;                              \
+    }
 
 class FusedStage {
   public:

@@ -229,10 +229,10 @@ __global__ void __launch_bounds__(256) k_mlp_infer(int n, const float* __restric
     }
 }
 
-// Features + inference fused over the elements of a state; p per element and, when estat is
-// given, the class: 0 smooth (p <= lo), 1 troubled (p >= hi), 2 unsure.  A block takes 32 elements:
+// Features + inference fused over the elements of a state; p (may be null) per element.  Classes: 0 smooth
+// (p <= lo), 1 troubled (p >= hi), 2 unsure.  A block takes 32 elements:
 // features by row threads into two 16-row BF16 tiles, then waves 0 and 1 run one tile each.
-// With MS.visc (and estat), the block then finishes ShockCapturing masked by the classes: the
+// With MS.visc, the block then finishes ShockCapturing masked by the classes: the
 // feature pass left the squares of the modal coefficients m = V (h + b) V^T in LDS, formed with
 // the sensor's arithmetic (ShockCapturing.okl:63-129), so four threads per element form the energy
 // sums from them in the okl's order; the viscosity is the sensor's value, or 0 where the class is
@@ -245,14 +245,10 @@ struct MaskedSensor {
     SensorConsts sc{};
     int audit = 0;
     unsigned long long* counters = nullptr;
-    // the device clock (see mlp_classify_sensor): skip a step issued after T
-    const double* clock = nullptr;
-    double T = 0.0;
-    int clock_mode = 0;
-    // a scenario of a batched ensemble: an element given viscosity marks itself and its face
-    // neighbours with `mark`; in stage 0 its viscosity also enters the scenario's maximum
+    // an element given viscosity marks itself and its face neighbours with `mark`; in stage 0 its
+    // viscosity also enters the scenario's maximum
     const StageScn* scn = nullptr;
-    int mark = 0;
+    int mark = 0, buffer = 0;
     int stage = 0;
 };
 
@@ -264,7 +260,7 @@ struct MaskedSensor {
 __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __restrict__ q,
                                     gptr<const double> __restrict__ B, gptr<const double> __restrict__ V,
                                     const MlpDev& W, float lo, float hi,
-                                    float* __restrict__ p, signed char* __restrict__ estat, const MaskedSensor& MS) {
+                                    float* __restrict__ p, const MaskedSensor& MS) {
     if (MS.counters && threadIdx.x == 0)
         atomicAdd(MS.counters + 4, (unsigned long long)min(FEPB, Nelem - e0));
     __shared__ __attribute__((aligned(16))) FeatLds L;
@@ -302,7 +298,6 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
             const float pv = sigmoidf_(sZ[w][l]);
             const signed char st = (pv <= lo) ? 0 : (pv >= hi ? 1 : 2);
             if (p) p[ee] = pv;
-            if (estat) estat[ee] = st;
             sSt[w * 16 + l] = st;
         }
     }
@@ -325,13 +320,11 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
             }
             glob(MS.visc)[e] = v;
             if (MS.visc_plot) glob(MS.visc_plot)[e] = v;
-            if (MS.scn) {
-                if (v != 0.0) mark_reach(*MS.scn, e, MS.mark, MS.stage);
-                // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
-                if (MS.stage == 0 && v > 0.0) atomicMax(&sMax, (unsigned long long)__double_as_longlong(v));
-            }
+            if (v != 0.0) mark_reach(*MS.scn, e, MS.mark, MS.buffer);
+            // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
+            if (MS.stage == 0 && v > 0.0) atomicMax(&sMax, (unsigned long long)__double_as_longlong(v));
         }
-        const bool to_max = MS.scn && MS.stage == 0;
+        const bool to_max = MS.stage == 0;
         if (MS.counters || to_max) {
             __syncthreads();
             if (threadIdx.x == 0) {
@@ -346,13 +339,8 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
 
 __global__ void __launch_bounds__(256) k_mlp_indicator(int Nelem, const double* __restrict__ q,
                                                        const double* __restrict__ B, const double* __restrict__ V,
-                                                       MlpDev W, float lo, float hi, float* __restrict__ p,
-                                                       signed char* __restrict__ estat, MaskedSensor MS) {
-    if (MS.clock) {
-        // a step issued after T changes nothing: no evaluation, no counts (uniform per block)
-        if ((MS.clock_mode == 1 && MS.clock[1] >= MS.T) || (MS.clock_mode == 2 && MS.clock[0] == 0.0)) return;
-    }
-    mlp_indicator_block(Nelem, (int)blockIdx.x * FEPB, glob(q), glob(B), glob(V), W, lo, hi, p, estat, MS);
+                                                       MlpDev W, float* __restrict__ p) {
+    mlp_indicator_block(Nelem, (int)blockIdx.x * FEPB, glob(q), glob(B), glob(V), W, 0.0f, 1.0f, p, MaskedSensor{});
 }
 
 // The indicator over the learned scenarios of a batched ensemble: block b takes tile tasks[b] (32
@@ -364,18 +352,21 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
                                                        float hi, int audit, unsigned long long* counters) {
     const StageTask tk = tasks[blockIdx.x];
     const StageScn& S = scns[tk.scn];
-    if (stage > 0 && S.clock[0] == 0.0) return;
+    if (stage > 0 && S.clock[0] <= 0.0) return;
     if (stage == 0 && S.clock[1] >= S.T) return;
     MaskedSensor MS;
     MS.visc = S.visc;
+    MS.visc_plot = S.visc_plot;
     MS.sc = S.sc;
     MS.audit = audit;
     MS.counters = counters;
     MS.scn = &S;
-    MS.mark = *mark + stage;
+    // (the step's first viscosity comes before its marks are advanced)
+    MS.mark = *mark + (stage == 0 ? STAGE_MARKS : stage);
+    MS.buffer = src;
     MS.stage = stage;
     mlp_indicator_block(S.Nelem, tk.e0, glob((const double*)S.q[src]), glob(S.B), glob(S.VdmInv), W, lo, hi, nullptr,
-                        nullptr, MS);
+                        MS);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -572,10 +563,9 @@ struct esdg_mlp {
 
 namespace esdg {
 int mlp_classify(esdg_ctx* ctx, const esdg_mlp* m, int Nelem, const double* q, const double* B, const double* VdmInv,
-                 float lo, float hi, float* p, signed char* estat) {
+                 float* p) {
     KernelScope ks(ctx, "mlp_indicator");
-    k_mlp_indicator<<<blocks_for(Nelem, FEPB), 256, 0, ctx->stream>>>(Nelem, q, B, VdmInv, m->dev(), lo, hi, p, estat,
-                                                                       MaskedSensor{});
+    k_mlp_indicator<<<blocks_for(Nelem, FEPB), 256, 0, ctx->stream>>>(Nelem, q, B, VdmInv, m->dev(), p);
     return launch_check(ctx, "mlp_indicator");
 }
 
@@ -586,26 +576,6 @@ int mlp_ensemble_indicator(esdg_ctx* ctx, const esdg_mlp* m, const StageScn* scn
     KernelScope ks(ctx, "ens_indicator");
     k_ens_indicator<<<ntask, 256, 0, ctx->stream>>>(scns, tasks, src, mark, stage, m->dev(), lo, hi, audit, counters);
     return launch_check(ctx, "ens_indicator");
-}
-
-int mlp_classify_sensor(esdg_ctx* ctx, const esdg_mlp* m, int Nelem, const double* q, const double* B,
-                        const double* VdmInv, float lo, float hi, signed char* estat, int audit,
-                        unsigned long long* counters, double* visc, double* visc_plot, const double* clock,
-                        double T, int clock_mode, hipStream_t stream) {
-    if (ctx->p.ngl != 8) return set_error(ctx, ESDG_ERR_ARG, "the learned indicator needs N = 7");
-    MaskedSensor MS;
-    MS.clock = clock;
-    MS.T = T;
-    MS.clock_mode = clock_mode;
-    MS.visc = visc;
-    MS.visc_plot = visc_plot;
-    MS.sc = SensorConsts{ctx->p.ZeroTOL, ctx->p.eps0, ctx->p.sigmaMin, ctx->p.sigmaMax};
-    MS.audit = audit;
-    MS.counters = counters;
-    KernelScope ks(ctx, "mlp_indicator");
-    hipStream_t st = stream ? stream : ctx->stream;
-    k_mlp_indicator<<<blocks_for(Nelem, FEPB), 256, 0, st>>>(Nelem, q, B, VdmInv, m->dev(), lo, hi, nullptr, estat, MS);
-    return launch_check(ctx, "mlp_indicator");
 }
 }  // namespace esdg
 
@@ -706,7 +676,7 @@ int esdg_mlp_indicator(esdg_mlp* M, int Nelem, const double* q, const double* B,
     ESDG_REQUIRE(M->ctx, Nelem >= 0 && q && B && VdmInv && p, "esdg_mlp_indicator: bad argument");
     ESDG_REQUIRE(M->ctx, M->ctx->p.ngl == 8, "esdg_mlp_indicator: the indicator is defined for N = 7 (ngl = 8)");
     if (Nelem == 0) return ESDG_OK;
-    return mlp_classify(M->ctx, M, Nelem, q, B, VdmInv, 0.0f, 1.0f, p, nullptr);
+    return mlp_classify(M->ctx, M, Nelem, q, B, VdmInv, p);
 }
 
 int esdg_mlp_loss_grad(esdg_mlp* M, int n, const float* feat, const float* label, const int* idx, float pos_weight,

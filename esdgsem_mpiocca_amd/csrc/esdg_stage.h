@@ -6,8 +6,8 @@
 // sides from the stage-start state (the neighbour's trace is read from the same buffer, so the two
 // elements of a face produce identical bits), then the flux-differencing volume term, the surface
 // lift, the low-storage RK step into the other state buffer and, on request, the positivity
-// limiter and the wave speed of the new state (the next step's lambda_max, reduced per scenario
-// with an atomic max).  dt is computed on the device; a whole step needs no host synchronisation,
+// limiter, the shock sensor and the wave speed of the new state (the next stage's viscosity and the next
+// step's lambda_max, reduced per scenario with an atomic max).  dt is computed on the device; a whole step needs no host synchronisation,
 // so steps are captured in a hipGraph.
 #pragma once
 
@@ -29,9 +29,9 @@ struct StageScn {
     const int *EdgeData, *E2E, *EMS, *EOR;
     double* q[2];       // ping-pong state buffers
     double* gRK;
-    double* clock;      // [0] dt of the current step (0 once t >= T), [1] t, [2] steps taken,
-                        // [3] dt of the last step taken, [4] 1 if a dt was not positive and finite,
-                        // [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
+    double* clock;      // [0] dt of the current step (-1: it changes nothing; 0: a failed scenario), [1] t,
+                        // [2] steps taken, [3] dt of the last step taken, [4] 1 if a dt was not positive
+                        // and finite ([5] that dt), [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
     unsigned long long* lmax;   // bit pattern of max lambda (non-negative doubles order as integers)
     // artificial viscosity (av = 1): the modal sensor, or with learned = 1 (N = 7) the learned
     // indicator with the sensor as fallback, evaluated on each stage's state; BR1 gradients and the
@@ -44,19 +44,25 @@ struct StageScn {
     double* gtr;        // side traces of the scaled velocity gradients [Nelem][4][4][ngl]
     double* Qv;         // viscous volume term [Nelem][2][ngl^2] (hu, hv)
     double* SPV;        // viscous face fluxes [Nfaces][2][ngl]
-    int* active;        // == mark: viscosity on the element or a face neighbour this stage
-    // the stage's marked elements, each once, with those of every scenario of the same degree and
-    // indicator (learned or not): mlist[0 .. mcount[s]) = {scenario, element} at stage s of a step
+    double* visc_plot;  // its copy (may be null)
+    // active[b][e] == the stage's mark: viscosity on the element or a face neighbour in the state of
+    // buffer b.  Those elements, each once, with those of every scenario of the same degree and
+    // indicator (learned or not): mlist[0 .. mcount[b]) = {scenario, element}
+    int* active[2];
     int2* mlist;
     int* mcount;
     int id;             // this scenario's index in the batch
+    int freeze;         // after a dt that was not positive and finite: 1 the state stays as it is, 0 it takes
+                        // q + 0 gRK
+    // a single solver's buffers (each may be null): the element wave speeds of the state after a step,
+    // and the analysis buffers, advanced after every step
+    double *lam, *arrival, *maxelev;
     unsigned long long* emax;   // bit pattern of the step's max viscosity
     // per element side, what its face flux needs from the connectivity (built by StageBatch::init
     // from E2E, EOR, EMS and EdgeData; one record per side, shared by the scenarios of a mesh):
     // x face, y EdgeData[0] (left element), z EdgeData[1] (right element), w bits: [0,2) left
     // side, [2,4) right side, 4 EdgeData[4] (reversed), 5 EOR, 6 EMS > 0, [8,16) EdgeData[5] + 2,
-    // [16,24) EdgeData[6] + 2
-    // (24: the face's geometry is one record of fgeo)
+    // [16,24) EdgeData[6] + 2, 24 the face's geometry is one record of fgeo
     const int4* srec;
     // one record per element and per face of a mesh with element-wise constant metrics (else null)
     const double *geo, *fgeo;
@@ -66,13 +72,14 @@ struct StageTask {
     int scn, e0, ngl, pad;
 };
 
-// An element with viscosity marks itself and its face neighbours for this stage (the elements whose
-// viscous terms can be non-zero), as the fused face pass does for both elements of every face with
-// viscosity on either side.  The first to mark an element this stage also lists it.
-__device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m, int stage) {
-    auto mark = [&](int k) {
-        if (atomicExch(S.active + k, m) != m) S.mlist[atomicAdd(S.mcount + stage, 1)] = make_int2(S.id, k);
-    };
+// An element with viscosity in the state of buffer b marks itself and its face neighbours for the stage that
+// starts from it (the elements whose viscous terms can be non-zero), as the fused face pass does for both
+// elements of every face with viscosity on either side.  The first to mark an element also lists it.
+__device__ __forceinline__ void mark_element(const StageScn& S, int k, int m, int b) {
+    if (atomicExch(S.active[b] + k, m) != m) S.mlist[atomicAdd(S.mcount + b, 1)] = make_int2(S.id, k);
+}
+__device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m, int b) {
+    auto mark = [&](int k) { mark_element(S, k, m, b); };
     mark(e);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -82,11 +89,14 @@ __device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m, int 
     }
 }
 
+// The mark of a stage: the step's base (advanced by STAGE_MARKS at each step, on the device, so that
+// replays of a captured step take fresh marks) plus the stage.
+constexpr int STAGE_MARKS = 8;
+
 // The marked-element lists of a batch: one for the modal-sensor scenarios of each degree (ngl - 3)
 // and one for the learned ones (MARK_LISTS - 1).  A pass over them takes, of each list, the blocks
 // [first, first + blocks) of its grid.
 constexpr int MARK_LISTS = 7;
-constexpr int MARK_STAGES = 8;          // counter slots of a list, one per stage of a step
 struct MarkLists {
     const int2* list[MARK_LISTS];
     const int* count[MARK_LISTS];
@@ -107,12 +117,17 @@ struct StageSchedule {
 // Host side: device copies of the scenario table and the task list, plus the per-step sequence.
 class StageBatch {
   public:
-    int init(esdg_ctx* ctx, const std::vector<StageScn>& scns);
+    // any_D: without it a degree's D must be the one that earlier batches of the process brought
+    int init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D = false);
     int set_schedule(esdg_ctx* ctx, const StageSchedule& sc);
     // initial lambda_max of every scenario from the state in buffer `src`
     int lambda(esdg_ctx* ctx, int src);
-    // one time step: [marks, viscosity,] dt kernel, then the RK stages [each after its viscosity
-    // and viscous terms]; src flips once per stage
+    // the sensor, marks and viscosity maximum of the state in buffer src; run() calls it when `primed`
+    // is not set, which whoever changes the state, or which scenarios are learned, clears
+    int prime(esdg_ctx* ctx, int src);
+    bool primed = false;
+    // one time step: dt kernel, then the RK stages [each after its viscous terms]; src flips once per
+    // stage
     int step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src);
     // `steps` steps: pairs of steps replayed from a captured graph (schedule.graph), the rest eager
     int run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src);
@@ -139,7 +154,7 @@ class StageBatch {
     StageTask *d_sens = nullptr, *d_ind = nullptr;
     int nsens = 0, nind = 0;
     int2* d_mlist = nullptr;                       // the marked-element lists, one after another
-    int* d_mcount = nullptr;                       // MARK_LISTS x MARK_STAGES lengths
+    int* d_mcount = nullptr;                       // MARK_LISTS x 2 lengths
     int64_t mfirst[MARK_LISTS + 1] = {0};          // where each list starts in d_mlist
     // With both modal-sensor and learned scenarios the stage runs as two streams of work: the
     // other scenarios (sensor pass, their AV terms, their stage launches) on the second stream and
@@ -161,7 +176,6 @@ class StageBatch {
     std::vector<void*> rec_bufs;    // side, element and face records, per distinct mesh
     int build_av_tasks(esdg_ctx* ctx);
     int reset_marks(esdg_ctx* ctx);
-    int av_pass(esdg_ctx* ctx, int src, int stage);     // viscosity of the stage's state + marks
     // gradients, viscous volume and face terms of the marked elements, of the lists [l0, l1), on
     // stream st
     int av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipStream_t st);

@@ -7,6 +7,8 @@
 //   calcRK + UpdateKernel                              (rkLS.okl, UpdateKernelLS.okl)
 //   [PosPres]                                          (PosPres.okl)
 //   [FindLambdaMax of the new state, last stage]      (FindLambdaMax.okl)
+//   [ShockCapturing of the new state]                 (ShockCapturing.okl, for the next stage)
+//   [ArrivalTimes, MaximumElevation, last stage]      (ArrivalTimes.okl, MaximumElevation.okl)
 // and the dt of DGtimeloop (src/deviceclass.cpp:899-930) runs on the device.
 #include "esdg_av_device.h"
 #include "esdg_device.h"
@@ -21,8 +23,8 @@
 namespace esdg {
 
 // Per element: the four planes of the volume sweep (VolCfg::ESZ), reused for the face fluxes
-// [side][v][k] once the sweeps have read them, and 16 doubles for the limiter's element means
-// (keeping consecutive elements 8 doubles apart modulo 16, as ESZ does).  At N = 7 a block of 8
+// [side][v][k] once the sweeps have read them, and 16 doubles: the side records, and the limiter's and the
+// sensor's sums (keeping consecutive elements 8 doubles apart modulo 16, as ESZ does).  At N = 7 a block of 8
 // elements then fits 8 blocks per CU.
 template <int NGL>
 struct StageCfg {
@@ -30,7 +32,7 @@ struct StageCfg {
     static constexpr int EPW = V::EPW;
     static constexpr int FSZ = 12 * NGL;              // face fluxes [side][v][k] of one element
     static_assert(FSZ <= 4 * V::PLANE, "the face fluxes fit in the element's planes");
-    static constexpr int ELDS = V::ESZ + 16;          // per element
+    static constexpr int ELDS = V::ESZ + 16;          // per element: planes, side records, sums
     static constexpr int LDS = EPW * ELDS;            // doubles of LDS per block
 };
 
@@ -43,6 +45,14 @@ template <int HI>
 struct MaxLds<HI, HI> {
     static constexpr int value = StageCfg<HI>::LDS;
 };
+
+// max of a non-negative double into a cell (non-negative doubles order as their bit patterns).  Most blocks
+// find a larger value there already and leave the cell alone: atomics of all blocks on one cell queue
+// up at about 12 ns each.
+__device__ __forceinline__ void max_into(unsigned long long* cell, double m) {
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    if (bits > __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(cell, bits);
+}
 
 // Volume term, surface lift, RK update, limiter and wave speed of one block of elements; the
 // face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
@@ -63,11 +73,13 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                                            gptr<const double> __restrict__ geo,
                                            gptr<const double> __restrict__ EleSizes,
                                            gptr<const double> __restrict__ GLw,
-                                           gptr<unsigned long long> __restrict__ lmax, const StageScn* SV, int mark,
-                                           const double* D) {
+                                           gptr<unsigned long long> __restrict__ lmax, const StageScn* SV, int src,
+                                           int mark, int next_mark, double* sD) {
     using C = VolCfg<NGL>;
     double* FS = P;                  // face fluxes, after the sweeps (the planes are free then)
-    double* MS = P + C::ESZ;         // the limiter's element means
+    const int4* rec = reinterpret_cast<const int4*>(P + C::ESZ);   // the element's side records
+    double* MS = P + C::ESZ + 8;     // the limiter's and the sensor's sums
+    const double* D = sD;
     const int lane = threadIdx.x;
     double h[NGL], hu[NGL], hv[NGL], u[NGL], v[NGL];
     double Y[AFF ? 1 : NGL], X[AFF ? 1 : NGL];
@@ -75,6 +87,16 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
     double G[8];                     // the element's geometry record (AFF)
 #pragma unroll
     for (int c = 0; c < NGL; ++c) { a1[c] = 0.0; a2[c] = 0.0; a3[c] = 0.0; }
+
+    // whether viscosity is in reach, and the element's own, loaded beside the row data
+    bool marked = false;
+    double eps0 = 0.0;
+    if constexpr (AV) {
+        if (act && SV->av) {
+            marked = glob(SV->active[src])[e] == mark;
+            eps0 = glob((const double*)SV->visc)[e];
+        }
+    }
 
     // ---- row phase: eta-row r ---------------------------------------------------------------
     if (act) {
@@ -100,6 +122,16 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 X[c] = Xeta[xb + c];
             }
         }
+        // a step that changes nothing has dt < 0: the state goes over to the other buffer as it is.  (dt is
+        // loaded beside the rows; a wave that waited for it before loading them cost 3 %.)
+        if (dt < 0.0) {
+#pragma unroll
+            for (int c = 0; c < NGL; ++c) {
+                qo[qb + c] = h[c];
+                qo[qb + C::NN + c] = hu[c];
+                qo[qb + 2 * C::NN + c] = hv[c];
+            }
+        } else {
         early();   // LDS stores of values loaded beside the row data
 #pragma unroll
         for (int c = 0; c < NGL; ++c) {
@@ -113,7 +145,9 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
         if constexpr (AFF) line_sweep<NGL, false>(D, g, h, hu, hv, u, v, ConstMetrics(G[0], G[1]), a1, a2, a3);
         else line_sweep<NGL, false>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, a1, a2, a3);
+        }
     }
+    if (dt < 0.0) return;
     __syncthreads();
 
     // ---- column phase: xi-column r ----------------------------------------------------------
@@ -208,10 +242,24 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             // after the surface lift: the viscous volume term (where the element's viscosity is not
             // zero), then the lift of the viscous face fluxes (VolumeKernelViscose.okl,
             // SurfaceKernelVisc.okl), as the fused volume pass adds them
-            const gptr<const int> E2E = glob(SV->E2E), EOR = glob(SV->EOR), EMS = glob(SV->EMS);
-            const gptr<const double> SPV = glob((const double*)SV->SPV);
-            if (SV->av && glob(SV->active)[e] == mark) {
-                if (glob(SV->visc)[e] != 0.0) {
+            if (marked) {
+                const gptr<const double> SPV = glob((const double*)SV->SPV);
+                // every load of the branch is issued before its sums: each side's face, orientation and
+                // sign come from its record
+                auto side = [&](int s, int& rev, double& nms) {
+                    const int4 R4 = rec[s];
+                    rev = (int)(((unsigned)R4.w >> 5) & 1u);
+                    nms = (((unsigned)R4.w >> 6) & 1u) ? -1.0 : 1.0;    // -EMS
+                    return SPV + (int64_t)R4.x * NGL * 2;
+                };
+                const bool edge = r == 0 || r == NGL - 1;
+                int rv0, rv2, rvc;
+                double m0, m2, mc;
+                const gptr<const double> f0 = side(0, rv0, m0), f2 = side(2, rv2, m2),
+                                         fc = side(r == NGL - 1 ? 1 : 3, rvc, mc);
+                const int l0 = rv0 ? r : NGL - 1 - r, l2 = rv2 ? r : NGL - 1 - r;
+                const double s02 = f0[l0], s03 = f0[l0 + NGL], s22 = f2[l2], s23 = f2[l2 + NGL];
+                if (eps0 != 0.0) {
                     const gptr<const double> qv = glob((const double*)SV->Qv) + (int64_t)e * C::NN * 2 + r;
 #pragma unroll
                     for (int k = 0; k < NGL; ++k) {
@@ -219,26 +267,16 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                         b3[k] += qv[C::NN + k * NGL];
                     }
                 }
-#pragma unroll
-                for (int ph = 0; ph < 2; ++ph) {
+                b2[0] += m0 * rJ[0] * s02;
+                b3[0] += m0 * rJ[0] * s03;
+                b2[NGL - 1] += m2 * rJ[NGL - 1] * s22;
+                b3[NGL - 1] += m2 * rJ[NGL - 1] * s23;
+                if (edge) {
 #pragma unroll
                     for (int k = 0; k < NGL; ++k) {
-                        int side = -1, t = 0;
-                        if (ph == 0) {
-                            if (k == 0) { side = 0; t = r; }
-                            else if (k == NGL - 1) { side = 2; t = r; }
-                        } else {
-                            if (r == NGL - 1) { side = 1; t = k; }
-                            else if (r == 0) { side = 3; t = k; }
-                        }
-                        if (side < 0) continue;
-                        const int ifa = E2E[e * 4 + side] - 1;
-                        const int rev = EOR[e * 4 + side];
-                        const int ms = EMS[e * 4 + side];
-                        const int inc = rev * t + (1 - rev) * (NGL - 1 - t);
-                        const int64_t fl = (int64_t)ifa * NGL * 2 + inc;
-                        b2[k] += -ms * rJ[k] * SPV[fl];
-                        b3[k] += -ms * rJ[k] * SPV[fl + NGL];
+                        const int l = rvc ? k : NGL - 1 - k;
+                        b2[k] += mc * rJ[k] * fc[l];
+                        b3[k] += mc * rJ[k] * fc[l + NGL];
                     }
                 }
             }
@@ -276,41 +314,40 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
     }
     if (positivity) {
-        // PosPres.okl on the new state: element means in the okl's serial order (xi outer, eta inner)
+        // PosPres.okl on the new state: the products h w, hu w, hv w (w = GLw[xi] GLw[eta] / Jinv) to the
+        // planes; three lanes of the element add them in the okl's serial order (xi outer, eta inner)
         __syncthreads();
+        double hmin = 0.0;
         if (act) {
+            const double gx = GLw[r];
 #pragma unroll
             for (int k = 0; k < NGL; ++k) {
-                P[0 * C::PLANE + k * C::RS + r] = b1[k];
-                P[1 * C::PLANE + k * C::RS + r] = b2[k];
-                P[2 * C::PLANE + k * C::RS + r] = b3[k];
-                P[3 * C::PLANE + k * C::RS + r] = rJ[k];
+                const double w = gx * GLw[k] / rJ[k];
+                P[0 * C::PLANE + k * C::RS + r] = b1[k] * w;
+                P[1 * C::PLANE + k * C::RS + r] = b2[k] * w;
+                P[2 * C::PLANE + k * C::RS + r] = b3[k] * w;
+                hmin = fmin(hmin, b1[k]);
             }
+            P[3 * C::PLANE + r] = hmin;
         }
         __syncthreads();
-        if (act && r == 0) {
-            double hmin = 0.0, ha = 0.0, hua = 0.0, hva = 0.0;
+        if (act && r < 3) {
+            const double* F = P + r * C::PLANE;
+            double a = 0.0;
             for (int l = 0; l < NGL; ++l)
-                for (int k = 0; k < NGL; ++k) {
-                    const int o = k * C::RS + l;
-                    const double w = GLw[l] * GLw[k] / P[3 * C::PLANE + o];
-                    ha += P[o] * w;
-                    hua += P[C::PLANE + o] * w;
-                    hva += P[2 * C::PLANE + o] * w;
-                    hmin = fmin(hmin, P[o]);
-                }
-            const double size = EleSizes[e];
-            ha = ha / size;
-            if (fabs(ha) < zero_tol) ha = 0.0;
-            MS[0] = ha;
-            MS[1] = hua / size;
-            MS[2] = hva / size;
-            MS[3] = (ha == hmin) ? 1.0 : fmin(1.0, ha / (ha - hmin));
-            MS[4] = hmin;
+                for (int k = 0; k < NGL; ++k) a += F[k * C::RS + l];
+            MS[r] = a;
         }
         __syncthreads();
         if (act) {
-            const double ha = MS[0], hua = MS[1], hva = MS[2], th = MS[3], hmin = MS[4];
+            hmin = 0.0;
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) hmin = fmin(hmin, P[3 * C::PLANE + k]);
+            const double size = EleSizes[e];
+            double ha = MS[0] / size;
+            if (fabs(ha) < zero_tol) ha = 0.0;
+            const double hua = MS[1] / size, hva = MS[2] / size;
+            const double th = (ha == hmin) ? 1.0 : fmin(1.0, ha / (ha - hmin));
 #pragma unroll
             for (int k = 0; k < NGL; ++k) {
                 if (hmin < 0.0) {
@@ -328,6 +365,17 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                     b2[k] = 0.0; b3[k] = 0.0;
                 }
             }
+        }
+    }
+    // b of row r for the sensor below, loaded before the stores
+    // (a step of a failed scenario has marks in its first stage only)
+    const bool sensor = AV && SV->av && !SV->learned && (dt != 0.0 || last);
+    double w[AV ? NGL : 1];
+    if constexpr (AV) {
+        if (sensor && act) {
+            const gptr<const double> B = glob(SV->B) + (int64_t)e * C::NN + r * NGL;
+#pragma unroll
+            for (int i = 0; i < NGL; ++i) w[i] = B[i];
         }
     }
     double lam = 0.0;
@@ -352,18 +400,115 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
     }
     if (last) {
-        for (int off = 32; off > 0; off >>= 1) lam = fmax(lam, __shfl_xor(lam, off));
-        if (lane == 0) atomicMax((unsigned long long*)lmax, (unsigned long long)__double_as_longlong(lam));
+        if (SV->lam) {
+            double m = 0.0;
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) m = fmax(m, __shfl(lam, lane - r + k));
+            if (act && r == 0) glob(SV->lam)[e] = m;
+        }
+        double m = lam;
+        for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+        if (lane == 0) max_into((unsigned long long*)lmax, m);
+        // ArrivalTimes.okl:16-62 and MaximumElevation.okl:16-55 on the state after the step, at its time
+        if (act && SV->arrival) {
+            const double t = glob(SV->clock)[1];
+            const gptr<double> arr = glob(SV->arrival);
+            const gptr<const double> B = glob(SV->B);
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) {
+                const int64_t x = xb + k * NGL;
+                if (arr[x] == 1000.0 && fabs((b1[k] + B[x]) - SV->h_zero) > 0.00005) arr[x] = t;
+            }
+        }
+        if (act && SV->maxelev) {
+            const gptr<double> mx = glob(SV->maxelev);
+            const gptr<const double> B = glob(SV->B);
+#pragma unroll
+            for (int k = 0; k < NGL; ++k) {
+                const int64_t x = xb + k * NGL;
+                mx[x] = fmax(mx[x], b1[k] + B[x] - SV->h_zero);
+            }
+        }
+    }
+    if constexpr (AV) {
+        // ShockCapturing.okl:63-217 on the new state (here 80 us at 512 x 512, N = 7; as a pass of its own
+        // over q 105), with the arithmetic of sensor_rows: lane r forms
+        // column r of T = V (h + b) from row r of h + b, then the squares of row r of T V^T; up to four
+        // lanes form the energy sums.  An element with viscosity marks what it reaches for the next stage,
+        // and after the last stage its viscosity enters the next step's maximum.
+        if (sensor) {
+            __syncthreads();
+            double* Tm = P + 1 * C::PLANE;
+            double* V = sD;
+            for (int t = lane; t < C::NN; t += 64) V[t] = glob(SV->VdmInv)[t];
+            if (act) {
+#pragma unroll
+                for (int k = 0; k < NGL; ++k) P[k * C::RS + r] = b1[k];
+            }
+            __syncthreads();
+            if (act) {
+#pragma unroll
+                for (int i = 0; i < NGL; ++i) w[i] = w[i] + P[r * C::RS + i];
+#pragma unroll
+                for (int a = 0; a < NGL; ++a) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int l = 0; l < NGL; ++l) s += V[a * NGL + l] * w[l];
+                    Tm[a * C::RS + r] = s;
+                }
+            }
+            __syncthreads();
+            if (act) {
+#pragma unroll
+                for (int l = 0; l < NGL; ++l) w[l] = Tm[r * C::RS + l];
+#pragma unroll
+                for (int c = 0; c < NGL; ++c) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int l = 0; l < NGL; ++l) s += w[l] * V[c * NGL + l];
+                    Tm[r * C::RS + c] = s * s;
+                }
+            }
+            __syncthreads();
+            if (act)
+                for (int k = r; k < 4; k += NGL) MS[k] = sensor_sum<NGL, C::RS, true>(Tm, k);
+            __syncthreads();
+            double eps = 0.0;
+            if (act && r == 0) {
+                eps = sensor_ramp(MS[0], MS[1], MS[2], MS[3], SV->sc);
+                glob(SV->visc)[e] = eps;
+                if (SV->visc_plot) glob(SV->visc_plot)[e] = eps;
+            }
+            // mark_reach by the element's lanes, a side each
+            if (__shfl(eps, lane - r) != 0.0 && act) {
+                for (int s = r; s < 4; s += NGL) {
+                    const int4 R4 = rec[s];
+                    const int cpuL = (int)(((unsigned)R4.w >> 8) & 255u) - 2, cpuR = (int)(((unsigned)R4.w >> 16) & 255u) - 2;
+                    if (s == 0) mark_element(*SV, e, next_mark, src ^ 1);
+                    if (cpuL == 0 && R4.y != e) mark_element(*SV, R4.y, next_mark, src ^ 1);
+                    if (cpuR == 0 && R4.z != e) mark_element(*SV, R4.z, next_mark, src ^ 1);
+                }
+            }
+            if (last) {
+                // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
+                double m = eps > 0.0 ? eps : 0.0;
+                for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+                if (lane == 0 && m > 0.0) max_into(SV->emax, m);
+            }
+        }
     }
 }
 
 
 template <int NGL, bool AV, bool AFF>
 __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, int src, double rkA,
-                                           double rkC, bool last, int mark) {
+                                           double rkC, bool last, int mark, int next_mark) {
     using C = VolCfg<NGL>;
     using SC = StageCfg<NGL>;
     const int lane = threadIdx.x;
+    // the marks of the stage's state have been used: the list that the next stage's marks go to is the
+    // other one, and this one is empty when its turn comes
+    if (AV && S.av && e0 == 0 && lane == 0) S.mcount[src] = 0;
     // D of this degree in LDS (wave-uniform reads, broadcast): keeps it out of the scalar registers
     for (int t = lane; t < NGL * NGL; t += 64) sD[t] = glob(S.D)[t];
     const int el = lane / NGL, r = lane % NGL;
@@ -375,8 +520,8 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     const double g = S.g;
 
     // The element's four side records (StageScn::srec) are loaded beside the row data and stored
-    // to the limiter's LDS area (free until the epilogue), so the face-flux reads after the sweeps
-    // need no dependent round trips through ElemToEdge and EdgeData.
+    // to LDS, so the face-flux reads after the sweeps need no dependent round trips through
+    // ElemToEdge and EdgeData.
     constexpr int FPL = (4 + NGL - 1) / NGL;   // sides per lane: lane r loads sides r, r + NGL, ...
     int4 rec[FPL];
 #pragma unroll
@@ -468,20 +613,21 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     };
 
     __syncthreads();   // sD written
-    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, glob(S.clock)[0],
-                             last, glob(S.clock)[6] != 0.0, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
+    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, glob(S.clock)[0], last,
+                             glob(S.clock)[6] != 0.0, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
                              glob(S.Xxi), glob(S.Jac), glob(S.Bx), glob(S.By), glob(S.geo), glob(S.EleSizes), glob(S.GLw),
-                             glob(S.lmax), &S, mark, sD);
+                             glob(S.lmax), &S, src, mark, next_mark, sD);
 }
 
 template <int LO, int HI, bool AV, bool AFF>
 __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, const StageTask& tk, double* lds,
-                                           double* sD, int src, double rkA, double rkC, bool last, int mark) {
+                                           double* sD, int src, double rkA, double rkC, bool last, int mark,
+                                           int next_mark) {
     const StageScn& S = scns[tk.scn];
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                \
     case n:                                                                         \
-        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, rkA, rkC, last, mark);    \
+        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, rkA, rkC, last, mark, next_mark);    \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -503,7 +649,7 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
                                                  int last, const int* __restrict__ markp, int stage) {
     __shared__ __attribute__((aligned(16))) double lds[MaxLds<LO, HI>::value];
     __shared__ double sD[HI * HI];
-    const int mark = AV ? *markp + stage : 0;
+    const int base = AV ? *markp : 0, mark = base + stage, next_mark = last ? base + STAGE_MARKS : mark + 1;
     const int b = blockIdx.x;
     int beg = 0, cnt = n, i0 = b, stride = gridDim.x;
     if (xcd) {
@@ -514,48 +660,59 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
         stride = gridDim.x >> 3;
     }
     if constexpr (!PERSIST) {
-        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i0], lds, sD, src, rkA, rkC, last != 0, mark);
+        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i0], lds, sD, src, rkA, rkC, last != 0, mark, next_mark);
     } else {
         const int nch = (cnt + tile - 1) / tile;
         for (int c = i0; c < nch; c += stride) {
             const int i1 = min(cnt, (c + 1) * tile);
             for (int i = c * tile; i < i1; ++i) {
                 if (i != i0 * tile) __syncthreads();   // LDS of the previous task is free
-                stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i], lds, sD, src, rkA, rkC, last != 0, mark);
+                stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i], lds, sD, src, rkA, rkC, last != 0, mark, next_mark);
             }
         }
     }
 }
 
-// lambda_max of the state in buffer src, per scenario (FindLambdaMax.okl + the host max loop)
+// lambda_max of the state in buffer src, per scenario (FindLambdaMax.okl + the host max loop).  A block
+// takes every gridDim.x-th task and keeps the maximum while the scenario stays the same (one wave per task,
+// each with an atomic, took 395 us at 512 x 512, N = 7; this takes 89).
 __global__ void __launch_bounds__(256) k_stage_lambda(const StageScn* __restrict__ scns,
-                                                      const StageTask* __restrict__ tasks, int src) {
-    const StageTask tk = tasks[blockIdx.x];
-    const StageScn& S = scns[tk.scn];
-    const int ngl2 = tk.ngl * tk.ngl;
-    const int epw = 64 / tk.ngl;
+                                                      const StageTask* __restrict__ tasks, int n, int src) {
+    __shared__ double part[4];
     double lam = 0.0;
-    for (int t = threadIdx.x; t < epw * ngl2; t += blockDim.x) {
-        const int e = tk.e0 + t / ngl2;
-        if (e >= S.Nelem) continue;
-        const int64_t id = (int64_t)e * ngl2 * 3 + t % ngl2;
-        const double* q = S.q[src];
-        const double hh = q[id];
-        const double Qinv = (hh > S.tol) ? 1.0 / hh : 0.0;
-        const double c = sqrt(S.g * hh);
-        lam = fmax(lam, c + fmax(fabs(q[id + ngl2] * Qinv), fabs(q[id + 2 * ngl2] * Qinv)));
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const StageTask tk = tasks[i];
+        const StageScn& S = scns[tk.scn];
+        const int ngl2 = tk.ngl * tk.ngl;
+        const int nodes = min(64 / tk.ngl, S.Nelem - tk.e0) * ngl2;
+        const gptr<const double> q = glob((const double*)S.q[src]) + (int64_t)tk.e0 * ngl2 * 3;
+        for (int t = threadIdx.x; t < nodes; t += 256) {
+            const int id = t / ngl2 * ngl2 * 3 + t % ngl2;
+            const double hh = q[id];
+            const double Qinv = (hh > S.tol) ? 1.0 / hh : 0.0;
+            const double c = sqrt(S.g * hh);
+            lam = fmax(lam, c + fmax(fabs(q[id + ngl2] * Qinv), fabs(q[id + 2 * ngl2] * Qinv)));
+        }
+        const int next = i + (int)gridDim.x;
+        if (next < n && tasks[next].scn == tk.scn) continue;
+        for (int off = 32; off > 0; off >>= 1) lam = fmax(lam, __shfl_xor(lam, off));
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = lam;
+        __syncthreads();
+        if (threadIdx.x == 0) max_into(S.lmax, fmax(fmax(part[0], part[1]), fmax(part[2], part[3])));
+        __syncthreads();
+        lam = 0.0;
     }
-    for (int off = 32; off > 0; off >>= 1) lam = fmax(lam, __shfl_xor(lam, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(S.lmax, (unsigned long long)__double_as_longlong(lam));
 }
 
 // DGtimeloop's dt (src/deviceclass.cpp:899-930) per scenario: while t < T, dt = min(T - t,
 // dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T (or after a dt that is not positive
-// and finite, which is flagged) dt = 0 and the stages leave the state unchanged.  lambda_max and
-// eps_max are reset for the next step's reductions.
-__global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
+// and finite, which is flagged) clock[0] = -1 and the stages leave the state unchanged.  (A batch that does
+// not freeze a failed state goes on with dt = 0 there: what is not finite spreads, as in
+// q + 0 gRK.)  lambda_max and eps_max are reset for the next step's reductions, and the step's marks begin.
+__global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn, int* mark) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nscn) return;
+    if (s == 0 && mark) *mark += STAGE_MARKS;
     const StageScn& S = scns[s];
     const double lm = __longlong_as_double((long long)*S.lmax);
     *S.lmax = 0ull;
@@ -566,7 +723,7 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
     }
     double* ck = S.clock;
     const double t = ck[1];
-    double dt = 0.0;
+    double dt = -1.0;
     if (t < S.T && ck[4] == 0.0) {
         const double dt_i = S.dti / lm;
         // with artificial viscosity also the viscous limit dvc / max eps (infinite where no element
@@ -574,7 +731,9 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
         dt = S.av ? fmin(S.T - t, fmin(dt_i, S.dvc / em)) : fmin(S.T - t, dt_i);
         if (!(dt > 0.0) || isinf(dt)) {
             ck[4] = 1.0;
-            dt = 0.0;
+            ck[5] = dt;
+            ck[6] = 1.0;
+            dt = S.freeze ? -1.0 : 0.0;
         } else {
             ck[1] = t + dt;
             ck[2] += 1.0;
@@ -582,14 +741,17 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
             // the step that ends the run leaves its RK register for a checkpoint
             ck[6] = (ck[2] == ck[7] || t + dt >= S.T) ? 1.0 : 0.0;
         }
+    } else if (ck[4] != 0.0 && !S.freeze) {
+        dt = 0.0;
     }
     ck[0] = dt;
 }
 
 // ---------------------------------------------------------------------------------------------
-// Artificial viscosity of the scenarios with av = 1.  Before each stage: the element viscosity of
-// the stage's state (ShockCapturing.okl, or the learned indicator's pass in esdg_mlp.hip), each
-// viscous element marking itself and its face neighbours with the stage's mark; the gradient pass
+// Artificial viscosity of the scenarios with av = 1.  The element viscosity of a stage's state comes from the
+// stage that wrote it (ShockCapturing.okl) or from the learned indicator's pass before the stage
+// (esdg_mlp.hip), each viscous element marking itself and its face neighbours with the stage's mark.
+// Before each stage: the gradient pass
 // (calcGradient + SurfaceKernelGradient + scaleGradient + VolumeKernelViscose) over the marked
 // elements; the viscous face fluxes (CollectEdgeDataGradient + calcNumFluxesViscose) of the faces
 // of marked elements.  The stage kernel then adds the viscous terms of the marked elements.  The
@@ -597,12 +759,12 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn) {
 // traces read from the state instead of a side-trace buffer: the same bits.
 // ---------------------------------------------------------------------------------------------
 
-// The marks of a step: stage s of the step marks with *mark + s.  Advanced by 8 at each step on
-// the device, so that replays of a captured step take fresh marks; the lists of every stage start
-// empty.
-__global__ void k_stage_mark(int* mark, int* mcount) {
-    if (threadIdx.x == 0) *mark += 8;
-    if (threadIdx.x < MARK_LISTS * MARK_STAGES) mcount[threadIdx.x] = 0;
+// Before the sensor pass of prime(): fresh marks, empty lists, no viscosity maximum.
+__global__ void k_stage_prime(const StageScn* __restrict__ scns, int nscn, int* mark, int* mcount) {
+    if (threadIdx.x == 0) *mark += STAGE_MARKS;
+    if (threadIdx.x < 2 * MARK_LISTS) mcount[threadIdx.x] = 0;
+    for (int s = threadIdx.x; s < nscn; s += blockDim.x)
+        if (scns[s].av) *scns[s].emax = 0ull;
 }
 
 template <int LO, int HI>
@@ -615,7 +777,7 @@ struct MaxRowLds<HI, HI> {
 };
 
 template <int NGL>
-__device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int src, int m, int stage, double* sV,
+__device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int src, int m, double* sV,
                                                 double* sT, double (*sSum)[4], unsigned long long* sMax) {
     if (threadIdx.x < NGL * NGL) sV[threadIdx.x] = glob(S.VdmInv)[threadIdx.x];
     const double v = sensor_rows<NGL>(S.Nelem, e0, S.sc, glob((const double*)S.q[src]), glob(S.B), sV, sT, sSum);
@@ -623,42 +785,39 @@ __device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int s
     const int e = e0 + el;
     if (el < RowBlock<NGL>::EPB && e < S.Nelem && r == 0) {
         glob(S.visc)[e] = v;
-        if (v != 0.0) mark_reach(S, e, m, stage);
+        if (S.visc_plot) glob(S.visc_plot)[e] = v;
+        if (v != 0.0) mark_reach(S, e, m, src);
         // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
-        if (stage == 0 && v > 0.0) atomicMax(sMax, (unsigned long long)__double_as_longlong(v));
+        if (v > 0.0) atomicMax(sMax, (unsigned long long)__double_as_longlong(v));
     }
 }
 
-// ShockCapturing of the stage's state over RowBlock tiles (tasks: {scenario, first element, ngl}).
-// A scenario whose time has reached T (or whose step has dt = 0) is skipped; in stage 0 the
-// block's largest viscosity enters the scenario's eps_max.
+// ShockCapturing of the state in buffer src over RowBlock tiles (tasks: {scenario, first element, ngl}), for
+// the first stage of a run: the stages evaluate it on the states that they write.  A block's largest
+// viscosity enters its scenario's eps_max; the marks are those of the next step's first stage.
 template <int LO, int HI>
 __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__ scns,
                                                     const StageTask* __restrict__ tasks, int src,
-                                                    const int* __restrict__ markp, int stage) {
+                                                    const int* __restrict__ markp) {
     __shared__ double sV[HI * HI];
     __shared__ double sT[MaxRowLds<LO, HI>::value];
     __shared__ double sSum[RowBlock<LO>::EPB][4];
     __shared__ unsigned long long sMax;
     const StageTask tk = tasks[blockIdx.x];
     const StageScn& S = scns[tk.scn];
-    if (stage > 0 && S.clock[0] == 0.0) return;
-    if (stage == 0 && S.clock[1] >= S.T) return;
-    const int m = *markp + stage;
+    const int m = *markp + STAGE_MARKS;
     if (threadIdx.x == 0) sMax = 0ull;   // published by the sensor's first barrier
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
-        if constexpr (n >= LO && n <= HI) ens_sensor_body<n>(S, tk.e0, src, m, stage, sV, sT, sSum, &sMax); \
+        if constexpr (n >= LO && n <= HI) ens_sensor_body<n>(S, tk.e0, src, m, sV, sT, sSum, &sMax); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
         default: break;
     }
-    if (stage == 0) {
-        __syncthreads();
-        if (threadIdx.x == 0 && sMax) atomicMax(S.emax, sMax);
-    }
+    __syncthreads();
+    if (threadIdx.x == 0 && sMax) atomicMax(S.emax, sMax);
 }
 
 // One list's marked elements, ElemBlock<NGL>::EPB at a time, one thread per node; the elements of a
@@ -690,14 +849,13 @@ __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns,
 // that crosses one part of a mesh spreads over the chip (one block per 256-element tile worked
 // through the tile's marked elements in sequence, 248 us for each launch of ten scenarios).
 template <int LO, int HI>
-__global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src,
-                                                  int stage) {
+__global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src) {
     __shared__ double sDh[256], sDs[256];
     __shared__ double sA[256], sB[256], sC[256], sE[256];
     __shared__ double sEps[ElemBlock<LO>::EPB];
     int l = l0;
     while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
-    const int blk = (int)blockIdx.x - L.first[l], cnt = L.count[l][stage];
+    const int blk = (int)blockIdx.x - L.first[l], cnt = L.count[l][src];
     if (blk >= L.blocks[l]) return;
     switch (L.ngl[l]) {
 #define ESDG_CASE(n)                                                                          \
@@ -714,14 +872,14 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
 // The viscous face fluxes over the side nodes of the listed elements; each face node once, by the
 // face's left element if that is marked, else by its right one (the faces a marked element reads
 // are exactly those).
-__global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1,
+__global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src,
                                                    const int* __restrict__ markp, int stage) {
     int l = l0;
     while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
     const int blk = (int)blockIdx.x - L.first[l];
     if (blk >= L.blocks[l]) return;
     const int m = *markp + stage, ngl = L.ngl[l];
-    const int64_t items = (int64_t)L.count[l][stage] * 4 * ngl;
+    const int64_t items = (int64_t)L.count[l][src] * 4 * ngl;
     for (int64_t it = (int64_t)blk * 256 + threadIdx.x; it < items; it += (int64_t)L.blocks[l] * 256) {
         const int li = (int)(it / (4 * ngl)), rem = (int)(it % (4 * ngl));
         const int side = rem / ngl, i = rem % ngl;
@@ -730,7 +888,7 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
         const int f = S.E2E[me.y * 4 + side] - 1;
         const int* E = S.EdgeData + 8 * (int64_t)f;
         const int iel = E[0], ier = E[1], isl = E[2], isr = E[3], rv = E[4], cpuL = E[5], cpuR = E[6];
-        const int owner = (cpuL == 0 && S.active[iel] == m) ? iel : ier;
+        const int owner = (cpuL == 0 && S.active[src][iel] == m) ? iel : ier;
         if (me.y != owner) continue;
         viscous_face_node(f, i, ngl, S.geomFace, iel, ier, isl, isr, rv, cpuL, cpuR, S.gtr, S.visc, S.nx, S.ny, S.scal,
                           S.SPV);
@@ -819,14 +977,14 @@ __global__ void __launch_bounds__(256) k_side_records(int Nelem, const int* __re
     rec[t] = make_int4(f, E[0], E[1], (int)w);
 }
 
-int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
+int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D) {
     host = scns;
     if (scns.empty()) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one scenario");
     for (const StageScn& S : scns) {
         if (S.ngl < 3 || S.ngl > 8) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage supports 2 <= N <= 7");
         if (S.Nelem <= 0) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one element");
     }
-    int rc = check_degree_operators(ctx, scns);
+    int rc = any_D ? ESDG_OK : check_degree_operators(ctx, scns);
     if (rc) return rc;
     // element and face records, once per distinct mesh and bottom (a mesh with varying metrics has
     // none), and side records, once per distinct connectivity and face records
@@ -924,7 +1082,7 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     // not depend on which scenarios are learned
     if (!d_mlist) {
         int rc = esdg_malloc(ctx, (void**)&d_mlist, (size_t)all * sizeof(int2));
-        if (!rc) rc = esdg_malloc(ctx, (void**)&d_mcount, MARK_LISTS * MARK_STAGES * sizeof(int));
+        if (!rc) rc = esdg_malloc(ctx, (void**)&d_mcount, MARK_LISTS * 2 * sizeof(int));
         if (rc) return rc;
     }
     for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + total[l];
@@ -933,7 +1091,7 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
         S.id = s;
         if (!S.av) continue;
         S.mlist = d_mlist + mfirst[list_of(S)];
-        S.mcount = d_mcount + MARK_STAGES * list_of(S);
+        S.mcount = d_mcount + 2 * list_of(S);
     }
     int rcs = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (rcs) return rcs;
@@ -960,6 +1118,7 @@ int StageBatch::set_indicator(esdg_ctx* ctx, const esdg_mlp* m, float lo, float 
     }
     if (m && !learned)
         return set_error(ctx, ESDG_ERR_ARG, "the learned indicator needs a scenario with N = 7 and artificial viscosity");
+    primed = false;
     mlp = m;
     ind_lo = lo;
     ind_hi = hi;
@@ -975,35 +1134,28 @@ int StageBatch::set_indicator(esdg_ctx* ctx, const esdg_mlp* m, float lo, float 
 int StageBatch::reset_marks(esdg_ctx* ctx) {
     int rc = esdg_fill(ctx, reinterpret_cast<double*>(d_mark), 0.0, 8);
     for (const StageScn& S : host)
-        if (!rc && S.av) rc = esdg_fill(ctx, reinterpret_cast<double*>(S.active), 0.0, ((size_t)S.Nelem + 1) / 2);
+        for (int* a : {S.active[0], S.active[1]})
+            if (!rc && S.av) rc = esdg_fill(ctx, reinterpret_cast<double*>(a), 0.0, ((size_t)S.Nelem + 1) / 2);
     marks_used = 0;
+    primed = false;
     return rc;
 }
 
-int StageBatch::av_pass(esdg_ctx* ctx, int src, int stage) {
-    if (nind && !mlp) return set_error(ctx, ESDG_ERR_STATE, "learned scenarios without a network");
-    // The modal-sensor and the learned scenarios are disjoint (each pass writes its own scenarios'
-    // viscosities, marks and maxima): with both present the sensor pass runs on the second stream
-    // beside the indicator pass (not under per-launch profiling, whose events are on the main
-    // stream).
-    const bool overlap = nsens && nind && ctx->side && !ctx->profile;
-    if (overlap) {
-        (void)hipEventRecord(ctx->fork, ctx->stream);
-        (void)hipStreamWaitEvent(ctx->side, ctx->fork, 0);
+int StageBatch::prime(esdg_ctx* ctx, int src) {
+    {
+        KernelScope ks(ctx, "stage_mark");
+        k_stage_prime<<<1, 64, 0, ctx->stream>>>(d_scn, (int)host.size(), d_mark, d_mcount);
+        int rc = launch_check(ctx, "stage_prime");
+        if (rc) return rc;
     }
+    marks_used += 1;
     if (nsens) {
         KernelScope ks(ctx, "ens_sensor");
-        k_ens_sensor<3, 8><<<nsens, 256, 0, overlap ? ctx->side : ctx->stream>>>(d_scn, d_sens, src, d_mark, stage);
+        k_ens_sensor<3, 8><<<nsens, 256, 0, ctx->stream>>>(d_scn, d_sens, src, d_mark);
         int rc = launch_check(ctx, "ens_sensor");
         if (rc) return rc;
     }
-    if (overlap) (void)hipEventRecord(ctx->join, ctx->side);
-    if (nind) {
-        int rc = mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, stage, ind_lo, ind_hi, ind_audit,
-                                        d_icount);
-        if (rc) return rc;
-    }
-    if (overlap) (void)hipStreamWaitEvent(ctx->stream, ctx->join, 0);
+    primed = true;
     return ESDG_OK;
 }
 
@@ -1016,7 +1168,7 @@ int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipS
         for (int l = l0; l < l1; ++l) {
             L.ngl[l] = l == MARK_LISTS - 1 ? 8 : l + 3;
             L.list[l] = d_mlist + mfirst[l];
-            L.count[l] = d_mcount + MARK_STAGES * l;
+            L.count[l] = d_mcount + 2 * l;
             L.first[l] = n;
             L.blocks[l] = (int)std::min<int64_t>(cap, per_block(mfirst[l + 1] - mfirst[l], L.ngl[l]));
             n += L.blocks[l];
@@ -1030,13 +1182,13 @@ int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipS
         });
         if (n == 0) return ESDG_OK;
         KernelScope ks(ctx, "ens_grad");
-        k_ens_grad<3, 8><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, stage);
+        k_ens_grad<3, 8><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src);
         int rc = launch_check(ctx, "ens_grad");
         if (rc) return rc;
     }
     const auto [L, n] = lay_out(512, [](int64_t e, int ngl) { return (e * 4 * ngl + 255) / 256; });
     KernelScope ks(ctx, "ens_viscous_face");
-    k_ens_vface<<<n, 256, 0, st>>>(d_scn, L, l0, l1, d_mark, stage);
+    k_ens_vface<<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, d_mark, stage);
     return launch_check(ctx, "ens_viscous_face");
 }
 
@@ -1144,7 +1296,7 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
 
 int StageBatch::lambda(esdg_ctx* ctx, int src) {
     KernelScope ks(ctx, "stage_lambda");
-    k_stage_lambda<<<ntask, 64, 0, ctx->stream>>>(d_scn, d_task, src);
+    k_stage_lambda<<<std::min(ntask, 4096), 256, 0, ctx->stream>>>(d_scn, d_task, ntask, src);
     return launch_check(ctx, "stage_lambda");
 }
 
@@ -1179,18 +1331,18 @@ static void launch_ranges(hipStream_t st, const StageBatch& b, const StageBatch:
 
 int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src) {
     const int ns = (int)host.size();
-    if (has_av) {
-        // the step's marks, then the viscosity of the step's state (its maximum enters the dt)
-        KernelScope ks(ctx, "stage_mark");
-        k_stage_mark<<<1, 64, 0, ctx->stream>>>(d_mark, d_mcount);
-        int rc = launch_check(ctx, "stage_mark");
-        if (!rc) rc = av_pass(ctx, src, 0);
-        if (rc) return rc;
-    }
+    if (nind && !mlp) return set_error(ctx, ESDG_ERR_STATE, "learned scenarios without a network");
+    auto indicator = [&](int s) {
+        return mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit, d_icount);
+    };
+    // the learned scenarios' viscosity of the step's state (its maximum enters the dt; the others' is
+    // there already)
+    int rc = nind ? indicator(0) : ESDG_OK;
+    if (rc) return rc;
     {
         KernelScope ks(ctx, "stage_dt");
-        k_stage_dt<<<(ns + 63) / 64, 64, 0, ctx->stream>>>(d_scn, ns);
-        int rc = launch_check(ctx, "stage_dt");
+        k_stage_dt<<<(ns + 63) / 64, 64, 0, ctx->stream>>>(d_scn, ns, d_mark);
+        rc = launch_check(ctx, "stage_dt");
         if (rc) return rc;
     }
     for (int s = 0; s < stages; ++s) {
@@ -1199,21 +1351,14 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
             // the other scenarios on the second stream, the learned ones on the main stream
             (void)hipEventRecord(ctx->fork, ctx->stream);
             (void)hipStreamWaitEvent(ctx->side, ctx->fork, 0);
-            int rc = ESDG_OK;
-            if (s > 0 && nsens) {
-                k_ens_sensor<3, 8><<<nsens, 256, 0, ctx->side>>>(d_scn, d_sens, src, d_mark, s);
-                rc = launch_check(ctx, "ens_sensor");
-            }
-            if (!rc) rc = av_terms(ctx, src, s, 0, MARK_LISTS - 1, ctx->side);
+            rc = av_terms(ctx, src, s, 0, MARK_LISTS - 1, ctx->side);
             for (const Range& r : ranges)
                 if (!rc && !r.learned) {
                     launch_ranges<true>(ctx->side, *this, r, src, A[s], C[s], last, s);
                     rc = launch_check(ctx, "stage");
                 }
             (void)hipEventRecord(ctx->join, ctx->side);
-            if (!rc && s > 0)
-                rc = mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit,
-                                            d_icount);
+            if (!rc && s > 0) rc = indicator(s);
             if (!rc) rc = av_terms(ctx, src, s, MARK_LISTS - 1, MARK_LISTS, ctx->stream);
             for (const Range& r : ranges)
                 if (!rc && r.learned) {
@@ -1226,7 +1371,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
             continue;
         }
         if (has_av) {
-            int rc = (s > 0) ? av_pass(ctx, src, s) : ESDG_OK;
+            if (nind && s > 0) rc = indicator(s);
             if (!rc) rc = av_terms(ctx, src, s, 0, MARK_LISTS, ctx->stream);
             if (rc) return rc;
         }
@@ -1234,7 +1379,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
             KernelScope ks(ctx, "stage");
             if (has_av) launch_ranges<true>(ctx->stream, *this, r, src, A[s], C[s], last, s);
             else launch_ranges<false>(ctx->stream, *this, r, src, A[s], C[s], last, s);
-            int rc = launch_check(ctx, "stage");
+            rc = launch_check(ctx, "stage");
             if (rc) return rc;
         }
         src ^= 1;
@@ -1245,11 +1390,10 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
 int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src) {
     int n = 0;
     if (has_av) {
-        // marks advance by 8 per step: start them afresh long before the int would wrap
-        if (marks_used + (int64_t)steps + 2 > (int64_t)(1 << 27)) {
-            int rc = reset_marks(ctx);
-            if (rc) return rc;
-        }
+        // marks advance by STAGE_MARKS per step: start them afresh long before the int would wrap
+        int rc = marks_used + (int64_t)steps + 2 > (int64_t)(1 << 27) ? reset_marks(ctx) : ESDG_OK;
+        if (!rc && !primed) rc = prime(ctx, src);
+        if (rc) return rc;
         marks_used += steps;
     }
     if (sched.graph && !ctx->profile && steps >= 2) {

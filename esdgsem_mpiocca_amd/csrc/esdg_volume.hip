@@ -712,7 +712,7 @@ int fused_volume(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA, double 
         return set_error(ctx, ESDG_ERR_STATE, "fused_volume: viscous terms need the stage marks and element list");
     KernelScope ks(ctx, "fused_volume");
     if (tr && !slot) return set_error(ctx, ESDG_ERR_STATE, "fused_volume: side traces need the face slots");
-    ESDG_NGL_DISPATCH(ctx->p.ngl, launch_volume_fused, ctx, a, rk, rkA, cdt, fstar, Qt, Qv, SPV, tr, slot, active,
+    ESDG_FUSED_DISPATCH(ctx->p.ngl, launch_volume_fused, ctx, a, rk, rkA, cdt, fstar, Qt, Qv, SPV, tr, slot, active,
                       list, acount);
     return launch_check(ctx, "fused_volume");
 }

@@ -15,10 +15,10 @@
  *
  * Thread-safety: one context is used from one host thread at a time (the reference's one rank
  * per device).  All of a context's work is ordered on its stream, esdg_stream(ctx).  Some work
- * runs on a second stream that the context owns: with the learned indicator its pass beside the
- * face fluxes, and in a batched ensemble with both learned and modal-sensor scenarios the latter's
- * passes and stage launches.  That work is forked from and joined back into the main stream inside the same call,
- * so synchronising esdg_stream(ctx) (or esdg_finish) covers it.
+ * runs on a second stream that the context owns: in a batched ensemble with both learned and
+ * modal-sensor scenarios the latter's viscous passes and stage launches.  That work is forked from
+ * and joined back into the main stream inside the same call, so synchronising esdg_stream(ctx) (or
+ * esdg_finish) covers it.
  */
 #ifndef ESDG_H
 #define ESDG_H
@@ -236,9 +236,10 @@ typedef struct esdg_run_params {
     int positivity;               /* PositivityPreserving */
     int rk_order, rk_ssp;         /* rkorder (3 or 4), rkSSP */
     int flux_differencing;        /* FluxDifferencing */
-    int fused;                    /* 0: the reference's kernel sequence; 1: fused stage kernels;
-                                     2: single-kernel stage (2 <= N <= 7; with artificial viscosity
-                                     the sensor, gradient and viscous face passes run before it) */
+    int fused;                    /* 0: the reference's kernel sequence; 1: fused stage kernels (at
+                                     2 <= N <= 7 the single-kernel stage); 2: the single-kernel stage
+                                     (2 <= N <= 7; with artificial viscosity the gradient and viscous
+                                     face passes run before it) */
     int arrival_times;            /* calcArrivalTimes: buffer "ArrivalTimings" (fused 0 or 1) */
     int maximum_elevation;        /* calcMaximumElevation: buffer "MaximumElevation" (fused 0 or 1) */
 } esdg_run_params;
@@ -258,8 +259,8 @@ int esdg_solver_create(esdg_ctx* ctx, const esdg_inputs* in, const esdg_run_para
                        esdg_solver** out);
 /* DGtimeloop with a step cap: at most max_steps steps or until t >= T.  Returns steps taken
  * and the final time.  dt is computed on the device; the fused and single-kernel schedules keep
- * the clock there and read it back every 64 steps (the fused schedule reads dt back every step
- * when analysis buffers are on). */
+ * the clock there and read it back every 64 steps (at N = 1, 8 and 9 the fused schedule reads dt
+ * back every step when analysis buffers are on). */
 int esdg_solver_run(esdg_solver* s, int max_steps, int* steps_taken, double* t_out);
 int esdg_solver_get_q(esdg_solver* s, double* host_q);        /* blocking D2H copy of q */
 int esdg_solver_set_q(esdg_solver* s, const double* host_q);  /* blocking H2D copy, t = 0 */

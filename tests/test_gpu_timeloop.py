@@ -433,3 +433,46 @@ def test_lowest_degrees(dev, N, av, pos, fused):
     qg, ng, tg = run_gpu(dev, case, rp, 6, fused=fused)
     assert ng == no == 6 and abs(tg - to) <= 1e-12 * to
     assert max(fields_rel_l2(case, qg, qo)) <= 1e-12
+
+
+@pytest.mark.parametrize("av", [0, 1])
+@pytest.mark.parametrize("mesh", ["affine", "affine_flat", "curved"])
+@pytest.mark.parametrize("N", range(1, 10))
+def test_fused_every_degree_equals_sequence_bitwise(dev, N, mesh, av):
+    """Every degree of the fused schedule, and the single-kernel stage where it exists (2 <= N <= 7), on
+    metrics and slopes from element records (affine_flat), metrics from records and slopes per node
+    (affine), and everything per node (curved): state, time and the analysis buffers of 3 + 2 steps
+    (each call an odd number) equal the reference sequence's, bit for bit."""
+    if av and N == 1:
+        pytest.skip("the sensor's two top shells need modes below them")
+    if mesh == "curved":
+        case, kw = Case.dam_break(N=N, nel=6, noise=1e-3, seed=N), dict(num_flux=3, h_zero=1.5)
+    elif mesh == "affine":
+        case, kw = Case.gaussian_bump(N=N, nel=6), dict(num_flux=0, h_zero=1.0)
+    else:
+        case, kw = Case.ocean_uplift(N=N, nel=6), dict(num_flux=3, bc_kind=2, h_zero=4000.0)
+    q = case["q"].reshape(case.Nelem, 3, -1).copy()
+    q[:, 0] *= 1.0 + 1e-3 * np.random.default_rng(N).uniform(-1.0, 1.0, q[:, 0].shape)
+    case = case.with_state(q)
+    rp = RunParams(artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05, arrival_times=1,
+                   maximum_elevation=1, **kw)
+    size = case.Nelem * case.ngl ** 2
+    outs = []
+    for fused in (0, 1, 2):
+        if fused == 2 and not 2 <= N <= 7:
+            continue
+        r = RunParams(**{**vars(rp), "arrival_times": int(fused < 2), "maximum_elevation": int(fused < 2)})
+        ctx = dev.Context(dev.make_params(case, r))
+        try:
+            s = dev.Solver(ctx, case, r, fused=fused)
+            n = s.run(3)[0] + s.run(2)[0]
+            extra = [s.view(b, size).download() for b in ("ArrivalTimings", "MaximumElevation")] if fused < 2 else []
+            outs.append((n, s.time(), s.get_q(), *extra))
+            s.close()
+        finally:
+            ctx.close()
+    ref = outs[0]
+    assert ref[0] == 5 and np.isfinite(ref[2]).all()
+    for o in outs[1:]:
+        assert o[:2] == ref[:2]
+        assert all(np.array_equal(a, b) for a, b in zip(o[2:], ref[2:]))
