@@ -743,14 +743,8 @@ int esdg_solver_indicator_counts(esdg_solver* s, int64_t* viscous, int64_t* fals
                                  int64_t* not_smooth, int64_t* element_stages) {
     if (!s) return set_error(nullptr, ESDG_ERR_ARG, "esdg_solver_indicator_counts: null solver");
     deviceclass& d = s->dc;
-    unsigned long long c[5] = {0, 0, 0, 0, 0};
-    unsigned long long* ic = d.stage_.d_icount;
-    if (ic) {
-        int rc = esdg_memcpy(d.ctx_, c, ic, sizeof c, ESDG_D2H);
-        if (!rc) rc = esdg_fill(d.ctx_, reinterpret_cast<double*>(ic), 0.0, 5);
-        if (!rc) rc = esdg_finish(d.ctx_);
-        if (rc) return rc;
-    }
+    unsigned long long c[5];
+    if (int rc = d.stage_.take_counts(d.ctx_, c)) return rc;
     if (viscous) *viscous = (int64_t)c[0];
     if (false_negatives) *false_negatives = (int64_t)c[1];
     if (sensor_positives) *sensor_positives = (int64_t)c[2];

@@ -305,8 +305,8 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
     };
     rc = copy_all(true);
     // the learned indicator's counts are restored after the trials as well
-    unsigned long long icount[5] = {0, 0, 0, 0, 0};
-    if (!rc && E->batch.d_icount) rc = esdg_memcpy(ctx, icount, E->batch.d_icount, sizeof icount, ESDG_D2H);
+    unsigned long long icount[5] = {0, 0, 0, 0, 0}, dropped[5];
+    if (!rc) rc = E->batch.take_counts(ctx, icount);
     const int src0 = E->src;
     const StageSchedule keep = E->batch.sched;
     StageSchedule best_s = keep;
@@ -352,6 +352,7 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
         trial(s);
     }
     esdg_free(ctx, snap);
+    if (!rc) rc = E->batch.take_counts(ctx, dropped);
     if (!rc && E->batch.d_icount) rc = esdg_memcpy(ctx, E->batch.d_icount, icount, sizeof icount, ESDG_H2D);
     if (!rc) rc = E->batch.set_schedule(ctx, best_s);
     if (rc) return rc;
@@ -375,13 +376,8 @@ int esdg_ensemble_indicator_audit(esdg_ensemble* E, int audit) {
 int esdg_ensemble_indicator_counts(esdg_ensemble* E, int64_t* viscous, int64_t* false_negatives,
                                    int64_t* sensor_positives, int64_t* not_smooth, int64_t* element_stages) {
     if (!E) return set_error(nullptr, ESDG_ERR_ARG, "esdg_ensemble_indicator_counts: null ensemble");
-    unsigned long long c[5] = {0, 0, 0, 0, 0};
-    if (E->batch.d_icount) {
-        int rc = esdg_memcpy(E->ctx, c, E->batch.d_icount, sizeof c, ESDG_D2H);
-        if (!rc) rc = esdg_fill(E->ctx, reinterpret_cast<double*>(E->batch.d_icount), 0.0, 5);
-        if (!rc) rc = esdg_finish(E->ctx);
-        if (rc) return rc;
-    }
+    unsigned long long c[5];
+    if (int rc = E->batch.take_counts(E->ctx, c)) return rc;
     if (viscous) *viscous = (int64_t)c[0];
     if (false_negatives) *false_negatives = (int64_t)c[1];
     if (sensor_positives) *sensor_positives = (int64_t)c[2];

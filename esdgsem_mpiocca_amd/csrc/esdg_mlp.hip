@@ -256,13 +256,14 @@ struct MaskedSensor {
 // LDS holds the feature pass's tiles (V, the modal coefficients, the row reductions); once the
 // sensor's energy sums are taken from the coefficients, the two 16-row BF16 feature tiles and the
 // hidden activations take their place.  The network's weights are read from global memory (8 KB,
-// cached), not staged per block: about 22 KB of LDS per block, 7 blocks per CU.
+// cached), not staged per block: about 22 KB of LDS per block, 7 blocks per CU.  At 65536 elements the
+// features and the network take 23 us and the whole pass 35: the ramp and the sums run in few wavefronts,
+// the marks a side per thread, the counts in IND_SLOTS copies (58 us with the ramp in every wavefront,
+// an element's marks in sequence from E2E and EdgeData, and all blocks' counts on one copy).
 __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __restrict__ q,
                                     gptr<const double> __restrict__ B, gptr<const double> __restrict__ V,
                                     const MlpDev& W, float lo, float hi,
                                     float* __restrict__ p, const MaskedSensor& MS) {
-    if (MS.counters && threadIdx.x == 0)
-        atomicAdd(MS.counters + 4, (unsigned long long)min(FEPB, Nelem - e0));
     __shared__ __attribute__((aligned(16))) FeatLds L;
     __shared__ float sZ[2][16];
     __shared__ signed char sSt[FEPB];
@@ -276,8 +277,10 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
     float xn[8], modal;
     row_features(q, B, L, e, act, xn, modal);
     // row_features leaves the squares of the modal coefficients m = V (h + b) V^T in L.T: the
-    // sensor's sums
-    if (MS.visc && act && r < 4) sSum[el][r] = sensor_sum<8, FRS, true>(L.T + el * FES, r);
+    // sensor's sums, one of the four per wave and an element per lane (with the four on an element's own
+    // lanes every wave ran all four chains of additions in turn)
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    if (MS.visc && l < FEPB && e0 + l < Nelem) sSum[l][w] = sensor_sum<8, FRS, true>(L.T + l * FES, w);
     __syncthreads();   // L.T is free
     uint16_t* sX = reinterpret_cast<uint16_t*>(L.T);   // [2][16][KP]
     uint16_t* sH = sX + 2 * 16 * KP;                   // [2][16][NH]
@@ -289,7 +292,6 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
         for (int k = NIN + r; k < KP; k += 8) row[k] = 0;   // the K padding of layer 1
     }
     __syncthreads();
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     if (w < 2) {
         mlp_tile(sX + w * 16 * KP, sH + w * 16 * NH, W.W1T, W.W2T, W.w3, W.bias, W.bias + NH, W.bias[2 * NH], sZ[w]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -307,7 +309,8 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
         if (threadIdx.x < 4) sCnt[threadIdx.x] = 0ull;
         if (threadIdx.x == 4) sMax = 0ull;
         __syncthreads();   // the classes are in sSt
-        if (act && r == 0) {
+        if ((int)threadIdx.x < FEPB && e0 + (int)threadIdx.x < Nelem) {   // an element per lane of one wave
+            const int el = threadIdx.x, e = e0 + el;
             double v = sensor_ramp(sSum[el][0], sSum[el][1], sSum[el][2], sSum[el][3], MS.sc);
             const int st = sSt[el];
             const double plain = v;
@@ -320,19 +323,24 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
             }
             glob(MS.visc)[e] = v;
             if (MS.visc_plot) glob(MS.visc_plot)[e] = v;
-            if (v != 0.0) mark_reach(*MS.scn, e, MS.mark, MS.buffer);
+            sSt[el] = v != 0.0;
             // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
             if (MS.stage == 0 && v > 0.0) atomicMax(&sMax, (unsigned long long)__double_as_longlong(v));
         }
-        const bool to_max = MS.stage == 0;
-        if (MS.counters || to_max) {
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                if (MS.counters)
-                    for (int k = 0; k < 4; ++k)
-                        if (sCnt[k]) atomicAdd(MS.counters + k, sCnt[k]);
-                if (to_max && sMax) atomicMax(MS.scn->emax, sMax);
+        __syncthreads();
+        // the elements with viscosity mark what they reach, a side per thread
+        if (threadIdx.x < 4 * FEPB) {
+            const int el = threadIdx.x >> 2, e = e0 + el;
+            if (e < Nelem && sSt[el]) {
+                const int sd = threadIdx.x & 3;
+                mark_side(*MS.scn, e, sd, side_record(*MS.scn, e, sd), MS.mark, MS.buffer);
             }
+        } else if (threadIdx.x < 4 * FEPB + 5) {
+            const int k = threadIdx.x - 4 * FEPB;
+            const unsigned long long c = k < 4 ? sCnt[k] : (unsigned long long)min(FEPB, Nelem - e0);
+            if (MS.counters && c) atomicAdd(MS.counters + k, c);
+        } else if (threadIdx.x == 4 * FEPB + 5) {
+            if (MS.stage == 0 && sMax) max_into(MS.scn->emax, __longlong_as_double((long long)sMax));
         }
     }
 }
@@ -359,7 +367,9 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
     MS.visc_plot = S.visc_plot;
     MS.sc = S.sc;
     MS.audit = audit;
-    MS.counters = counters;
+    // each block adds to one of IND_SLOTS copies of the counts (all blocks' atomics on one copy queued up
+    // for 20 us at 65536 elements)
+    MS.counters = counters + 8 * (blockIdx.x % IND_SLOTS);
     MS.scn = &S;
     // (the step's first viscosity comes before its marks are advanced)
     MS.mark = *mark + (stage == 0 ? STAGE_MARKS : stage);

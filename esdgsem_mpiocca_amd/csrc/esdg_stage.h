@@ -72,26 +72,38 @@ struct StageTask {
     int scn, e0, ngl, pad;
 };
 
+// max of a non-negative double into a cell (non-negative doubles order as their bit patterns).  Most blocks
+// find a larger value there already and leave the cell alone: atomics of all blocks on one cell queue
+// up at about 12 ns each.
+__device__ __forceinline__ void max_into(unsigned long long* cell, double m) {
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    if (bits > __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(cell, bits);
+}
+
 // An element with viscosity in the state of buffer b marks itself and its face neighbours for the stage that
 // starts from it (the elements whose viscous terms can be non-zero), as the fused face pass does for both
 // elements of every face with viscosity on either side.  The first to mark an element also lists it.
 __device__ __forceinline__ void mark_element(const StageScn& S, int k, int m, int b) {
     if (atomicExch(S.active[b] + k, m) != m) S.mlist[atomicAdd(S.mcount + b, 1)] = make_int2(S.id, k);
 }
-__device__ __forceinline__ void mark_reach(const StageScn& S, int e, int m, int b) {
-    auto mark = [&](int k) { mark_element(S, k, m, b); };
-    mark(e);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const gptr<const int> E = glob(S.EdgeData) + 8 * (int64_t)(glob(S.E2E)[e * 4 + s] - 1);
-        if (E[5] == 0) mark(E[0]);
-        if (E[6] == 0) mark(E[1]);
-    }
+// Side `side` of element e (record R, StageScn::srec): the neighbour there, and with side 0 the element itself.
+__device__ __forceinline__ void mark_side(const StageScn& S, int e, int side, const int4& R, int m, int b) {
+    const int cpuL = (int)(((unsigned)R.w >> 8) & 255u) - 2, cpuR = (int)(((unsigned)R.w >> 16) & 255u) - 2;
+    if (side == 0) mark_element(S, e, m, b);
+    if (cpuL == 0 && R.y != e) mark_element(S, R.y, m, b);
+    if (cpuR == 0 && R.z != e) mark_element(S, R.z, m, b);
+}
+__device__ __forceinline__ int4 side_record(const StageScn& S, int e, int side) {
+    // one 16-byte load (a vector type: int4's assignment would take a generic reference)
+    using i4v = int __attribute__((ext_vector_type(4)));
+    const i4v v = ((gptr<const i4v>)glob(S.srec))[(int64_t)e * 4 + side];
+    return make_int4(v.x, v.y, v.z, v.w);
 }
 
 // The mark of a stage: the step's base (advanced by STAGE_MARKS at each step, on the device, so that
 // replays of a captured step take fresh marks) plus the stage.
 constexpr int STAGE_MARKS = 8;
+constexpr int IND_SLOTS = 64;
 
 // The marked-element lists of a batch: one for the modal-sensor scenarios of each degree (ngl - 3)
 // and one for the learned ones (MARK_LISTS - 1).  A pass over them takes, of each list, the blocks
@@ -162,7 +174,9 @@ class StageBatch {
     // indicator overlaps the other scenarios' stage.  Their marked elements are in lists of their own.
     bool split = false;
     int* d_mark = nullptr;
-    unsigned long long* d_icount = nullptr;        // learned indicator counts (5, as the solver's)
+    // the learned indicator's 5 counts: IND_SLOTS copies, 8 words apart, to be added
+    unsigned long long* d_icount = nullptr;
+    int take_counts(esdg_ctx* ctx, unsigned long long c[5]);   // since the last call
     const esdg_mlp* mlp = nullptr;
     float ind_lo = 0.5f, ind_hi = 0.5f;
     int ind_audit = 0;

@@ -46,14 +46,6 @@ struct MaxLds<HI, HI> {
     static constexpr int value = StageCfg<HI>::LDS;
 };
 
-// max of a non-negative double into a cell (non-negative doubles order as their bit patterns).  Most blocks
-// find a larger value there already and leave the cell alone: atomics of all blocks on one cell queue
-// up at about 12 ns each.
-__device__ __forceinline__ void max_into(unsigned long long* cell, double m) {
-    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
-    if (bits > __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(cell, bits);
-}
-
 // Volume term, surface lift, RK update, limiter and wave speed of one block of elements; the
 // face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
 // parameters are __restrict__ so that the geometry loads schedule as in a kernel taking them as
@@ -479,15 +471,9 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 glob(SV->visc)[e] = eps;
                 if (SV->visc_plot) glob(SV->visc_plot)[e] = eps;
             }
-            // mark_reach by the element's lanes, a side each
+            // the marks of an element with viscosity, a side per lane
             if (__shfl(eps, lane - r) != 0.0 && act) {
-                for (int s = r; s < 4; s += NGL) {
-                    const int4 R4 = rec[s];
-                    const int cpuL = (int)(((unsigned)R4.w >> 8) & 255u) - 2, cpuR = (int)(((unsigned)R4.w >> 16) & 255u) - 2;
-                    if (s == 0) mark_element(*SV, e, next_mark, src ^ 1);
-                    if (cpuL == 0 && R4.y != e) mark_element(*SV, R4.y, next_mark, src ^ 1);
-                    if (cpuR == 0 && R4.z != e) mark_element(*SV, R4.z, next_mark, src ^ 1);
-                }
+                for (int s = r; s < 4; s += NGL) mark_side(*SV, e, s, rec[s], next_mark, src ^ 1);
             }
             if (last) {
                 // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
@@ -528,12 +514,7 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     for (int j = 0; j < FPL; ++j) {
         const int sd = r + j * NGL;
         rec[j] = make_int4(0, 0, 0, 0);
-        if (act && sd < 4) {
-            // one 16-byte load (a vector type: int4's assignment would take a generic reference)
-            using i4v = int __attribute__((ext_vector_type(4)));
-            const i4v v = ((gptr<const i4v>)glob(S.srec))[(int64_t)e * 4 + sd];
-            rec[j] = make_int4(v.x, v.y, v.z, v.w);
-        }
+        if (act && sd < 4) rec[j] = side_record(S, e, sd);
     }
     int4* RS = reinterpret_cast<int4*>(P + C::ESZ);
     auto early = [&]() {
@@ -786,7 +767,8 @@ __device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int s
     if (el < RowBlock<NGL>::EPB && e < S.Nelem && r == 0) {
         glob(S.visc)[e] = v;
         if (S.visc_plot) glob(S.visc_plot)[e] = v;
-        if (v != 0.0) mark_reach(S, e, m, src);
+        if (v != 0.0)
+            for (int s = 0; s < 4; ++s) mark_side(S, e, s, side_record(S, e, s), m, src);
         // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
         if (v > 0.0) atomicMax(sMax, (unsigned long long)__double_as_longlong(v));
     }
@@ -1052,9 +1034,9 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
     if (!rc) rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (!rc && has_av) {
         rc = esdg_malloc(ctx, (void**)&d_mark, 64);
-        if (!rc) rc = esdg_malloc(ctx, (void**)&d_icount, 5 * sizeof(unsigned long long));
+        if (!rc) rc = esdg_malloc(ctx, (void**)&d_icount, 8 * IND_SLOTS * sizeof(unsigned long long));
         if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_mark), 0.0, 8);
-        if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_icount), 0.0, 5);
+        if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_icount), 0.0, 8 * IND_SLOTS);
         if (!rc) rc = build_av_tasks(ctx);
     }
     if (!rc) rc = set_schedule(ctx, StageSchedule{});
@@ -1106,6 +1088,18 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     };
     int rc = put(sens, d_sens, nsens);
     if (!rc) rc = put(ind, d_ind, nind);
+    return rc;
+}
+
+int StageBatch::take_counts(esdg_ctx* ctx, unsigned long long c[5]) {
+    for (int k = 0; k < 5; ++k) c[k] = 0;
+    if (!d_icount) return ESDG_OK;
+    unsigned long long all[8 * IND_SLOTS];
+    int rc = esdg_memcpy(ctx, all, d_icount, sizeof all, ESDG_D2H);
+    if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_icount), 0.0, 8 * IND_SLOTS);
+    if (!rc) rc = esdg_finish(ctx);
+    for (int i = 0; i < IND_SLOTS && !rc; ++i)
+        for (int k = 0; k < 5; ++k) c[k] += all[8 * i + k];
     return rc;
 }
 

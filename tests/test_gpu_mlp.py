@@ -218,3 +218,34 @@ def test_loss_gradient_batch_sizes(dev, state, n):
                  (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.NPARAM)):
         scale = np.abs(go[a:b]).max()
         assert np.abs(g[a:b] - go[a:b]).max() <= 2e-3 * scale + 1e-9, (a, np.abs(g[a:b] - go[a:b]).max(), scale)
+
+
+@pytest.mark.parametrize("nel", [2, 5, 6, 12])
+def test_learned_indicator_element_tiles(dev, nel):
+    """With lo = 0 no element is smooth, so the network's pass gives every element the modal sensor's value: the
+    run equals the one without a network bit for bit, marks and viscosity maximum included, on meshes of
+    part of a 32-element tile, one tile and a remainder, and whole tiles with a remainder."""
+    case = Case.dam_break(N=7, nel=nel, noise=1e-3, seed=nel)
+    rp = RunParams(num_flux=3, artificial_viscosity=1, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+    outs = []
+    for learned in (False, True):
+        ctx = dev.Context(dev.make_params(case, rp))
+        try:
+            s = dev.Solver(ctx, case, rp, fused=1)
+            net = dev.MLP(ctx, seed=1) if learned else None
+            if learned:
+                s.set_indicator(net, 0.0, 1.0)
+                s.indicator_audit(True)
+            n, t = s.run(5)
+            outs.append((n, t, s.get_q()))
+            if learned:
+                c = s.indicator_counts()
+                assert c["element_stages"] == c["not_smooth"] == 25 * case.Nelem
+                assert c["false_negatives"] == 0 and 0 < c["viscous"] == c["sensor_positives"]
+            s.close()
+            if net:
+                net.close()
+        finally:
+            ctx.close()
+    assert outs[0][:2] == outs[1][:2]
+    assert np.array_equal(outs[0][2], outs[1][2])
