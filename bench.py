@@ -90,7 +90,8 @@ KERNELS = ["volume_kernel", "collect_edge_data", "calc_num_fluxes", "surface_ker
            "volume_kernel_viscose", "calc_num_fluxes_viscose", "surface_kernel_visc",
            "find_lambda_max", "reduce_max", "pos_pres", "fused_face", "fused_volume", "fused_av",
            "fused_viscous_face", "fused_clock", "mlp_indicator", "write_traces", "stage", "stage_dt", "stage_lambda",
-           "stage_mark", "ens_sensor", "ens_indicator", "ens_grad", "ens_viscous_face"]
+           "stage_mark", "ens_sensor", "ens_indicator", "ens_grad", "ens_viscous_face", "sequence_faces",
+           "sequence_gradient", "sequence_viscous_faces", "sequence_volume"]
 
 
 def c1_params(RunParams):
@@ -644,14 +645,17 @@ def main():
         v["share"] = v["total_ms"] / gpu_ms if gpu_ms else None
 
     on_stage = 3 <= case.ngl <= 8
-    vol_name = ("stage" if on_stage else "fused_volume") if args.fused else "volume_kernel"
+    vol_name = ("stage" if on_stage else "fused_volume") if args.fused else "sequence_volume"
     roofline = None
     if vol_name in per_kernel:
         avg_s = per_kernel[vol_name]["avg_us"] * 1e-6
         # this workload's viscosity is the modal sensor alone, which the fused schedule evaluates
         # inside the state update
         if not args.fused:
-            alg = volume_bytes(case.Nelem, case.ngl)
+            # the update pass with Qt stored and every element's viscous terms read
+            av = 1 if rp.artificial_viscosity else 0
+            alg = (fused_volume_bytes(case.Nelem, case.ngl, av, False, limiter=bool(rp.positivity)) +
+                   8 * case.Nelem * ((3 + 2 * av) * case.ngl ** 2 + 8 * av * case.ngl))
         elif on_stage:
             alg = stage_bytes(case.Nelem, case.ngl, sensor=bool(rp.artificial_viscosity), stages=5)
         else:

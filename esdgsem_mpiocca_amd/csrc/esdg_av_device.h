@@ -16,13 +16,16 @@
 namespace esdg {
 
 // Face states of face f as CollectEdgeData stores them into qL / qR, read from the face slots of
-// the side-trace buffer or straight from the state.
+// the side-trace buffer or straight from the state.  store: the scaled gradients at the element's nodes
+// (nothing but their side traces is kept here).
 struct TraceFromSides {
     const double* tr;
     __device__ __forceinline__ FaceState operator()(int ngl, int f, const int* E, bool left, int k, double nx,
                                                     double ny, const GatherConsts& gc, double bl, double br) const {
         return gathered_tr(tr, ngl, f, E, left, k, nx, ny, gc, bl, br);
     }
+    template <int NN>
+    __device__ __forceinline__ void store(int, int, double, double, double, double) const {}
 };
 struct TraceFromState {
     const double* q;
@@ -30,6 +33,8 @@ struct TraceFromState {
                                                     const GatherConsts& gc, double bl, double br) const {
         return gathered(q, ngl, E, left, k, nx, ny, gc, bl, br);
     }
+    template <int NN>
+    __device__ __forceinline__ void store(int, int, double, double, double, double) const {}
 };
 
 // calcNumFluxesGradient.okl:16-135 at face node i: the BR1 face fluxes of u and v (x and y parts)
@@ -70,30 +75,47 @@ struct AvMesh {
 // fluxes of the element's sides), scaled by h, its side traces, and the viscous volume term
 // Qv = J^-1 Dstrong (eps J grad) in the contravariant form.  Called by every thread of the block;
 // act = whether this thread's element takes part, eps its viscosity.  LDS: sDh, sDs (ngl^2), and
-// sA, sB, sC, sE (EPB ngl^2 each), sEps (EPB); the call ends with the LDS free.
+// sA, sB, sC, sE (EPB ngl^2 each), sF (EPB 16 ngl), sEps (EPB); the call ends with the LDS free.  Every load
+// is issued before the first barrier: the side fluxes' chain of dependent loads (ElemToEdge, face, traces)
+// runs once, beside those of the state and the metrics.
 template <int NGL, class Src>
 __device__ __forceinline__ void av_element_block(const AvMesh& M, const Src& src, int e, bool act, double eps,
                                                  const double* sDh, const double* sDs, double* sA, double* sB,
-                                                 double* sC, double* sE, double* sEps) {
+                                                 double* sC, double* sE, double* sF, double* sEps) {
     constexpr int NN = NGL * NGL;
     const int el = threadIdx.x / NN, n = threadIdx.x % NN;
     if (act && n == 0) sEps[el] = eps;
     const int a = n % NGL, c = n / NGL;
     const int64_t xid = (int64_t)e * NN + n;
     double h = 0.0, hu = 0.0, hv = 0.0;
+    double ye = 0.0, yx = 0.0, xe = 0.0, xx = 0.0, rJ = 0.0;
     if (act) {
         const int64_t id = (int64_t)e * NN * ESDG_NEQ + n;
         h = M.q[id]; hu = M.q[id + NN]; hv = M.q[id + 2 * NN];
         const double Qinv = (h > M.tol) ? 1.0 / h : 0.0;
         sB[threadIdx.x] = hu * Qinv;                // u at node n
         sC[threadIdx.x] = hv * Qinv;                // v at node n
+        ye = M.Yeta[xid]; yx = M.Yxi[xid]; xe = M.Xeta[xid]; xx = M.Xxi[xid]; rJ = M.Jac[xid];
+        // the BR1 face fluxes of the element's side nodes, each by one thread
+        for (int m = n; m < 4 * NGL; m += NN) {
+            const int side = m / NGL, t = m % NGL;
+            const int ifa = M.E2E[e * 4 + side] - 1;
+            const int rev = M.EOR[e * 4 + side];
+            const int ms = M.EMS[e * 4 + side];
+            const int inc = rev * t + (1 - rev) * (NGL - 1 - t);
+            const int64_t fn = (int64_t)ifa * NGL + inc;
+            const Br1Flux F = br1_face_flux(src, NGL, ifa, M.ED + 8 * (int64_t)ifa, inc, M.nx[fn], M.ny[fn], M.scal[fn],
+                                            M.bL[fn], M.bR[fn], M.gc, M.tol, M.geomFace);
+            double* f = sF + el * 16 * NGL + side * 4 * NGL + t;
+            f[0] = ms * F.x0; f[NGL] = ms * F.x1;
+            f[2 * NGL] = ms * F.y0; f[3 * NGL] = ms * F.y1;
+        }
     }
     __syncthreads();
     // ---- BR1 gradient (weak form volume part) ----
     const double* u = sB + el * NN;
     const double* v = sC + el * NN;
     double gx0 = 0.0, gx1 = 0.0, gy0 = 0.0, gy1 = 0.0;
-    double ye = 0.0, yx = 0.0, xe = 0.0, xx = 0.0, rJ = 0.0;
     if (act) {
         double u_xi = 0.0, u_eta = 0.0, v_xi = 0.0, v_eta = 0.0;
 #pragma unroll
@@ -103,39 +125,26 @@ __device__ __forceinline__ void av_element_block(const AvMesh& M, const Src& src
             v_xi += sDh[a * NGL + l] * v[c * NGL + l];
             v_eta += sDh[c * NGL + l] * v[l * NGL + a];
         }
-        ye = M.Yeta[xid]; yx = M.Yxi[xid]; xe = M.Xeta[xid]; xx = M.Xxi[xid]; rJ = M.Jac[xid];
         const double u_x = ye * u_xi - yx * u_eta;
         const double v_x = ye * v_xi - yx * v_eta;
         const double u_y = -xe * u_xi + xx * u_eta;
         const double v_y = -xe * v_xi + xx * v_eta;
         gx0 = rJ * u_x; gx1 = rJ * v_x; gy0 = rJ * u_y; gy1 = rJ * v_y;
-        // surface lift of the BR1 face fluxes: sides 0/2 first, then 1/3 (SurfaceKernelGradient.okl)
-#pragma unroll
-        for (int ph = 0; ph < 2; ++ph) {
-            int side = -1, t = 0;
-            if (ph == 0) {
-                if (c == 0) { side = 0; t = a; }
-                else if (c == NGL - 1) { side = 2; t = a; }
-            } else {
-                if (a == NGL - 1) { side = 1; t = c; }
-                else if (a == 0) { side = 3; t = c; }
-            }
-            if (side < 0) continue;
-            const int ifa = M.E2E[e * 4 + side] - 1;
-            const int rev = M.EOR[e * 4 + side];
-            const int ms = M.EMS[e * 4 + side];
-            const int inc = rev * t + (1 - rev) * (NGL - 1 - t);
-            const int64_t fn = (int64_t)ifa * NGL + inc;
-            const Br1Flux F = br1_face_flux(src, NGL, ifa, M.ED + 8 * (int64_t)ifa, inc, M.nx[fn], M.ny[fn], M.scal[fn],
-                                            M.bL[fn], M.bR[fn], M.gc, M.tol, M.geomFace);
-            if (ph == 0) gx0 += ms * F.x0 * rJ;
-            else gx0 += ms * rJ * F.x0;
-            gx1 += ms * rJ * F.x1;
-            gy0 += ms * rJ * F.y0;
-            gy1 += ms * rJ * F.y1;
-        }
+        // surface lift of the BR1 face fluxes: sides 0/2 first, then 1/3 (SurfaceKernelGradient.okl); sF
+        // holds ms F (ms = +-1, so the sign is exact wherever it is applied)
+        const double* F = sF + el * 16 * NGL;
+        auto lift = [&](int side, int t) {
+            const double* f = F + side * 4 * NGL + t;
+            gx0 += f[0] * rJ; gx1 += f[NGL] * rJ;
+            gy0 += f[2 * NGL] * rJ; gy1 += f[3 * NGL] * rJ;
+        };
+        if (c == 0) lift(0, a);
+        else if (c == NGL - 1) lift(2, a);
+        if (a == NGL - 1) lift(1, c);
+        else if (a == 0) lift(3, c);
         // scaleGradient: multiply by h
         gx0 = h * gx0; gx1 = h * gx1; gy0 = h * gy0; gy1 = h * gy1;
+        src.template store<NN>(e, n, gx0, gx1, gy0, gy1);
         // side traces of the scaled gradients, [e][side][gX0, gX1, gY0, gY1][k] (k in the side's order)
         double* T = M.gtr + (int64_t)e * 16 * NGL;
         auto put = [&](int side, int k) {

@@ -15,6 +15,7 @@
 #include "esdg_fused.h"
 #include "esdg_internal.h"
 #include "esdg_mlp_internal.h"
+#include "esdg_sequence.h"
 #include "esdg_stage.h"
 
 namespace esdg {
@@ -50,11 +51,15 @@ class deviceclass {
         I(&o_ElemEdgeOrientation, (size_t)Nelem * 4);
         if (rp.artificial_viscosity) {
             A(&o_qGradientX, nodes * 2); A(&o_qGradientY, nodes * 2);
-            A(&o_SurfGradientX, fn * 2); A(&o_SurfGradientY, fn * 2);
-            A(&o_qGradientXL, fn * 2); A(&o_qGradientXR, fn * 2);
-            A(&o_qGradientYL, fn * 2); A(&o_qGradientYR, fn * 2);
             A(&o_SurfacePartsVisc, fn * 2);
-            A(&o_ViscParaL, Nfaces); A(&o_ViscParaR, Nfaces);
+            if (fewer_passes()) {
+                A(&o_gtr, (size_t)Nelem * 16 * ngl); A(&o_Qv, nodes * 2);
+            } else if (rp.fused == 0) {
+                A(&o_SurfGradientX, fn * 2); A(&o_SurfGradientY, fn * 2);
+                A(&o_qGradientXL, fn * 2); A(&o_qGradientXR, fn * 2);
+                A(&o_qGradientYL, fn * 2); A(&o_qGradientYR, fn * 2);
+                A(&o_ViscParaL, Nfaces); A(&o_ViscParaR, Nfaces);
+            }
         }
         // analysis buffers (src/deviceclass.cpp:324-342): arrival times start at 1000.0, maximum
         // elevations at 0
@@ -114,6 +119,15 @@ class deviceclass {
     // 512, N = 7, with viscosity 3.73 ms on the passes and 3.26 on the stage kernel, at 301 x 223, N = 4, with
     // viscosity 685 and 505 us, at 93 x 71, N = 5, without 115 and 94.
     bool element_stage() const { return rp_.fused == 2 || (rp_.fused == 1 && ngl >= 3 && ngl <= 8); }
+
+    // The kernel sequence in fewer passes (esdg_sequence.hip): flux differencing, a low-storage RK, boundaries
+    // without the time or the node positions.  Per step at 160 x 160, N = 7, with viscosity 0.92 ms and kernel
+    // by kernel 1.75; at 16 x 16, N = 4, without 102 and 170 us.
+    bool fewer_passes() const {
+        const int bc = ctx_->p.bc_kind;
+        return rp_.fused == 0 && rp_.flux_differencing && !rp_.rk_ssp &&
+               (bc == ESDG_BC_WALLS || bc == ESDG_BC_INNER_OUTER || bc == ESDG_BC_OCEAN);
+    }
 
     // buildDeviceKernels (src/deviceclass.cpp:349-544): kernels are compiled ahead of time; here the
     // run flags are checked against what is implemented.
@@ -198,6 +212,13 @@ class deviceclass {
 
     // The reference's kernel sequence for one RK stage (src/deviceclass.cpp:938-1126).
     int stage(int s, double dt) {
+        if (fewer_passes()) {
+            const SequenceArgs a = sequence_args();
+            int rc = sequence_faces(ctx_, a);
+            if (!rc && rp_.artificial_viscosity && s > 0) rc = viscosity();
+            if (!rc) rc = sequence_update(ctx_, a, A[s], Cc[s] * dt);
+            return rc;
+        }
         int rc = esdg_collect_edge_data(ctx_, Nfaces, o_EdgeData, o_q, o_x, o_y, o_nx, o_ny, o_bL, o_bR, o_qL, o_qR,
                                         t + (rp_.rk_ssp ? rkD[s] : Bc[s]) * dt);
         if (rc) return rc;
@@ -491,14 +512,31 @@ class deviceclass {
             if (p) esdg_free(ctx_, p);
         fused_.release(ctx_);
         stage_.release(ctx_);
-        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_gtr,
+        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_gtr, (void*)o_Qv,
                         (void*)o_active[0], (void*)o_active[1], (void*)o_emax})
             if (p) esdg_free(ctx_, p);
-        o_q2 = o_clock = o_gtr = nullptr;
+        o_q2 = o_clock = o_gtr = o_Qv = nullptr;
         o_lmax = o_emax = nullptr;
         o_active[0] = o_active[1] = nullptr;
         o_q = o_Qt = o_gRK = o_Qtmp = nullptr;
         return ESDG_OK;
+    }
+
+    SequenceArgs sequence_args() {
+        SequenceArgs a;
+        a.Nelem = Nelem; a.Nfaces = Nfaces;
+        a.artificial_viscosity = rp_.artificial_viscosity; a.positivity = rp_.positivity;
+        a.q = o_q; a.gRK = o_gRK; a.Qt = o_Qt;
+        a.Jac = o_Jac; a.Yxi = o_Yxi; a.Yeta = o_Yeta; a.Xxi = o_Xxi; a.Xeta = o_Xeta;
+        a.Bx = o_Bx; a.By = o_By; a.D = o_D; a.Dhat = o_Dhat; a.Dstrong = o_Dstrong;
+        a.GLw = o_GLw; a.EleSizes = o_EleSizes;
+        a.nx = o_nx; a.ny = o_ny; a.scal = o_scal; a.bL = o_bL; a.bR = o_bR; a.ViscPara = o_ViscPara;
+        a.EdgeData = o_EdgeData; a.EdgeReversed = o_EdgeReversed; a.ElemToEdge = o_ElemToEdge;
+        a.EMS = o_ElemEdgeMasterSlave; a.EOR = o_ElemEdgeOrientation;
+        a.qL = o_qL; a.qR = o_qR; a.SurfaceParts = o_SurfaceParts;
+        a.qGradientX = o_qGradientX; a.qGradientY = o_qGradientY; a.SurfacePartsVisc = o_SurfacePartsVisc;
+        a.gtr = o_gtr; a.Qv = o_Qv;
+        return a;
     }
 
     FusedArgs fused_args() {
@@ -560,6 +598,7 @@ class deviceclass {
     unsigned long long* o_lmax = nullptr;
     // single-kernel stage with artificial viscosity
     double* o_gtr = nullptr;
+    double* o_Qv = nullptr;      // the sequence's viscous volume term
     int* o_active[2] = {nullptr, nullptr};
     unsigned long long* o_emax = nullptr;
     // a captured step of the fused schedule (clock_timeloop) and the settings it was captured with

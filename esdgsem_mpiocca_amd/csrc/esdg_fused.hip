@@ -31,8 +31,8 @@
 
 namespace esdg {
 
-int fused_volume(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA, double cdt, const double* fstar, double* Qt,
-                 const double* Qv, const double* SPV, double* tr, const int* slot, const int* active = nullptr,
+int fused_volume(esdg_ctx* ctx, const FusedArgs& a, double rkA, double cdt, const double* fstar, const double* Qv,
+                 const double* SPV, double* tr, const int* slot, const int* active = nullptr,
                  const int* list = nullptr, const int* acount = nullptr);
 int write_traces(esdg_ctx* ctx, int Nelem, const double* q, double* tr, const int* slot);
 int trace_slots(esdg_ctx* ctx, int Nelem, const int* E2E, const int* ED, int* slot);
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) k_fused_av(int Nelem, AvMesh M, const dou
     constexpr int NN = NGL * NGL;
     const int seq = acount[2];
     __shared__ double sDh[NN], sDs[NN];
-    __shared__ double sA[EB::THREADS], sB[EB::THREADS], sC[EB::THREADS], sE[EB::THREADS];
+    __shared__ double sA[EB::THREADS], sB[EB::THREADS], sC[EB::THREADS], sE[EB::THREADS], sF[EB::EPB * 16 * NGL];
     __shared__ double sEps[EB::EPB];
     if (threadIdx.x < NN) {
         sDh[threadIdx.x] = Dh[threadIdx.x];
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(256) k_fused_av(int Nelem, AvMesh M, const dou
         const int idx = grp * EB::EPB + el;
         const bool act = idx < cnt;
         const int e = act ? alist[idx] : 0;
-        av_element_block<NGL>(M, TraceFromSides{tr}, e, act, act ? visc[e] : 0.0, sDh, sDs, sA, sB, sC, sE, sEps);
+        av_element_block<NGL>(M, TraceFromSides{tr}, e, act, act ? visc[e] : 0.0, sDh, sDs, sA, sB, sC, sE, sF, sEps);
     }
 }
 
@@ -332,7 +332,7 @@ int FusedStage::stage(esdg_ctx* ctx, int, double rkA, double cdt, const FusedArg
     if (!av) {
         // volume + surface + RK (+ the limiter on the new state) in one element pass, which writes
         // the side traces of the state it stores
-        return fused_volume(ctx, A, true, rkA, cdt, fstar, nullptr, nullptr, nullptr, tr, slot);
+        return fused_volume(ctx, A, rkA, cdt, fstar, nullptr, nullptr, tr, slot);
     }
     int rc = ESDG_OK;
     {
@@ -351,7 +351,7 @@ int FusedStage::stage(esdg_ctx* ctx, int, double rkA, double cdt, const FusedArg
         if (rc) return rc;
     }
     // volume + surface + viscous terms + RK (+ the limiter on the new state) in one element pass
-    return fused_volume(ctx, A, true, rkA, cdt, fstar, nullptr, qvisc, fvisc, tr, slot, active, alist, acount);
+    return fused_volume(ctx, A, rkA, cdt, fstar, qvisc, fvisc, tr, slot, active, alist, acount);
 }
 
 void FusedStage::release(esdg_ctx* ctx) {

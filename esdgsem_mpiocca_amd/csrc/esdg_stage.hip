@@ -807,7 +807,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
 template <int NGL>
 __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns, const int2* __restrict__ list, int cnt,
                                               int blk, int nblk, int src, double* sDh, double* sDs, double* sA,
-                                              double* sB, double* sC, double* sE, double* sEps) {
+                                              double* sB, double* sC, double* sE, double* sF, double* sEps) {
     using EB = ElemBlock<NGL>;
     constexpr int NN = NGL * NGL;
     const int el = threadIdx.x / NN, n = threadIdx.x % NN;
@@ -823,7 +823,7 @@ __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns,
                        S.nx, S.ny, S.scal, S.bL, S.bR, GatherConsts{S.bc, S.h_zero}, S.geomFace, S.tol, S.gtr, S.Qv};
         const int o = (el < EB::EPB ? el : 0) * NN;
         av_element_block<NGL>(M, TraceFromState{S.q[src]}, me.y, act, act ? S.visc[me.y] : 0.0, sDh + o, sDs + o, sA,
-                              sB, sC, sE, sEps);
+                              sB, sC, sE, sF, sEps);
     }
 }
 
@@ -834,6 +834,7 @@ template <int LO, int HI>
 __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src) {
     __shared__ double sDh[256], sDs[256];
     __shared__ double sA[256], sB[256], sC[256], sE[256];
+    __shared__ double sF[ElemBlock<LO>::EPB * 16 * LO];   // (the most at the lowest degree)
     __shared__ double sEps[ElemBlock<LO>::EPB];
     int l = l0;
     while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
@@ -843,7 +844,7 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
         if constexpr (n >= LO && n <= HI)                                                     \
-            ens_grad_body<n>(scns, L.list[l], cnt, blk, L.blocks[l], src, sDh, sDs, sA, sB, sC, sE, sEps); \
+            ens_grad_body<n>(scns, L.list[l], cnt, blk, L.blocks[l], src, sDh, sDs, sA, sB, sC, sE, sF, sEps); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE

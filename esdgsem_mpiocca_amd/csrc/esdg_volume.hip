@@ -18,20 +18,21 @@
 #include "esdg_device.h"
 #include "esdg_fused.h"
 #include "esdg_internal.h"
+#include "esdg_sequence.h"
 
 namespace esdg {
 
 // What the flux-differencing kernel does after the volume term of its nodes:
 //   VOL_ONLY      store Qt (the reference's VolumeKernel)
-//   VOL_SURF      add the surface lift of the face fluxes (okl/DG/SurfaceKernel.okl, DBSurf = 0), store Qt
-//   VOL_SURF_RK   as VOL_SURF, then the low-storage RK step gRK = A gRK + Qt, q += cdt gRK in place
-//                 (okl/RungeKutta/rkLS.okl + UpdateKernelLS.okl); Qt never reaches HBM
+//   VOL_SURF_RK   add the surface lift of the face fluxes (okl/DG/SurfaceKernel.okl, DBSurf = 0), then the
+//                 low-storage RK step gRK = A gRK + Qt, q += cdt gRK in place (okl/RungeKutta/rkLS.okl +
+//                 UpdateKernelLS.okl); Qt is stored where the caller keeps it
 //   VOL_SURF_VISC_RK  as VOL_SURF_RK with the viscous terms of the artificial viscosity added
 //                 after the surface lift, in the reference's order: the viscous volume term
 //                 (VolumeKernelViscose.okl, precomputed per node; skipped where the element's
 //                 viscosity is zero, where it is +-0) and the viscous surface lift
 //                 (SurfaceKernelVisc.okl)
-enum VolMode { VOL_ONLY = 0, VOL_SURF = 1, VOL_SURF_RK = 2, VOL_SURF_VISC_RK = 3 };
+enum VolMode { VOL_ONLY, VOL_SURF_RK, VOL_SURF_VISC_RK };
 
 struct SurfIn {
     const int *E2E, *EMS, *EOR;
@@ -51,7 +52,8 @@ struct SurfIn {
     double* lam;           // FindLambdaMax's element maximum wave speed
     double tol;            // PosPresTOL (velocities are 0 where h <= tol)
     // VOL_SURF_VISC_RK: elements with active[e] != the stage mark have zero viscosity on
-    // themselves and on every face neighbour; their viscous terms are +-0 and are not read
+    // themselves and on every face neighbour; their viscous terms are +-0 and are not read (null: every
+    // element takes its viscous terms)
     const int* active;
     // the marked elements (list[0 .. acount[m & 1]), m = acount[2] the stage mark): with them
     // given, VOL_SURF_RK leaves the marked elements out and VOL_SURF_VISC_RK runs over the list
@@ -294,8 +296,8 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
                 }
             }
         }
-        if (MODE == VOL_SURF_VISC_RK && si.active[e] == seq) {
-            if (si.visc[e] != 0.0) {
+        if (MODE == VOL_SURF_VISC_RK && (!si.active || si.active[e] == seq)) {
+            if (!si.active || si.visc[e] != 0.0) {
                 const double* qv = si.Qv + (int64_t)e * C::NN * 2 + r;
 #pragma unroll
                 for (int k = 0; k < NGL; ++k) {
@@ -359,6 +361,11 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
 #pragma unroll
             for (int k = 0; k < NGL; ++k) {
                 const int64_t id = ob + k * NGL;
+                if (Qt) {
+                    Qt[id] = b1[k];
+                    Qt[id + C::NN] = b2[k];
+                    Qt[id + 2 * C::NN] = b3[k];
+                }
                 double g1, g2, g3;
                 if constexpr (kDma) {
                     g1 = gk[0][k]; g2 = gk[1][k]; g3 = gk[2][k];
@@ -653,25 +660,23 @@ void launch_volume_fluxdiff(esdg_ctx* ctx, int Nelem, const double* Jac, const d
 }
 
 template <int NGL>
-void launch_volume_fused(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA, double cdt, const double* fstar,
-                         double* Qt, const double* Qv, const double* SPV, double* tr, const int* slot,
+void launch_volume_fused(esdg_ctx* ctx, const FusedArgs& a, double rkA, double cdt, const double* fstar,
+                         const double* Qv, const double* SPV, double* tr, const int* slot,
                          const int* active, const int* list, const int* acount) {
     using C = VolCfg<NGL>;
-    SurfIn si{a.ElemToEdge, a.EMS, a.EOR, fstar, rkA, cdt, a.gRK, Qv, a.ViscPara, SPV, rk ? tr : nullptr, slot};
+    SurfIn si{a.ElemToEdge, a.EMS, a.EOR, fstar, rkA, cdt, a.gRK, Qv, a.ViscPara, SPV, tr, slot};
     si.active = active;
     si.list = list;
     si.acount = acount;
     si.dtp = a.dt_dev;
     si.Cs = a.C_stage;
-    if (rk) {
-        // PosPres on the new state before it is stored (okl/Positivity/PosPres.okl)
-        si.tol = ctx->p.PosPresTOL;
-        si.limit = a.positivity;
-        si.EleSizes = a.EleSizes;
-        si.GLw = a.GLw;
-        si.zero_tol = ctx->p.ZeroTOL;
-    }
-    if (rk && tr) {
+    // PosPres on the new state before it is stored (okl/Positivity/PosPres.okl)
+    si.tol = ctx->p.PosPresTOL;
+    si.limit = a.positivity;
+    si.EleSizes = a.EleSizes;
+    si.GLw = a.GLw;
+    si.zero_tol = ctx->p.ZeroTOL;
+    if (tr) {
         // the updated state's viscosity and wave speed, for the next stage or time step
         si.visc_next = a.next_visc;
         si.visc_plot = a.next_visc ? a.next_visc_plot : nullptr;
@@ -680,7 +685,7 @@ void launch_volume_fused(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA,
         si.sc = SensorConsts{ctx->p.ZeroTOL, ctx->p.eps0, ctx->p.sigmaMin, ctx->p.sigmaMax};
         si.lam = a.next_lambda;
     }
-    if (rk && Qv) {
+    if (Qv) {
         // the listed marked elements and the unmarked ones (disjoint sets, each updated once;
         // nothing else is read or written by both) in one launch
         // (at ngl = 10 the two bodies in one kernel spill far more than each alone: two launches
@@ -695,24 +700,47 @@ void launch_volume_fused(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA,
             k_volume_fluxdiff<NGL, VOL_SURF_RK><<<nb, 64, 0, ctx->stream>>>(
                 a.Nelem, ctx->p.g, a.Jac, a.Yxi, a.Yeta, a.Xxi, a.Xeta, a.q, a.D, a.Bx, a.By, nullptr, si);
         }
-    } else if (rk)
+    } else {
         k_volume_fluxdiff<NGL, VOL_SURF_RK><<<blocks_for(a.Nelem, C::EPW), 64, 0, ctx->stream>>>(
             a.Nelem, ctx->p.g, a.Jac, a.Yxi, a.Yeta, a.Xxi, a.Xeta, a.q, a.D, a.Bx, a.By, nullptr, si);
-    else
-        k_volume_fluxdiff<NGL, VOL_SURF><<<blocks_for(a.Nelem, C::EPW), 64, 0, ctx->stream>>>(
-            a.Nelem, ctx->p.g, a.Jac, a.Yxi, a.Yeta, a.Xxi, a.Xeta, a.q, a.D, a.Bx, a.By, Qt, si);
+    }
 }
 
-// Fused volume + surface lift (+ viscous terms when Qv is given) (+ RK update in place when rk,
-// with the side traces of the new state written to tr when given): called by the fused stage.
-int fused_volume(esdg_ctx* ctx, const FusedArgs& a, bool rk, double rkA, double cdt, const double* fstar, double* Qt,
-                 const double* Qv, const double* SPV, double* tr, const int* slot, const int* active,
+// The sequence's update: Qt stored, every element's viscous terms taken, no side traces.
+template <int NGL>
+void launch_sequence_volume(esdg_ctx* ctx, const SequenceArgs& a, double rkA, double cdt) {
+    using C = VolCfg<NGL>;
+    SurfIn si{a.ElemToEdge, a.EMS, a.EOR, a.SurfaceParts, rkA, cdt, a.gRK, a.Qv, a.ViscPara, a.SurfacePartsVisc};
+    si.tol = ctx->p.PosPresTOL;
+    si.limit = a.positivity;
+    si.EleSizes = a.EleSizes;
+    si.GLw = a.GLw;
+    si.zero_tol = ctx->p.ZeroTOL;
+    const unsigned nb = blocks_for(a.Nelem, C::EPW);
+    if (a.artificial_viscosity)
+        k_volume_fluxdiff<NGL, VOL_SURF_VISC_RK><<<nb, 64, 0, ctx->stream>>>(
+            a.Nelem, ctx->p.g, a.Jac, a.Yxi, a.Yeta, a.Xxi, a.Xeta, a.q, a.D, a.Bx, a.By, a.Qt, si);
+    else
+        k_volume_fluxdiff<NGL, VOL_SURF_RK><<<nb, 64, 0, ctx->stream>>>(
+            a.Nelem, ctx->p.g, a.Jac, a.Yxi, a.Yeta, a.Xxi, a.Xeta, a.q, a.D, a.Bx, a.By, a.Qt, si);
+}
+
+int sequence_volume(esdg_ctx* ctx, const SequenceArgs& a, double rkA, double cdt) {
+    KernelScope ks(ctx, "sequence_volume");
+    ESDG_NGL_DISPATCH(ctx->p.ngl, launch_sequence_volume, ctx, a, rkA, cdt);
+    return launch_check(ctx, "sequence_volume");
+}
+
+// Fused volume + surface lift (+ viscous terms when Qv is given) + RK update in place, with the side
+// traces of the new state written to tr when given: called by the fused stage.
+int fused_volume(esdg_ctx* ctx, const FusedArgs& a, double rkA, double cdt, const double* fstar, const double* Qv,
+                 const double* SPV, double* tr, const int* slot, const int* active,
                  const int* list, const int* acount) {
     if (Qv && !(active && list && acount))
         return set_error(ctx, ESDG_ERR_STATE, "fused_volume: viscous terms need the stage marks and element list");
     KernelScope ks(ctx, "fused_volume");
     if (tr && !slot) return set_error(ctx, ESDG_ERR_STATE, "fused_volume: side traces need the face slots");
-    ESDG_FUSED_DISPATCH(ctx->p.ngl, launch_volume_fused, ctx, a, rk, rkA, cdt, fstar, Qt, Qv, SPV, tr, slot, active,
+    ESDG_FUSED_DISPATCH(ctx->p.ngl, launch_volume_fused, ctx, a, rkA, cdt, fstar, Qv, SPV, tr, slot, active,
                       list, acount);
     return launch_check(ctx, "fused_volume");
 }

@@ -236,7 +236,9 @@ typedef struct esdg_run_params {
     int positivity;               /* PositivityPreserving */
     int rk_order, rk_ssp;         /* rkorder (3 or 4), rkSSP */
     int flux_differencing;        /* FluxDifferencing */
-    int fused;                    /* 0: the reference's kernel sequence; 1: fused stage kernels (at
+    int fused;                    /* 0: the reference's kernel sequence (its arrays, in fewer passes
+                                     with flux differencing, a low-storage RK and walls, inner/outer
+                                     or ocean boundaries); 1: fused stage kernels (at
                                      2 <= N <= 7 the single-kernel stage); 2: the single-kernel stage
                                      (2 <= N <= 7; with artificial viscosity the gradient and viscous
                                      face passes run before it) */
