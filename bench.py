@@ -89,7 +89,7 @@ KERNELS = ["volume_kernel", "collect_edge_data", "calc_num_fluxes", "surface_ker
            "surface_kernel_gradient", "scale_gradient", "collect_edge_data_gradient",
            "volume_kernel_viscose", "calc_num_fluxes_viscose", "surface_kernel_visc",
            "find_lambda_max", "reduce_max", "pos_pres", "fused_face", "fused_volume", "fused_av",
-           "fused_viscous_face", "fused_clock", "mlp_indicator", "write_traces", "stage", "stage_dt", "stage_lambda",
+           "fused_viscous_face", "fused_clock", "mlp_indicator", "write_traces", "stage", "stage_lambda",
            "stage_mark", "ens_sensor", "ens_indicator", "ens_grad", "ens_viscous_face", "sequence_faces",
            "sequence_gradient", "sequence_viscous_faces", "sequence_volume"]
 
@@ -261,7 +261,7 @@ def ensemble_av_bench(dev, args):
             ctx.profile_reset()
             ens.run(1)
             kern = {}
-            for kn in ("stage", "ens_sensor", "ens_indicator", "ens_grad", "ens_viscous_face", "stage_dt", "stage_mark"):
+            for kn in ("stage", "ens_sensor", "ens_indicator", "ens_grad", "ens_viscous_face", "stage_mark"):
                 launches, ms = ctx.profile_query(kn)
                 if launches:
                     kern[kn] = {"launches": launches, "ms_per_step": round(ms, 3)}

@@ -70,17 +70,17 @@ class deviceclass {
         if (rp.maximum_elevation) A(&o_MaximumElevation, nodes);
         if (rc == ESDG_OK && rp.fused == 1 && !element_stage())
             rc = fused_.init(ctx_, Nelem, Nfaces, rp.artificial_viscosity != 0);
-        if (rp.fused) A(&o_clock, 8);   // the device clock
+        if (rp.fused) A(&o_clock, 16);   // the device clock (the stage kernel's two)
         if (element_stage()) {
             // the stage kernel: second state buffer (ping-pong), lambda_max cell
-            A(&o_q2, nodes * 3); A(reinterpret_cast<double**>(&o_lmax), 1);
+            A(&o_q2, nodes * 3); A(reinterpret_cast<double**>(&o_lmax), 2);
             if (rp.artificial_viscosity) {
                 // the stage's gradient side traces, marks (one array per state buffer) and viscosity
                 // maximum (the viscous volume term goes to qGradientX, the viscous face fluxes to
                 // SurfacePartsVisc); allocations are zero-filled
                 A(&o_gtr, (size_t)Nelem * 16 * ngl);
                 for (int*& a : o_active) A(reinterpret_cast<double**>(&a), ((size_t)Nelem + 1) / 2);
-                A(reinterpret_cast<double**>(&o_emax), 1);
+                A(reinterpret_cast<double**>(&o_emax), 2);
             }
         }
         return rc;
@@ -476,7 +476,7 @@ class deviceclass {
         // the state is in o_q at every entry; the clock restarts from the host's t
         double ck[8] = {0.0, t, 0.0, last_dt, 0.0, 0.0, 0.0, (double)max_steps};
         rc = esdg_memcpy(ctx_, o_clock, ck, sizeof ck, ESDG_H2D);
-        if (!rc) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_lmax), 0.0, 1);
+        if (!rc) rc = esdg_fill(ctx_, reinterpret_cast<double*>(o_lmax), 0.0, 2);
         int src = 0;
         if (!rc) rc = stage_.lambda(ctx_, src);
         stage_.primed = false;   // q may have been set since the last call
@@ -484,7 +484,7 @@ class deviceclass {
         while (!rc && issued < max_steps && ck[1] < rp_.T && ck[4] == 0.0) {
             const int chunk = std::min(max_steps - issued, 64);
             rc = stage_.run(ctx_, A, Cc, stages, chunk, src);
-            if (!rc) rc = esdg_memcpy(ctx_, ck, o_clock, sizeof ck, ESDG_D2H);
+            if (!rc) rc = esdg_memcpy(ctx_, ck, o_clock + 8 * src, sizeof ck, ESDG_D2H);
             issued += chunk;
         }
         if (!rc && src == 1)

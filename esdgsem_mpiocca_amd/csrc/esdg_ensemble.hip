@@ -22,9 +22,9 @@ struct esdg_ensemble {
     std::map<std::pair<const void*, size_t>, void*> up;  // host (pointer, bytes) -> device copy
     std::map<std::tuple<const void*, const void*, int, int>, std::pair<double*, double*>> btr;
     std::vector<void*> owned;
-    double* clocks = nullptr;             // 8 doubles per scenario
-    unsigned long long* lmax = nullptr;   // one per scenario
-    unsigned long long* emax = nullptr;   // one per scenario (artificial viscosity)
+    double* clocks = nullptr;             // 2 x 8 doubles per scenario
+    unsigned long long* lmax = nullptr;   // two per scenario
+    unsigned long long* emax = nullptr;   // two per scenario (artificial viscosity)
     StageBatch batch;
     int src = 0;
     bool need_lambda = true;
@@ -59,7 +59,7 @@ struct esdg_ensemble {
 
     int start() {
         if (!need_lambda) return ESDG_OK;
-        int rc = esdg_fill(ctx, reinterpret_cast<double*>(lmax), 0.0, scn.size());
+        int rc = esdg_fill(ctx, reinterpret_cast<double*>(lmax), 0.0, 2 * scn.size());
         if (!rc) rc = batch.lambda(ctx, src);
         if (!rc) need_lambda = false;
         return rc;
@@ -117,10 +117,10 @@ int esdg_ensemble_create(esdg_ctx* ctx, int nscn, const esdg_params* params, con
     double Bdummy[5];
     if (esdg_rk_coefficients(rp[0].rk_order, 0, &E->stages, E->A, Bdummy, E->C) != 0)
         rc = set_error(ctx, ESDG_ERR_ARG, "esdg_ensemble_create: RK coefficients");
-    if (!rc) E->clocks = (double*)E->alloc((size_t)nscn * 8 * sizeof(double), &rc);
-    if (!rc) E->lmax = (unsigned long long*)E->alloc((size_t)nscn * sizeof(unsigned long long), &rc);
-    if (!rc) E->emax = (unsigned long long*)E->alloc((size_t)nscn * sizeof(unsigned long long), &rc);
-    if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(E->emax), 0.0, nscn);
+    if (!rc) E->clocks = (double*)E->alloc((size_t)nscn * 16 * sizeof(double), &rc);
+    if (!rc) E->lmax = (unsigned long long*)E->alloc((size_t)nscn * 2 * sizeof(unsigned long long), &rc);
+    if (!rc) E->emax = (unsigned long long*)E->alloc((size_t)nscn * 2 * sizeof(unsigned long long), &rc);
+    if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(E->emax), 0.0, 2 * (size_t)nscn);
     const size_t dd = sizeof(double), di = sizeof(int);
     for (int i = 0; i < nscn && !rc; ++i) {
         const esdg_params& p = params[i];
@@ -174,9 +174,9 @@ int esdg_ensemble_create(esdg_ctx* ctx, int nscn, const esdg_params* params, con
             if (!in.q) rc = set_error(ctx, ESDG_ERR_ARG, "esdg_ensemble_create: missing q");
             else rc = esdg_memcpy(ctx, S.q[0], in.q, nodes * 3 * dd, ESDG_H2D);
         }
-        S.clock = E->clocks + 8 * (size_t)i;
-        S.lmax = E->lmax + i;
-        S.emax = E->emax + i;
+        S.clock = E->clocks + 16 * (size_t)i;
+        S.lmax = E->lmax + 2 * (size_t)i;
+        S.emax = E->emax + 2 * (size_t)i;
         if (r.artificial_viscosity) {
             // the element viscosity and the BR1 / viscous work buffers, private to the scenario;
             // the dt limit of src/deviceclass.cpp:922 with the solver's constant
@@ -248,7 +248,7 @@ int esdg_ensemble_status(esdg_ensemble* E, int i, double* t, int* steps_taken, d
     if (!E) return set_error(nullptr, ESDG_ERR_ARG, "esdg_ensemble_status: null ensemble");
     ESDG_REQUIRE(E->ctx, i >= 0 && i < (int)E->scn.size(), "esdg_ensemble_status: scenario out of range");
     double ck[8];
-    int rc = esdg_memcpy(E->ctx, ck, E->clocks + 8 * (size_t)i, sizeof ck, ESDG_D2H);
+    int rc = esdg_memcpy(E->ctx, ck, E->clocks + 16 * (size_t)i + 8 * E->src, sizeof ck, ESDG_D2H);
     if (rc) return rc;
     if (t) *t = ck[1];
     if (steps_taken) *steps_taken = (int)ck[2];
@@ -280,7 +280,7 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
     size_t total = 0;
     for (size_t c : E->qcount) total += c;
     double* snap = nullptr;
-    rc = esdg_malloc(ctx, (void**)&snap, (total + 9 * (size_t)ns) * sizeof(double));
+    rc = esdg_malloc(ctx, (void**)&snap, (total + 18 * (size_t)ns) * sizeof(double));
     if (rc) return rc;
     auto copy_all = [&](bool save) {
         size_t off = 0;
@@ -292,12 +292,12 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
             off += E->qcount[i];
         }
         if (!r) r = hip_check(ctx, hipMemcpyAsync(save ? snap + off : E->clocks, save ? E->clocks : snap + off,
-                                                  (size_t)ns * 8 * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream),
+                                                  (size_t)ns * 16 * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream),
                               "autotune snapshot");
-        off += (size_t)ns * 8;
+        off += (size_t)ns * 16;
         if (!r) r = hip_check(ctx, hipMemcpyAsync(save ? (void*)(snap + off) : (void*)E->lmax,
                                                   save ? (const void*)E->lmax : (const void*)(snap + off),
-                                                  (size_t)ns * sizeof(unsigned long long), hipMemcpyDeviceToDevice,
+                                                  (size_t)ns * 2 * sizeof(unsigned long long), hipMemcpyDeviceToDevice,
                                                   ctx->stream),
                               "autotune snapshot");
         if (!r) r = esdg_finish(ctx);

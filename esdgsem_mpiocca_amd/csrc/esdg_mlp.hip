@@ -340,7 +340,7 @@ __device__ void mlp_indicator_block(int Nelem, int e0, gptr<const double> __rest
             const unsigned long long c = k < 4 ? sCnt[k] : (unsigned long long)min(FEPB, Nelem - e0);
             if (MS.counters && c) atomicAdd(MS.counters + k, c);
         } else if (threadIdx.x == 4 * FEPB + 5) {
-            if (MS.stage == 0 && sMax) max_into(MS.scn->emax, __longlong_as_double((long long)sMax));
+            if (MS.stage == 0 && sMax) max_into(MS.scn->emax + MS.buffer, __longlong_as_double((long long)sMax));
         }
     }
 }
@@ -360,8 +360,9 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
                                                        float hi, int audit, unsigned long long* counters) {
     const StageTask tk = tasks[blockIdx.x];
     const StageScn& S = scns[tk.scn];
-    if (stage > 0 && S.clock[0] <= 0.0) return;
-    if (stage == 0 && S.clock[1] >= S.T) return;
+    const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
+    if (stage > 0 && S.clock[8 * (p ^ 1)] <= 0.0) return;
+    if (stage == 0 && S.clock[8 * p + 1] >= S.T) return;
     MaskedSensor MS;
     MS.visc = S.visc;
     MS.visc_plot = S.visc_plot;
@@ -371,8 +372,7 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
     // for 20 us at 65536 elements)
     MS.counters = counters + 8 * (blockIdx.x % IND_SLOTS);
     MS.scn = &S;
-    // (the step's first viscosity comes before its marks are advanced)
-    MS.mark = *mark + (stage == 0 ? STAGE_MARKS : stage);
+    MS.mark = mark[p] + stage;
     MS.buffer = src;
     MS.stage = stage;
     mlp_indicator_block(S.Nelem, tk.e0, glob((const double*)S.q[src]), glob(S.B), glob(S.VdmInv), W, lo, hi, nullptr,

@@ -29,10 +29,13 @@ struct StageScn {
     const int *EdgeData, *E2E, *EMS, *EOR;
     double* q[2];       // ping-pong state buffers
     double* gRK;
-    double* clock;      // [0] dt of the current step (-1: it changes nothing; 0: a failed scenario), [1] t,
+    // Of the clock, the maxima and the marks there are two, used by steps in turn: a step that starts from the
+    // state in buffer p takes half p and leaves the other half for the next (the stages of a step are odd
+    // in number, so that one starts from buffer p ^ 1).
+    double* clock;      // 2 x 8: [0] dt of the current step (-1: it changes nothing; 0: a failed scenario), [1] t,
                         // [2] steps taken, [3] dt of the last step taken, [4] 1 if a dt was not positive
                         // and finite ([5] that dt), [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
-    unsigned long long* lmax;   // bit pattern of max lambda (non-negative doubles order as integers)
+    unsigned long long* lmax;   // 2: bit pattern of max lambda (non-negative doubles order as integers)
     // artificial viscosity (av = 1): the modal sensor, or with learned = 1 (N = 7) the learned
     // indicator with the sensor as fallback, evaluated on each stage's state; BR1 gradients and the
     // viscous terms only where viscosity is in reach (active[e] == the stage's mark)
@@ -57,7 +60,7 @@ struct StageScn {
     // a single solver's buffers (each may be null): the element wave speeds of the state after a step,
     // and the analysis buffers, advanced after every step
     double *lam, *arrival, *maxelev;
-    unsigned long long* emax;   // bit pattern of the step's max viscosity
+    unsigned long long* emax;   // 2: bit pattern of the step's max viscosity
     // per element side, what its face flux needs from the connectivity (built by StageBatch::init
     // from E2E, EOR, EMS and EdgeData; one record per side, shared by the scenarios of a mesh):
     // x face, y EdgeData[0] (left element), z EdgeData[1] (right element), w bits: [0,2) left

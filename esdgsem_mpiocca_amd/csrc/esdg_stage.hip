@@ -46,6 +46,13 @@ struct MaxLds<HI, HI> {
     static constexpr int value = StageCfg<HI>::LDS;
 };
 
+// a double that is the same in all lanes, as a scalar
+__device__ __forceinline__ double uniform(double x) {
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // Volume term, surface lift, RK update, limiter and wave speed of one block of elements; the
 // face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
 // parameters are __restrict__ so that the geometry loads schedule as in a kernel taking them as
@@ -53,11 +60,10 @@ struct MaxLds<HI, HI> {
 // AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
 // record per element instead of five doubles per node; the bottom slopes too where they are constant.
 // The kernel moves its bytes at what streaming kernels reach here, so bytes are time.
-template <int NGL, bool AV, bool AFF, class Faces, class Early>
+template <int NGL, bool AV, bool AFF, class Faces, class Early, class Dt>
 __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, const Faces& faces, const Early& early,
-                                           double g, double tol,
-                                           double zero_tol, int positivity, double rkA, double rkC, double dt, bool last,
-                                           bool keep, gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
+                                           const Dt& step_dt, double g, double tol,
+                                           double zero_tol, int positivity, double rkA, double rkC, bool last, gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
                                            gptr<double> __restrict__ gRK, gptr<const double> __restrict__ Yeta,
                                            gptr<const double> __restrict__ Xeta, gptr<const double> __restrict__ Yxi,
                                            gptr<const double> __restrict__ Xxi, gptr<const double> __restrict__ Jac,
@@ -65,7 +71,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                                            gptr<const double> __restrict__ geo,
                                            gptr<const double> __restrict__ EleSizes,
                                            gptr<const double> __restrict__ GLw,
-                                           gptr<unsigned long long> __restrict__ lmax, const StageScn* SV, int src,
+                                           const StageScn* SV, int src, int p,
                                            int mark, int next_mark, double* sD) {
     using C = VolCfg<NGL>;
     double* FS = P;                  // face fluxes, after the sweeps (the planes are free then)
@@ -80,6 +86,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 #pragma unroll
     for (int c = 0; c < NGL; ++c) { a1[c] = 0.0; a2[c] = 0.0; a3[c] = 0.0; }
 
+    double dt = 0.0;
     // whether viscosity is in reach, and the element's own, loaded beside the row data
     bool marked = false;
     double eps0 = 0.0;
@@ -116,6 +123,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
         // a step that changes nothing has dt < 0: the state goes over to the other buffer as it is.  (dt is
         // loaded beside the rows; a wave that waited for it before loading them cost 3 %.)
+        dt = step_dt();
         if (dt < 0.0) {
 #pragma unroll
             for (int c = 0; c < NGL; ++c) {
@@ -139,6 +147,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         else line_sweep<NGL, false>(D, g, h, hu, hv, u, v, LineMetrics<NGL>{Y, X}, a1, a2, a3);
         }
     }
+    dt = uniform(dt);   // (lane 0 has an element)
     if (dt < 0.0) return;
     __syncthreads();
 
@@ -289,7 +298,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 b3[k] = rkA * gRK[id + 2 * C::NN] + b3[k];
             }
         }
-        if (!last || keep) {
+        if (!last || glob((const double*)SV->clock)[8 * (p ^ 1) + 6] != 0.0) {
 #pragma unroll
             for (int k = 0; k < NGL; ++k) {
                 const int64_t id = ob + k * NGL;
@@ -400,10 +409,10 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
         double m = lam;
         for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-        if (lane == 0) max_into((unsigned long long*)lmax, m);
+        if (lane == 0) max_into(SV->lmax + (p ^ 1), m);
         // ArrivalTimes.okl:16-62 and MaximumElevation.okl:16-55 on the state after the step, at its time
         if (act && SV->arrival) {
-            const double t = glob(SV->clock)[1];
+            const double t = glob(SV->clock)[8 * (p ^ 1) + 1];
             const gptr<double> arr = glob(SV->arrival);
             const gptr<const double> B = glob(SV->B);
 #pragma unroll
@@ -479,22 +488,68 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 // non-negative doubles order as their bit patterns; a NaN stays out, as fmax leaves it
                 double m = eps > 0.0 ? eps : 0.0;
                 for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-                if (lane == 0 && m > 0.0) max_into(SV->emax, m);
+                if (lane == 0 && m > 0.0) max_into(SV->emax + (p ^ 1), m);
             }
         }
     }
 }
 
 
+// DGtimeloop's dt (src/deviceclass.cpp:899-930) of the step that starts from the scenario's clock ck: while
+// t < T, dt = min(T - t, dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T (or after a dt that is not
+// positive and finite, which is flagged) dt = -1 and the stages leave the state unchanged.  (A batch that does
+// not freeze a failed state goes on with dt = 0 there: what is not finite spreads, as in q + 0 gRK.)  Every
+// wave of a step's first stage forms it from the maxima that the last step's last stage left, beside its
+// row loads; the clock after it is written to `next` by one of them (as a launch of its own before the
+// stages it took 4 to 5 us per step).
+__device__ __forceinline__ double first_dt(const StageScn& S, gptr<const double> ck, double lm, double em,
+                                           gptr<double> next) {
+    const double t = ck[1], steps = ck[2], failed = ck[4], until = ck[7];
+    double dt = -1.0, t1 = t, n1 = steps, last = ck[3], err = failed, bad = ck[5], keep = ck[6];
+    if (t < S.T && failed == 0.0) {
+        const double dt_i = S.dti / lm;
+        // with artificial viscosity also the viscous limit dvc / max eps (infinite where no element
+        // has viscosity), in the order of src/deviceclass.cpp:920-926
+        dt = S.av ? fmin(S.T - t, fmin(dt_i, S.dvc / em)) : fmin(S.T - t, dt_i);
+        if (!(dt > 0.0) || isinf(dt)) {
+            err = 1.0;
+            bad = dt;
+            keep = 1.0;
+            dt = S.freeze ? -1.0 : 0.0;
+        } else {
+            t1 = t + dt;
+            n1 = steps + 1.0;
+            last = dt;
+            // the step that ends the run leaves its RK register for a checkpoint
+            keep = (n1 == until || t1 >= S.T) ? 1.0 : 0.0;
+        }
+    } else if (failed != 0.0 && !S.freeze) {
+        dt = 0.0;
+    }
+    if (next) {
+        next[0] = dt; next[1] = t1; next[2] = n1; next[3] = last;
+        next[4] = err; next[5] = bad; next[6] = keep; next[7] = until;
+    }
+    return dt;
+}
+
 template <int NGL, bool AV, bool AFF>
-__device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, int src, double rkA,
-                                           double rkC, bool last, int mark, int next_mark) {
+__device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, int src, int stage,
+                                           double rkA, double rkC, bool last, int mark, int next_mark, int* markp) {
     using C = VolCfg<NGL>;
     using SC = StageCfg<NGL>;
     const int lane = threadIdx.x;
+    const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
     // the marks of the stage's state have been used: the list that the next stage's marks go to is the
     // other one, and this one is empty when its turn comes
     if (AV && S.av && e0 == 0 && lane == 0) S.mcount[src] = 0;
+    if (stage == 1 && e0 == 0 && lane == 0) {
+        // the first stage has read the step's maxima: they are empty when the next step's last stage adds
+        // to them; and the next step's marks
+        S.lmax[p] = 0ull;
+        if (AV && S.av) S.emax[p] = 0ull;
+        if (AV && S.id == 0) markp[p ^ 1] = markp[p] + STAGE_MARKS;
+    }
     // D of this degree in LDS (wave-uniform reads, broadcast): keeps it out of the scalar registers
     for (int t = lane; t < NGL * NGL; t += 64) sD[t] = glob(S.D)[t];
     const int el = lane / NGL, r = lane % NGL;
@@ -593,22 +648,29 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
         flux(3, b);
     };
 
+    auto step_dt = [&]() -> double {
+        const gptr<double> ck = glob(S.clock);
+        if (stage) return ck[8 * (p ^ 1)];
+        const double lm = __longlong_as_double((long long)glob(S.lmax)[p]);
+        const double em = S.av ? __longlong_as_double((long long)glob(S.emax)[p]) : 0.0;
+        return first_dt(S, ck + 8 * p, lm, em, e0 == 0 && lane == 0 ? ck + 8 * (p ^ 1) : nullptr);
+    };
+
     __syncthreads();   // sD written
-    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, glob(S.clock)[0], last,
-                             glob(S.clock)[6] != 0.0, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
+    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, step_dt, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, last, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
                              glob(S.Xxi), glob(S.Jac), glob(S.Bx), glob(S.By), glob(S.geo), glob(S.EleSizes), glob(S.GLw),
-                             glob(S.lmax), &S, src, mark, next_mark, sD);
+                             &S, src, p, mark, next_mark, sD);
 }
 
 template <int LO, int HI, bool AV, bool AFF>
 __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, const StageTask& tk, double* lds,
-                                           double* sD, int src, double rkA, double rkC, bool last, int mark,
-                                           int next_mark) {
+                                           double* sD, int src, int stage, double rkA, double rkC, bool last, int mark,
+                                           int next_mark, int* markp) {
     const StageScn& S = scns[tk.scn];
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                \
     case n:                                                                         \
-        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, rkA, rkC, last, mark, next_mark);    \
+        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, stage, rkA, rkC, last, mark, next_mark, markp); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -627,10 +689,10 @@ __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, co
 template <int LO, int HI, bool PERSIST, bool AV, bool AFF>
 __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ scns, const StageTask* __restrict__ tasks,
                                                  int n, int xcd, int tile, int src, double rkA, double rkC,
-                                                 int last, const int* __restrict__ markp, int stage) {
+                                                 int last, int* markp, int stage) {
     __shared__ __attribute__((aligned(16))) double lds[MaxLds<LO, HI>::value];
     __shared__ double sD[HI * HI];
-    const int base = AV ? *markp : 0, mark = base + stage, next_mark = last ? base + STAGE_MARKS : mark + 1;
+    const int base = AV ? markp[src ^ (stage & 1)] : 0, mark = base + stage, next_mark = last ? base + STAGE_MARKS : mark + 1;
     const int b = blockIdx.x;
     int beg = 0, cnt = n, i0 = b, stride = gridDim.x;
     if (xcd) {
@@ -640,15 +702,17 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
         i0 = b >> 3;
         stride = gridDim.x >> 3;
     }
+    // (the tasks of a single scenario need no list)
+    auto task = [&](int i) { return tasks ? tasks[i] : StageTask{0, i * (64 / LO), LO, 0}; };
     if constexpr (!PERSIST) {
-        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i0], lds, sD, src, rkA, rkC, last != 0, mark, next_mark);
+        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, task(beg + i0), lds, sD, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
     } else {
         const int nch = (cnt + tile - 1) / tile;
         for (int c = i0; c < nch; c += stride) {
             const int i1 = min(cnt, (c + 1) * tile);
             for (int i = c * tile; i < i1; ++i) {
                 if (i != i0 * tile) __syncthreads();   // LDS of the previous task is free
-                stage_task<LO, HI, AV, AFF>(scns, tasks[beg + i], lds, sD, src, rkA, rkC, last != 0, mark, next_mark);
+                stage_task<LO, HI, AV, AFF>(scns, task(beg + i), lds, sD, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
             }
         }
     }
@@ -679,53 +743,10 @@ __global__ void __launch_bounds__(256) k_stage_lambda(const StageScn* __restrict
         for (int off = 32; off > 0; off >>= 1) lam = fmax(lam, __shfl_xor(lam, off));
         if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = lam;
         __syncthreads();
-        if (threadIdx.x == 0) max_into(S.lmax, fmax(fmax(part[0], part[1]), fmax(part[2], part[3])));
+        if (threadIdx.x == 0) max_into(S.lmax + src, fmax(fmax(part[0], part[1]), fmax(part[2], part[3])));
         __syncthreads();
         lam = 0.0;
     }
-}
-
-// DGtimeloop's dt (src/deviceclass.cpp:899-930) per scenario: while t < T, dt = min(T - t,
-// dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T (or after a dt that is not positive
-// and finite, which is flagged) clock[0] = -1 and the stages leave the state unchanged.  (A batch that does
-// not freeze a failed state goes on with dt = 0 there: what is not finite spreads, as in
-// q + 0 gRK.)  lambda_max and eps_max are reset for the next step's reductions, and the step's marks begin.
-__global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn, int* mark) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nscn) return;
-    if (s == 0 && mark) *mark += STAGE_MARKS;
-    const StageScn& S = scns[s];
-    const double lm = __longlong_as_double((long long)*S.lmax);
-    *S.lmax = 0ull;
-    double em = 0.0;
-    if (S.av) {
-        em = __longlong_as_double((long long)*S.emax);
-        *S.emax = 0ull;
-    }
-    double* ck = S.clock;
-    const double t = ck[1];
-    double dt = -1.0;
-    if (t < S.T && ck[4] == 0.0) {
-        const double dt_i = S.dti / lm;
-        // with artificial viscosity also the viscous limit dvc / max eps (infinite where no element
-        // has viscosity), in the order of src/deviceclass.cpp:920-926
-        dt = S.av ? fmin(S.T - t, fmin(dt_i, S.dvc / em)) : fmin(S.T - t, dt_i);
-        if (!(dt > 0.0) || isinf(dt)) {
-            ck[4] = 1.0;
-            ck[5] = dt;
-            ck[6] = 1.0;
-            dt = S.freeze ? -1.0 : 0.0;
-        } else {
-            ck[1] = t + dt;
-            ck[2] += 1.0;
-            ck[3] = dt;
-            // the step that ends the run leaves its RK register for a checkpoint
-            ck[6] = (ck[2] == ck[7] || t + dt >= S.T) ? 1.0 : 0.0;
-        }
-    } else if (ck[4] != 0.0 && !S.freeze) {
-        dt = 0.0;
-    }
-    ck[0] = dt;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -741,11 +762,11 @@ __global__ void k_stage_dt(const StageScn* __restrict__ scns, int nscn, int* mar
 // ---------------------------------------------------------------------------------------------
 
 // Before the sensor pass of prime(): fresh marks, empty lists, no viscosity maximum.
-__global__ void k_stage_prime(const StageScn* __restrict__ scns, int nscn, int* mark, int* mcount) {
-    if (threadIdx.x == 0) *mark += STAGE_MARKS;
+__global__ void k_stage_prime(const StageScn* __restrict__ scns, int nscn, int src, int* mark, int* mcount) {
+    if (threadIdx.x == 0) mark[src] = max(mark[0], mark[1]) + STAGE_MARKS;
     if (threadIdx.x < 2 * MARK_LISTS) mcount[threadIdx.x] = 0;
     for (int s = threadIdx.x; s < nscn; s += blockDim.x)
-        if (scns[s].av) *scns[s].emax = 0ull;
+        if (scns[s].av) scns[s].emax[0] = scns[s].emax[1] = 0ull;
 }
 
 template <int LO, int HI>
@@ -787,7 +808,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
     __shared__ unsigned long long sMax;
     const StageTask tk = tasks[blockIdx.x];
     const StageScn& S = scns[tk.scn];
-    const int m = *markp + STAGE_MARKS;
+    const int m = markp[src];
     if (threadIdx.x == 0) sMax = 0ull;   // published by the sensor's first barrier
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                          \
@@ -799,7 +820,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
         default: break;
     }
     __syncthreads();
-    if (threadIdx.x == 0 && sMax) atomicMax(S.emax, sMax);
+    if (threadIdx.x == 0 && sMax) max_into(S.emax + src, __longlong_as_double((long long)sMax));
 }
 
 // One list's marked elements, ElemBlock<NGL>::EPB at a time, one thread per node; the elements of a
@@ -861,7 +882,7 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
     while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
     const int blk = (int)blockIdx.x - L.first[l];
     if (blk >= L.blocks[l]) return;
-    const int m = *markp + stage, ngl = L.ngl[l];
+    const int m = markp[src ^ (stage & 1)] + stage, ngl = L.ngl[l];
     const int64_t items = (int64_t)L.count[l][src] * 4 * ngl;
     for (int64_t it = (int64_t)blk * 256 + threadIdx.x; it < items; it += (int64_t)L.blocks[l] * 256) {
         const int li = (int)(it / (4 * ngl)), rem = (int)(it % (4 * ngl));
@@ -1139,7 +1160,7 @@ int StageBatch::reset_marks(esdg_ctx* ctx) {
 int StageBatch::prime(esdg_ctx* ctx, int src) {
     {
         KernelScope ks(ctx, "stage_mark");
-        k_stage_prime<<<1, 64, 0, ctx->stream>>>(d_scn, (int)host.size(), d_mark, d_mcount);
+        k_stage_prime<<<1, 64, 0, ctx->stream>>>(d_scn, (int)host.size(), src, d_mark, d_mcount);
         int rc = launch_check(ctx, "stage_prime");
         if (rc) return rc;
     }
@@ -1298,15 +1319,16 @@ int StageBatch::lambda(esdg_ctx* ctx, int src) {
 template <int LO, int HI, bool AV>
 static void launch_stage(hipStream_t st, const StageBatch& b, const StageBatch::Range& r, int src, double rkA,
                          double rkC, int last, int stage) {
+    const StageTask* tasks = b.host.size() == 1 && LO == HI ? nullptr : b.d_task + r.beg;
     if (r.persistent)
         // (the records of a Cartesian mesh serve the launches of one block per task)
-        k_stage<LO, HI, true, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, b.sched.tile,
+        k_stage<LO, HI, true, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, b.sched.tile,
                                                                 src, rkA, rkC, last, b.d_mark, stage);
     else if (r.affine)
-        k_stage<LO, HI, false, AV, true><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, 1, src, rkA,
+        k_stage<LO, HI, false, AV, true><<<r.grid, 64, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, 1, src, rkA,
                                                                 rkC, last, b.d_mark, stage);
     else
-        k_stage<LO, HI, false, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, b.d_task + r.beg, r.n, b.sched.xcd, 1, src, rkA,
+        k_stage<LO, HI, false, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, 1, src, rkA,
                                                                  rkC, last, b.d_mark, stage);
 }
 
@@ -1325,7 +1347,6 @@ static void launch_ranges(hipStream_t st, const StageBatch& b, const StageBatch:
 }
 
 int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src) {
-    const int ns = (int)host.size();
     if (nind && !mlp) return set_error(ctx, ESDG_ERR_STATE, "learned scenarios without a network");
     auto indicator = [&](int s) {
         return mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit, d_icount);
@@ -1334,12 +1355,6 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
     // there already)
     int rc = nind ? indicator(0) : ESDG_OK;
     if (rc) return rc;
-    {
-        KernelScope ks(ctx, "stage_dt");
-        k_stage_dt<<<(ns + 63) / 64, 64, 0, ctx->stream>>>(d_scn, ns, d_mark);
-        rc = launch_check(ctx, "stage_dt");
-        if (rc) return rc;
-    }
     for (int s = 0; s < stages; ++s) {
         const int last = (s == stages - 1);
         if (split && ctx->side && !ctx->profile) {

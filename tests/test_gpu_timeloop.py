@@ -476,3 +476,26 @@ def test_fused_every_degree_equals_sequence_bitwise(dev, N, mesh, av):
     for o in outs[1:]:
         assert o[:2] == ref[:2]
         assert all(np.array_equal(a, b) for a, b in zip(o[2:], ref[2:]))
+
+
+@pytest.mark.parametrize("av", [0, 1])
+@pytest.mark.parametrize("fused", [1, 2])
+def test_step_counts_of_either_parity(dev, fused, av):
+    """The step's clock, maxima and marks alternate between two halves: calls of odd and even step counts, a
+    call of no steps, and a new state between calls equal one run of the same steps, bit for bit."""
+    case = Case.dam_break(N=4, nel=9, noise=1e-3, seed=6)
+    rp = RunParams(num_flux=3, artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        a, b = dev.Solver(ctx, case, rp, fused=fused), dev.Solver(ctx, case, rp, fused=fused)
+        assert a.run(9)[0] == 9
+        assert [b.run(k)[0] for k in (1, 2, 0, 3, 1, 2)] == [1, 2, 0, 3, 1, 2]
+        assert a.time() == b.time() and np.array_equal(a.get_q(), b.get_q())
+        for s, parts in ((a, (4,)), (b, (3, 1))):
+            s.set_q(case["q"])
+            assert sum(s.run(k)[0] for k in parts) == 4
+        assert np.array_equal(a.get_q(), b.get_q()) and a.last_dt() == b.last_dt()
+        a.close()
+        b.close()
+    finally:
+        ctx.close()
