@@ -60,7 +60,20 @@ __device__ __forceinline__ double uniform(double x) {
 // AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
 // record per element instead of five doubles per node; the bottom slopes too where they are constant.
 // The kernel moves its bytes at what streaming kernels reach here, so bytes are time.
-template <int NGL, bool AV, bool AFF, class Faces, class Early, class Dt>
+// LDS accesses of a wave complete in order: the lanes of a block of one wave, or with MW of the wave that the
+// caller is, see each other's.
+template <bool MW>
+__device__ __forceinline__ void wave_sync() {
+    if constexpr (MW) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
+template <int NGL, bool AV, bool AFF, bool MW, class Faces, class Early, class Dt>
 __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, const Faces& faces, const Early& early,
                                            const Dt& step_dt, double g, double tol,
                                            double zero_tol, int positivity, double rkA, double rkC, bool last, gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
@@ -72,9 +85,9 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                                            gptr<const double> __restrict__ EleSizes,
                                            gptr<const double> __restrict__ GLw,
                                            const StageScn* SV, int src, int p,
-                                           int mark, int next_mark, double* sD) {
+                                           int mark, int next_mark, double* sD, double* mwFS) {
     using C = VolCfg<NGL>;
-    double* FS = P;                  // face fluxes, after the sweeps (the planes are free then)
+    double* FS = MW ? mwFS : P;      // face fluxes, after the sweeps (the planes are free then)
     const int4* rec = reinterpret_cast<const int4*>(P + C::ESZ);   // the element's side records
     double* MS = P + C::ESZ + 8;     // the limiter's and the sensor's sums
     const double* D = sD;
@@ -148,8 +161,11 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
     }
     dt = uniform(dt);   // (lane 0 has an element)
-    if (dt < 0.0) return;
-    __syncthreads();
+    if (dt < 0.0) {
+        if constexpr (MW) __syncthreads();   // (every wave of the block meets one barrier)
+        return;
+    }
+    wave_sync<MW>();
 
     // ---- column phase: xi-column r ----------------------------------------------------------
     const int64_t xb = (int64_t)e * C::NN + r;
@@ -168,7 +184,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             }
         }
     }
-    __syncthreads();
+    wave_sync<MW>();
     if (act) {
 #pragma unroll
         for (int c = 0; c < NGL; ++c) {
@@ -177,7 +193,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             P[2 * C::PLANE + r * C::RS + c] = a3[c];
         }
     }
-    __syncthreads();
+    wave_sync<MW>();
     double b1[NGL], b2[NGL], b3[NGL], rJ[NGL];
     if (act) {
 #pragma unroll
@@ -213,9 +229,13 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
     }
     // the face fluxes of the element's sides (from the stage-start state) into the planes, which
     // every lane has read by now
-    __syncthreads();
-    if (act) faces(FS);
-    __syncthreads();
+    if constexpr (MW) {
+        __syncthreads();     // the block's other waves have written them
+    } else {
+        __syncthreads();
+        if (act) faces(FS);
+        __syncthreads();
+    }
     if (act) {
         // surface lift: bottom/top sides first, then right/left (SurfaceKernel.okl).  FS holds
         // -ms F* (ms = +-1, so the sign is exact and -ms F* rJ equals the okl's -ms rJ F* bitwise).
@@ -317,7 +337,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
     if (positivity) {
         // PosPres.okl on the new state: the products h w, hu w, hv w (w = GLw[xi] GLw[eta] / Jinv) to the
         // planes; three lanes of the element add them in the okl's serial order (xi outer, eta inner)
-        __syncthreads();
+        wave_sync<MW>();
         double hmin = 0.0;
         if (act) {
             const double gx = GLw[r];
@@ -331,7 +351,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             }
             P[3 * C::PLANE + r] = hmin;
         }
-        __syncthreads();
+        wave_sync<MW>();
         if (act && r < 3) {
             const double* F = P + r * C::PLANE;
             double a = 0.0;
@@ -339,7 +359,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 for (int k = 0; k < NGL; ++k) a += F[k * C::RS + l];
             MS[r] = a;
         }
-        __syncthreads();
+        wave_sync<MW>();
         if (act) {
             hmin = 0.0;
 #pragma unroll
@@ -438,7 +458,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         // lanes form the energy sums.  An element with viscosity marks what it reaches for the next stage,
         // and after the last stage its viscosity enters the next step's maximum.
         if (sensor) {
-            __syncthreads();
+            wave_sync<MW>();
             double* Tm = P + 1 * C::PLANE;
             double* V = sD;
             for (int t = lane; t < C::NN; t += 64) V[t] = glob(SV->VdmInv)[t];
@@ -446,7 +466,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 #pragma unroll
                 for (int k = 0; k < NGL; ++k) P[k * C::RS + r] = b1[k];
             }
-            __syncthreads();
+            wave_sync<MW>();
             if (act) {
 #pragma unroll
                 for (int i = 0; i < NGL; ++i) w[i] = w[i] + P[r * C::RS + i];
@@ -458,7 +478,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                     Tm[a * C::RS + r] = s;
                 }
             }
-            __syncthreads();
+            wave_sync<MW>();
             if (act) {
 #pragma unroll
                 for (int l = 0; l < NGL; ++l) w[l] = Tm[r * C::RS + l];
@@ -470,10 +490,10 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                     Tm[r * C::RS + c] = s * s;
                 }
             }
-            __syncthreads();
+            wave_sync<MW>();
             if (act)
                 for (int k = r; k < 4; k += NGL) MS[k] = sensor_sum<NGL, C::RS, true>(Tm, k);
-            __syncthreads();
+            wave_sync<MW>();
             double eps = 0.0;
             if (act && r == 0) {
                 eps = sensor_ramp(MS[0], MS[1], MS[2], MS[3], SV->sc);
@@ -533,17 +553,18 @@ __device__ __forceinline__ double first_dt(const StageScn& S, gptr<const double>
     return dt;
 }
 
-template <int NGL, bool AV, bool AFF>
-__device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, int src, int stage,
+template <int NGL, bool AV, bool AFF, bool MW>
+__device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* lds, double* sD, double* mwF, int src, int stage,
                                            double rkA, double rkC, bool last, int mark, int next_mark, int* markp) {
     using C = VolCfg<NGL>;
     using SC = StageCfg<NGL>;
-    const int lane = threadIdx.x;
+    const int lane = MW ? threadIdx.x & 63 : threadIdx.x;
+    const int wave = MW ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
     // the marks of the stage's state have been used: the list that the next stage's marks go to is the
     // other one, and this one is empty when its turn comes
-    if (AV && S.av && e0 == 0 && lane == 0) S.mcount[src] = 0;
-    if (stage == 1 && e0 == 0 && lane == 0) {
+    if (AV && S.av && e0 == 0 && lane == 0 && wave == 0) S.mcount[src] = 0;
+    if (stage == 1 && e0 == 0 && lane == 0 && wave == 0) {
         // the first stage has read the step's maxima: they are empty when the next step's last stage adds
         // to them; and the next step's marks
         S.lmax[p] = 0ull;
@@ -551,7 +572,8 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
         if (AV && S.id == 0) markp[p ^ 1] = markp[p] + STAGE_MARKS;
     }
     // D of this degree in LDS (wave-uniform reads, broadcast): keeps it out of the scalar registers
-    for (int t = lane; t < NGL * NGL; t += 64) sD[t] = glob(S.D)[t];
+    if (wave == 0)
+        for (int t = lane; t < NGL * NGL; t += 64) sD[t] = glob(S.D)[t];
     const int el = lane / NGL, r = lane % NGL;
     const int e = e0 + el;
     const bool act = (el < C::EPW) && (e < S.Nelem);
@@ -569,7 +591,7 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     for (int j = 0; j < FPL; ++j) {
         const int sd = r + j * NGL;
         rec[j] = make_int4(0, 0, 0, 0);
-        if (act && sd < 4) rec[j] = side_record(S, e, sd);
+        if (act && sd < 4 && wave == 0) rec[j] = side_record(S, e, sd);
     }
     int4* RS = reinterpret_cast<int4*>(P + C::ESZ);
     auto early = [&]() {
@@ -595,7 +617,7 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
             double nx, ny, sc, bl, br;
         };
         auto load = [&](int s, Side& d) {
-            const int4 R4 = RS[s];
+            const int4 R4 = MW ? side_record(S, e, s) : RS[s];
             const int f = R4.x;
             d.w = (unsigned)R4.w;
             d.rev = (int)((d.w >> 5) & 1u);
@@ -638,6 +660,11 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
             FS[(s * 3 + 2) * NGL + r] = nms * (d.sc * S.geomFace * F2);
         };
         Side a, b;
+        if constexpr (MW) {
+            load(wave - 1, a);
+            flux(wave - 1, a);
+            return;
+        }
         load(0, a);
         load(1, b);
         flux(0, a);
@@ -656,21 +683,29 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
         return first_dt(S, ck + 8 * p, lm, em, e0 == 0 && lane == 0 ? ck + 8 * (p ^ 1) : nullptr);
     };
 
-    __syncthreads();   // sD written
-    stage_core<NGL, AV, AFF>(e, r, act, P, faces, early, step_dt, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, last, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
+    double* const FSx = MW ? mwF + (act ? el : 0) * SC::FSZ : nullptr;
+    if constexpr (MW) {
+        if (wave > 0) {
+            if (act) faces(FSx);
+            __syncthreads();
+            return;
+        }
+    }
+    wave_sync<MW>();   // sD written
+    stage_core<NGL, AV, AFF, MW>(e, r, act, P, faces, early, step_dt, g, S.tol, S.zero_tol, S.positivity, rkA, rkC, last, qi, qo, glob(S.gRK), glob(S.Yeta), glob(S.Xeta), glob(S.Yxi),
                              glob(S.Xxi), glob(S.Jac), glob(S.Bx), glob(S.By), glob(S.geo), glob(S.EleSizes), glob(S.GLw),
-                             &S, src, p, mark, next_mark, sD);
+                             &S, src, p, mark, next_mark, sD, FSx);
 }
 
-template <int LO, int HI, bool AV, bool AFF>
+template <int LO, int HI, bool AV, bool AFF, bool MW = false>
 __device__ __forceinline__ void stage_task(const StageScn* __restrict__ scns, const StageTask& tk, double* lds,
-                                           double* sD, int src, int stage, double rkA, double rkC, bool last, int mark,
+                                           double* sD, double* mwF, int src, int stage, double rkA, double rkC, bool last, int mark,
                                            int next_mark, int* markp) {
     const StageScn& S = scns[tk.scn];
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                \
     case n:                                                                         \
-        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF>(S, tk.e0, lds, sD, src, stage, rkA, rkC, last, mark, next_mark, markp); \
+        if constexpr (n >= LO && n <= HI) stage_body<n, AV, AFF, MW>(S, tk.e0, lds, sD, mwF, src, stage, rkA, rkC, last, mark, next_mark, markp); \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -705,17 +740,40 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
     // (the tasks of a single scenario need no list)
     auto task = [&](int i) { return tasks ? tasks[i] : StageTask{0, i * (64 / LO), LO, 0}; };
     if constexpr (!PERSIST) {
-        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, task(beg + i0), lds, sD, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
+        if (i0 < cnt) stage_task<LO, HI, AV, AFF>(scns, task(beg + i0), lds, sD, nullptr, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
     } else {
         const int nch = (cnt + tile - 1) / tile;
         for (int c = i0; c < nch; c += stride) {
             const int i1 = min(cnt, (c + 1) * tile);
             for (int i = c * tile; i < i1; ++i) {
                 if (i != i0 * tile) __syncthreads();   // LDS of the previous task is free
-                stage_task<LO, HI, AV, AFF>(scns, task(beg + i), lds, sD, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
+                stage_task<LO, HI, AV, AFF>(scns, task(beg + i), lds, sD, nullptr, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
             }
         }
     }
+}
+
+// The same stage for short lists of tasks of one degree, where a stage takes as long as one wave's chain of
+// loads, sweeps and face fluxes: five waves per block, one for the elements and one for each of their
+// sides, whose fluxes are ready when the sweeps are.  16 x 16, N = 4: 11.6 us per stage with one wave per block,
+// 7.5 with five.
+template <int NGL, bool AV, bool AFF>
+__global__ void __launch_bounds__(320, 2) k_stage_wide(const StageScn* __restrict__ scns,
+                                                       const StageTask* __restrict__ tasks, int n, int xcd, int src,
+                                                       double rkA, double rkC, int last, int* markp, int stage) {
+    __shared__ __attribute__((aligned(16))) double lds[StageCfg<NGL>::LDS];
+    __shared__ double sD[NGL * NGL], mwF[StageCfg<NGL>::EPW * StageCfg<NGL>::FSZ];
+    const int base = AV ? markp[src ^ (stage & 1)] : 0, mark = base + stage, next_mark = last ? base + STAGE_MARKS : mark + 1;
+    int i = blockIdx.x, beg = 0, cnt = n;
+    if (xcd) {
+        const int q = n >> 3, rr = n & 7, x = i & 7;
+        cnt = q + (x < rr ? 1 : 0);
+        beg = x * q + (x < rr ? x : rr);
+        i >>= 3;
+    }
+    if (i >= cnt) return;
+    const StageTask tk = tasks ? tasks[beg + i] : StageTask{0, (beg + i) * (64 / NGL), NGL, 0};
+    stage_body<NGL, AV, AFF, true>(scns[tk.scn], tk.e0, lds, sD, mwF, src, stage, rkA, rkC, last != 0, mark, next_mark, markp);
 }
 
 // lambda_max of the state in buffer src, per scenario (FindLambdaMax.okl + the host max loop).  A block
@@ -1316,10 +1374,28 @@ int StageBatch::lambda(esdg_ctx* ctx, int src) {
     return launch_check(ctx, "stage_lambda");
 }
 
+// k_stage_wide where its blocks of five waves are all resident at once: one per CU, two at ngl <= 5, whose waves
+// need fewer registers.  us per step there and with k_stage: 16 x 16, N = 4, 45 and 68, 48 x 48 50 and 70, 64 x 64
+// (342 tasks) 74 and 78; 16 x 16, N = 7, 62 and 86, 45 x 45 (254 tasks) 70 and 92.  Beyond it k_stage has more
+// waves at work: 56 x 56, N = 7 (392 tasks) 115 and 99, 64 x 64, N = 5 (410 tasks) 88 and 86, 80 x 80, N = 4 (534
+// tasks) 97 and 86.
+static constexpr int wide_blocks_per_cu(int ngl) { return ngl <= 5 ? 2 : 1; }
+
 template <int LO, int HI, bool AV>
 static void launch_stage(hipStream_t st, const StageBatch& b, const StageBatch::Range& r, int src, double rkA,
                          double rkC, int last, int stage) {
     const StageTask* tasks = b.host.size() == 1 && LO == HI ? nullptr : b.d_task + r.beg;
+    if constexpr (LO == HI) {
+        if (!r.persistent && r.n <= b.ncu * wide_blocks_per_cu(LO)) {
+            if (r.affine)
+                k_stage_wide<LO, AV, true><<<r.grid, 320, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, src, rkA, rkC, last,
+                                                                   b.d_mark, stage);
+            else
+                k_stage_wide<LO, AV, false><<<r.grid, 320, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, src, rkA, rkC, last,
+                                                                    b.d_mark, stage);
+            return;
+        }
+    }
     if (r.persistent)
         // (the records of a Cartesian mesh serve the launches of one block per task)
         k_stage<LO, HI, true, AV, false><<<r.grid, 64, 0, st>>>(b.d_scn, tasks, r.n, b.sched.xcd, b.sched.tile,

@@ -499,3 +499,15 @@ def test_step_counts_of_either_parity(dev, fused, av):
         b.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("N,nel", [(2, 103), (2, 104), (4, 78), (4, 79), (5, 50), (5, 51), (7, 45), (7, 46), (7, 3)])
+def test_wide_blocks_up_to_one_round(dev, N, nel):
+    """Meshes on either side of the size up to which a block has five waves, and a mesh of one partly filled
+    block: the state after three steps equals the reference sequence's, bit for bit."""
+    case = Case.dam_break(N=N, nel=nel, noise=1e-3, seed=N)
+    rp = RunParams(num_flux=3, artificial_viscosity=1, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+    qa, na, ta = run_gpu(dev, case, rp, 3, fused=0)
+    qb, nb, tb = run_gpu(dev, case, rp, 3, fused=1)
+    assert na == nb == 3 and ta == tb
+    assert np.array_equal(qa, qb)
