@@ -336,16 +336,14 @@ __device__ __forceinline__ void flux_roe(const FluxConsts& c, double nx, double 
 __device__ __forceinline__ void numerical_flux(int kind, const FluxConsts& c, int cpuR, double nx, double ny,
                                                double hL, double huL, double hvL, double hR, double huR, double hvR,
                                                double bL, double bR, double& F0, double& F1, double& F2) {
-    switch (kind) {
-        case ESDG_FLUX_ES_ROTATED: flux_es_rotated(c, nx, ny, hL, huL, hvL, hR, huR, hvR, bL, bR, F0, F1, F2); break;
-        case ESDG_FLUX_LF: flux_lf(c, nx, ny, hL, huL, hvL, hR, huR, hvR, F0, F1, F2); break;
-        case ESDG_FLUX_ROE: flux_roe(c, nx, ny, hL, huL, hvL, hR, huR, hvR, F0, F1, F2); break;
-        case ESDG_FLUX_OCEAN:
-            if (cpuR == -1 && bL < 6.7) flux_roe(c, nx, ny, hL, huL, hvL, hR, huR, hvR, F0, F1, F2);
-            else flux_es_rotated(c, nx, ny, hL, huL, hvL, hR, huR, hvR, bL, bR, F0, F1, F2);
-            break;
-        default: flux_es(c, nx, ny, hL, huL, hvL, hR, huR, hvR, bL, bR, F0, F1, F2); break;
-    }
+    // one copy of each flux, the others out of the way of the rotated ES flux (which most runs take): the stage
+    // kernel is 40 to 70 KB of code, and what lies between the executed parts costs instruction fetches
+    const bool roe = kind == ESDG_FLUX_OCEAN ? (cpuR == -1 && bL < 6.7) : kind == ESDG_FLUX_ROE;
+    const bool rotated = kind == ESDG_FLUX_ES_ROTATED || (kind == ESDG_FLUX_OCEAN && !roe);
+    if (__builtin_expect(rotated, 1)) flux_es_rotated(c, nx, ny, hL, huL, hvL, hR, huR, hvR, bL, bR, F0, F1, F2);
+    else if (roe) flux_roe(c, nx, ny, hL, huL, hvL, hR, huR, hvR, F0, F1, F2);
+    else if (kind == ESDG_FLUX_LF) flux_lf(c, nx, ny, hL, huL, hvL, hR, huR, hvR, F0, F1, F2);
+    else flux_es(c, nx, ny, hL, huL, hvL, hR, huR, hvR, bL, bR, F0, F1, F2);
 }
 
 __device__ __forceinline__ int surf_node(int ngl, int side, int k) {

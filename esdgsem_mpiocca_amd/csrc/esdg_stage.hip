@@ -607,8 +607,7 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
         const GatherConsts gc{S.bc, S.h_zero};
         const gptr<const double> nxp = glob(S.nx), nyp = glob(S.ny), scp = glob(S.scal), bLp = glob(S.bL),
                                  bRp = glob(S.bR);
-        // one side's decoded record and loads: side s+1's loads are issued before side s's flux
-        // is evaluated, so a wave waits for memory once per element rather than once per side
+        // one side's decoded record and loads
         struct Side {
             int E[8];
             int ir, rev;     // the reversed face node (EdgeData[4]) of the lane's node; EOR
@@ -665,14 +664,18 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
             flux(wave - 1, a);
             return;
         }
-        load(0, a);
-        load(1, b);
-        flux(0, a);
-        load(2, a);
-        flux(1, b);
-        load(3, b);
-        flux(2, a);
-        flux(3, b);
+        // two sides at a time, in a loop of one copy of the code: unrolled over the four sides, with each
+        // side's loads issued before the fluxes of the one before it, the N = 7 kernels were 87 to 99 KB of
+        // code, more than the 64 KB of instruction cache, and slower (us per step with and without the
+        // loop: 256 x 256, N = 7, single kernel 596 and 624, 192 x 192 with analysis 352 and 390, 24 mixed
+        // scenarios 1073 and 1174, 512 x 512 with viscosity 3155 and 3228)
+#pragma unroll 1
+        for (int s = 0; s < 4; s += 2) {
+            load(s, a);
+            load(s + 1, b);
+            flux(s, a);
+            flux(s + 1, b);
+        }
     };
 
     auto step_dt = [&]() -> double {
