@@ -384,6 +384,34 @@ __device__ __forceinline__ double sensor_sum(const double* m, int which) {
     return s;
 }
 
+// The same sum of stored squares where the lanes of a wave take different ones: the two large sums share a loop
+// over all modes (one leaves terms out as + 0.0, the same bits), the two shell sums another; four branches in
+// turn took twice the additions.
+template <int NGL, int RS>
+__device__ __forceinline__ double sensor_sum_lane(const double* m, int which) {
+    constexpr int N = NGL - 1;
+    double s = 0.0;
+    if (which >= 2) {
+        const int n = which == 2 ? NGL : N;
+#pragma unroll
+        for (int i = 0; i < NGL; ++i)
+#pragma unroll
+            for (int j = 0; j < NGL; ++j) {
+                const double v = m[i * RS + j];
+                s += (i < n && j < n) ? v : 0.0;
+            }
+    } else {
+        const int k = N - which;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const double v = m[i * RS + k] + m[k * RS + i];
+            s += i < k ? v : 0.0;
+        }
+        s += m[k * RS + k];
+    }
+    return s;
+}
+
 // sigma = log10(max(z1/n1, z2/n2)) and the sine ramp to eps0 (ShockCapturing.okl:198-217)
 __device__ __forceinline__ double sensor_ramp(double z1, double z2, double n1, double n2, const SensorConsts& c) {
     const double t1 = (n1 < c.ZeroTOL) ? 0.0 : z1 / n1;
@@ -456,7 +484,7 @@ __device__ __forceinline__ double sensor_rows(int Nelem, int e0, const SensorCon
     }
     __syncthreads();
     if (act)
-        for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum<NGL, RB::RS, true>(T, w);   // (NGL = 3: lane 0 two)
+        for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum_lane<NGL, RB::RS>(T, w);   // (NGL = 3: lane 0 two)
     __syncthreads();
     double v = 0.0;
     if (act && r == 0) {

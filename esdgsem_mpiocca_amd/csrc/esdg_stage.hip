@@ -492,7 +492,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
             }
             wave_sync<MW>();
             if (act)
-                for (int k = r; k < 4; k += NGL) MS[k] = sensor_sum<NGL, C::RS, true>(Tm, k);
+                for (int k = r; k < 4; k += NGL) MS[k] = sensor_sum_lane<NGL, C::RS>(Tm, k);
             wave_sync<MW>();
             double eps = 0.0;
             if (act && r == 0) {

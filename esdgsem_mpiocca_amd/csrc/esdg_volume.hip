@@ -544,7 +544,7 @@ __device__ __forceinline__ void volume_body(int blk, VolLds<NGL>& L, int Nelem, 
                 }
                 __syncthreads();
                 if (act)
-                    for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum<NGL, C::RS, true>(Tm, w);
+                    for (int w = r; w < 4; w += NGL) sSum[el][w] = sensor_sum_lane<NGL, C::RS>(Tm, w);
                 __syncthreads();
                 if (act && r == 0) {
                     const double v = sensor_ramp(sSum[el][0], sSum[el][1], sSum[el][2], sSum[el][3], si.sc);
