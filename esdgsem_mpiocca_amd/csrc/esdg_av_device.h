@@ -1,6 +1,7 @@
-// esdg_av_device.h -- the artificial-viscosity element and face work, shared by the fused stage
-// (esdg_fused.hip: one mesh, face traces from the side-trace buffer) and the batched ensembles
-// (esdg_stage.hip: many meshes, face traces gathered from the state).  Both give the same bits.
+// esdg_av_device.h -- the artificial-viscosity element and face work, shared by the default schedule
+// (esdg_sequence.hip: face traces from qL and qR), the fused schedule's passes (esdg_fused.hip: from the
+// side-trace buffer) and the stage kernel's (esdg_stage.hip: many meshes, gathered from the state).  All give
+// the same bits.
 //
 //   br1_face_flux      calcNumFluxesGradient.okl:16-135 at one face node
 //   av_element_block   calcGradient.okl:18-156 + SurfaceKernelGradient.okl:16-148 +

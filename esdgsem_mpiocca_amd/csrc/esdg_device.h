@@ -385,8 +385,8 @@ __device__ __forceinline__ double sensor_sum(const double* m, int which) {
 }
 
 // The same sum of stored squares where the lanes of a wave take different ones: the two large sums share a loop
-// over all modes (one leaves terms out as + 0.0, the same bits), the two shell sums another; four branches in
-// turn took twice the additions.
+// over all modes (one leaves terms out as + 0.0, the same bits), the two shell sums another; four branches in turn
+// took twice the additions (160 x 160, N = 7, the default schedule with viscosity: 921 us per step, now 907).
 template <int NGL, int RS>
 __device__ __forceinline__ double sensor_sum_lane(const double* m, int which) {
     constexpr int N = NGL - 1;

@@ -141,6 +141,7 @@ class StageBatch {
     // is not set, which whoever changes the state, or which scenarios are learned, clears
     int prime(esdg_ctx* ctx, int src);
     bool primed = false;
+    int issued = 0;     // steps that run() has been asked for (as far as it matters)
     // one time step: dt kernel, then the RK stages [each after its viscous terms]; src flips once per
     // stage
     int step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src);

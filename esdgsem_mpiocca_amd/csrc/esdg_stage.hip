@@ -53,13 +53,6 @@ __device__ __forceinline__ double uniform(double x) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Volume term, surface lift, RK update, limiter and wave speed of one block of elements; the
-// face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
-// parameters are __restrict__ so that the geometry loads schedule as in a kernel taking them as
-// arguments, and global (gptr) so that they compile to global loads and stores.
-// AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
-// record per element instead of five doubles per node; the bottom slopes too where they are constant.
-// The kernel moves its bytes at what streaming kernels reach here, so bytes are time.
 // LDS accesses of a wave complete in order: the lanes of a block of one wave, or with MW of the wave that the
 // caller is, see each other's.
 template <bool MW>
@@ -73,10 +66,22 @@ __device__ __forceinline__ void wave_sync() {
     }
 }
 
+// Volume term, surface lift, RK update, limiter and wave speed of one block of elements; the
+// face fluxes of the elements' sides come from `faces`, into LDS (FS) after the sweeps.  Pointer
+// parameters are __restrict__ so that the geometry loads schedule as in a kernel taking them as
+// arguments, and global (gptr) so that they compile to global loads and stores.
+// AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
+// record per element instead of five doubles per node; the bottom slopes too where they are constant.
+// MW: the caller is the element wave of a block of five (k_stage_wide), the face fluxes come in mwFS.
+// What bounds it: on curved meshes the memory path (512 x 512, N = 7, with viscosity 2.71 GB in 610 us per
+// stage, 4.4 TB/s; an add of three large arrays reaches 5.65 here), on Cartesian meshes, whose records
+// leave 11 doubles per node, instruction issue (256 x 256, N = 7: 121 us per stage, 157 with metrics per
+// node), and on small ones one wave's chain of dependent steps.
 template <int NGL, bool AV, bool AFF, bool MW, class Faces, class Early, class Dt>
 __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, const Faces& faces, const Early& early,
                                            const Dt& step_dt, double g, double tol,
-                                           double zero_tol, int positivity, double rkA, double rkC, bool last, gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
+                                           double zero_tol, int positivity, double rkA, double rkC, bool last,
+                                           gptr<const double> __restrict__ qi, gptr<double> __restrict__ qo,
                                            gptr<double> __restrict__ gRK, gptr<const double> __restrict__ Yeta,
                                            gptr<const double> __restrict__ Xeta, gptr<const double> __restrict__ Yxi,
                                            gptr<const double> __restrict__ Xxi, gptr<const double> __restrict__ Jac,
@@ -787,7 +792,7 @@ __global__ void __launch_bounds__(256) k_stage_lambda(const StageScn* __restrict
     __shared__ double part[4];
     double lam = 0.0;
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const StageTask tk = tasks[i];
+        const StageTask tk = tasks ? tasks[i] : StageTask{0, i * (64 / scns[0].ngl), scns[0].ngl, 0};
         const StageScn& S = scns[tk.scn];
         const int ngl2 = tk.ngl * tk.ngl;
         const int nodes = min(64 / tk.ngl, S.Nelem - tk.e0) * ngl2;
@@ -800,7 +805,7 @@ __global__ void __launch_bounds__(256) k_stage_lambda(const StageScn* __restrict
             lam = fmax(lam, c + fmax(fabs(q[id + ngl2] * Qinv), fabs(q[id + 2 * ngl2] * Qinv)));
         }
         const int next = i + (int)gridDim.x;
-        if (next < n && tasks[next].scn == tk.scn) continue;
+        if (next < n && (!tasks || tasks[next].scn == tk.scn)) continue;
         for (int off = 32; off > 0; off >>= 1) lam = fmax(lam, __shfl_xor(lam, off));
         if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = lam;
         __syncthreads();
@@ -991,6 +996,8 @@ __global__ void __launch_bounds__(64) k_geo_records(int Nelem, int nn, const dou
     const int n = threadIdx.x;      // nn <= 64
     const double* a[7] = {Yeta, Xeta, Yxi, Xxi, Jac, Bx, By};
     for (int e = blockIdx.x; e < Nelem; e += gridDim.x) {
+        // (on a curved mesh the first elements settle it)
+        if (__hip_atomic_load(bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
         bool metrics = true, slopes = true;
         double first[7];
         for (int k = 0; k < 7; ++k) {
@@ -1076,32 +1083,27 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
             continue;
         }
         S.geo = S.fgeo = nullptr;
+        // one buffer (zero-filled): the flag, the element, face and side records.  (Where the mesh turns out to have
+        // no element and face records their part, 2 % of the mesh's arrays, stays unused: an
+        // allocation and a free of their own took as long as the passes.)
         int bad = 0;
-        double* geo = (double*)buffer((size_t)S.Nelem * 8 * sizeof(double));
-        int* dbad = (int*)buffer(sizeof(int));      // zero-filled
-        if (!rc) {
-            k_geo_records<<<(unsigned)std::min(S.Nelem, 16384), 64, 0, ctx->stream>>>(
-                S.Nelem, S.ngl * S.ngl, S.Yeta, S.Xeta, S.Yxi, S.Xxi, S.Jac, S.Bx, S.By, geo, dbad);
-            rc = launch_check(ctx, "geometry records");
-        }
+        char* buf = (char*)buffer(64 + ((size_t)S.Nelem * 2 + S.Nfaces) * 64);
+        int* dbad = (int*)buf;
+        double* geo = (double*)(buf + 64);
+        double* fgeo = geo + (size_t)S.Nelem * 8;
+        int4* d = (int4*)(fgeo + (size_t)S.Nfaces * 8);
+        if (rc) break;
+        k_geo_records<<<(unsigned)std::min(S.Nelem, 16384), 64, 0, ctx->stream>>>(
+            S.Nelem, S.ngl * S.ngl, S.Yeta, S.Xeta, S.Yxi, S.Xxi, S.Jac, S.Bx, S.By, geo, dbad);
+        rc = launch_check(ctx, "geometry records");
         if (!rc) rc = esdg_memcpy(ctx, &bad, dbad, sizeof bad, ESDG_D2H);
-        auto drop = [&](void* d) {
-            rec_bufs.erase(std::find(rec_bufs.begin(), rec_bufs.end(), d));
-            esdg_free(ctx, d);
-        };
-        if (!rc) drop(dbad);
-        if (!rc && bad) drop(geo);
         if (!rc && !bad) {
+            k_face_records<<<blocks_for(S.Nfaces, 256), 256, 0, ctx->stream>>>(S.Nfaces, S.ngl, S.nx, S.ny, S.scal, S.bL,
+                                                                               S.bR, fgeo);
+            rc = launch_check(ctx, "face records");
             S.geo = geo;
-            double* fgeo = (double*)buffer((size_t)S.Nfaces * 8 * sizeof(double));
-            if (!rc) {
-                k_face_records<<<blocks_for(S.Nfaces, 256), 256, 0, ctx->stream>>>(S.Nfaces, S.ngl, S.nx, S.ny, S.scal,
-                                                                                   S.bL, S.bR, fgeo);
-                rc = launch_check(ctx, "face records");
-            }
             S.fgeo = fgeo;
         }
-        int4* d = (int4*)buffer((size_t)S.Nelem * 4 * sizeof(int4));
         if (rc) break;
         k_side_records<<<blocks_for((int64_t)S.Nelem * 4, 256), 256, 0, ctx->stream>>>(S.Nelem, S.E2E, S.EOR, S.EMS,
                                                                                      S.EdgeData, S.fgeo, d);
@@ -1118,9 +1120,7 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
     if (!rc && has_av) {
         rc = esdg_malloc(ctx, (void**)&d_mark, 64);
         if (!rc) rc = esdg_malloc(ctx, (void**)&d_icount, 8 * IND_SLOTS * sizeof(unsigned long long));
-        if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_mark), 0.0, 8);
-        if (!rc) rc = esdg_fill(ctx, reinterpret_cast<double*>(d_icount), 0.0, 8 * IND_SLOTS);
-        if (!rc) rc = build_av_tasks(ctx);
+        if (!rc) rc = build_av_tasks(ctx);     // (allocations are zero-filled)
     }
     if (!rc) rc = set_schedule(ctx, StageSchedule{});
     return rc;
@@ -1356,14 +1356,17 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     add_group(0, nother);
     cur_learned = 1;
     add_group(nother, (int)tasks.size());
-    if (d_task && (int)tasks.size() != ntask) {
-        esdg_free(ctx, d_task);
-        d_task = nullptr;
+    // (the tasks of a single scenario follow from their index)
+    if (ns > 1) {
+        if (d_task && (int)tasks.size() != ntask) {
+            esdg_free(ctx, d_task);
+            d_task = nullptr;
+        }
+        int rc = ESDG_OK;
+        if (!d_task) rc = esdg_malloc(ctx, (void**)&d_task, tasks.size() * sizeof(StageTask));
+        if (!rc) rc = esdg_memcpy(ctx, d_task, tasks.data(), tasks.size() * sizeof(StageTask), ESDG_H2D);
+        if (rc) return rc;
     }
-    int rc = ESDG_OK;
-    if (!d_task) rc = esdg_malloc(ctx, (void**)&d_task, tasks.size() * sizeof(StageTask));
-    if (!rc) rc = esdg_memcpy(ctx, d_task, tasks.data(), tasks.size() * sizeof(StageTask), ESDG_H2D);
-    if (rc) return rc;
     ntask = (int)tasks.size();
     ranges = rg;
     sched = sc;
@@ -1387,7 +1390,7 @@ static constexpr int wide_blocks_per_cu(int ngl) { return ngl <= 5 ? 2 : 1; }
 template <int LO, int HI, bool AV>
 static void launch_stage(hipStream_t st, const StageBatch& b, const StageBatch::Range& r, int src, double rkA,
                          double rkC, int last, int stage) {
-    const StageTask* tasks = b.host.size() == 1 && LO == HI ? nullptr : b.d_task + r.beg;
+    const StageTask* tasks = b.d_task ? b.d_task + r.beg : nullptr;
     if constexpr (LO == HI) {
         if (!r.persistent && r.n <= b.ncu * wide_blocks_per_cu(LO)) {
             if (r.affine)
@@ -1485,7 +1488,11 @@ int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages,
         if (rc) return rc;
         marks_used += steps;
     }
-    if (sched.graph && !ctx->profile && steps >= 2) {
+    // A captured pair of steps takes about 100 us to capture and instantiate: the first few steps of a batch
+    // are launched one by one.
+    const int before = issued;
+    issued = (int)std::min<int64_t>((int64_t)issued + steps, 1 << 20);
+    if (sched.graph && !ctx->profile && steps >= 2 && (exec[src] || steps >= 8 || before >= 8)) {
         // two steps flip the buffers an even number of times, so the graph that starts from buffer
         // `src` ends there and can be replayed
         const int start = src;
