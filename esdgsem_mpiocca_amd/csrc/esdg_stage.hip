@@ -1042,9 +1042,11 @@ __global__ void __launch_bounds__(256) k_side_records(int Nelem, const int* __re
     if (t >= (int64_t)Nelem * 4) return;
     const int f = E2E[t] - 1;
     const int* E = ED + 8 * (int64_t)f;
+    // (of another rank only that it is one matters)
+    auto rank = [](int c) { return (unsigned)(min(max(c, -2), 253) + 2); };
     const unsigned w = (unsigned)(E[2] & 3) | ((unsigned)(E[3] & 3) << 2) | ((unsigned)(E[4] & 1) << 4) |
                        ((unsigned)(EOR[t] & 1) << 5) | ((EMS[t] > 0 ? 1u : 0u) << 6) |
-                       (((unsigned)(E[5] + 2) & 255u) << 8) | (((unsigned)(E[6] + 2) & 255u) << 16) |
+                       (rank(E[5]) << 8) | (rank(E[6]) << 16) |
                        ((fgeo && fgeo[8 * (int64_t)f + 7] != 0.0 ? 1u : 0u) << 24);
     rec[t] = make_int4(f, E[0], E[1], (int)w);
 }
