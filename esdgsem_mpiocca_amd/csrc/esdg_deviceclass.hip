@@ -459,9 +459,15 @@ class deviceclass {
                 S.SPV = o_SurfacePartsVisc;
                 S.active[0] = o_active[0]; S.active[1] = o_active[1];
             }
+            // a learned indicator that is set by now goes in at once
+            S.learned = rp_.artificial_viscosity && ind_ ? 1 : 0;
             rc = stage_.init(ctx_, std::vector<StageScn>{S}, rp_.fused == 1);
             if (rc) return rc;
             stage_ready = true;
+            stage_.mlp = S.learned ? ind_ : nullptr;
+            stage_.ind_lo = ind_lo;
+            stage_.ind_hi = ind_hi;
+            ind_changed = false;
         }
         // the learned indicator as last set on the solver
         if (rp_.artificial_viscosity && ind_changed) {

@@ -358,7 +358,7 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
                                                        const StageTask* __restrict__ tasks, int src,
                                                        const int* __restrict__ mark, int stage, MlpDev W, float lo,
                                                        float hi, int audit, unsigned long long* counters) {
-    const StageTask tk = tasks[blockIdx.x];
+    const StageTask tk = tasks ? tasks[blockIdx.x] : StageTask{0, (int)blockIdx.x * FEPB, 8, 0};
     const StageScn& S = scns[tk.scn];
     const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
     if (stage > 0 && S.clock[8 * (p ^ 1)] <= 0.0) return;

@@ -169,6 +169,7 @@ class StageBatch {
     bool has_av = false;
     StageTask *d_sens = nullptr, *d_ind = nullptr;
     int nsens = 0, nind = 0;
+    char* d_av = nullptr;                          // the allocation that holds the marks, lists and counts
     int2* d_mlist = nullptr;                       // the marked-element lists, one after another
     int* d_mcount = nullptr;                       // MARK_LISTS x 2 lengths
     int64_t mfirst[MARK_LISTS + 1] = {0};          // where each list starts in d_mlist

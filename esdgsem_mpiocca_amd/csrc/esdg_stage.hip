@@ -872,7 +872,8 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
     __shared__ double sT[MaxRowLds<LO, HI>::value];
     __shared__ double sSum[RowBlock<LO>::EPB][4];
     __shared__ unsigned long long sMax;
-    const StageTask tk = tasks[blockIdx.x];
+    const StageTask tk = tasks ? tasks[blockIdx.x]
+                               : StageTask{0, (int)blockIdx.x * (256 / scns[0].ngl), scns[0].ngl, 0};
     const StageScn& S = scns[tk.scn];
     const int m = markp[src];
     if (threadIdx.x == 0) sMax = 0ull;   // published by the sensor's first barrier
@@ -1120,9 +1121,20 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
     rc = esdg_malloc(ctx, (void**)&d_scn, host.size() * sizeof(StageScn));
     if (!rc) rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (!rc && has_av) {
-        rc = esdg_malloc(ctx, (void**)&d_mark, 64);
-        if (!rc) rc = esdg_malloc(ctx, (void**)&d_icount, 8 * IND_SLOTS * sizeof(unsigned long long));
-        if (!rc) rc = build_av_tasks(ctx);     // (allocations are zero-filled)
+        // one allocation (zero-filled): marks, list lengths, counts, and the lists, which hold every element of
+        // their scenarios at most once a stage; their total size does not depend on which are learned
+        size_t all = 0;
+        for (const StageScn& S : host)
+            if (S.av) all += S.Nelem;
+        const size_t counts = 8 * IND_SLOTS * sizeof(unsigned long long);
+        rc = esdg_malloc(ctx, (void**)&d_av, 128 + counts + all * sizeof(int2));
+        if (!rc) {
+            d_mark = (int*)d_av;
+            d_mcount = (int*)(d_av + 64);
+            d_icount = (unsigned long long*)(d_av + 128);
+            d_mlist = (int2*)(d_av + 128 + counts);
+            rc = build_av_tasks(ctx);
+        }
     }
     if (!rc) rc = set_schedule(ctx, StageSchedule{});
     return rc;
@@ -1132,7 +1144,7 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
 // (32-element tiles), and the layout of the marked-element lists.
 int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     std::vector<StageTask> sens, ind;
-    int64_t total[MARK_LISTS] = {0}, all = 0;
+    int64_t total[MARK_LISTS] = {0};
     auto list_of = [](const StageScn& S) { return S.learned ? MARK_LISTS - 1 : S.ngl - 3; };
     for (int s = 0; s < (int)host.size(); ++s) {
         const StageScn& S = host[s];
@@ -1143,14 +1155,6 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
         else
             for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
         total[list_of(S)] += S.Nelem;
-        all += S.Nelem;
-    }
-    // the lists hold every element of their scenarios at most once a stage; their total size does
-    // not depend on which scenarios are learned
-    if (!d_mlist) {
-        int rc = esdg_malloc(ctx, (void**)&d_mlist, (size_t)all * sizeof(int2));
-        if (!rc) rc = esdg_malloc(ctx, (void**)&d_mcount, MARK_LISTS * 2 * sizeof(int));
-        if (rc) return rc;
     }
     for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + total[l];
     for (int s = 0; s < (int)host.size(); ++s) {
@@ -1166,7 +1170,7 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
         if (d) esdg_free(ctx, d);
         d = nullptr;
         n = (int)v.size();
-        if (v.empty()) return ESDG_OK;
+        if (v.empty() || host.size() == 1) return ESDG_OK;   // (a single scenario's follow from their index)
         int rc = esdg_malloc(ctx, (void**)&d, v.size() * sizeof(StageTask));
         if (!rc) rc = esdg_memcpy(ctx, d, v.data(), v.size() * sizeof(StageTask), ESDG_H2D);
         return rc;
@@ -1534,10 +1538,8 @@ void StageBatch::release(esdg_ctx* ctx) {
     if (d_scn) esdg_free(ctx, d_scn);
     for (void* p : rec_bufs) esdg_free(ctx, p);
     rec_bufs.clear();
-    if (d_mark) esdg_free(ctx, d_mark);
-    if (d_icount) esdg_free(ctx, d_icount);
-    if (d_mlist) esdg_free(ctx, d_mlist);
-    if (d_mcount) esdg_free(ctx, d_mcount);
+    if (d_av) esdg_free(ctx, d_av);
+    d_av = nullptr;
     d_mlist = nullptr;
     d_mcount = nullptr;
     d_scn = nullptr;
