@@ -43,7 +43,7 @@ class deviceclass {
         A(&o_B, nodes); A(&o_Bx, nodes); A(&o_By, nodes); A(&o_x, nodes); A(&o_y, nodes);
         A(&o_nx, fn); A(&o_ny, fn); A(&o_scal, fn);
         A(&o_qL, fn * 3); A(&o_qR, fn * 3); A(&o_bL, fn); A(&o_bR, fn); A(&o_SurfaceParts, fn * 3);
-        A(&o_DBSurf1, fn); A(&o_DBSurf2, fn);
+        if (rp.fused == 0 && !fewer_passes()) { A(&o_DBSurf1, fn); A(&o_DBSurf2, fn); }
         A(&o_EleSizes, Nelem); A(&o_LambdaMax, Nelem); A(&o_ViscPara, Nelem); A(&o_ViscForPlot, Nelem);
         A(&o_red, 4);
         I(&o_EdgeData, (size_t)Nfaces * 8); I(&o_EdgeReversed, Nfaces);
@@ -74,6 +74,7 @@ class deviceclass {
         if (element_stage()) {
             // the stage kernel: second state buffer (ping-pong), lambda_max cell
             A(&o_q2, nodes * 3); A(reinterpret_cast<double**>(&o_lmax), 2);
+            A(&o_rec, record_bytes(Nelem, Nfaces) / sizeof(double));
             if (rp.artificial_viscosity) {
                 // the stage's gradient side traces, marks (one array per state buffer) and viscosity
                 // maximum (the viscous volume term goes to qGradientX, the viscous face fluxes to
@@ -447,6 +448,7 @@ class deviceclass {
             S.EdgeData = o_EdgeData; S.E2E = o_ElemToEdge; S.EMS = o_ElemEdgeMasterSlave; S.EOR = o_ElemEdgeOrientation;
             S.q[0] = o_q; S.q[1] = o_q2; S.gRK = o_gRK; S.clock = o_clock; S.lmax = o_lmax;
             S.emax = o_emax;
+            S.rec = o_rec;
             S.B = o_B;
             S.arrival = o_ArrivalTimings; S.maxelev = o_MaximumElevation;
             if (rp_.fused == 1) { S.lam = o_LambdaMax; S.freeze = 1; }
@@ -518,10 +520,10 @@ class deviceclass {
             if (p) esdg_free(ctx_, p);
         fused_.release(ctx_);
         stage_.release(ctx_);
-        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_gtr, (void*)o_Qv,
+        for (void* p : {(void*)o_q2, (void*)o_clock, (void*)o_lmax, (void*)o_rec, (void*)o_gtr, (void*)o_Qv,
                         (void*)o_active[0], (void*)o_active[1], (void*)o_emax})
             if (p) esdg_free(ctx_, p);
-        o_q2 = o_clock = o_gtr = o_Qv = nullptr;
+        o_q2 = o_clock = o_rec = o_gtr = o_Qv = nullptr;
         o_lmax = o_emax = nullptr;
         o_active[0] = o_active[1] = nullptr;
         o_q = o_Qt = o_gRK = o_Qtmp = nullptr;
@@ -600,7 +602,7 @@ class deviceclass {
     bool ind_changed = false;                // since the stage batch was given it
     float ind_lo = 0.0f, ind_hi = 1.0f;
     int ind_audit = 0;
-    double *o_q2 = nullptr, *o_clock = nullptr;
+    double *o_q2 = nullptr, *o_clock = nullptr, *o_rec = nullptr;
     unsigned long long* o_lmax = nullptr;
     // single-kernel stage with artificial viscosity
     double* o_gtr = nullptr;

@@ -69,7 +69,11 @@ struct StageScn {
     const int4* srec;
     // one record per element and per face of a mesh with element-wise constant metrics (else null)
     const double *geo, *fgeo;
+    void* rec;          // record_bytes of zeroed memory for them, or null: StageBatch::init allocates it
 };
+
+// bytes of a mesh's records (StageScn::rec)
+inline size_t record_bytes(int Nelem, int Nfaces) { return 64 + ((size_t)Nelem * 2 + Nfaces) * 64; }
 
 struct StageTask {
     int scn, e0, ngl, pad;

@@ -1090,7 +1090,7 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
         // no element and face records their part, 2 % of the mesh's arrays, stays unused: an
         // allocation and a free of their own took as long as the passes.)
         int bad = 0;
-        char* buf = (char*)buffer(64 + ((size_t)S.Nelem * 2 + S.Nfaces) * 64);
+        char* buf = S.rec ? (char*)S.rec : (char*)buffer(record_bytes(S.Nelem, S.Nfaces));
         int* dbad = (int*)buf;
         double* geo = (double*)(buf + 64);
         double* fgeo = geo + (size_t)S.Nelem * 8;
