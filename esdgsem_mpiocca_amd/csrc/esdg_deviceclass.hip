@@ -495,6 +495,11 @@ class deviceclass {
             if (!rc) rc = esdg_memcpy(ctx_, ck, o_clock + 8 * src, sizeof ck, ESDG_D2H);
             issued += chunk;
         }
+        if (!rc && ck[4] != 0.0 && rp_.fused == 1) {
+            // the state stays where the last good step left it, and that step did not know that the run ends with it
+            src = (int)ck[2] & 1;
+            if (ck[2] > 0.0) rc = stage_.repeat_last_stage(ctx_, A, Cc, stages, src, ck);
+        }
         if (!rc && src == 1)
             rc = hip_check(ctx_, hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double), hipMemcpyDeviceToDevice,
                                                 ctx_->stream), "state copy");

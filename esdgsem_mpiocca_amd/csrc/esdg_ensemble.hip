@@ -305,7 +305,7 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
     };
     rc = copy_all(true);
     // the learned indicator's counts are restored after the trials as well
-    unsigned long long icount[5] = {0, 0, 0, 0, 0}, dropped[5];
+    unsigned long long icount[5] = {0, 0, 0, 0, 0};
     if (!rc) rc = E->batch.take_counts(ctx, icount);
     const int src0 = E->src;
     const StageSchedule keep = E->batch.sched;
@@ -352,8 +352,7 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
         trial(s);
     }
     esdg_free(ctx, snap);
-    if (!rc) rc = E->batch.take_counts(ctx, dropped);
-    if (!rc && E->batch.d_icount) rc = esdg_memcpy(ctx, E->batch.d_icount, icount, sizeof icount, ESDG_H2D);
+    if (!rc) rc = E->batch.put_counts(ctx, icount);
     if (!rc) rc = E->batch.set_schedule(ctx, best_s);
     if (rc) return rc;
     if (best) esdg_ensemble_get_schedule(E, best);

@@ -373,9 +373,11 @@ __global__ void __launch_bounds__(256) k_ens_indicator(const StageScn* __restric
     MS.counters = counters + 8 * (blockIdx.x % IND_SLOTS);
     MS.scn = &S;
     MS.mark = mark[p] + stage;
-    MS.buffer = src;
+    // (a frozen failed scenario's state stays in the buffer of its last good step, which buffer 0 began)
+    const int buf = stage == 0 && S.freeze && S.clock[8 * p + 4] != 0.0 ? (int)S.clock[8 * p + 2] & 1 : src;
+    MS.buffer = buf;
     MS.stage = stage;
-    mlp_indicator_block(S.Nelem, tk.e0, glob((const double*)S.q[src]), glob(S.B), glob(S.VdmInv), W, lo, hi, nullptr,
+    mlp_indicator_block(S.Nelem, tk.e0, glob((const double*)S.q[buf]), glob(S.B), glob(S.VdmInv), W, lo, hi, nullptr,
                         MS);
 }
 

@@ -32,7 +32,7 @@ struct StageScn {
     // Of the clock, the maxima and the marks there are two, used by steps in turn: a step that starts from the
     // state in buffer p takes half p and leaves the other half for the next (the stages of a step are odd
     // in number, so that one starts from buffer p ^ 1).
-    double* clock;      // 2 x 8: [0] dt of the current step (-1: it changes nothing; 0: a failed scenario), [1] t,
+    double* clock;      // 2 x 8: [0] dt of the current step (-1: it changes nothing; -2 or 0: a failed scenario), [1] t,
                         // [2] steps taken, [3] dt of the last step taken, [4] 1 if a dt was not positive
                         // and finite ([5] that dt), [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
     unsigned long long* lmax;   // 2: bit pattern of max lambda (non-negative doubles order as integers)
@@ -55,8 +55,8 @@ struct StageScn {
     int2* mlist;
     int* mcount;
     int id;             // this scenario's index in the batch
-    int freeze;         // after a dt that was not positive and finite: 1 the state stays as it is, 0 it takes
-                        // q + 0 gRK
+    int freeze;         // after a dt that was not positive and finite: 1 both state buffers stay as they are, 0
+                        // the state takes q + 0 gRK
     // a single solver's buffers (each may be null): the element wave speeds of the state after a step,
     // and the analysis buffers, advanced after every step
     double *lam, *arrival, *maxelev;
@@ -142,8 +142,9 @@ class StageBatch {
     // initial lambda_max of every scenario from the state in buffer `src`
     int lambda(esdg_ctx* ctx, int src);
     // the sensor, marks and viscosity maximum of the state in buffer src; run() calls it when `primed`
-    // is not set, which whoever changes the state, or which scenarios are learned, clears
-    int prime(esdg_ctx* ctx, int src);
+    // is not set, which whoever changes the state, or which scenarios are learned, clears.  stage (even): the
+    // stage of the next step that the marks are for
+    int prime(esdg_ctx* ctx, int src, int stage = 0);
     bool primed = false;
     int issued = 0;     // steps that run() has been asked for (as far as it matters)
     // one time step: dt kernel, then the RK stages [each after its viscous terms]; src flips once per
@@ -151,6 +152,10 @@ class StageBatch {
     int step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src);
     // `steps` steps: pairs of steps replayed from a captured graph (schedule.graph), the rest eager
     int run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src);
+    // A batch of one scenario that freezes a failed state, after a run that failed: the last stage of the last good
+    // step again, from buffer dst ^ 1 into buffer dst, for the RK register, which a step stores to the end only
+    // where the run is known to end with it.  ck: the clock that the run left.
+    int repeat_last_stage(esdg_ctx* ctx, const double* A, const double* C, int stages, int dst, const double* ck);
     void release(esdg_ctx* ctx);
 
     struct Range {
@@ -186,6 +191,7 @@ class StageBatch {
     // the learned indicator's 5 counts: IND_SLOTS copies, 8 words apart, to be added
     unsigned long long* d_icount = nullptr;
     int take_counts(esdg_ctx* ctx, unsigned long long c[5]);   // since the last call
+    int put_counts(esdg_ctx* ctx, const unsigned long long c[5]);
     const esdg_mlp* mlp = nullptr;
     float ind_lo = 0.5f, ind_hi = 0.5f;
     int ind_audit = 0;
@@ -199,6 +205,10 @@ class StageBatch {
     std::vector<void*> rec_bufs;    // side, element and face records, per distinct mesh
     int build_av_tasks(esdg_ctx* ctx);
     int reset_marks(esdg_ctx* ctx);
+    // the learned scenarios' viscosities and marks of the state in buffer src, for stage s
+    int indicator(esdg_ctx* ctx, int src, int s);
+    // the stage's launches, one after another on the main stream
+    int launch_all(esdg_ctx* ctx, int src, double A, double C, int last, int s);
     // gradients, viscous volume and face terms of the marked elements, of the lists [l0, l1), on
     // stream st
     int av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipStream_t st);

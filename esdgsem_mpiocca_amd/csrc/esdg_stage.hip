@@ -139,15 +139,18 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 X[c] = Xeta[xb + c];
             }
         }
-        // a step that changes nothing has dt < 0: the state goes over to the other buffer as it is.  (dt is
-        // loaded beside the rows; a wave that waited for it before loading them cost 3 %.)
+        // a step that changes nothing has dt < 0: the state goes over to the other buffer as it is, or with -2
+        // both buffers keep theirs.  (dt is loaded beside the rows; a wave that waited for it before loading
+        // them cost 3 %.)
         dt = step_dt();
         if (dt < 0.0) {
+            if (dt != -2.0) {
 #pragma unroll
-            for (int c = 0; c < NGL; ++c) {
-                qo[qb + c] = h[c];
-                qo[qb + C::NN + c] = hu[c];
-                qo[qb + 2 * C::NN + c] = hv[c];
+                for (int c = 0; c < NGL; ++c) {
+                    qo[qb + c] = h[c];
+                    qo[qb + C::NN + c] = hu[c];
+                    qo[qb + 2 * C::NN + c] = hv[c];
+                }
             }
         } else {
         early();   // LDS stores of values loaded beside the row data
@@ -521,16 +524,18 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 
 
 // DGtimeloop's dt (src/deviceclass.cpp:899-930) of the step that starts from the scenario's clock ck: while
-// t < T, dt = min(T - t, dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T (or after a dt that is not
-// positive and finite, which is flagged) dt = -1 and the stages leave the state unchanged.  (A batch that does
-// not freeze a failed state goes on with dt = 0 there: what is not finite spreads, as in q + 0 gRK.)  Every
+// t < T, dt = min(T - t, dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T dt = -1 and the stages carry
+// the state over unchanged.  From a dt that is not positive and finite on, which is flagged, dt = -2 and nothing is
+// written: the last good step's state and the one before its last stage stay where they are (see
+// StageBatch::repeat_last_stage).  (A batch that does not freeze a failed state goes on with dt = 0 there: what
+// is not finite spreads, as in q + 0 gRK.)  Every
 // wave of a step's first stage forms it from the maxima that the last step's last stage left, beside its
 // row loads; the clock after it is written to `next` by one of them (as a launch of its own before the
 // stages it took 4 to 5 us per step).
 __device__ __forceinline__ double first_dt(const StageScn& S, gptr<const double> ck, double lm, double em,
                                            gptr<double> next) {
     const double t = ck[1], steps = ck[2], failed = ck[4], until = ck[7];
-    double dt = -1.0, t1 = t, n1 = steps, last = ck[3], err = failed, bad = ck[5], keep = ck[6];
+    double dt = failed != 0.0 ? -2.0 : -1.0, t1 = t, n1 = steps, last = ck[3], err = failed, bad = ck[5], keep = ck[6];
     if (t < S.T && failed == 0.0) {
         const double dt_i = S.dti / lm;
         // with artificial viscosity also the viscous limit dvc / max eps (infinite where no element
@@ -540,7 +545,7 @@ __device__ __forceinline__ double first_dt(const StageScn& S, gptr<const double>
             err = 1.0;
             bad = dt;
             keep = 1.0;
-            dt = S.freeze ? -1.0 : 0.0;
+            dt = S.freeze ? -2.0 : 0.0;
         } else {
             t1 = t + dt;
             n1 = steps + 1.0;
@@ -863,11 +868,11 @@ __device__ __forceinline__ void ens_sensor_body(const StageScn& S, int e0, int s
 
 // ShockCapturing of the state in buffer src over RowBlock tiles (tasks: {scenario, first element, ngl}), for
 // the first stage of a run: the stages evaluate it on the states that they write.  A block's largest
-// viscosity enters its scenario's eps_max; the marks are those of the next step's first stage.
+// viscosity enters its scenario's eps_max; the marks are those of stage `stage` (even) of the next step.
 template <int LO, int HI>
 __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__ scns,
                                                     const StageTask* __restrict__ tasks, int src,
-                                                    const int* __restrict__ markp) {
+                                                    const int* __restrict__ markp, int stage) {
     __shared__ double sV[HI * HI];
     __shared__ double sT[MaxRowLds<LO, HI>::value];
     __shared__ double sSum[RowBlock<LO>::EPB][4];
@@ -875,7 +880,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
     const StageTask tk = tasks ? tasks[blockIdx.x]
                                : StageTask{0, (int)blockIdx.x * (256 / scns[0].ngl), scns[0].ngl, 0};
     const StageScn& S = scns[tk.scn];
-    const int m = markp[src];
+    const int m = markp[src] + stage;
     if (threadIdx.x == 0) sMax = 0ull;   // published by the sensor's first barrier
     switch (tk.ngl) {
 #define ESDG_CASE(n)                                                                          \
@@ -1192,6 +1197,13 @@ int StageBatch::take_counts(esdg_ctx* ctx, unsigned long long c[5]) {
     return rc;
 }
 
+int StageBatch::put_counts(esdg_ctx* ctx, const unsigned long long c[5]) {
+    if (!d_icount) return ESDG_OK;
+    int rc = esdg_fill(ctx, reinterpret_cast<double*>(d_icount), 0.0, 8 * IND_SLOTS);
+    if (!rc) rc = esdg_memcpy(ctx, d_icount, c, 5 * sizeof c[0], ESDG_H2D);
+    return rc;
+}
+
 int StageBatch::set_indicator(esdg_ctx* ctx, const esdg_mlp* m, float lo, float hi) {
     if (m && !(lo <= hi)) return set_error(ctx, ESDG_ERR_ARG, "set_indicator: lo > hi");
     int learned = 0;
@@ -1224,7 +1236,7 @@ int StageBatch::reset_marks(esdg_ctx* ctx) {
     return rc;
 }
 
-int StageBatch::prime(esdg_ctx* ctx, int src) {
+int StageBatch::prime(esdg_ctx* ctx, int src, int stage) {
     {
         KernelScope ks(ctx, "stage_mark");
         k_stage_prime<<<1, 64, 0, ctx->stream>>>(d_scn, (int)host.size(), src, d_mark, d_mcount);
@@ -1234,7 +1246,7 @@ int StageBatch::prime(esdg_ctx* ctx, int src) {
     marks_used += 1;
     if (nsens) {
         KernelScope ks(ctx, "ens_sensor");
-        k_ens_sensor<3, 8><<<nsens, 256, 0, ctx->stream>>>(d_scn, d_sens, src, d_mark);
+        k_ens_sensor<3, 8><<<nsens, 256, 0, ctx->stream>>>(d_scn, d_sens, src, d_mark, stage);
         int rc = launch_check(ctx, "ens_sensor");
         if (rc) return rc;
     }
@@ -1434,14 +1446,27 @@ static void launch_ranges(hipStream_t st, const StageBatch& b, const StageBatch:
     }
 }
 
+int StageBatch::indicator(esdg_ctx* ctx, int src, int s) {
+    if (!nind) return ESDG_OK;
+    return mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit, d_icount);
+}
+
+int StageBatch::launch_all(esdg_ctx* ctx, int src, double A, double C, int last, int s) {
+    for (const Range& r : ranges) {
+        KernelScope ks(ctx, "stage");
+        if (has_av) launch_ranges<true>(ctx->stream, *this, r, src, A, C, last, s);
+        else launch_ranges<false>(ctx->stream, *this, r, src, A, C, last, s);
+        const int rc = launch_check(ctx, "stage");
+        if (rc) return rc;
+    }
+    return ESDG_OK;
+}
+
 int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src) {
     if (nind && !mlp) return set_error(ctx, ESDG_ERR_STATE, "learned scenarios without a network");
-    auto indicator = [&](int s) {
-        return mlp_ensemble_indicator(ctx, mlp, d_scn, d_ind, nind, src, d_mark, s, ind_lo, ind_hi, ind_audit, d_icount);
-    };
     // the learned scenarios' viscosity of the step's state (its maximum enters the dt; the others' is
     // there already)
-    int rc = nind ? indicator(0) : ESDG_OK;
+    int rc = indicator(ctx, src, 0);
     if (rc) return rc;
     for (int s = 0; s < stages; ++s) {
         const int last = (s == stages - 1);
@@ -1456,7 +1481,7 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
                     rc = launch_check(ctx, "stage");
                 }
             (void)hipEventRecord(ctx->join, ctx->side);
-            if (!rc && s > 0) rc = indicator(s);
+            if (!rc && s > 0) rc = indicator(ctx, src, s);
             if (!rc) rc = av_terms(ctx, src, s, MARK_LISTS - 1, MARK_LISTS, ctx->stream);
             for (const Range& r : ranges)
                 if (!rc && r.learned) {
@@ -1469,20 +1494,34 @@ int StageBatch::step(esdg_ctx* ctx, const double* A, const double* C, int stages
             continue;
         }
         if (has_av) {
-            if (nind && s > 0) rc = indicator(s);
+            if (s > 0) rc = indicator(ctx, src, s);
             if (!rc) rc = av_terms(ctx, src, s, 0, MARK_LISTS, ctx->stream);
             if (rc) return rc;
         }
-        for (const Range& r : ranges) {
-            KernelScope ks(ctx, "stage");
-            if (has_av) launch_ranges<true>(ctx->stream, *this, r, src, A[s], C[s], last, s);
-            else launch_ranges<false>(ctx->stream, *this, r, src, A[s], C[s], last, s);
-            rc = launch_check(ctx, "stage");
-            if (rc) return rc;
-        }
+        rc = launch_all(ctx, src, A[s], C[s], last, s);
+        if (rc) return rc;
         src ^= 1;
     }
     return ESDG_OK;
+}
+
+// Everything of that stage is computed anew from the state before it, the viscosities and marks too, so it writes the
+// same bits as it did.  Its clock is in the half that the good step left (ck: the clock after that step).
+int StageBatch::repeat_last_stage(esdg_ctx* ctx, const double* A, const double* C, int stages, int dst, const double* ck) {
+    const int src = dst ^ 1, s = stages - 1;
+    const double clock[8] = {ck[3], ck[1], ck[2], ck[3], 0.0, 0.0, 1.0, ck[7]};
+    unsigned long long counts[5];
+    int rc = esdg_memcpy(ctx, host[0].clock + 8 * dst, clock, sizeof clock, ESDG_H2D);
+    if (!rc) rc = take_counts(ctx, counts);
+    if (!rc && has_av) rc = prime(ctx, src, s);
+    if (!rc) rc = indicator(ctx, src, s);
+    if (!rc && has_av) rc = av_terms(ctx, src, s, 0, MARK_LISTS, ctx->stream);
+    if (!rc) rc = launch_all(ctx, src, A[s], C[s], 1, s);
+    // the network's viscosities are those of the state that the failed step started from
+    if (!rc) rc = indicator(ctx, dst, 0);
+    if (!rc) rc = put_counts(ctx, counts);
+    primed = false;
+    return rc;
 }
 
 int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src) {

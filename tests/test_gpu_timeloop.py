@@ -511,3 +511,81 @@ def test_wide_blocks_up_to_one_round(dev, N, nel):
     qb, nb, tb = run_gpu(dev, case, rp, 3, fused=1)
     assert na == nb == 3 and ta == tb
     assert np.array_equal(qa, qb)
+
+
+def register_run(dev, case, rp, fused, calls, net=None, fails=False):
+    """(steps, time, last dt, q, gRK) after the calls of run(), the last of which must fail with `fails`; `net`: (lo, hi)
+    of a learned indicator."""
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        s = dev.Solver(ctx, case, rp, fused=fused)
+        mlp = dev.MLP(ctx, seed=1) if net else None
+        if net:
+            s.set_indicator(mlp, *net)
+        n = 0
+        for k in calls[:-1] if fails else calls:
+            n += s.run(k)[0]
+        if fails:
+            with pytest.raises(dev.EsdgDeviceError, match="not positive and finite"):
+                s.run(calls[-1])
+        q = s.get_q()
+        out = (n, s.time(), s.last_dt(), q, s.view("gRK", q.size).download())
+        extra = [s.view(b, case.Nelem).download() for b in ("ViscPara", "ViscForPlot", "LambdaMax")]
+        s.close()
+        if mlp:
+            mlp.close()
+    finally:
+        ctx.close()
+    return out, extra
+
+
+@pytest.mark.parametrize("end", ["odd", "even", "chunks", "T"])
+@pytest.mark.parametrize("rk", [3, 4])
+@pytest.mark.parametrize("fused,N,av", [(1, 1, 0), (1, 4, 0), (2, 4, 0), (1, 7, 1), (2, 7, 1), (1, 8, 1)])
+def test_register_after_a_run(dev, fused, N, av, rk, end):
+    """The low-storage RK register that a run leaves (buffer "gRK", which a checkpoint holds) is the reference
+    sequence's, bit for bit: after odd and even step counts, more steps than are issued at a time, and a run that
+    ends at T."""
+    case = Case.dam_break(N=N, nel=5, noise=1e-3, seed=N)
+    kw = dict(num_flux=3, rk_order=rk, artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05, CFL=0.2)
+    calls = dict(odd=(2, 3), even=(1, 4), chunks=(67,), T=(100,))[end]
+    if end == "T":
+        kw["T"] = 4.5 * run_gpu(dev, case, RunParams(**kw), 1)[2]
+    rp = RunParams(**kw)
+    ref = register_run(dev, case, rp, 0, calls)[0]
+    got = register_run(dev, case, rp, fused, calls)[0]
+    assert np.abs(ref[4]).max() > 0 and np.isfinite(ref[4]).all()
+    assert got[:3] == ref[:3]
+    assert np.array_equal(got[3], ref[3]) and np.array_equal(got[4], ref[4])
+
+
+@pytest.mark.parametrize("split", [0, 1, 2])
+@pytest.mark.parametrize("N,kind", [(4, "overflow"), (7, "overflow"), (7, "viscosity"), (7, "learned")])
+def test_register_after_a_failed_step(dev, N, kind, split):
+    """A run that ends because the next dt is not positive and finite leaves q and the RK register as the last good
+    step left them, bit for bit, and the wave speeds and viscosities of that state: with a wave speed that has
+    overflowed (no finite end time bounds dt), and with DFL = 0, which gives dt = 0 once an element has viscosity.
+    split: steps taken by a first call, so that the failing step starts from either state buffer."""
+    case = Case.gaussian_bump(N=N, nel=5)
+    if kind == "overflow":
+        rp = RunParams(num_flux=3, CFL=8.0, T=np.inf)
+    else:
+        rp = RunParams(num_flux=3, artificial_viscosity=1, eps0=0.005, sigma_min=-4.0, sigma_max=-2.0, DFL=0.0)
+    ref, _ = register_run(dev, case, rp, 0, (split, 150), fails=True)
+    got, extra = register_run(dev, case, rp, 1, (split, 150), net=(0.0, 1.0) if kind == "learned" else None, fails=True)
+    assert ref[1] > 0 and (kind == "overflow" or np.isfinite(ref[4]).all() and np.abs(ref[4]).max() > 0)
+    assert got[:3] == ref[:3]
+    assert np.array_equal(got[3], ref[3], equal_nan=True)
+    assert np.array_equal(got[4], ref[4], equal_nan=True)
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        E = case.Nelem
+        dq, lam, visc, plot = ctx.array(got[3]), ctx.empty(E), ctx.empty(E), ctx.empty(E)
+        ctx.find_lambda_max(E, dq, lam)
+        assert np.array_equal(extra[2], lam.download(), equal_nan=True)
+        if rp.artificial_viscosity:
+            ctx.shock_capturing(E, dq, ctx.array(case["b"]), ctx.array(case["VdmInv"]), ctx.array(case["EleSizes"]), visc, plot)
+            assert np.array_equal(extra[0], visc.download()) and np.array_equal(extra[1], plot.download())
+            assert (extra[0] > 0).any()
+    finally:
+        ctx.close()
