@@ -503,6 +503,8 @@ class deviceclass {
         if (!rc && src == 1)
             rc = hip_check(ctx_, hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double), hipMemcpyDeviceToDevice,
                                                 ctx_->stream), "state copy");
+        // the stages leave ViscPara and ViscForPlot of the state that they write; a call without a step has none
+        if (!rc && issued == 0 && rp_.fused == 2 && rp_.artificial_viscosity && !ind_) rc = viscosity();
         if (!rc) rc = esdg_finish(ctx_);
         if (rc) return rc;
         t = ck[1];

@@ -589,3 +589,28 @@ def test_register_after_a_failed_step(dev, N, kind, split):
             assert (extra[0] > 0).any()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("steps", [0, 2])
+@pytest.mark.parametrize("ended", [False, True])
+def test_single_kernel_viscosity_of_the_state(dev, ended, steps):
+    """The single-kernel schedule leaves ViscPara and ViscForPlot of the state that a call ends with, also where the
+    call takes no step: none asked for, or the end time reached."""
+    case = Case.dam_break(N=4, nel=6, noise=1e-3, seed=3)
+    rp = RunParams(num_flux=3, artificial_viscosity=1, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05,
+                   T=0.0 if ended else 1e30)
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        E = case.Nelem
+        s = dev.Solver(ctx, case, rp, fused=2)
+        for q in (case["q"], 1.5 * case["q"].reshape(E, 3, -1)[::-1].ravel()):
+            s.set_q(q)
+            assert s.run(steps)[0] == (0 if ended else steps)
+            dq, visc, plot = ctx.array(s.get_q()), ctx.empty(E), ctx.empty(E)
+            ctx.shock_capturing(E, dq, ctx.array(case["b"]), ctx.array(case["VdmInv"]), ctx.array(case["EleSizes"]), visc, plot)
+            assert (visc.download() > 0).any()
+            assert np.array_equal(s.view("ViscPara", E).download(), visc.download())
+            assert np.array_equal(s.view("ViscForPlot", E).download(), plot.download())
+        s.close()
+    finally:
+        ctx.close()
