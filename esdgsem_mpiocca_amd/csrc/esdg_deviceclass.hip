@@ -470,6 +470,9 @@ class deviceclass {
             stage_.ind_lo = ind_lo;
             stage_.ind_hi = ind_hi;
             ind_changed = false;
+        } else if (bottom_shared) {
+            rc = stage_.refresh_faces(ctx_);
+            if (rc) return rc;
         }
         // the learned indicator as last set on the solver
         if (rp_.artificial_viscosity && ind_changed) {
@@ -575,8 +578,10 @@ class deviceclass {
         if (n == "gRK") return o_gRK;
         if (n == "qL") return o_qL;
         if (n == "qR") return o_qR;
-        if (n == "bL") return o_bL;
-        if (n == "bR") return o_bR;
+        if (n == "bL" || n == "bR") {
+            bottom_shared = true;
+            return n == "bL" ? o_bL : o_bR;
+        }
         if (n == "SurfaceParts") return o_SurfaceParts;
         if (n == "LambdaMax") return o_LambdaMax;
         if (n == "ViscPara") return o_ViscPara;
@@ -600,6 +605,7 @@ class deviceclass {
     const double rkD[3] = {0.0, 1.0, 0.5};
     double t = 0.0, last_dt = 0.0;
     bool bottom_done = false;
+    bool bottom_shared = false;     // a program has o_bL or o_bR and may write there between two calls
     bool lambda_fresh = false, visc_fresh = false;   // o_LambdaMax / o_ViscPara hold those of o_q
     FusedStage fused_;
     StageBatch stage_;

@@ -139,6 +139,8 @@ class StageBatch {
     // any_D: without it a degree's D must be the one that earlier batches of the process brought
     int init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D = false);
     int set_schedule(esdg_ctx* ctx, const StageSchedule& sc);
+    // a batch of one scenario: its face records anew, after something has written the arrays they are made from
+    int refresh_faces(esdg_ctx* ctx);
     // initial lambda_max of every scenario from the state in buffer `src`
     int lambda(esdg_ctx* ctx, int src);
     // the sensor, marks and viscosity maximum of the state in buffer src; run() calls it when `primed`

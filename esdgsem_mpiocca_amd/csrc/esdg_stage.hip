@@ -1057,6 +1057,20 @@ __global__ void __launch_bounds__(256) k_side_records(int Nelem, const int* __re
     rec[t] = make_int4(f, E[0], E[1], (int)w);
 }
 
+static int face_records(esdg_ctx* ctx, const StageScn& S, double* fgeo, int4* rec) {
+    if (fgeo)
+        k_face_records<<<blocks_for(S.Nfaces, 256), 256, 0, ctx->stream>>>(S.Nfaces, S.ngl, S.nx, S.ny, S.scal, S.bL, S.bR,
+                                                                           fgeo);
+    k_side_records<<<blocks_for((int64_t)S.Nelem * 4, 256), 256, 0, ctx->stream>>>(S.Nelem, S.E2E, S.EOR, S.EMS, S.EdgeData,
+                                                                                 fgeo, rec);
+    return launch_check(ctx, "face and side records");
+}
+
+int StageBatch::refresh_faces(esdg_ctx* ctx) {
+    const StageScn& S = host[0];
+    return S.fgeo ? face_records(ctx, S, const_cast<double*>(S.fgeo), const_cast<int4*>(S.srec)) : ESDG_OK;
+}
+
 int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D) {
     host = scns;
     if (scns.empty()) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one scenario");
@@ -1105,17 +1119,12 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
             S.Nelem, S.ngl * S.ngl, S.Yeta, S.Xeta, S.Yxi, S.Xxi, S.Jac, S.Bx, S.By, geo, dbad);
         rc = launch_check(ctx, "geometry records");
         if (!rc) rc = esdg_memcpy(ctx, &bad, dbad, sizeof bad, ESDG_D2H);
-        if (!rc && !bad) {
-            k_face_records<<<blocks_for(S.Nfaces, 256), 256, 0, ctx->stream>>>(S.Nfaces, S.ngl, S.nx, S.ny, S.scal, S.bL,
-                                                                               S.bR, fgeo);
-            rc = launch_check(ctx, "face records");
+        if (rc) break;
+        rc = face_records(ctx, S, bad ? nullptr : fgeo, d);
+        if (!bad) {
             S.geo = geo;
             S.fgeo = fgeo;
         }
-        if (rc) break;
-        k_side_records<<<blocks_for((int64_t)S.Nelem * 4, 256), 256, 0, ctx->stream>>>(S.Nelem, S.E2E, S.EOR, S.EMS,
-                                                                                     S.EdgeData, S.fgeo, d);
-        rc = launch_check(ctx, "side records");
         S.srec = d;
     }
     if (rc) return rc;

@@ -3,6 +3,7 @@
 Acceptance bar: relative L2 <= 1e-12 after a fixed number of steps; lake at rest
 keeps |u|, |v| <= 1e-13.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -614,3 +615,33 @@ def test_single_kernel_viscosity_of_the_state(dev, ended, steps):
         s.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("fused", SCHEDULES, ids=SCHEDULE_IDS)
+@pytest.mark.parametrize("mesh", ["affine", "curved"])
+def test_bottom_traces_written_between_runs(dev, mesh, fused):
+    """The buffers "bL" and "bR" are the bottom traces that the face fluxes read: what a program writes there between
+    two calls counts in the second, also where a Cartesian mesh's face geometry comes from records."""
+    case = Case.ocean_uplift(N=4, nel=6) if mesh == "affine" else Case.dam_break(N=4, nel=6, noise=1e-3, seed=2)
+    rp = RunParams(num_flux=3, **(dict(bc_kind=2, h_zero=4000.0) if mesh == "affine" else {}))
+    add = 0.01 * np.arange(case.Nfaces)[:, None] * (1.0 + np.outer(np.arange(case.Nfaces) % 2, np.arange(case.ngl)))
+    outs = []
+    for change in (False, True):
+        for f in (0, fused):
+            ctx = dev.Context(dev.make_params(case, rp))
+            try:
+                s = dev.Solver(ctx, case, rp, fused=f)
+                bufs = [s.view(b, case.Nfaces * case.ngl) for b in ("bL", "bR")]
+                s.run(2)
+                if change:
+                    for b in bufs:
+                        v = b.download() + add.ravel() / case.Nfaces
+                        ctx.check(dev.lib().esdg_memcpy(ctx.handle, ctypes.c_void_p(b.ptr), v.ctypes.data_as(ctypes.c_void_p),
+                                                        v.nbytes, dev.ESDG_H2D))
+                s.run(2)
+                outs.append(s.get_q())
+                s.close()
+            finally:
+                ctx.close()
+    assert np.array_equal(outs[0], outs[1]) and not np.array_equal(outs[0], outs[2])
+    assert np.array_equal(outs[2], outs[3])
