@@ -503,6 +503,10 @@ class deviceclass {
             src = (int)ck[2] & 1;
             if (ck[2] > 0.0) rc = stage_.repeat_last_stage(ctx_, A, Cc, stages, src, ck);
         }
+        if (!rc && faces_shared) {
+            double* q[2] = {o_q, o_q2};
+            rc = leave_faces(issued == 0 ? nullptr : q[ck[4] != 0.0 ? src : src ^ 1], q[src]);
+        }
         if (!rc && src == 1)
             rc = hip_check(ctx_, hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double), hipMemcpyDeviceToDevice,
                                                 ctx_->stream), "state copy");
@@ -572,6 +576,18 @@ class deviceclass {
         return a;
     }
 
+    // The fused schedule's buffers "FStar" (the numerical fluxes of the last stage's state; null: as they are) and
+    // "Traces" (the side traces of the state).  The stage kernel forms neither in memory: kept once a program has
+    // asked for one of them.
+    int leave_faces(const double* before, const double* q) {
+        int rc = ESDG_OK;
+        if (before) {
+            rc = fused_.begin(ctx_, before, o_ElemToEdge, o_EdgeData);
+            if (!rc) rc = fused_.faces(ctx_, fused_args());
+        }
+        return rc ? rc : fused_.begin(ctx_, q, o_ElemToEdge, o_EdgeData);
+    }
+
     void* buffer(const std::string& n) {
         if (n == "q") return o_q;
         if (n == "Qt") return o_Qt;
@@ -591,6 +607,15 @@ class deviceclass {
         if (n == "qGradientX") return o_qGradientX;
         if (n == "qGradientY") return o_qGradientY;
         if (element_stage()) {
+            if (rp_.fused == 1 && !faces_shared && (n == "FStar" || n == "Traces")) {
+                if (fused_.init(ctx_, Nelem, Nfaces, false) != ESDG_OK) {
+                    fused_.release(ctx_);
+                    return nullptr;
+                }
+                faces_shared = true;
+                // (after an odd number of steps both state buffers hold the last state by now)
+                if (stage_.issued > 0 && (leave_faces(o_q2, o_q) != ESDG_OK || esdg_finish(ctx_) != ESDG_OK)) return nullptr;
+            }
             if (n == "Grad") return o_gtr;
             if (n == "FVisc") return o_SurfacePartsVisc;
             if (n == "QVisc") return o_qGradientX;
@@ -605,6 +630,7 @@ class deviceclass {
     const double rkD[3] = {0.0, 1.0, 0.5};
     double t = 0.0, last_dt = 0.0;
     bool bottom_done = false;
+    bool faces_shared = false;      // a program has "FStar" or "Traces" of the stage kernel's fused schedule
     bool bottom_shared = false;     // a program has o_bL or o_bR and may write there between two calls
     bool lambda_fresh = false, visc_fresh = false;   // o_LambdaMax / o_ViscPara hold those of o_q
     FusedStage fused_;

@@ -49,6 +49,8 @@ class FusedStage {
     // One RK stage: residual, low-storage accumulate and update (gRK = rkA gRK + Qt; q += cdt gRK).
     // With AV: face -> AV element pass -> viscous face -> volume + surface + viscous + RK [-> limiter].
     int stage(esdg_ctx* ctx, int s, double rkA, double cdt, const FusedArgs& a);
+    // its face pass: F* from the side traces (with AV also the marks)
+    int faces(esdg_ctx* ctx, const FusedArgs& a);
     // side traces of q (the face pass reads them; each stage's update refreshes them): called
     // whenever q was set from outside the stages.  E2E, ED: the mesh's ElemToEdge and EdgeData
     // (the trace slots of the element sides are derived from them once)

@@ -284,13 +284,38 @@ int FusedStage::begin(esdg_ctx* ctx, const double* q, const int* E2E, const int*
     return write_traces(ctx, Nelem, q, tr, slot);
 }
 
-int FusedStage::stage(esdg_ctx* ctx, int, double rkA, double cdt, const FusedArgs& A) {
-    if (!ready) return set_error(ctx, ESDG_ERR_STATE, "fused stage used before init");
+int FusedStage::faces(esdg_ctx* ctx, const FusedArgs& A) {
     const int ngl = ctx->p.ngl;
     const int kind = ctx->p.num_flux;
     FluxConsts fc{ctx->p.g, ctx->p.geomFace, ctx->p.PosPresTOL, ctx->p.ES};
     GatherConsts gc{ctx->p.bc_kind, ctx->p.h_zero};
     const unsigned fb = blocks_for((int64_t)A.Nfaces * ngl, 256);
+    KernelScope ks(ctx, "fused_face");
+    auto launch = [&](auto av_tag, auto kind_tag) {
+        constexpr bool AVK = decltype(av_tag)::value;
+        constexpr int KK = decltype(kind_tag)::value;
+        k_fused_face<AVK, KK><<<fb, 256, 0, ctx->stream>>>(A.Nfaces, ngl, fc, gc, A.EdgeData, tr, A.nx, A.ny,
+                                                         A.scal, A.bL, A.bR, fstar, AVK ? A.ViscPara : nullptr,
+                                                         AVK ? active : nullptr, A.Nelem,
+                                                         AVK ? alist : nullptr, AVK ? acount : nullptr);
+    };
+    auto by_kind = [&](auto av_tag) {
+        switch (kind) {
+            case ESDG_FLUX_ES: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ES>{}); break;
+            case ESDG_FLUX_LF: launch(av_tag, std::integral_constant<int, ESDG_FLUX_LF>{}); break;
+            case ESDG_FLUX_ES_ROTATED: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ES_ROTATED>{}); break;
+            case ESDG_FLUX_ROE: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ROE>{}); break;
+            default: launch(av_tag, std::integral_constant<int, ESDG_FLUX_OCEAN>{}); break;
+        }
+    };
+    if (av) by_kind(std::true_type{});
+    else by_kind(std::false_type{});
+    return launch_check(ctx, "fused_face");
+}
+
+int FusedStage::stage(esdg_ctx* ctx, int, double rkA, double cdt, const FusedArgs& A) {
+    if (!ready) return set_error(ctx, ESDG_ERR_STATE, "fused stage used before init");
+    const int ngl = ctx->p.ngl;
     if (av) {
         // stage mark of the elements with viscosity in reach, advanced on the device (replays of a
         // captured step take fresh marks); the marks of earlier stages are other values, so
@@ -305,36 +330,13 @@ int FusedStage::stage(esdg_ctx* ctx, int, double rkA, double cdt, const FusedArg
         }
         if (rc) return rc;
     }
-    {
-        KernelScope ks(ctx, "fused_face");
-        auto launch = [&](auto av_tag, auto kind_tag) {
-            constexpr bool AVK = decltype(av_tag)::value;
-            constexpr int KK = decltype(kind_tag)::value;
-            k_fused_face<AVK, KK><<<fb, 256, 0, ctx->stream>>>(A.Nfaces, ngl, fc, gc, A.EdgeData, tr, A.nx, A.ny,
-                                                             A.scal, A.bL, A.bR, fstar, AVK ? A.ViscPara : nullptr,
-                                                             AVK ? active : nullptr, A.Nelem,
-                                                             AVK ? alist : nullptr, AVK ? acount : nullptr);
-        };
-        auto by_kind = [&](auto av_tag) {
-            switch (kind) {
-                case ESDG_FLUX_ES: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ES>{}); break;
-                case ESDG_FLUX_LF: launch(av_tag, std::integral_constant<int, ESDG_FLUX_LF>{}); break;
-                case ESDG_FLUX_ES_ROTATED: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ES_ROTATED>{}); break;
-                case ESDG_FLUX_ROE: launch(av_tag, std::integral_constant<int, ESDG_FLUX_ROE>{}); break;
-                default: launch(av_tag, std::integral_constant<int, ESDG_FLUX_OCEAN>{}); break;
-            }
-        };
-        if (av) by_kind(std::true_type{});
-        else by_kind(std::false_type{});
-        int rc = launch_check(ctx, "fused_face");
-        if (rc) return rc;
-    }
+    int rc = faces(ctx, A);
+    if (rc) return rc;
     if (!av) {
         // volume + surface + RK (+ the limiter on the new state) in one element pass, which writes
         // the side traces of the state it stores
         return fused_volume(ctx, A, rkA, cdt, fstar, nullptr, nullptr, tr, slot);
     }
-    int rc = ESDG_OK;
     {
         KernelScope ks(ctx, "fused_av");
         ESDG_FUSED_DISPATCH(ngl, launch_fused_av, ctx, A, *this);

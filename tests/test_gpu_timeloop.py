@@ -645,3 +645,38 @@ def test_bottom_traces_written_between_runs(dev, mesh, fused):
                 ctx.close()
     assert np.array_equal(outs[0], outs[1]) and not np.array_equal(outs[0], outs[2])
     assert np.array_equal(outs[2], outs[3])
+
+
+@pytest.mark.parametrize("late", [False, True])
+@pytest.mark.parametrize("calls", [(2,), (3,), (2, 3, 0)], ids=["even", "odd", "calls"])
+@pytest.mark.parametrize("N,av", [(2, 0), (4, 1), (7, 1), (8, 0)])
+def test_fused_face_buffers(dev, N, av, calls, late):
+    """The fused schedule's buffers "FStar" and "Traces", which programs can ask for before a run or after it: the
+    numerical fluxes of the last stage's state (the reference sequence's SurfaceParts) and the side traces of the
+    state, in face slots.  (Asked for after an odd number of steps, FStar starts with the next call.)"""
+    case = Case.dam_break(N=N, nel=6, noise=1e-3, seed=N)
+    rp = RunParams(num_flux=3, artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+    n, F = case.ngl, case.Nfaces
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        a, s = dev.Solver(ctx, case, rp, fused=0), dev.Solver(ctx, case, rp, fused=1)
+        if not late:
+            s.view("FStar", F * 3 * n), s.view("Traces", F * 6 * n)
+        for k in calls:
+            assert a.run(k)[0] == s.run(k)[0] == k
+        tr, fs = s.view("Traces", F * 6 * n).download().reshape(F, 2, 3, n), s.view("FStar", F * 3 * n).download()
+        q = s.get_q().reshape(case.Nelem, 3, n * n)
+        assert np.array_equal(q.ravel(), a.get_q())
+        k = np.arange(n)
+        node = np.stack([k, (k + 1) * n - 1, n * n - n + k, k * n])
+        E = case["EdgeData"].reshape(F, 8)
+        for f in range(F):
+            for side in (0, 1):
+                if E[f, 5 + side] == 0:
+                    assert np.array_equal(tr[f, side], q[E[f, side]][:, node[E[f, 2 + side]]]), (f, side)
+        if not (late and sum(calls) % 2):
+            assert np.array_equal(fs, a.view("SurfaceParts", F * 3 * n).download())
+        a.close()
+        s.close()
+    finally:
+        ctx.close()
