@@ -507,9 +507,11 @@ class deviceclass {
             double* q[2] = {o_q, o_q2};
             rc = leave_faces(issued == 0 ? nullptr : q[ck[4] != 0.0 ? src : src ^ 1], q[src]);
         }
-        if (!rc && src == 1)
-            rc = hip_check(ctx_, hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double), hipMemcpyDeviceToDevice,
-                                                ctx_->stream), "state copy");
+        if (src == 1) {   // (also after an error: q is the state of the steps that were taken)
+            const hipError_t e = hipMemcpyAsync(o_q, o_q2, (size_t)Nelem * ngl2 * 3 * sizeof(double),
+                                                hipMemcpyDeviceToDevice, ctx_->stream);
+            if (!rc) rc = hip_check(ctx_, e, "state copy");
+        }
         // the stages leave ViscPara and ViscForPlot of the state that they write; a call without a step has none
         if (!rc && issued == 0 && rp_.fused == 2 && rp_.artificial_viscosity && !ind_) rc = viscosity();
         if (!rc) rc = esdg_finish(ctx_);

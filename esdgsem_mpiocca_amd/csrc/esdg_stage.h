@@ -205,6 +205,10 @@ class StageBatch {
 
   private:
     std::vector<void*> rec_bufs;    // side, element and face records, per distinct mesh
+    bool graph_ok = true;           // no capture has been refused
+    // two steps from buffer `start` into exec[start], without running them.  A capture that the runtime refuses is no
+    // error: exec[start] stays null and this batch's steps are launched one by one.
+    int capture(esdg_ctx* ctx, const double* A, const double* C, int stages, int start);
     int build_av_tasks(esdg_ctx* ctx);
     int reset_marks(esdg_ctx* ctx);
     // the learned scenarios' viscosities and marks of the state in buffer src, for stage s

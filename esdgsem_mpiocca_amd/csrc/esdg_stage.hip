@@ -1533,6 +1533,25 @@ int StageBatch::repeat_last_stage(esdg_ctx* ctx, const double* A, const double* 
     return rc;
 }
 
+int StageBatch::capture(esdg_ctx* ctx, const double* A, const double* C, int stages, int start) {
+    if (hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+        (void)hipGetLastError();
+        graph_ok = false;
+        return ESDG_OK;
+    }
+    int rc = ESDG_OK, src = start;
+    for (int k = 0; k < 2 && !rc; ++k) rc = step(ctx, A, C, stages, src);
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
+    if (!rc && (e != hipSuccess || !g || hipGraphInstantiate(&exec[start], g, nullptr, nullptr, 0) != hipSuccess)) {
+        (void)hipGetLastError();
+        exec[start] = nullptr;
+        graph_ok = false;
+    }
+    if (g) (void)hipGraphDestroy(g);
+    return rc;
+}
+
 int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src) {
     int n = 0;
     if (has_av) {
@@ -1546,29 +1565,15 @@ int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages,
     // are launched one by one.
     const int before = issued;
     issued = (int)std::min<int64_t>((int64_t)issued + steps, 1 << 20);
-    if (sched.graph && !ctx->profile && steps >= 2 && (exec[src] || steps >= 8 || before >= 8)) {
+    if (sched.graph && graph_ok && !ctx->profile && steps >= 2 && (exec[src] || steps >= 8 || before >= 8)) {
         // two steps flip the buffers an even number of times, so the graph that starts from buffer
         // `src` ends there and can be replayed
-        const int start = src;
-        if (!exec[start]) {
-            hipGraph_t gph = nullptr;
-            int rc = hip_check(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "graph capture");
-            if (rc) return rc;
-            int s2 = start;
-            for (int k = 0; k < 2 && rc == ESDG_OK; ++k) rc = step(ctx, A, C, stages, s2);
-            const hipError_t e = hipStreamEndCapture(ctx->stream, &gph);
-            if (rc) {
-                if (gph) (void)hipGraphDestroy(gph);
-                return rc;
-            }
-            rc = hip_check(ctx, e, "graph capture end");
-            if (rc) return rc;
-            rc = hip_check(ctx, hipGraphInstantiate(&exec[start], gph, nullptr, nullptr, 0), "graph instantiate");
-            (void)hipGraphDestroy(gph);
+        if (!exec[src]) {
+            const int rc = capture(ctx, A, C, stages, src);
             if (rc) return rc;
         }
-        for (; n + 2 <= steps; n += 2) {
-            int rc = hip_check(ctx, hipGraphLaunch(exec[start], ctx->stream), "graph launch");
+        for (; exec[src] && n + 2 <= steps; n += 2) {
+            int rc = hip_check(ctx, hipGraphLaunch(exec[src], ctx->stream), "graph launch");
             if (rc) return rc;
         }
     }

@@ -5,6 +5,8 @@ keeps |u|, |v| <= 1e-13.
 """
 import ctypes
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -680,3 +682,42 @@ def test_fused_face_buffers(dev, N, av, calls, late):
         s.close()
     finally:
         ctx.close()
+
+
+REFUSED = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)     # before the library: its calls bind here first
+import numpy as np
+import esdgsem_mpiocca_amd as E
+dev = E.device()
+case = E.Case.dam_break(N=4, nel=6, noise=1e-3, seed=2)
+rp = E.RunParams(num_flux=3, artificial_viscosity=1, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+ctx = dev.Context(dev.make_params(case, rp))
+outs = []
+for fused in (0, 1, 2):
+    s = dev.Solver(ctx, case, rp, fused=fused)
+    outs.append((s.run(3)[0] + s.run(20)[0], s.time(), s.get_q()))
+    s.close()
+ens = dev.Ensemble(ctx, [(case, rp, None)])
+ens.run(23)
+outs.append((ens.status(0)[1], ens.status(0)[0], ens.get_q(0)))
+ens.close()
+ctx.close()
+assert ctypes.c_int.in_dll(shim, "refused").value == 3
+assert all(o[:2] == outs[0][:2] and np.array_equal(o[2], outs[0][2]) for o in outs)
+print("same states")
+"""
+
+
+@pytest.mark.parametrize("call", ["int hipStreamBeginCapture(void* s, int mode) { return ++refused, 900; }",
+                                  "int hipGraphInstantiate(void** e, void* g, void** n, char* l, unsigned long k) { return ++refused, 2; }"],
+                         ids=["begin", "instantiate"])
+def test_refused_graph_capture_runs_eagerly(tmp_path, call):
+    """Where the runtime refuses to capture steps or to instantiate the graph, they are launched one by one: the same
+    states and times.  (In a process of its own, with that one call of the runtime replaced by a refusal.)"""
+    src, lib = tmp_path / "refuse.c", tmp_path / "librefuse.so"
+    src.write_text("int refused = 0;\n" + call + "\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    r = subprocess.run([sys.executable, "-c", REFUSED, str(lib)], capture_output=True, text=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0 and "same states" in r.stdout, r.stdout + r.stderr
