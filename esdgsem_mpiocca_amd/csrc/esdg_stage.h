@@ -50,10 +50,12 @@ struct StageScn {
     double* visc_plot;  // its copy (may be null)
     // active[b][e] == the stage's mark: viscosity on the element or a face neighbour in the state of
     // buffer b.  Those elements, each once, with those of every scenario of the same degree and
-    // indicator (learned or not): mlist[0 .. mcount[b]) = {scenario, element}
+    // indicator (learned or not), as {scenario, element} in MARK_SLOTS parts of a list: part s is
+    // mlist[s mcap .. s mcap + mark_count(mcount, b, s))
     int* active[2];
     int2* mlist;
     int* mcount;
+    int mcap;
     int id;             // this scenario's index in the batch
     int freeze;         // after a dt that was not positive and finite: 1 both state buffers stay as they are, 0
                         // the state takes q + 0 gRK
@@ -87,11 +89,33 @@ __device__ __forceinline__ void max_into(unsigned long long* cell, double m) {
     if (bits > __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(cell, bits);
 }
 
+// The part of its list that an element goes to, and the length of a part.  One length for all was a queue: where every
+// element has viscosity the stage took 1057 us at 300 x 300, N = 4, and 223 at 128 x 128, N = 7, and takes 128 and 51 with
+// 64 lengths in cache lines of their own.  Four consecutive elements go together (a group of the gradient pass at
+// N = 7); any 256 consecutive ones are dealt out evenly, the higher bits keep a front that crosses the rows of a mesh
+// from meeting in few parts.
+constexpr int MARK_SLOTS = 64, MARK_STRIDE = 16;
+__host__ __device__ constexpr int mark_capacity(int Nelem) { return 4 * ((Nelem + 255) / 256); }
+__host__ __device__ constexpr int mark_slot(int k) { return ((k >> 2) ^ (k >> 8) ^ (k >> 14) ^ (k >> 20)) & (MARK_SLOTS - 1); }
+constexpr bool deals_out(int first) {      // 256 elements from `first`: four to each part
+    int n[MARK_SLOTS] = {};
+    for (int k = 0; k < 256; ++k) n[mark_slot(first + k)] += 1;
+    for (int c : n)
+        if (c != 4) return false;
+    return true;
+}
+static_assert(deals_out(0) && deals_out(256) && deals_out(77 * 256) && deals_out(0x2a500 * 256), "a part holds mark_capacity elements");
+template <class P>
+__device__ __forceinline__ P mark_count(P mcount, int b, int slot) { return mcount + (b * MARK_SLOTS + slot) * MARK_STRIDE; }
+
 // An element with viscosity in the state of buffer b marks itself and its face neighbours for the stage that
 // starts from it (the elements whose viscous terms can be non-zero), as the fused face pass does for both
 // elements of every face with viscosity on either side.  The first to mark an element also lists it.
 __device__ __forceinline__ void mark_element(const StageScn& S, int k, int m, int b) {
-    if (atomicExch(S.active[b] + k, m) != m) S.mlist[atomicAdd(S.mcount + b, 1)] = make_int2(S.id, k);
+    if (atomicExch(S.active[b] + k, m) != m) {
+        const int s = mark_slot(k);
+        S.mlist[s * S.mcap + atomicAdd(mark_count(S.mcount, b, s), 1)] = make_int2(S.id, k);
+    }
 }
 // Side `side` of element e (record R, StageScn::srec): the neighbour there, and with side 0 the element itself.
 __device__ __forceinline__ void mark_side(const StageScn& S, int e, int side, const int4& R, int m, int b) {
@@ -114,12 +138,12 @@ constexpr int IND_SLOTS = 64;
 
 // The marked-element lists of a batch: one for the modal-sensor scenarios of each degree (ngl - 3)
 // and one for the learned ones (MARK_LISTS - 1).  A pass over them takes, of each list, the blocks
-// [first, first + blocks) of its grid.
+// [first, first + blocks) of its grid, every MARK_SLOTS-th of them for the same part.
 constexpr int MARK_LISTS = 7;
 struct MarkLists {
     const int2* list[MARK_LISTS];
     const int* count[MARK_LISTS];
-    int ngl[MARK_LISTS], first[MARK_LISTS], blocks[MARK_LISTS];
+    int ngl[MARK_LISTS], first[MARK_LISTS], blocks[MARK_LISTS], cap[MARK_LISTS];
 };
 
 // How the tasks of a stage are ordered and launched (the autotuner's search space).
@@ -182,7 +206,8 @@ class StageBatch {
     int nsens = 0, nind = 0;
     char* d_av = nullptr;                          // the allocation that holds the marks, lists and counts
     int2* d_mlist = nullptr;                       // the marked-element lists, one after another
-    int* d_mcount = nullptr;                       // MARK_LISTS x 2 lengths
+    int* d_mcount = nullptr;                       // MARK_LISTS x 2 x MARK_SLOTS lengths, MARK_STRIDE apart
+    int mcap[MARK_LISTS] = {0};                    // elements that a part of each list has room for
     int64_t mfirst[MARK_LISTS + 1] = {0};          // where each list starts in d_mlist
     // With both modal-sensor and learned scenarios the stage runs as two streams of work: the
     // other scenarios (sensor pass, their AV terms, their stage launches) on the second stream and

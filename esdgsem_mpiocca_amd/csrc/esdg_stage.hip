@@ -573,7 +573,7 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
     // the marks of the stage's state have been used: the list that the next stage's marks go to is the
     // other one, and this one is empty when its turn comes
-    if (AV && S.av && e0 == 0 && lane == 0 && wave == 0) S.mcount[src] = 0;
+    if (AV && S.av && e0 == 0 && wave == 0) *mark_count(S.mcount, src, lane) = 0;   // (a part per lane)
     if (stage == 1 && e0 == 0 && lane == 0 && wave == 0) {
         // the first stage has read the step's maxima: they are empty when the next step's last stage adds
         // to them; and the next step's marks
@@ -835,7 +835,7 @@ __global__ void __launch_bounds__(256) k_stage_lambda(const StageScn* __restrict
 // Before the sensor pass of prime(): fresh marks, empty lists, no viscosity maximum.
 __global__ void k_stage_prime(const StageScn* __restrict__ scns, int nscn, int src, int* mark, int* mcount) {
     if (threadIdx.x == 0) mark[src] = max(mark[0], mark[1]) + STAGE_MARKS;
-    if (threadIdx.x < 2 * MARK_LISTS) mcount[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < 2 * MARK_LISTS * MARK_SLOTS; i += blockDim.x) mcount[i * MARK_STRIDE] = 0;
     for (int s = threadIdx.x; s < nscn; s += blockDim.x)
         if (scns[s].av) scns[s].emax[0] = scns[s].emax[1] = 0ull;
 }
@@ -931,13 +931,15 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
     __shared__ double sEps[ElemBlock<LO>::EPB];
     int l = l0;
     while (l + 1 < l1 && (int)blockIdx.x >= L.first[l] + L.blocks[l]) ++l;
-    const int blk = (int)blockIdx.x - L.first[l], cnt = L.count[l][src];
+    const int blk = (int)blockIdx.x - L.first[l], slot = blk % MARK_SLOTS, cnt = *mark_count(L.count[l], src, slot);
     if (blk >= L.blocks[l]) return;
+    const int2* list = L.list[l] + slot * L.cap[l];
     switch (L.ngl[l]) {
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
         if constexpr (n >= LO && n <= HI)                                                     \
-            ens_grad_body<n>(scns, L.list[l], cnt, blk, L.blocks[l], src, sDh, sDs, sA, sB, sC, sE, sF, sEps); \
+            ens_grad_body<n>(scns, list, cnt, blk / MARK_SLOTS, L.blocks[l] / MARK_SLOTS, src, sDh, sDs, sA, sB, sC, sE, \
+                             sF, sEps);                                                       \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
 #undef ESDG_CASE
@@ -955,11 +957,13 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
     const int blk = (int)blockIdx.x - L.first[l];
     if (blk >= L.blocks[l]) return;
     const int m = markp[src ^ (stage & 1)] + stage, ngl = L.ngl[l];
-    const int64_t items = (int64_t)L.count[l][src] * 4 * ngl;
-    for (int64_t it = (int64_t)blk * 256 + threadIdx.x; it < items; it += (int64_t)L.blocks[l] * 256) {
+    const int slot = blk % MARK_SLOTS;
+    const int2* list = L.list[l] + slot * L.cap[l];
+    const int64_t items = (int64_t)*mark_count(L.count[l], src, slot) * 4 * ngl;
+    for (int64_t it = (int64_t)(blk / MARK_SLOTS) * 256 + threadIdx.x; it < items; it += (int64_t)(L.blocks[l] / MARK_SLOTS) * 256) {
         const int li = (int)(it / (4 * ngl)), rem = (int)(it % (4 * ngl));
         const int side = rem / ngl, i = rem % ngl;
-        const int2 me = L.list[l][li];
+        const int2 me = list[li];
         const StageScn& S = scns[me.x];
         const int f = S.E2E[me.y * 4 + side] - 1;
         const int* E = S.EdgeData + 8 * (int64_t)f;
@@ -1139,14 +1143,15 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
         // their scenarios at most once a stage; their total size does not depend on which are learned
         size_t all = 0;
         for (const StageScn& S : host)
-            if (S.av) all += S.Nelem;
+            if (S.av) all += (size_t)mark_capacity(S.Nelem) * MARK_SLOTS;
         const size_t counts = 8 * IND_SLOTS * sizeof(unsigned long long);
-        rc = esdg_malloc(ctx, (void**)&d_av, 128 + counts + all * sizeof(int2));
+        const size_t lengths = 2 * MARK_LISTS * MARK_SLOTS * MARK_STRIDE * sizeof(int);
+        rc = esdg_malloc(ctx, (void**)&d_av, 128 + counts + lengths + all * sizeof(int2));
         if (!rc) {
             d_mark = (int*)d_av;
-            d_mcount = (int*)(d_av + 64);
             d_icount = (unsigned long long*)(d_av + 128);
-            d_mlist = (int2*)(d_av + 128 + counts);
+            d_mcount = (int*)(d_av + 128 + counts);
+            d_mlist = (int2*)(d_av + 128 + counts + lengths);
             rc = build_av_tasks(ctx);
         }
     }
@@ -1158,7 +1163,7 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_
 // (32-element tiles), and the layout of the marked-element lists.
 int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     std::vector<StageTask> sens, ind;
-    int64_t total[MARK_LISTS] = {0};
+    for (int& c : mcap) c = 0;
     auto list_of = [](const StageScn& S) { return S.learned ? MARK_LISTS - 1 : S.ngl - 3; };
     for (int s = 0; s < (int)host.size(); ++s) {
         const StageScn& S = host[s];
@@ -1168,15 +1173,16 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
             for (int e0 = 0; e0 < S.Nelem; e0 += 32) ind.push_back(StageTask{s, e0, ngl, 0});
         else
             for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
-        total[list_of(S)] += S.Nelem;
+        mcap[list_of(S)] += mark_capacity(S.Nelem);
     }
-    for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + total[l];
+    for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + (int64_t)mcap[l] * MARK_SLOTS;
     for (int s = 0; s < (int)host.size(); ++s) {
         StageScn& S = host[s];
         S.id = s;
         if (!S.av) continue;
         S.mlist = d_mlist + mfirst[list_of(S)];
-        S.mcount = d_mcount + 2 * list_of(S);
+        S.mcount = d_mcount + 2 * MARK_SLOTS * MARK_STRIDE * list_of(S);
+        S.mcap = mcap[list_of(S)];
     }
     int rcs = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (rcs) return rcs;
@@ -1248,7 +1254,7 @@ int StageBatch::reset_marks(esdg_ctx* ctx) {
 int StageBatch::prime(esdg_ctx* ctx, int src, int stage) {
     {
         KernelScope ks(ctx, "stage_mark");
-        k_stage_prime<<<1, 64, 0, ctx->stream>>>(d_scn, (int)host.size(), src, d_mark, d_mcount);
+        k_stage_prime<<<1, 256, 0, ctx->stream>>>(d_scn, (int)host.size(), src, d_mark, d_mcount);
         int rc = launch_check(ctx, "stage_prime");
         if (rc) return rc;
     }
@@ -1272,9 +1278,10 @@ int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipS
         for (int l = l0; l < l1; ++l) {
             L.ngl[l] = l == MARK_LISTS - 1 ? 8 : l + 3;
             L.list[l] = d_mlist + mfirst[l];
-            L.count[l] = d_mcount + 2 * l;
+            L.count[l] = d_mcount + 2 * MARK_SLOTS * MARK_STRIDE * l;
+            L.cap[l] = mcap[l];
             L.first[l] = n;
-            L.blocks[l] = (int)std::min<int64_t>(cap, per_block(mfirst[l + 1] - mfirst[l], L.ngl[l]));
+            L.blocks[l] = (int)std::min<int64_t>(cap / MARK_SLOTS, per_block(mcap[l], L.ngl[l])) * MARK_SLOTS;
             n += L.blocks[l];
         }
         return std::make_pair(L, n);

@@ -223,3 +223,46 @@ def test_every_element_marked(dev, learned):
         want, nw, tw, _ = alone(dev, case, rp, q, 2)
         assert n == nw == 2 and t == tw
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("learned", [False, True], ids=["sensor", "learned"])
+def test_every_element_marked_part_sizes(dev, learned):
+    """The lists of marked elements are kept in parts that every 256 consecutive elements fill evenly: meshes of a few
+    elements, of exactly 256 and of 256 and a remainder, every element with viscosity, three of them in one list."""
+    kw = dict(sigma_min=-40.0, sigma_max=-2.5, eps0=1e-4, DFL=0.05)
+    mem = [(Case.dam_break(N=N, nel=nel, noise=1e-3, seed=nel, ratio=2.0, angle=0.4), av(**kw), None)
+           for N, nel in ((7, 2), (7, 16), (7, 17), (4, 3), (4, 32), (2, 33))]
+    seed, lo, hi = (3, -1.0, 2.0) if learned else (None, 0.5, 0.5)     # every element unsure
+    res, _ = run_ensemble(dev, mem, 3, net_seed=seed, lo=lo, hi=hi)
+    for (case, rp, q), (got, t, n) in zip(mem, res):
+        want, nw, tw, _ = alone(dev, case, rp, q, 3, fused=0)
+        assert n == nw == 3 and t == tw
+        assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("N,nel", [(4, 200), (7, 128)])
+def test_marking_every_element_is_not_serial(dev, N, nel):
+    """Viscosity on every element costs the stage little more than viscosity nowhere (both evaluate the sensor): with
+    one length for the whole list of marked elements, which all marks queued up for, it took 4 to 8 times as long."""
+    us = []
+    for smin in (-40.0, 40.0):
+        case = Case.dam_break(N=N, nel=nel, noise=1e-3, seed=1, build=False)
+        rp = av(sigma_min=smin, sigma_max=smin + 37.5, eps0=1e-4)
+        ctx = dev.Context(dev.make_params(case, rp))
+        try:
+            mesh = dev.DeviceCase(ctx, case)
+            s = dev.Solver(ctx, mesh, rp, fused=1)
+            s.run(2)
+            ctx.profile(True)
+            ctx.profile_reset()
+            s.run(3)
+            launches, ms = ctx.profile_query("stage")
+            assert launches == 15
+            visc = s.view("ViscPara", mesh.Nelem).download()
+            assert (visc > 0).all() if smin < 0 else (visc == 0).all()
+            us.append(ms / launches * 1e3)
+            s.close()
+            mesh.close()
+        finally:
+            ctx.close()
+    assert us[0] < 2.5 * us[1], us
