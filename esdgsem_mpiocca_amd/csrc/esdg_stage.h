@@ -32,7 +32,7 @@ struct StageScn {
     // Of the clock, the maxima and the marks there are two, used by steps in turn: a step that starts from the
     // state in buffer p takes half p and leaves the other half for the next (the stages of a step are odd
     // in number, so that one starts from buffer p ^ 1).
-    double* clock;      // 2 x 8: [0] dt of the current step (-1: it changes nothing; -2 or 0: a failed scenario), [1] t,
+    double* clock;      // 2 x 8: [0] dt of the current step (-1 or -2: it changes nothing; 0: a failed scenario), [1] t,
                         // [2] steps taken, [3] dt of the last step taken, [4] 1 if a dt was not positive
                         // and finite ([5] that dt), [6] 1 in the step that brings [2] to [7] or t to T: it stores gRK to the end
     unsigned long long* lmax;   // 2: bit pattern of max lambda (non-negative doubles order as integers)

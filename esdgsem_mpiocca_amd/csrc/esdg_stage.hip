@@ -139,7 +139,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
                 X[c] = Xeta[xb + c];
             }
         }
-        // a step that changes nothing has dt < 0: the state goes over to the other buffer as it is, or with -2
+        // a step that changes nothing has dt < 0: with -1 the state goes over to the other buffer as it is, with -2
         // both buffers keep theirs.  (dt is loaded beside the rows; a wave that waited for it before loading
         // them cost 3 %.)
         dt = step_dt();
@@ -524,9 +524,10 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 
 
 // DGtimeloop's dt (src/deviceclass.cpp:899-930) of the step that starts from the scenario's clock ck: while
-// t < T, dt = min(T - t, dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T dt = -1 and the stages carry
-// the state over unchanged.  From a dt that is not positive and finite on, which is flagged, dt = -2 and nothing is
-// written: the last good step's state and the one before its last stage stay where they are (see
+// t < T, dt = min(T - t, dti / lambda_max[, dvc / eps_max]) and t += dt; once t >= T the
+// steps change nothing: dt = -1 in the first stage, which carries the state over to the other buffer, and -2, with
+// which nothing is written, from there on.  From a dt that is not positive and finite on, which is flagged, dt = -2 at
+// once: the last good step's state and the one before its last stage stay where they are (see
 // StageBatch::repeat_last_stage).  (A batch that does not freeze a failed state goes on with dt = 0 there: what
 // is not finite spreads, as in q + 0 gRK.)  Every
 // wave of a step's first stage forms it from the maxima that the last step's last stage left, beside its
@@ -535,7 +536,7 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
 __device__ __forceinline__ double first_dt(const StageScn& S, gptr<const double> ck, double lm, double em,
                                            gptr<double> next) {
     const double t = ck[1], steps = ck[2], failed = ck[4], until = ck[7];
-    double dt = failed != 0.0 ? -2.0 : -1.0, t1 = t, n1 = steps, last = ck[3], err = failed, bad = ck[5], keep = ck[6];
+    double dt = failed != 0.0 || ck[0] < 0.0 ? -2.0 : -1.0, t1 = t, n1 = steps, last = ck[3], err = failed, bad = ck[5], keep = ck[6];
     if (t < S.T && failed == 0.0) {
         const double dt_i = S.dti / lm;
         // with artificial viscosity also the viscous limit dvc / max eps (infinite where no element
@@ -690,7 +691,10 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
 
     auto step_dt = [&]() -> double {
         const gptr<double> ck = glob(S.clock);
-        if (stage) return ck[8 * (p ^ 1)];
+        if (stage) {
+            const double dt = ck[8 * (p ^ 1)];
+            return dt < 0.0 ? -2.0 : dt;
+        }
         const double lm = __longlong_as_double((long long)glob(S.lmax)[p]);
         const double em = S.av ? __longlong_as_double((long long)glob(S.emax)[p]) : 0.0;
         return first_dt(S, ck + 8 * p, lm, em, e0 == 0 && lane == 0 ? ck + 8 * (p ^ 1) : nullptr);

@@ -266,3 +266,27 @@ def test_marking_every_element_is_not_serial(dev, N, nel):
         finally:
             ctx.close()
     assert us[0] < 2.5 * us[1], us
+
+
+def test_ended_scenario_stays(dev, mem):
+    """A scenario whose end time has passed keeps its state and time through further calls of odd and even step counts,
+    a new schedule among them, while the others go on as they would alone."""
+    case0, rp0, _ = mem[0]
+    ctx = dev.Context(dev.make_params(case0, rp0))
+    try:
+        ens = dev.Ensemble(ctx, mem)
+        ens.run(5)                       # the last scenario ends with its fifth step
+        end = ens.get_q(5)
+        for k in (1, 2):
+            ens.run(k)
+            assert np.array_equal(ens.get_q(5), end) and ens.status(5)[:2] == (mem[5][1].T, 5)
+        ens.autotune(trial_steps=3)
+        ens.run(STEPS - 8)
+        assert np.array_equal(ens.get_q(5), end) and ens.status(5)[:2] == (mem[5][1].T, 5)
+        for i, (case, rp, q) in enumerate(mem[:5]):
+            assert np.array_equal(ens.get_q(i), alone(dev, case, rp, q, STEPS)[0]), i
+        ens.close()
+    finally:
+        ctx.close()
+    case, rp, q = mem[5]
+    assert np.array_equal(end, alone(dev, case, rp, q, STEPS)[0])

@@ -721,3 +721,33 @@ def test_refused_graph_capture_runs_eagerly(tmp_path, call):
     r = subprocess.run([sys.executable, "-c", REFUSED, str(lib)], capture_output=True, text=True, timeout=100,
                        cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     assert r.returncode == 0 and "same states" in r.stdout, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("fused", [1, 2])
+def test_steps_after_the_end_write_nothing(dev, fused):
+    """Steps issued after t has reached T leave the state, which both buffers hold by then, without writing it again: a
+    launch of theirs takes a sixth of a stage's time (carrying the state over in every stage took a third)."""
+    case = Case.gaussian_bump(N=7, nel=256, build=False)
+    us, outs = [], []
+    for T in (1e30, 1e-9):
+        rp = RunParams(num_flux=3, T=T)
+        ctx = dev.Context(dev.make_params(case, rp))
+        try:
+            mesh = dev.DeviceCase(ctx, case)
+            s = dev.Solver(ctx, mesh, rp, fused=fused)
+            q0 = s.get_q()
+            s.run(1)
+            s.set_q(q0)
+            ctx.profile(True)
+            ctx.profile_reset()
+            n, t = s.run(4 if T > 1 else 64)
+            launches, ms = ctx.profile_query("stage")
+            assert (n, launches) == ((4, 20) if T > 1 else (1, 320))
+            us.append(ms / launches * 1e3)
+            outs.append((t, s.get_q(), q0))
+            s.close()
+            mesh.close()
+        finally:
+            ctx.close()
+    assert outs[1][0] == 1e-9 and np.abs(outs[1][1] - outs[1][2]).max() < 1e-6
+    assert us[1] < 0.25 * us[0], us
