@@ -463,7 +463,7 @@ class deviceclass {
             }
             // a learned indicator that is set by now goes in at once
             S.learned = rp_.artificial_viscosity && ind_ ? 1 : 0;
-            rc = stage_.init(ctx_, std::vector<StageScn>{S}, rp_.fused == 1);
+            rc = stage_.init(ctx_, std::vector<StageScn>{S});
             if (rc) return rc;
             stage_ready = true;
             stage_.mlp = S.learned ? ind_ : nullptr;

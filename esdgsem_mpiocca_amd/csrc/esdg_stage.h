@@ -160,8 +160,7 @@ struct StageSchedule {
 // Host side: device copies of the scenario table and the task list, plus the per-step sequence.
 class StageBatch {
   public:
-    // any_D: without it a degree's D must be the one that earlier batches of the process brought
-    int init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D = false);
+    int init(esdg_ctx* ctx, const std::vector<StageScn>& scns);
     int set_schedule(esdg_ctx* ctx, const StageSchedule& sc);
     // a batch of one scenario: its face records anew, after something has written the arrays they are made from
     int refresh_faces(esdg_ctx* ctx);

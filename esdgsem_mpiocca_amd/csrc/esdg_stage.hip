@@ -16,9 +16,6 @@
 #include "esdg_stage.h"
 
 #include <algorithm>
-#include <cstring>
-#include <map>
-#include <mutex>
 
 namespace esdg {
 
@@ -979,26 +976,6 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
     }
 }
 
-// Each degree has one D per device: a later batch must bring the same.
-static int check_degree_operators(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
-    static std::mutex mtx;
-    static std::map<int, std::map<int, std::vector<double>>> loaded;   // device -> ngl -> D
-    std::lock_guard<std::mutex> lock(mtx);
-    for (const StageScn& S : scns) {
-        const int n2 = S.ngl * S.ngl;
-        std::vector<double> D(n2);
-        int rc = esdg_memcpy(ctx, D.data(), S.D, n2 * sizeof(double), ESDG_D2H);
-        if (rc) return rc;
-        auto& slot = loaded[ctx->device][S.ngl];
-        if (slot.empty()) {
-            slot = D;
-        } else if (std::memcmp(slot.data(), D.data(), n2 * sizeof(double)) != 0) {
-            return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage: D differs from the one loaded for this degree");
-        }
-    }
-    return ESDG_OK;
-}
-
 // One record per element (StageScn::geo) of a mesh whose metrics are the same, bit for bit, at all nodes
 // of each element: {Yeta, Xeta, Yxi, Xxi, 1/J, Bx, By, 1 if Bx and By are the same at all nodes}.  *bad is
 // set where an element's metrics vary: the mesh then has no records.  One wave per element.
@@ -1079,15 +1056,14 @@ int StageBatch::refresh_faces(esdg_ctx* ctx) {
     return S.fgeo ? face_records(ctx, S, const_cast<double*>(S.fgeo), const_cast<int4*>(S.srec)) : ESDG_OK;
 }
 
-int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns, bool any_D) {
+int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
     host = scns;
     if (scns.empty()) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one scenario");
     for (const StageScn& S : scns) {
         if (S.ngl < 3 || S.ngl > 8) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage supports 2 <= N <= 7");
         if (S.Nelem <= 0) return set_error(ctx, ESDG_ERR_ARG, "the single-kernel stage needs at least one element");
     }
-    int rc = any_D ? ESDG_OK : check_degree_operators(ctx, scns);
-    if (rc) return rc;
+    int rc = ESDG_OK;
     // element and face records, once per distinct mesh and bottom (a mesh with varying metrics has
     // none), and side records, once per distinct connectivity and face records
     auto same_mesh = [](const StageScn& A, const StageScn& B) {

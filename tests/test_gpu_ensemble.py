@@ -144,3 +144,37 @@ def test_autotune_keeps_state(dev, mem, ensemble_default):
     for i in range(len(mem)):
         assert res[i][1:] == ensemble_default[i][1:], i
         assert np.array_equal(res[i][0], ensemble_default[i][0]), i
+
+
+def test_each_scenario_brings_its_own_D(dev):
+    """The single-kernel stage reads the flux-differencing operator of the scenario at hand: scenarios of one degree
+    whose D differ, next to each other and after one another in a process, equal the reference sequence's runs."""
+    cases = [Case.dam_break(N=4, nel=6, noise=1e-3, seed=2) for _ in range(2)]
+    cases[1].arrays["D"] = cases[1]["D"] * (1.0 + 2.0 ** -10)
+    rp = RunParams(num_flux=3, CFL=0.2)
+
+    def alone(case, fused):
+        ctx = dev.Context(dev.make_params(case, rp))
+        try:
+            s = dev.Solver(ctx, case, rp, fused=fused)
+            n, t = s.run(5)
+            q = s.get_q()
+            s.close()
+        finally:
+            ctx.close()
+        return n, t, q
+    ref = [alone(c, 0) for c in cases]
+    assert not np.array_equal(ref[0][2], ref[1][2])
+    for fused in (1, 2):
+        for c, r in zip(cases, ref):
+            got = alone(c, fused)
+            assert got[:2] == r[:2] and np.array_equal(got[2], r[2]), fused
+    ctx = dev.Context(dev.make_params(cases[0], rp))
+    try:
+        ens = dev.Ensemble(ctx, [(c, rp, None) for c in cases])
+        ens.run(5)
+        for i, r in enumerate(ref):
+            assert ens.status(i)[:2] == (r[1], r[0]) and np.array_equal(ens.get_q(i), r[2]), i
+        ens.close()
+    finally:
+        ctx.close()
