@@ -320,6 +320,8 @@ int esdg_ensemble_autotune(esdg_ensemble* E, int trial_steps, esdg_ensemble_sche
                     s.order = order; s.blocks_per_cu = bpc; s.per_degree = pd; s.xcd = xcd; s.graph = keep.graph;
                     cand.push_back(s);
                 }
+    // (a batch's first steps run without a graph: the trials' do not, so that none of them is captured while it is timed)
+    E->batch.issued = std::max(E->batch.issued, StageBatch::EAGER_STEPS);
     auto trial = [&](const StageSchedule& s) {
         rc = E->batch.set_schedule(ctx, s);
         if (!rc) rc = E->batch.run(ctx, E->A, E->C, E->stages, 2, E->src);   // warm-up, captures the graph

@@ -171,7 +171,10 @@ class StageBatch {
     // stage of the next step that the marks are for
     int prime(esdg_ctx* ctx, int src, int stage = 0);
     bool primed = false;
-    int issued = 0;     // steps that run() has been asked for (as far as it matters)
+    // steps that run() has been asked for (as far as it matters).  A captured pair of steps takes about 100 us to
+    // capture and instantiate: a batch's first EAGER_STEPS, unless asked for at once, are launched one by one.
+    int issued = 0;
+    static constexpr int EAGER_STEPS = 8;
     // one time step: dt kernel, then the RK stages [each after its viscous terms]; src flips once per
     // stage
     int step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src);

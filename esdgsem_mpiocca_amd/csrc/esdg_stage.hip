@@ -1548,11 +1548,9 @@ int StageBatch::run(esdg_ctx* ctx, const double* A, const double* C, int stages,
         if (rc) return rc;
         marks_used += steps;
     }
-    // A captured pair of steps takes about 100 us to capture and instantiate: the first few steps of a batch
-    // are launched one by one.
     const int before = issued;
     issued = (int)std::min<int64_t>((int64_t)issued + steps, 1 << 20);
-    if (sched.graph && graph_ok && !ctx->profile && steps >= 2 && (exec[src] || steps >= 8 || before >= 8)) {
+    if (sched.graph && graph_ok && !ctx->profile && steps >= 2 && (exec[src] || std::max(steps, before) >= EAGER_STEPS)) {
         // two steps flip the buffers an even number of times, so the graph that starts from buffer
         // `src` ends there and can be replayed
         if (!exec[src]) {

@@ -5,6 +5,10 @@ solver (single-kernel schedule, itself bitwise equal to the fused and reference 
 within 1e-12 of the oracle; the task ordering, launch shape, graph replay and autotuning must not
 change a bit.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -178,3 +182,35 @@ def test_each_scenario_brings_its_own_D(dev):
         ens.close()
     finally:
         ctx.close()
+
+
+COUNT_GRAPHS = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)     # before the library: its calls bind here first
+import esdgsem_mpiocca_amd as E
+dev = E.device()
+dev.lib()
+hip = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+real = ctypes.cast(ctypes.CDLL(hip).hipGraphInstantiate, ctypes.c_void_p)
+ctypes.c_void_p.in_dll(shim, "real").value = real.value
+case, rp = E.Case.gaussian_bump(N=4, nel=4), E.RunParams(num_flux=0)
+ctx = dev.Context(dev.make_params(case, rp))
+ens = dev.Ensemble(ctx, [(case, rp, None)] * 2)
+ens.autotune(trial_steps=2)
+ens.close()
+ctx.close()
+print("graphs", ctypes.c_int.in_dll(shim, "count").value)
+"""
+
+
+def test_autotune_trials_replay_graphs(tmp_path):
+    """Every trial of the autotuner captures its steps in its warm-up, the first ones of a new ensemble too, so that
+    what is timed is what runs afterwards: one graph for each of the 38 schedules."""
+    src, lib = tmp_path / "count.c", tmp_path / "libcount.so"
+    src.write_text("int count = 0;\nvoid* real = 0;\n"
+                   "int hipGraphInstantiate(void** e, void* g, void** n, char* l, unsigned long k) {\n"
+                   "    ++count;\n    return ((int (*)(void**, void*, void**, char*, unsigned long))real)(e, g, n, l, k);\n}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    r = subprocess.run([sys.executable, "-c", COUNT_GRAPHS, str(lib)], capture_output=True, text=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0 and "graphs 38" in r.stdout, r.stdout + r.stderr
