@@ -290,3 +290,20 @@ def test_ended_scenario_stays(dev, mem):
         ctx.close()
     case, rp, q = mem[5]
     assert np.array_equal(end, alone(dev, case, rp, q, STEPS)[0])
+
+
+def test_per_degree_cartesian_ensemble(dev):
+    """Viscous scenarios on Cartesian meshes only, launched degree by degree: element records in launches of one degree,
+    on either side of the size up to which a block has five waves."""
+    mem = []
+    for N, nel, s in ((4, 40, 1), (4, 70, 2), (7, 30, 3), (7, 40, 4), (5, 9, 5)):
+        case = Case.gaussian_bump(N=N, nel=nel)
+        q = case["q"].reshape(case.Nelem, 3, -1).copy()
+        q[:, 0] *= 1.0 + 1e-3 * np.random.default_rng(s).uniform(-1.0, 1.0, q[:, 0].shape)
+        mem.append((case, av(num_flux=0, CFL=0.2, DFL=0.05, sigma_min=-9.0, sigma_max=-5.0), q.ravel()))
+    want = [alone(dev, case, rp, q, 4, fused=0, plot=True) for case, rp, q in mem]
+    assert all((w[3] > 0).any() for w in want)
+    for schedule in (dict(order=1, per_degree=1), dict(order=0, per_degree=1, xcd=1), dict(order=0, per_degree=0)):
+        res, _ = run_ensemble(dev, mem, 4, schedule=schedule)
+        for (w, n, t, _), got in zip(want, res):
+            assert (n, t) == (got[2], got[1]) and np.array_equal(got[0], w)

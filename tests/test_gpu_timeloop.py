@@ -751,3 +751,39 @@ def test_steps_after_the_end_write_nothing(dev, fused):
             ctx.close()
     assert outs[1][0] == 1e-9 and np.abs(outs[1][1] - outs[1][2]).max() < 1e-6
     assert us[1] < 0.25 * us[0], us
+
+
+@pytest.mark.parametrize("av", [0, 1])
+@pytest.mark.parametrize("mesh", ["slopes", "flat"])
+@pytest.mark.parametrize("N,nel", [(2, 103), (2, 104), (3, 6), (4, 78), (4, 79), (5, 7), (6, 6), (7, 45), (7, 46)])
+def test_element_records_around_one_round(dev, N, nel, mesh, av):
+    """Cartesian meshes, whose metrics come from element records (the slopes too where the bottom is flat), on either
+    side of the size up to which a block has five waves, with and without viscosity: both fused schedules' state, register
+    and viscosity equal the reference sequence's, bit for bit."""
+    if mesh == "slopes":
+        case, kw = Case.gaussian_bump(N=N, nel=nel), dict(num_flux=0)
+    else:
+        case, kw = Case.ocean_uplift(N=N, nel=nel), dict(num_flux=3, bc_kind=2, h_zero=4000.0)
+    q = case["q"].reshape(case.Nelem, 3, -1).copy()
+    rng = np.random.default_rng(N)
+    rough = rng.uniform(size=(case.Nelem, 1)) < 0.3       # the others stay smooth
+    q[:, 0] *= 1.0 + 1e-3 * rough * rng.uniform(-1.0, 1.0, q[:, 0].shape)
+    case = case.with_state(q)
+    rp = RunParams(artificial_viscosity=av, eps0=0.005, sigma_min=-9.0, sigma_max=-5.0, DFL=0.05, CFL=0.2, **kw)
+    outs = []
+    for fused in (0, 1, 2):
+        ctx = dev.Context(dev.make_params(case, rp))
+        try:
+            s = dev.Solver(ctx, case, rp, fused=fused)
+            n, t = s.run(3)
+            visc = s.view("ViscPara", case.Nelem).download()
+            outs.append((n, t, s.get_q(), s.view("gRK", q.size).download(), visc))
+            s.close()
+        finally:
+            ctx.close()
+    ref = outs[0]
+    assert ref[0] == 3 and np.isfinite(ref[2]).all()
+    assert not av or (ref[4] > 0).any() and (ref[4] == 0).any()
+    for o in outs[1:]:
+        assert o[:2] == ref[:2] and np.array_equal(o[2], ref[2]) and np.array_equal(o[3], ref[3])
+    assert np.array_equal(outs[1][4], outs[2][4])
