@@ -419,17 +419,20 @@ __global__ void __launch_bounds__(256) k_train_fwd_bwd(int n, const float* __res
             sx[f][s] = srow[s] >= 0 ? rbf(feat[(int64_t)srow[s] * NIN + f]) : 0.0f;
         }
         __syncthreads();
-        // thread (j, k): hidden unit j of samples 4 k .. 4 k + 3; every sum runs in index order
+        // thread (j, k): hidden unit j of samples 4 k .. 4 k + 3; every sum runs in index order.  A place without a
+        // sample holds zeros throughout, whatever the parameters (an infinite one times its zeros would be NaN).
+        bool ok[4];
+        for (int c = 0; c < 4; ++c) ok[c] = srow[4 * k + c] >= 0;
         floatx4 z1 = {0.f, 0.f, 0.f, 0.f};
         for (int i = 0; i < NIN; ++i) z1 += four(&sx[i][4 * k]) * sW[OFF_W1 + i * NH + j];
         z1 += sW[OFF_B1 + j];
-        for (int c = 0; c < 4; ++c) sa1[j][4 * k + c] = rbf(fmaxf(z1[c], 0.0f));
+        for (int c = 0; c < 4; ++c) sa1[j][4 * k + c] = ok[c] ? rbf(fmaxf(z1[c], 0.0f)) : 0.0f;
         __syncthreads();
         floatx4 z2 = {0.f, 0.f, 0.f, 0.f};
         for (int i = 0; i < NH; ++i) z2 += four(&sa1[i][4 * k]) * sW[OFF_W2 + i * NH + j];
         z2 += sW[OFF_B2 + j];
         for (int c = 0; c < 4; ++c) {
-            const float a2 = rbf(fmaxf(z2[c], 0.0f));
+            const float a2 = ok[c] ? rbf(fmaxf(z2[c], 0.0f)) : 0.0f;
             sa2[j][4 * k + c] = a2;
             sdz2[j][4 * k + c] = a2 * sW[OFF_W3 + j];
         }
@@ -448,11 +451,11 @@ __global__ void __launch_bounds__(256) k_train_fwd_bwd(int n, const float* __res
             sloss[t] = ok ? pos_weight * y * sp_neg + (1.0f - y) * sp_pos : 0.0f;
         }
         __syncthreads();
-        for (int c = 0; c < 4; ++c) sdz2[j][4 * k + c] = (z2[c] > 0.0f) ? sW[OFF_W3 + j] * sdz3[4 * k + c] : 0.0f;
+        for (int c = 0; c < 4; ++c) sdz2[j][4 * k + c] = (ok[c] && z2[c] > 0.0f) ? sW[OFF_W3 + j] * sdz3[4 * k + c] : 0.0f;
         __syncthreads();
         floatx4 da = {0.f, 0.f, 0.f, 0.f};
         for (int i = 0; i < NH; ++i) da += four(&sdz2[i][4 * k]) * sW2T[i][j];
-        for (int c = 0; c < 4; ++c) sdz1[j][4 * k + c] = (z1[c] > 0.0f) ? da[c] : 0.0f;
+        for (int c = 0; c < 4; ++c) sdz1[j][4 * k + c] = (ok[c] && z1[c] > 0.0f) ? da[c] : 0.0f;
         __syncthreads();
         for (int s = 0; s < TS; s += 4) {
             const floatx4 d1 = four(&sdz1[j][s]), d2 = four(&sdz2[j][s]);

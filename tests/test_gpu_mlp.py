@@ -249,3 +249,31 @@ def test_learned_indicator_element_tiles(dev, nel):
             ctx.close()
     assert outs[0][:2] == outs[1][:2]
     assert np.array_equal(outs[0][2], outs[1][2])
+
+
+@pytest.mark.parametrize("where", ["b1", "b2", "w3", "W2"])
+def test_loss_gradient_infinite_parameter(dev, state, where):
+    """A batch of one sample and one of 32 copies of it have the same mean loss and gradient, also where a parameter
+    has overflowed: the 31 places of a block that the first leaves empty add nothing, not 0 times infinity."""
+    case, rp, _ = state
+    w = np.abs(random_params(23)) * 0.1
+    at = {"b1": M.OFF_B1 + 3, "b2": M.OFF_B2 + 3, "w3": M.OFF_W3 + 3, "W2": M.OFF_W2 + 3}[where]
+    w[at] = np.inf
+    x = np.random.default_rng(24).uniform(0.1, 1.0, (1, 72)).astype(np.float32)
+    got = []
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        net = dev.MLP(ctx, params=w)
+        for n in (32, 1):
+            dX, dy = ctx.array(np.repeat(x, n, 0)), ctx.array(np.zeros(n, np.float32))
+            dg, dl = ctx.empty(M.NPARAM, np.float32), ctx.empty(1, np.float32)
+            net.loss_grad(n, dX, dy, None, 1.0, dg, dl)
+            got.append(np.append(dg.download(), dl.download()))
+        net.close()
+    finally:
+        ctx.close()
+    full, one = got
+    assert not np.isfinite(full).all() and np.isfinite(full).any()
+    assert np.array_equal(np.isnan(full), np.isnan(one)) and np.array_equal(np.isinf(full), np.isinf(one))
+    ok = np.isfinite(full)
+    assert np.allclose(one[ok], full[ok], rtol=1e-5, atol=1e-30)
