@@ -74,7 +74,7 @@ class deviceclass {
         if (element_stage()) {
             // the stage kernel: second state buffer (ping-pong), lambda_max cell
             A(&o_q2, nodes * 3); A(reinterpret_cast<double**>(&o_lmax), 2);
-            A(&o_rec, record_bytes(Nelem, Nfaces) / sizeof(double));
+            A(&o_rec, batch_bytes(Nelem, Nfaces, rp.artificial_viscosity != 0) / sizeof(double));
             if (rp.artificial_viscosity) {
                 // the stage's gradient side traces, marks (one array per state buffer) and viscosity
                 // maximum (the viscous volume term goes to qGradientX, the viscous face fluxes to

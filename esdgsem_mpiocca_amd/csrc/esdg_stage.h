@@ -71,10 +71,11 @@ struct StageScn {
     const int4* srec;
     // one record per element and per face of a mesh with element-wise constant metrics (else null)
     const double *geo, *fgeo;
-    void* rec;          // record_bytes of zeroed memory for them, or null: StageBatch::init allocates it
+    void* rec;          // batch_bytes of zeroed memory for a batch of this scenario alone, or null: StageBatch::init
+                        // allocates it
 };
 
-// bytes of a mesh's records (StageScn::rec)
+// bytes of a mesh's records
 inline size_t record_bytes(int Nelem, int Nfaces) { return 64 + ((size_t)Nelem * 2 + Nfaces) * 64; }
 
 struct StageTask {
@@ -146,6 +147,18 @@ struct MarkLists {
     int ngl[MARK_LISTS], first[MARK_LISTS], blocks[MARK_LISTS], cap[MARK_LISTS];
 };
 
+// bytes of a batch's marks, counts and marked-element lists, of `slots` elements in all
+inline size_t mark_bytes(size_t slots) {
+    return 128 + 8 * IND_SLOTS * sizeof(unsigned long long) + 2 * MARK_LISTS * MARK_SLOTS * MARK_STRIDE * sizeof(int) +
+           slots * sizeof(int2);
+}
+// bytes of what a batch of one scenario keeps beside the scenario's arrays (StageScn::rec): its records, its entry of the
+// scenario table, its marks
+inline size_t batch_bytes(int Nelem, int Nfaces, bool av) {
+    return record_bytes(Nelem, Nfaces) + (sizeof(StageScn) + 63) / 64 * 64 +
+           (av ? mark_bytes((size_t)mark_capacity(Nelem) * MARK_SLOTS) : 0);
+}
+
 // How the tasks of a stage are ordered and launched (the autotuner's search space).
 struct StageSchedule {
     int order = 0;          // 0 scenario by scenario; 1 tiles of geometry-sharing scenarios
@@ -206,7 +219,6 @@ class StageBatch {
     bool has_av = false;
     StageTask *d_sens = nullptr, *d_ind = nullptr;
     int nsens = 0, nind = 0;
-    char* d_av = nullptr;                          // the allocation that holds the marks, lists and counts
     int2* d_mlist = nullptr;                       // the marked-element lists, one after another
     int* d_mcount = nullptr;                       // MARK_LISTS x 2 x MARK_SLOTS lengths, MARK_STRIDE apart
     int mcap[MARK_LISTS] = {0};                    // elements that a part of each list has room for
@@ -231,7 +243,7 @@ class StageBatch {
     void drop_graphs();
 
   private:
-    std::vector<void*> rec_bufs;    // side, element and face records, per distinct mesh
+    std::vector<void*> rec_bufs;    // allocations: the records of each distinct mesh; table, marks, lists and counts
     bool graph_ok = true;           // no capture has been refused
     // two steps from buffer `start` into exec[start], without running them.  A capture that the runtime refuses is no
     // error: exec[start] stays null and this batch's steps are launched one by one.

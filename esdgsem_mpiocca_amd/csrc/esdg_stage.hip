@@ -1116,24 +1116,26 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
     if (rc) return rc;
     has_av = false;
     for (const StageScn& S : scns) has_av = has_av || S.av;
-    rc = esdg_malloc(ctx, (void**)&d_scn, host.size() * sizeof(StageScn));
-    if (!rc) rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
+    // the scenario table; marks, list lengths, counts, and the lists (zero-filled), which hold every element of their
+    // scenarios at most once a stage and whose total size does not depend on which are learned
+    size_t all = 0;
+    for (const StageScn& S : host)
+        if (S.av) all += (size_t)mark_capacity(S.Nelem) * MARK_SLOTS;
+    const size_t table = (host.size() * sizeof(StageScn) + 63) / 64 * 64;
+    char* own = host.size() == 1 ? (char*)host[0].rec : nullptr;
+    char* buf = own ? own + record_bytes(host[0].Nelem, host[0].Nfaces) : (char*)buffer(table + (has_av ? mark_bytes(all) : 0));
+    if (rc) return rc;
+    d_scn = (StageScn*)buf;
+    rc = esdg_memcpy(ctx, d_scn, host.data(), host.size() * sizeof(StageScn), ESDG_H2D);
     if (!rc && has_av) {
-        // one allocation (zero-filled): marks, list lengths, counts, and the lists, which hold every element of
-        // their scenarios at most once a stage; their total size does not depend on which are learned
-        size_t all = 0;
-        for (const StageScn& S : host)
-            if (S.av) all += (size_t)mark_capacity(S.Nelem) * MARK_SLOTS;
         const size_t counts = 8 * IND_SLOTS * sizeof(unsigned long long);
         const size_t lengths = 2 * MARK_LISTS * MARK_SLOTS * MARK_STRIDE * sizeof(int);
-        rc = esdg_malloc(ctx, (void**)&d_av, 128 + counts + lengths + all * sizeof(int2));
-        if (!rc) {
-            d_mark = (int*)d_av;
-            d_icount = (unsigned long long*)(d_av + 128);
-            d_mcount = (int*)(d_av + 128 + counts);
-            d_mlist = (int2*)(d_av + 128 + counts + lengths);
-            rc = build_av_tasks(ctx);
-        }
+        buf += table;
+        d_mark = (int*)buf;
+        d_icount = (unsigned long long*)(buf + 128);
+        d_mcount = (int*)(buf + 128 + counts);
+        d_mlist = (int2*)(buf + 128 + counts + lengths);
+        rc = build_av_tasks(ctx);
     }
     if (!rc) rc = set_schedule(ctx, StageSchedule{});
     return rc;
@@ -1142,14 +1144,15 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
 // Element tiles of the AV scenarios for the sensor (RowBlock tiles) and the learned indicator
 // (32-element tiles), and the layout of the marked-element lists.
 int StageBatch::build_av_tasks(esdg_ctx* ctx) {
-    std::vector<StageTask> sens, ind;
+    std::vector<StageTask> sens, ind;      // (a single scenario's follow from their index)
     for (int& c : mcap) c = 0;
     auto list_of = [](const StageScn& S) { return S.learned ? MARK_LISTS - 1 : S.ngl - 3; };
     for (int s = 0; s < (int)host.size(); ++s) {
         const StageScn& S = host[s];
         if (!S.av) continue;
         const int ngl = S.ngl;
-        if (S.learned)
+        if (host.size() == 1) {
+        } else if (S.learned)
             for (int e0 = 0; e0 < S.Nelem; e0 += 32) ind.push_back(StageTask{s, e0, ngl, 0});
         else
             for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
@@ -1170,13 +1173,18 @@ int StageBatch::build_av_tasks(esdg_ctx* ctx) {
         if (d) esdg_free(ctx, d);
         d = nullptr;
         n = (int)v.size();
-        if (v.empty() || host.size() == 1) return ESDG_OK;   // (a single scenario's follow from their index)
+        if (v.empty()) return ESDG_OK;
         int rc = esdg_malloc(ctx, (void**)&d, v.size() * sizeof(StageTask));
         if (!rc) rc = esdg_memcpy(ctx, d, v.data(), v.size() * sizeof(StageTask), ESDG_H2D);
         return rc;
     };
     int rc = put(sens, d_sens, nsens);
     if (!rc) rc = put(ind, d_ind, nind);
+    if (host.size() == 1) {
+        const StageScn& S = host[0];
+        const int per = S.learned ? 32 : 256 / S.ngl;
+        (S.learned ? nind : nsens) = (S.Nelem + per - 1) / per;
+    }
     return rc;
 }
 
@@ -1298,10 +1306,11 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     for (int s = 0; s < ns; ++s) scn[s] = s;
     if (sc.order == 2 || sc.per_degree)
         std::stable_sort(scn.begin(), scn.end(), [&](int a, int b) { return host[a].ngl > host[b].ngl; });
-    std::vector<StageTask> tasks;
+    std::vector<StageTask> tasks;      // (those of a single scenario follow from their index)
     auto tiles = [&](int s) { const int epw = 64 / host[s].ngl; return (host[s].Nelem + epw - 1) / epw; };
     auto task = [&](int s, int t) { return StageTask{s, t * (64 / host[s].ngl), host[s].ngl, 0}; };
-    if (sc.order == 1) {
+    if (ns == 1) {
+    } else if (sc.order == 1) {
         // groups of scenarios on the same geometry, in order of first appearance; tile-major inside
         std::vector<int> done(ns, 0);
         for (int a = 0; a < ns; ++a) {
@@ -1326,7 +1335,8 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     // with both modal-sensor and learned scenarios: the other scenarios' tasks first, then the
     // learned ones', each group in the schedule's order and launched on its own stream
     split = has_av && nsens > 0 && nind > 0;
-    int nother = (int)tasks.size();
+    const int ntasks = ns == 1 ? tiles(0) : (int)tasks.size();
+    int nother = ntasks;
     if (split) {
         std::stable_partition(tasks.begin(), tasks.end(), [&](const StageTask& t) { return !host[t.scn].learned; });
         nother = 0;
@@ -1338,8 +1348,8 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     auto add_range = [&](int beg, int n, int lo, int hi) {
         if (n <= 0) return;
         Range r{beg, n, lo, hi, n, 0, cur_learned, 1};
-        for (int i = beg; i < beg + n; ++i)
-            if (!host[tasks[i].scn].geo) { r.affine = 0; break; }
+        for (int i = beg; i < beg + (ns == 1 ? 1 : n); ++i)
+            if (!host[ns == 1 ? 0 : tasks[i].scn].geo) { r.affine = 0; break; }
         // chunks of sc.tile tasks; with xcd every XCD's part is chunked on its own
         const int nch = sc.xcd ? 8 * (((n + 7) / 8 + sc.tile - 1) / sc.tile) : (n + sc.tile - 1) / sc.tile;
         const int pgrid = sc.blocks_per_cu * ncu;
@@ -1353,7 +1363,9 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
         rg.push_back(r);
     };
     auto add_group = [&](int g0, int g1) {
-        if (sc.per_degree) {
+        if (ns == 1) {
+            add_range(g0, g1 - g0, host[0].ngl, host[0].ngl);
+        } else if (sc.per_degree) {
             int beg = g0;
             while (beg < g1) {
                 int end = beg;
@@ -1369,10 +1381,9 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
     };
     add_group(0, nother);
     cur_learned = 1;
-    add_group(nother, (int)tasks.size());
-    // (the tasks of a single scenario follow from their index)
+    add_group(nother, ntasks);
     if (ns > 1) {
-        if (d_task && (int)tasks.size() != ntask) {
+        if (d_task && ntasks != ntask) {
             esdg_free(ctx, d_task);
             d_task = nullptr;
         }
@@ -1381,7 +1392,7 @@ int StageBatch::set_schedule(esdg_ctx* ctx, const StageSchedule& sc) {
         if (!rc) rc = esdg_memcpy(ctx, d_task, tasks.data(), tasks.size() * sizeof(StageTask), ESDG_H2D);
         if (rc) return rc;
     }
-    ntask = (int)tasks.size();
+    ntask = ntasks;
     ranges = rg;
     sched = sc;
     drop_graphs();
@@ -1573,11 +1584,8 @@ void StageBatch::release(esdg_ctx* ctx) {
     drop_graphs();
     for (StageTask** p : {&d_task, &d_sens, &d_ind})
         if (*p) { esdg_free(ctx, *p); *p = nullptr; }
-    if (d_scn) esdg_free(ctx, d_scn);
     for (void* p : rec_bufs) esdg_free(ctx, p);
     rec_bufs.clear();
-    if (d_av) esdg_free(ctx, d_av);
-    d_av = nullptr;
     d_mlist = nullptr;
     d_mcount = nullptr;
     d_scn = nullptr;

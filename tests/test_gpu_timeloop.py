@@ -787,3 +787,20 @@ def test_element_records_around_one_round(dev, N, nel, mesh, av):
     for o in outs[1:]:
         assert o[:2] == ref[:2] and np.array_equal(o[2], ref[2]) and np.array_equal(o[3], ref[3])
     assert np.array_equal(outs[1][4], outs[2][4])
+
+
+@pytest.mark.parametrize("av", [0, 1])
+@pytest.mark.parametrize("fused,N", [(0, 4), (1, 4), (2, 4), (1, 8)])
+def test_first_run_allocates_nothing(dev, fused, N, av):
+    """All device memory of a solver is allocated with it: no run pays for an allocation, the first one included."""
+    case = Case.dam_break(N=N, nel=6, noise=1e-3, seed=2)
+    rp = RunParams(num_flux=3, artificial_viscosity=av, eps0=0.005, sigma_min=-4.5, sigma_max=-2.5, DFL=0.05)
+    ctx = dev.Context(dev.make_params(case, rp))
+    try:
+        s = dev.Solver(ctx, case, rp, fused=fused)
+        before = ctx.bytes_allocated()
+        assert s.run(3)[0] == 3 and s.run(12)[0] == 12
+        assert ctx.bytes_allocated() == before
+        s.close()
+    finally:
+        ctx.close()
