@@ -898,7 +898,7 @@ __global__ void __launch_bounds__(256) k_ens_sensor(const StageScn* __restrict__
 
 // One list's marked elements, ElemBlock<NGL>::EPB at a time, one thread per node; the elements of a
 // block may be of different scenarios, so every element brings its own operators and pointers.
-template <int NGL>
+template <int NGL, bool ONE>
 __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns, const int2* __restrict__ list, int cnt,
                                               int blk, int nblk, int src, double* sDh, double* sDs, double* sA,
                                               double* sB, double* sC, double* sE, double* sF, double* sEps) {
@@ -908,7 +908,7 @@ __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns,
     for (int g = blk * EB::EPB; g < cnt; g += nblk * EB::EPB) {
         const bool act = el < EB::EPB && g + el < cnt;
         const int2 me = list[act ? g + el : g];
-        const StageScn& S = scns[me.x];
+        const StageScn& S = scns[ONE ? 0 : me.x];
         if (el < EB::EPB) {
             sDh[threadIdx.x] = S.Dhat[n];
             sDs[threadIdx.x] = S.Dstrong[n];
@@ -923,8 +923,11 @@ __device__ __forceinline__ void ens_grad_body(const StageScn* __restrict__ scns,
 
 // The gradient pass over the lists of marked elements.  A list's blocks stride over it, so a front
 // that crosses one part of a mesh spreads over the chip (one block per 256-element tile worked
-// through the tile's marked elements in sequence, 248 us for each launch of ten scenarios).
-template <int LO, int HI>
+// through the tile's marked elements in sequence, 248 us for each launch of ten scenarios).  ONE: a batch of one
+// scenario, whose pointers are the same in all lanes, and of one degree, whose registers and LDS are all that is
+// held: 43 us where every element of 128 x 128, N = 7, has viscosity and 394 at 400 x 400, with the pointers per lane
+// and all degrees in one kernel 60 and 675.
+template <int LO, int HI, bool ONE>
 __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src) {
     __shared__ double sDh[256], sDs[256];
     __shared__ double sA[256], sB[256], sC[256], sE[256];
@@ -939,7 +942,7 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
 #define ESDG_CASE(n)                                                                          \
     case n:                                                                                   \
         if constexpr (n >= LO && n <= HI)                                                     \
-            ens_grad_body<n>(scns, list, cnt, blk / MARK_SLOTS, L.blocks[l] / MARK_SLOTS, src, sDh, sDs, sA, sB, sC, sE, \
+            ens_grad_body<n, ONE>(scns, list, cnt, blk / MARK_SLOTS, L.blocks[l] / MARK_SLOTS, src, sDh, sDs, sA, sB, sC, sE, \
                              sF, sEps);                                                       \
         break;
         ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7) ESDG_CASE(8)
@@ -951,6 +954,7 @@ __global__ void __launch_bounds__(256) k_ens_grad(const StageScn* __restrict__ s
 // The viscous face fluxes over the side nodes of the listed elements; each face node once, by the
 // face's left element if that is marked, else by its right one (the faces a marked element reads
 // are exactly those).
+template <bool ONE>
 __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ scns, MarkLists L, int l0, int l1, int src,
                                                    const int* __restrict__ markp, int stage) {
     int l = l0;
@@ -965,7 +969,7 @@ __global__ void __launch_bounds__(256) k_ens_vface(const StageScn* __restrict__ 
         const int li = (int)(it / (4 * ngl)), rem = (int)(it % (4 * ngl));
         const int side = rem / ngl, i = rem % ngl;
         const int2 me = list[li];
-        const StageScn& S = scns[me.x];
+        const StageScn& S = scns[ONE ? 0 : me.x];
         const int f = S.E2E[me.y * 4 + side] - 1;
         const int* E = S.EdgeData + 8 * (int64_t)f;
         const int iel = E[0], ier = E[1], isl = E[2], isr = E[3], rv = E[4], cpuL = E[5], cpuR = E[6];
@@ -1281,13 +1285,23 @@ int StageBatch::av_terms(esdg_ctx* ctx, int src, int stage, int l0, int l1, hipS
         });
         if (n == 0) return ESDG_OK;
         KernelScope ks(ctx, "ens_grad");
-        k_ens_grad<3, 8><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src);
+        if (host.size() == 1) {
+            switch (host[0].ngl) {
+#define ESDG_CASE(g) case g: k_ens_grad<g, g, true><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src); break;
+                ESDG_CASE(3) ESDG_CASE(4) ESDG_CASE(5) ESDG_CASE(6) ESDG_CASE(7)
+                default: k_ens_grad<8, 8, true><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src); break;
+#undef ESDG_CASE
+            }
+        } else {
+            k_ens_grad<3, 8, false><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src);
+        }
         int rc = launch_check(ctx, "ens_grad");
         if (rc) return rc;
     }
     const auto [L, n] = lay_out(512, [](int64_t e, int ngl) { return (e * 4 * ngl + 255) / 256; });
     KernelScope ks(ctx, "ens_viscous_face");
-    k_ens_vface<<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, d_mark, stage);
+    if (host.size() == 1) k_ens_vface<true><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, d_mark, stage);
+    else k_ens_vface<false><<<n, 256, 0, st>>>(d_scn, L, l0, l1, src, d_mark, stage);
     return launch_check(ctx, "ens_viscous_face");
 }
 
