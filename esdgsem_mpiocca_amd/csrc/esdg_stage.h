@@ -55,7 +55,7 @@ struct StageScn {
     int* active[2];
     int2* mlist;
     int* mcount;
-    int mcap;
+    int mcap, mbase;    // the scenarios of a list number their elements one after another: this one's from mbase on
     int id;             // this scenario's index in the batch
     int freeze;         // after a dt that was not positive and finite: 1 both state buffers stay as they are, 0
                         // the state takes q + 0 gRK
@@ -94,9 +94,11 @@ __device__ __forceinline__ void max_into(unsigned long long* cell, double m) {
 // element has viscosity the stage took 1057 us at 300 x 300, N = 4, and 223 at 128 x 128, N = 7, and takes 128 and 51 with
 // 64 lengths in cache lines of their own.  Four consecutive elements go together (a group of the gradient pass at
 // N = 7); any 256 consecutive ones are dealt out evenly, the higher bits keep a front that crosses the rows of a mesh
-// from meeting in few parts.
+// from meeting in few parts.  k counts over all scenarios of the list, so that many small meshes fill the parts evenly
+// too (numbered mesh by mesh, 512 of 4 x 4 elements met in four parts: 707 us per step instead of 213).
 constexpr int MARK_SLOTS = 64, MARK_STRIDE = 16;
-__host__ __device__ constexpr int mark_capacity(int Nelem) { return 4 * ((Nelem + 255) / 256); }
+__host__ __device__ constexpr int mark_capacity(int elements) { return 4 * ((elements + 255) / 256); }
+constexpr int mark_elements(int Nelem) { return (Nelem + 3) / 4 * 4; }     // a scenario's share of the numbers
 __host__ __device__ constexpr int mark_slot(int k) { return ((k >> 2) ^ (k >> 8) ^ (k >> 14) ^ (k >> 20)) & (MARK_SLOTS - 1); }
 constexpr bool deals_out(int first) {      // 256 elements from `first`: four to each part
     int n[MARK_SLOTS] = {};
@@ -114,7 +116,7 @@ __device__ __forceinline__ P mark_count(P mcount, int b, int slot) { return mcou
 // elements of every face with viscosity on either side.  The first to mark an element also lists it.
 __device__ __forceinline__ void mark_element(const StageScn& S, int k, int m, int b) {
     if (atomicExch(S.active[b] + k, m) != m) {
-        const int s = mark_slot(k);
+        const int s = mark_slot(S.mbase + k);
         S.mlist[s * S.mcap + atomicAdd(mark_count(S.mcount, b, s), 1)] = make_int2(S.id, k);
     }
 }
@@ -147,16 +149,17 @@ struct MarkLists {
     int ngl[MARK_LISTS], first[MARK_LISTS], blocks[MARK_LISTS], cap[MARK_LISTS];
 };
 
-// bytes of a batch's marks, counts and marked-element lists, of `slots` elements in all
-inline size_t mark_bytes(size_t slots) {
+// bytes of a batch's marks, counts and marked-element lists, whose scenarios have `elements` numbers in all (each list
+// is rounded up to 256)
+inline size_t mark_bytes(size_t elements) {
     return 128 + 8 * IND_SLOTS * sizeof(unsigned long long) + 2 * MARK_LISTS * MARK_SLOTS * MARK_STRIDE * sizeof(int) +
-           slots * sizeof(int2);
+           (elements + 256 * MARK_LISTS) * sizeof(int2);
 }
 // bytes of what a batch of one scenario keeps beside the scenario's arrays (StageScn::rec): its records, its entry of the
 // scenario table, its marks
 inline size_t batch_bytes(int Nelem, int Nfaces, bool av) {
     return record_bytes(Nelem, Nfaces) + (sizeof(StageScn) + 63) / 64 * 64 +
-           (av ? mark_bytes((size_t)mark_capacity(Nelem) * MARK_SLOTS) : 0);
+           (av ? mark_bytes(mark_elements(Nelem)) : 0);
 }
 
 // How the tasks of a stage are ordered and launched (the autotuner's search space).

@@ -571,7 +571,8 @@ __device__ __forceinline__ void stage_body(const StageScn& S, int e0, double* ld
     const int p = src ^ (stage & 1);     // the step's half of the clocks, maxima and marks
     // the marks of the stage's state have been used: the list that the next stage's marks go to is the
     // other one, and this one is empty when its turn comes
-    if (AV && S.av && e0 == 0 && wave == 0) *mark_count(S.mcount, src, lane) = 0;   // (a part per lane)
+    // (the list's first scenario does, a part per lane)
+    if (AV && S.av && S.mbase == 0 && e0 == 0 && wave == 0) *mark_count(S.mcount, src, lane) = 0;
     if (stage == 1 && e0 == 0 && lane == 0 && wave == 0) {
         // the first stage has read the step's maxima: they are empty when the next step's last stage adds
         // to them; and the next step's marks
@@ -1124,7 +1125,7 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
     // scenarios at most once a stage and whose total size does not depend on which are learned
     size_t all = 0;
     for (const StageScn& S : host)
-        if (S.av) all += (size_t)mark_capacity(S.Nelem) * MARK_SLOTS;
+        if (S.av) all += mark_elements(S.Nelem);
     const size_t table = (host.size() * sizeof(StageScn) + 63) / 64 * 64;
     char* own = host.size() == 1 ? (char*)host[0].rec : nullptr;
     char* buf = own ? own + record_bytes(host[0].Nelem, host[0].Nfaces) : (char*)buffer(table + (has_av ? mark_bytes(all) : 0));
@@ -1149,20 +1150,24 @@ int StageBatch::init(esdg_ctx* ctx, const std::vector<StageScn>& scns) {
 // (32-element tiles), and the layout of the marked-element lists.
 int StageBatch::build_av_tasks(esdg_ctx* ctx) {
     std::vector<StageTask> sens, ind;      // (a single scenario's follow from their index)
-    for (int& c : mcap) c = 0;
+    int elements[MARK_LISTS] = {0};
     auto list_of = [](const StageScn& S) { return S.learned ? MARK_LISTS - 1 : S.ngl - 3; };
     for (int s = 0; s < (int)host.size(); ++s) {
-        const StageScn& S = host[s];
+        StageScn& S = host[s];
         if (!S.av) continue;
+        S.mbase = elements[list_of(S)];
+        elements[list_of(S)] += mark_elements(S.Nelem);
         const int ngl = S.ngl;
         if (host.size() == 1) {
         } else if (S.learned)
             for (int e0 = 0; e0 < S.Nelem; e0 += 32) ind.push_back(StageTask{s, e0, ngl, 0});
         else
             for (int e0 = 0; e0 < S.Nelem; e0 += 256 / ngl) sens.push_back(StageTask{s, e0, ngl, 0});
-        mcap[list_of(S)] += mark_capacity(S.Nelem);
     }
-    for (int l = 0; l < MARK_LISTS; ++l) mfirst[l + 1] = mfirst[l] + (int64_t)mcap[l] * MARK_SLOTS;
+    for (int l = 0; l < MARK_LISTS; ++l) {
+        mcap[l] = mark_capacity(elements[l]);
+        mfirst[l + 1] = mfirst[l] + (int64_t)mcap[l] * MARK_SLOTS;
+    }
     for (int s = 0; s < (int)host.size(); ++s) {
         StageScn& S = host[s];
         S.id = s;

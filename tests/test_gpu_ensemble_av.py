@@ -307,3 +307,16 @@ def test_per_degree_cartesian_ensemble(dev):
         res, _ = run_ensemble(dev, mem, 4, schedule=schedule)
         for (w, n, t, _), got in zip(want, res):
             assert (n, t) == (got[2], got[1]) and np.array_equal(got[0], w)
+
+
+def test_many_small_scenarios_in_one_list(dev):
+    """40 meshes of 4 x 4 and 5 x 5 elements, every element with viscosity, numbered one after another in one list whose
+    parts they fill unevenly mesh by mesh; with a few scenarios of another list among them."""
+    kw = dict(sigma_min=-40.0, sigma_max=-2.5, eps0=1e-4, DFL=0.05)
+    kinds = [(Case.dam_break(N=N, nel=nel, noise=1e-3, seed=nel, ratio=2.0, angle=0.4), av(**kw))
+             for N, nel in ((4, 4), (4, 5), (2, 3))]
+    want = [alone(dev, case, rp, None, 3, fused=0) for case, rp in kinds]
+    pick = [(0, 1, 0, 2)[i % 4] if i < 20 else i % 2 for i in range(40)]
+    res, _ = run_ensemble(dev, [(*kinds[k], None) for k in pick], 3)
+    for k, (got, t, n) in zip(pick, res):
+        assert (n, t) == want[k][1:3] and np.array_equal(got, want[k][0])
