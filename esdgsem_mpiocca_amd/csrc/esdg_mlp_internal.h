@@ -15,7 +15,7 @@ int mlp_classify(esdg_ctx* ctx, const esdg_mlp* m, int Nelem, const double* q, c
 // in the same pass the modal sensor with zero viscosity where the class is smooth (from the modal
 // coefficients the features already formed).  Each viscous element marks itself and its face neighbours
 // for stage `stage` of the step; in stage 0 the viscosities enter each scenario's maximum.  A scenario
-// whose time has reached its end is skipped.  counters (may be null, 5 entries, accumulated):
+// whose time has reached its end is skipped.  counters (IND_SLOTS copies of 5 entries, 8 apart, accumulated):
 // [0] element-stages with viscosity, [1] sensor positives declared smooth (audit), [2] sensor positives
 // (audit), [3] element-stages not declared smooth, [4] element-stages classified.
 int mlp_ensemble_indicator(esdg_ctx* ctx, const esdg_mlp* m, const StageScn* scns, const StageTask* tasks, int ntask,

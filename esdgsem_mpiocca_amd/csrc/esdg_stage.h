@@ -191,8 +191,8 @@ class StageBatch {
     // capture and instantiate: a batch's first EAGER_STEPS, unless asked for at once, are launched one by one.
     int issued = 0;
     static constexpr int EAGER_STEPS = 8;
-    // one time step: dt kernel, then the RK stages [each after its viscous terms]; src flips once per
-    // stage
+    // one time step: the RK stages, the first of which forms dt [each after its viscous terms]; src flips
+    // once per stage
     int step(esdg_ctx* ctx, const double* A, const double* C, int stages, int& src);
     // `steps` steps: pairs of steps replayed from a captured graph (schedule.graph), the rest eager
     int run(esdg_ctx* ctx, const double* A, const double* C, int stages, int steps, int& src);

@@ -70,10 +70,10 @@ __device__ __forceinline__ void wave_sync() {
 // AFF: every element's metrics are the same at all of its nodes (a Cartesian mesh), and come from one
 // record per element instead of five doubles per node; the bottom slopes too where they are constant.
 // MW: the caller is the element wave of a block of five (k_stage_wide), the face fluxes come in mwFS.
-// What bounds it: on curved meshes the memory path (512 x 512, N = 7, with viscosity 2.71 GB in 610 us per
-// stage, 4.4 TB/s; an add of three large arrays reaches 5.65 here), on Cartesian meshes, whose records
-// leave 11 doubles per node, instruction issue (256 x 256, N = 7: 121 us per stage, 157 with metrics per
-// node), and on small ones one wave's chain of dependent steps.
+// What bounds it: on curved meshes the memory path (512 x 512, N = 7, with viscosity: 618 us per stage for 3.34 GB
+// moved, 5.4 TB/s, of which it cannot do without 2.71; an add of three large arrays reaches 5.65 here), on
+// Cartesian meshes, whose records leave 11 doubles per node, instruction issue (256 x 256, N = 7: 120 us per
+// stage, 157 with metrics per node), and on small ones one wave's chain of dependent steps.
 template <int NGL, bool AV, bool AFF, bool MW, class Faces, class Early, class Dt>
 __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, const Faces& faces, const Early& early,
                                            const Dt& step_dt, double g, double tol,
@@ -457,8 +457,8 @@ __device__ __forceinline__ void stage_core(int e, int r, bool act, double* P, co
         }
     }
     if constexpr (AV) {
-        // ShockCapturing.okl:63-217 on the new state (here 80 us at 512 x 512, N = 7; as a pass of its own
-        // over q 105), with the arithmetic of sensor_rows: lane r forms
+        // ShockCapturing.okl:63-217 on the new state (here 46 us at 512 x 512, N = 7, the stage 573 and without it
+        // 527; as a pass of its own 81), with the arithmetic of sensor_rows: lane r forms
         // column r of T = V (h + b) from row r of h + b, then the squares of row r of T V^T; up to four
         // lanes form the energy sums.  An element with viscosity marks what it reaches for the next stage,
         // and after the last stage its viscosity enters the next step's maximum.
@@ -770,8 +770,8 @@ __global__ void __launch_bounds__(64, 2) k_stage(const StageScn* __restrict__ sc
 
 // The same stage for short lists of tasks of one degree, where a stage takes as long as one wave's chain of
 // loads, sweeps and face fluxes: five waves per block, one for the elements and one for each of their
-// sides, whose fluxes are ready when the sweeps are.  16 x 16, N = 4: 11.6 us per stage with one wave per block,
-// 7.5 with five.
+// sides, whose fluxes are ready when the sweeps are.  16 x 16, N = 4: 12.2 us per stage with one wave per block,
+// 7.6 with five.
 template <int NGL, bool AV, bool AFF>
 __global__ void __launch_bounds__(320, 2) k_stage_wide(const StageScn* __restrict__ scns,
                                                        const StageTask* __restrict__ tasks, int n, int xcd, int src,
@@ -1425,10 +1425,10 @@ int StageBatch::lambda(esdg_ctx* ctx, int src) {
 }
 
 // k_stage_wide where its blocks of five waves are all resident at once: one per CU, two at ngl <= 5, whose waves
-// need fewer registers.  us per step there and with k_stage: 16 x 16, N = 4, 45 and 68, 48 x 48 50 and 70, 64 x 64
-// (342 tasks) 74 and 78; 16 x 16, N = 7, 62 and 86, 45 x 45 (254 tasks) 70 and 92.  Beyond it k_stage has more
-// waves at work: 56 x 56, N = 7 (392 tasks) 115 and 99, 64 x 64, N = 5 (410 tasks) 88 and 86, 80 x 80, N = 4 (534
-// tasks) 97 and 86.
+// need fewer registers.  us per step with it and with k_stage, runs of 40 steps on Cartesian meshes: 16 x 16, N = 4,
+// 38 and 61, 48 x 48 43 and 64, 64 x 64 (342 tasks) 67 and 72; 16 x 16, N = 7, 55 and 77, 45 x 45 (254 tasks) 63 and
+// 84.  Beyond it k_stage has more waves at work: 56 x 56, N = 7 (392 tasks) 110 and 91, 64 x 64, N = 5 (410 tasks) 82
+// and 79, 80 x 80, N = 4 (534 tasks) 89 and 79.
 static constexpr int wide_blocks_per_cu(int ngl) { return ngl <= 5 ? 2 : 1; }
 
 template <int LO, int HI, bool AV>

@@ -276,7 +276,9 @@ int esdg_solver_time(const esdg_solver* s, double* t);
 int esdg_solver_checkpoint(esdg_solver* s, const char* path);
 int esdg_solver_restart(esdg_solver* s, const char* path);
 int esdg_solver_last_dt(const esdg_solver* s, double* dt);
-/* Device pointer of a named solver buffer ("q","Qt","gRK","ViscPara","LambdaMax", ...). */
+/* Device pointer of a named solver buffer ("q","Qt","gRK","ViscPara","LambdaMax", ...).  With fused = 1 also
+ * "FStar" [Nfaces][3][ngl] and "Traces" [Nfaces][2][3][ngl]: at 2 <= N <= 7 filled from the first request on
+ * (after each esdg_solver_run). */
 int esdg_solver_buffer(esdg_solver* s, const char* name, void** dptr);
 int esdg_solver_destroy(esdg_solver* s);
 
